@@ -90,10 +90,8 @@ struct LiftWaves {
 // Accumulator tile (f-tile t): lane l holds Phi^T[16t + 4(l>>4) + i][row (l & 15)].
 //
 // FROM_BITS: Omega is not read from memory; each workgroup builds it in LDS from the packed Rademacher
-// table bits[D/64][3] (the reference's native boundary, kernels/fwht_cuda.cpp:29-32): wave w takes
-// columns j of block m in turn, column j of H d1 is (-1)^popcount(lane & j) d1_j in lane `lane`, then the
-// d2 / d3 sign flips and two wave64 butterflies (fwht_wave) give Omega[64m + lane][j] * 8 exactly, and
-// each lane writes its element into the A fragment that the staged copy would hold.
+// table bits[D/64][3] (the reference's native boundary, kernels/fwht_cuda.cpp:29-32), one 64-feature block
+// per wave at a time (build_omega_block).
 // Output staging tile (16 rows of 128 bytes per wave): chunk c (16 bytes) of row r sits at chunk
 // position c ^ ((r >> 1) & 7).  With bf16 output each lane stores 8 bytes (one half of a chunk) of its row,
 // and the halves of a chunk are swapped in rows with h(r) = (r ^ (r >> 1)) & 1 = 1.  8-byte stores are
@@ -117,6 +115,64 @@ __device__ __forceinline__ u32x4 stage_read(const unsigned char* stg, int r, int
   } else {
     return *reinterpret_cast<const u32x4*>(c);
   }
+}
+
+// Omega of block m (features 64m .. 64m + 63) as the A fragments lift_kernel stages, by one wave from the
+// packed sign table, on MFMA.  With G = H d2 (one wave64 butterfly), Omega_m^T / d1 has the entries
+//   sum_i d3_i G[i ^ j] (-1)^popcount(i & f)        (H diag(d2) H is the dyadic matrix G[i ^ j])
+// i.e. a 64 x 64 x 64 product of the signed, permuted G (integers up to 64) with the Sylvester signs: both
+// exact in bf16, the sums (integers up to 4096) exact in fp32.  32 MFMAs and 32 LDS reads per block.  (Two
+// butterflies per column, each six dependent cross-lane exchanges, took 45 us a workgroup of four waves at
+// D = 512 and 21 us of eight: the lift of 4084 fp32 rows 55.7 us against 11.4 with this, of 524,288 bf16
+// rows 136.8 against 118.1; the staged table takes 10.9 and 118.3.)  `g` is 64 floats of the wave's own; the fragments are written to `so` (the table's block).
+__device__ __forceinline__ void build_omega_block(const int64_t* __restrict__ bits, int m, float* g, bf16x8* so, int lane) {
+  const int64_t b1 = bits[3 * m + 0], b2 = bits[3 * m + 1], b3 = bits[3 * m + 2];
+  g[lane] = fwht_wave<64>(sign_of(b2, lane), lane);
+  wave_lds_sync();
+  const int q = lane >> 4, c = lane & 15;
+  // lane's depth indices of fragment kb: i = 32kb + 8q + s
+  float r[4][8];  // G[i ^ j] for rows j = 16 jt + c: r[jt ^ 2kb][s]
+#pragma unroll
+  for (int hi = 0; hi < 4; ++hi)
+#pragma unroll
+    for (int s = 0; s < 8; ++s) r[hi][s] = g[16 * (hi ^ (q >> 1)) + ((8 * (q & 1) + s) ^ c)];
+  u32x4 sg;  // (-1)^popcount(i & c) as bf16, the columns f = 16 ft + c up to the sign of bits 4, 5
+#pragma unroll
+  for (int s2 = 0; s2 < 4; ++s2) {
+    const unsigned lo = __builtin_popcount((8 * (q & 1) + 2 * s2) & c) & 1, hi = __builtin_popcount((8 * (q & 1) + 2 * s2 + 1) & c) & 1;
+    sg[s2] = 0x3F803F80u | (lo << 15) | (hi << 31);
+  }
+  bf16x8 hf[4][2];
+#pragma unroll
+  for (int ft = 0; ft < 4; ++ft)
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      const unsigned flip = (((ft & 1) & (q >> 1)) ^ ((ft >> 1) & kb)) ? 0x80008000u : 0u;
+      hf[ft][kb] = __builtin_bit_cast(bf16x8, (u32x4)(sg ^ flip));
+    }
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt) {
+    bf16x8 a[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        const float v = r[jt ^ (2 * kb)][s];
+        a[kb][s] = (__bf16)(((b3 >> (32 * kb + 8 * q + s)) & 1) ? -v : v);
+      }
+    f32x4 d1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d1[i] = 0.125f * sign_of(b1, 16 * jt + 4 * q + i);
+#pragma unroll
+    for (int ft = 0; ft < 4; ++ft) {
+      const f32x4 acc = PrecBF16::mma(PrecBF16::mma(zero4(), a[0], hf[ft][0]), a[1], hf[ft][1]) * d1;
+      // rows j = 16 jt + 4q + i of feature 16 ft + c: half of the 16 bytes of lane c + 16 ((j & 31) >> 3)
+      __bf16* dst = reinterpret_cast<__bf16*>(so + (ft * 2 + (jt >> 1)) * 64 + c + 16 * (2 * (jt & 1) + (q >> 1))) + 4 * (q & 1);
+      const float v[4] = {acc[0], acc[1], acc[2], acc[3]};
+      store4<__bf16>(dst, v);
+    }
+  }
+  wave_lds_sync();
 }
 
 template <typename InT, typename OutT, int D, bool FROM_BITS>
@@ -147,18 +203,9 @@ __global__ void __launch_bounds__((64 * LiftWaves<InT, OutT, D>::value)) lift_ke
 
   // Stage Omega as A fragments: lane l of fragment (t, kb) holds Omega[16t + (l&15)][32kb + 8(l>>4) .. +8].
   if constexpr (FROM_BITS) {
-    __bf16* so = reinterpret_cast<__bf16*>(s_omega);
-    for (int cj = wave; cj < D; cj += NW) {
-      const int m = cj >> 6, j = cj & 63;
-      const int64_t b1 = bits[3 * m + 0], b2 = bits[3 * m + 1], b3 = bits[3 * m + 2];
-      float v = (__builtin_popcount(lane & j) & 1) ? -sign_of(b1, j) : sign_of(b1, j);
-      v *= sign_of(b2, lane);
-      v = fwht_wave<64>(v, lane);
-      v *= sign_of(b3, lane);
-      v = fwht_wave<64>(v, lane);
-      const int f = 64 * m + lane;  // feature row of this lane's element
-      so[(((f >> 4) * 2 + (j >> 5)) * 64 + (f & 15) + 16 * ((j & 31) >> 3)) * 8 + (j & 7)] = (__bf16)(v * 0.125f);
-    }
+    // the staging tile of the wave is free until its first output rows: it holds the wave's G
+    float* g = reinterpret_cast<float*>(s_stage[wave]);
+    for (int m = wave; m < D / 64; m += NW) build_omega_block(bits, m, g, s_omega + m * 8 * 64, lane);
   } else {
     for (int idx = threadIdx.x; idx < NT * 2 * 64; idx += 64 * NW) {
       const int l = idx & 63, tk = idx >> 6, t = tk >> 1, kb = tk & 1;
@@ -302,6 +349,122 @@ __global__ void __launch_bounds__((64 * LiftWaves<InT, OutT, D>::value)) lift_ke
   }
 }
 
+// The lift of few rows: one workgroup per 16-row tile, its D / 64 waves each taking one 64-feature block
+// (lift_kernel's waves each take whole rows, so that a short call keeps a few of them busy for 32 feature
+// tiles in a row while the rest of the GPU idles).  Omega's block is the wave's own, built from the sign
+// table (FROM_BITS) or read as fragments, so only the rows' sums of squares cross the waves.  The wave's
+// 8 KB of Omega become its output staging tile once the last fragment is in registers.
+template <typename InT, typename OutT, int D, bool FROM_BITS>
+__global__ void __launch_bounds__(D) lift_rows16_kernel(const InT* __restrict__ x, int64_t rows, int64_t xs, int normalize,
+                                                        const __bf16* __restrict__ omega, const int64_t* __restrict__ bits,
+                                                        const float* __restrict__ phase, float inv_tau,
+                                                        OutT* __restrict__ out, int64_t os) {
+  constexpr int NW = D / 64;
+  constexpr int NSPLIT = XFrag<InT>::NSPLIT;
+  constexpr int TG = 128 / (16 * (int)sizeof(OutT));  // feature tiles per staged group: 128 bytes of a row
+  __shared__ __attribute__((aligned(16))) unsigned char s_buf[NW][FROM_BITS ? 8192 : 2048];
+  __shared__ float s_g[FROM_BITS ? NW : 1][64];
+  __shared__ float s_ss[NW][16];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row0 = (int64_t)blockIdx.x * 16;
+  const int64_t row = row0 + (lane & 15);
+  const bool valid = row < rows;
+  float xv[2][8];
+  {
+    const InT* src = x + (valid ? row : rows - 1) * xs + 8 * (lane >> 4);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      load8<InT>(src + 32 * kb, xv[kb]);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) xv[kb][s] = valid ? xv[kb][s] : 0.f;
+    }
+  }
+  f32x4 ph[4];
+  bf16x8 om[4][2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) ph[t] = *reinterpret_cast<const f32x4*>(phase + 64 * wave + 16 * t + 4 * (lane >> 4)) * 0.15915494309189535f;
+  if constexpr (FROM_BITS) {
+    bf16x8* so = reinterpret_cast<bf16x8*>(s_buf[wave]);
+    build_omega_block(bits, wave, s_g[wave], so, lane);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) om[t][kb] = so[(t * 2 + kb) * 64 + lane];
+    wave_lds_sync();
+  } else {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        om[t][kb] = *reinterpret_cast<const bf16x8*>(omega + (64 * wave + 16 * t + (lane & 15)) * 64 + 32 * kb + 8 * (lane >> 4));
+  }
+  if (normalize) {
+    float ss = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int s = 0; s < 8; ++s) ss += xv[kb][s] * xv[kb][s];
+    ss = sum_over_lane_groups(ss);
+    const float inv = 1.0f / fmaxf(sqrtf(ss), 1e-6f);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        const float y = xv[kb][s] * inv;
+        xv[kb][s] = (NSPLIT == 1) ? (float)(__bf16)y : y;  // F.normalize output keeps x's dtype
+      }
+  }
+  bf16x8 xb[2][NSPLIT];
+  split_frag<NSPLIT>(xv[0], xb[0]);
+  split_frag<NSPLIT>(xv[1], xb[1]);
+  const float ang_scale = inv_tau * 0.15915494309189535f;  // radians -> revolutions folded in
+  const float amp = sqrtf(2.0f / (float)D);
+  float c[4][4];
+  float ss = 0.f;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    f32x4 acc = zero4();
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int p = 0; p < NSPLIT; ++p) acc = PrecBF16::mma(acc, om[t][kb], xb[kb][p]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float cv = __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(acc[i] * ang_scale + ph[t][i]));
+      c[t][i] = cv;
+      ss += cv * cv;
+    }
+  }
+  ss = sum_over_lane_groups(ss);
+  if (lane < 16) s_ss[wave][lane] = ss;
+  __syncthreads();
+  ss = s_ss[0][lane & 15];
+#pragma unroll
+  for (int v = 1; v < NW; ++v) ss += s_ss[v][lane & 15];
+  const float scale = amp / (amp * sqrtf(ss) + 1e-8f);
+  unsigned char* stg = s_buf[wave];
+#pragma unroll
+  for (int gr = 0; gr < 4 / TG; ++gr) {
+#pragma unroll
+    for (int tp = 0; tp < TG; ++tp) {
+      const int t = TG * gr + tp;
+      const float v[4] = {c[t][0] * scale, c[t][1] * scale, c[t][2] * scale, c[t][3] * scale};
+      store4<OutT>(reinterpret_cast<OutT*>(stg + stage_off<OutT>(lane & 15, (int)sizeof(OutT) * (16 * tp + 4 * (lane >> 4)))), v);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int q = 64 * j + lane, r = q >> 3, pos = q & 7, ch = pos ^ ((r >> 1) & 7);
+      const u32x4 val = stage_read<OutT>(stg, r, pos);
+      const int64_t grow = row0 + r;
+      if (grow < rows)
+        *reinterpret_cast<u32x4*>(reinterpret_cast<unsigned char*>(out + grow * os + 64 * wave + 16 * TG * gr) + 16 * ch) = val;
+    }
+    wave_lds_sync();
+  }
+}
+
 // ------------------------------------------------------------------------------------------------
 // The same lift with the projection by in-register butterflies instead of the MFMA product (the design
 // of the reference's CUDA P3 kernel, kernels/in_register_fwht.cu:10-93 / .cuh, with the semantics of
@@ -376,6 +539,11 @@ static void launch_lift_butterfly(const void* x, int64_t rows, int64_t xs, int n
                      xs, normalize, bits, phase, inv_tau, (OutT*)out, os);
 }
 
+// Up to one 16-row tile per CU the lift takes lift_rows16_kernel, which fills the GPU with one round of
+// workgroups; past that lift_kernel, whose waves keep Omega over several tiles.  D = 512, us per call in a
+// graph, rows16 / persistent: 1021 rows 6.4 / 10.9 (fp32), 5.4 / 9.4 (bf16); 4084 rows 7.7 / 11.4, 6.0 / 9.7;
+// 8192 rows 12.0 / 12.0, 10.4 / 10.1; 16384 rows 19.2 / 13.8, 19.1 / 10.5.
+
 template <typename InT, typename OutT, int D>
 static void launch_lift(const void* x, int64_t rows, int64_t xs, int normalize, const void* omega, const int64_t* bits,
                         const float* phase, float inv_tau, void* out, int64_t os, hipStream_t st) {
@@ -387,6 +555,15 @@ static void launch_lift(const void* x, int64_t rows, int64_t xs, int normalize, 
   const int per_cu = (int)(CU_LDS_BYTES / lds) > 0 ? (int)(CU_LDS_BYTES / lds) : 1;
   const int cus = device_cus() > 0 ? device_cus() : 256;
   const int64_t cap = (int64_t)cus * per_cu;
+  if (ntiles <= cus) {
+    if (bits)
+      hipLaunchKernelGGL((lift_rows16_kernel<InT, OutT, D, true>), dim3((unsigned)ntiles), dim3(D), 0, st, (const InT*)x, rows,
+                         xs, normalize, nullptr, bits, phase, inv_tau, (OutT*)out, os);
+    else
+      hipLaunchKernelGGL((lift_rows16_kernel<InT, OutT, D, false>), dim3((unsigned)ntiles), dim3(D), 0, st, (const InT*)x, rows,
+                         xs, normalize, (const __bf16*)omega, nullptr, phase, inv_tau, (OutT*)out, os);
+    return;
+  }
   if (wgs > cap) wgs = cap;
   if (bits)
     hipLaunchKernelGGL((lift_kernel<InT, OutT, D, true>), dim3((unsigned)wgs), dim3(64 * NW), 0, st, (const InT*)x, rows, xs,

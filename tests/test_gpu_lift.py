@@ -181,6 +181,27 @@ def test_lift_bits_equals_table_lift(D, seed, dtype, normalize):
     assert rel_l2(a.float().cpu().numpy(), ol.lift(xr.numpy(), op)) < tol
 
 
+@pytest.mark.parametrize("D", [128, 256, 512])
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                             (torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("extra", [0, 1])
+def test_lift_at_the_one_tile_per_cu_line(D, dtype, out_dtype, extra):
+    """One 16-row tile per CU (a workgroup per tile, a wave per 64 features) and one row more (persistent
+    waves over whole rows): the sign-table and the table form agree bit for bit on either side, and match
+    the oracle on the first and last rows (1e-5: fp32 sums and the hardware cosine; 1e-2: bf16 outputs)."""
+    rows = 16 * torch.cuda.get_device_properties(0).multi_processor_count + extra
+    p, op = FastWalshHadamardProjection(64, D, 5), ol.make_projection(64, D, 5)
+    x = (torch.randn(rows, 64, generator=torch.Generator().manual_seed(D)) * 1.3).to(dtype)
+    xd = x.to(DEV)
+    a = ops.lift_bits(xd, p.device_bits(DEV), p.device_phase(DEV), p.tau_star_inv, out_dtype=out_dtype)
+    b = ops.lift(xd, p.device_omega(DEV), p.device_phase(DEV), p.tau_star_inv, out_dtype=out_dtype)
+    torch.cuda.synchronize()
+    assert a.shape == (rows, D) and a.dtype == out_dtype and torch.equal(a, b)
+    pick = torch.cat([torch.arange(40), torch.arange(rows - 40, rows)])
+    tol = 1e-5 if out_dtype == torch.float32 else 1e-2
+    assert rel_l2(a[pick.to(DEV)].float().cpu().numpy(), ol.lift(x[pick].float().numpy(), op)) < tol
+
+
 def test_reference_call_site_shim(proj, oproj):
     """The drop-in for the reference's extension module: kernel_deltanet_cuda.fwht_forward called with the
     reference's argument list (kernels/fwht.py:120) plus phase=self.b, no Omega."""
