@@ -21,46 +21,67 @@ constexpr int SRV_D = 512;   // lifted features
 constexpr int SRV_DK = 64;   // input features
 
 // ---- split ----------------------------------------------------------------------------------------
-// One workgroup: thread t counts the decode / prefill sequences of its contiguous range, an inclusive
-// Hillis-Steele scan over the 1024 counts gives each range its output offsets, and the ranges are then
-// written in sequence order.  The lists are first filled with skip entries (slot -1, no tokens), so
-// that a launch sized from host counts that differ from the device offsets reads no unwritten entry.
-// A sequence whose slot lies outside [0, num_slots) (a negative slot is the padding convention) keeps
-// its place in its list with slot -1 and no tokens: the decode and scan kernels skip it, its state is
-// not touched and its y rows are not written.
-__global__ void __launch_bounds__(1024) ragged_split_kernel(const int64_t* __restrict__ cu, const int32_t* __restrict__ slots,
+constexpr int PLAN_THREADS = 1024;
+
+// Exclusive prefix of v over the 1024 threads of a workgroup, and its total: shuffles inside the waves and
+// one exchange of the 16 wave sums (s_w), where ten rounds of shared-memory adds took twenty barriers.
+__device__ __forceinline__ int64_t plan_scan(int64_t v, int64_t* s_w, int64_t& total) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int64_t inc = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int64_t u = __shfl_up(inc, o);
+    if (lane >= o) inc += u;
+  }
+  __syncthreads();  // the previous scan's sums have been read
+  if (lane == 63) s_w[wv] = inc;
+  __syncthreads();
+  int64_t base = 0;
+  total = 0;
+#pragma unroll
+  for (int q = 0; q < PLAN_THREADS / 64; ++q) {
+    const int64_t w = s_w[q];
+    base += q < wv ? w : 0;
+    total += w;
+  }
+  return base + inc - v;
+}
+
+// One workgroup: thread t counts the decode / prefill sequences of its contiguous range (decodes in the low
+// half of a 64-bit count, prefills in the high half; n < 2^31), a scan gives each range its output offsets,
+// and the ranges are then written in sequence order.  The lists are first filled with skip entries (slot
+// -1, no tokens), so that a launch sized from host counts that differ from the device offsets reads no
+// unwritten entry.  A sequence whose slot lies outside [0, num_slots) (a negative slot is the padding
+// convention) keeps its place in its list with slot -1 and no tokens: the decode and scan kernels skip it,
+// its state is not touched and its y rows are not written.
+__global__ void __launch_bounds__(PLAN_THREADS) ragged_split_kernel(const int64_t* __restrict__ cu, const int32_t* __restrict__ slots,
                                                             int64_t n, int64_t num_slots, int64_t* __restrict__ dec_row,
                                                             int32_t* __restrict__ dec_slot, int64_t* __restrict__ pre_lo,
                                                             int64_t* __restrict__ pre_hi, int32_t* __restrict__ pre_slot) {
-  __shared__ int64_t s_d[1024], s_p[1024];
+  __shared__ int64_t s_w[PLAN_THREADS / 64];
   const int t = threadIdx.x;
-  for (int64_t i = t; i < n; i += 1024) {
-    dec_row[i] = 0;
-    dec_slot[i] = -1;
-    pre_lo[i] = 0;
-    pre_hi[i] = 0;
-    pre_slot[i] = -1;
-  }
-  __syncthreads();
-  const int64_t per = (n + 1023) / 1024;
+  const int64_t per = (n + PLAN_THREADS - 1) / PLAN_THREADS;
   const int64_t i0 = t * per, i1 = (i0 + per < n) ? i0 + per : n;
-  int64_t nd = 0, np = 0;
+  int64_t cnt = 0;
   for (int64_t i = i0; i < i1; ++i) {
     const int64_t len = cu[i + 1] - cu[i];
-    nd += len == 1;
-    np += len >= 2;
+    cnt += len == 1 ? 1 : len >= 2 ? (int64_t)1 << 32 : 0;
   }
-  s_d[t] = nd;
-  s_p[t] = np;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const int64_t ad = t >= off ? s_d[t - off] : 0, ap = t >= off ? s_p[t - off] : 0;
-    __syncthreads();
-    s_d[t] += ad;
-    s_p[t] += ap;
-    __syncthreads();
+  int64_t tot;
+  const int64_t off = plan_scan(cnt, s_w, tot);
+  const int64_t nd = tot & 0xffffffff, np = tot >> 32;
+  for (int64_t i = t; i < n; i += PLAN_THREADS) {
+    if (i >= nd) {
+      dec_row[i] = 0;
+      dec_slot[i] = -1;
+    }
+    if (i >= np) {
+      pre_lo[i] = 0;
+      pre_hi[i] = 0;
+      pre_slot[i] = -1;
+    }
   }
-  int64_t od = s_d[t] - nd, op = s_p[t] - np;
+  int64_t od = off & 0xffffffff, op = off >> 32;
   for (int64_t i = i0; i < i1; ++i) {
     const int64_t lo = cu[i], hi = cu[i + 1];
     const int32_t sl = slots[i];
@@ -202,39 +223,30 @@ __global__ void __launch_bounds__(RUN_THREADS) slot_runs_kernel(const void* __re
 // entry i takes ceil(len / 64) chunk slots and one spare when it has tokens, none otherwise; off[i] is the
 // exclusive prefix of those counts (off[cap] = *total) and first[w] the entry holding slot w * win (for
 // windows past the total, the last entry).  One workgroup: thread t sums a contiguous range of entries and
-// an inclusive scan over the 1024 sums gives each range its offset.
-__global__ void __launch_bounds__(1024) flat_plan_kernel(const int64_t* __restrict__ lo, const int64_t* __restrict__ hi,
+// a scan over the 1024 sums gives each range its offset.
+__device__ __forceinline__ int64_t flat_slots(int64_t len) { return len >= 2 ? (len + 63) / 64 + 1 : 0; }
+
+__global__ void __launch_bounds__(PLAN_THREADS) flat_plan_kernel(const int64_t* __restrict__ lo, const int64_t* __restrict__ hi,
                                                          int64_t cap, int64_t win, int64_t nwin, int64_t* __restrict__ off,
                                                          int64_t* __restrict__ first, int64_t* __restrict__ total) {
-  __shared__ int64_t s_c[1024];
+  __shared__ int64_t s_w[PLAN_THREADS / 64];
   const int t = threadIdx.x;
-  const int64_t per = (cap + 1023) / 1024;
+  const int64_t per = (cap + PLAN_THREADS - 1) / PLAN_THREADS;
   const int64_t i0 = t * per < cap ? t * per : cap, i1 = (i0 + per < cap) ? i0 + per : cap;
-  auto slots_of = [&](int64_t i) -> int64_t {
-    const int64_t len = hi[i] - lo[i];
-    return len >= 2 ? (len + 63) / 64 + 1 : 0;
-  };
   int64_t cnt = 0;
-  for (int64_t i = i0; i < i1; ++i) cnt += slots_of(i);
-  s_c[t] = cnt;
-  __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    const int64_t a = t >= o ? s_c[t - o] : 0;
-    __syncthreads();
-    s_c[t] += a;
-    __syncthreads();
-  }
-  int64_t acc = s_c[t] - cnt;
+  for (int64_t i = i0; i < i1; ++i) cnt += flat_slots(hi[i] - lo[i]);
+  int64_t tot;
+  int64_t acc = plan_scan(cnt, s_w, tot);
   for (int64_t i = i0; i < i1; ++i) {
     off[i] = acc;
-    acc += slots_of(i);
+    acc += flat_slots(hi[i] - lo[i]);
   }
-  if (t == 1023) {
-    off[cap] = s_c[1023];
-    *total = s_c[1023];
+  if (t == PLAN_THREADS - 1) {
+    off[cap] = tot;
+    *total = tot;
   }
   __syncthreads();  // off[] complete (the block's global writes are visible to its own threads after the barrier)
-  for (int64_t w = t; w < nwin; w += 1024) {
+  for (int64_t w = t; w < nwin; w += PLAN_THREADS) {
     const int64_t g = w * win;
     int64_t a = 0, b = cap;  // the last i in [0, cap) with off[i] <= g
     while (b - a > 1) {
@@ -243,6 +255,110 @@ __global__ void __launch_bounds__(1024) flat_plan_kernel(const int64_t* __restri
       else b = m;
     }
     first[w] = a;
+  }
+}
+
+// The whole plan of a step of at most SLOT_PLAN_TOKENS tokens in one workgroup: what slot_count_kernel,
+// slot_runs_kernel, ragged_split_kernel and flat_plan_kernel leave for the kernels that follow (the decode
+// and prefill lists, the packed layout), without the runs in between.  Thread t owns 8 consecutive tokens
+// and reads the token before and after them: a token that starts a run is a decode if the next one starts
+// a run too (or there is none), else a prefill, whose last token is the next one before a start; so one
+// scan over the counts places every entry.  Four launches of one to four microseconds each, back to back,
+// were most of a small decode step on the GPU (17.6 of 36 us at 9 decodes; the step 88 -> 38 us with this and
+// one stream).
+constexpr int SLOT_PLAN_TOKENS = 8 * PLAN_THREADS;
+
+__global__ void __launch_bounds__(PLAN_THREADS) slot_plan_kernel(
+    const void* __restrict__ sm, int slot_bytes, int64_t n, int64_t cap, int64_t num_slots, int32_t* __restrict__ status,
+    int64_t* __restrict__ dec_row, int32_t* __restrict__ dec_slot, int64_t* __restrict__ pre_lo, int64_t* __restrict__ pre_hi,
+    int32_t* __restrict__ pre_slot, int64_t win, int64_t nwin, int64_t* __restrict__ off, int64_t* __restrict__ first,
+    int64_t* __restrict__ total) {
+  __shared__ int64_t s_w[PLAN_THREADS / 64];
+  __shared__ int s_lo[SLOT_PLAN_TOKENS / 2], s_hi[SLOT_PLAN_TOKENS / 2];  // the prefills (two tokens or more each)
+  const int t = threadIdx.x;
+  const int64_t i0 = 8 * (int64_t)t;
+  int64_t v[10];  // tokens i0 - 1 .. i0 + 8
+#pragma unroll
+  for (int k = 0; k < 10; ++k) {
+    const int64_t i = i0 - 1 + k;
+    v[k] = (i >= 0 && i < n) ? slot_at(sm, slot_bytes, i) : 0;
+  }
+  unsigned start = 0;  // bit k: token i0 - 1 + k starts a run (or is the end of the map)
+#pragma unroll
+  for (int k = 1; k < 10; ++k) {
+    const int64_t i = i0 - 1 + k;
+    if (i == 0 || i == n || (i < n && v[k] != v[k - 1])) start |= 1u << k;
+  }
+  int64_t cnt = 0;
+#pragma unroll
+  for (int k = 1; k < 9; ++k)
+    if (i0 - 1 + k < n && (start >> k & 1)) cnt += (start >> (k + 1) & 1) ? 1 : (int64_t)1 << 32;
+  int64_t tot;
+  const int64_t at = plan_scan(cnt, s_w, tot);
+  int64_t nd = tot & 0xffffffff, np = tot >> 32;
+  const bool over = nd + np > cap;  // distinct runs do not have distinct slots: nothing runs
+  if (over) nd = np = 0;
+  else {
+    int64_t od = at & 0xffffffff, op = at >> 32;
+#pragma unroll
+    for (int k = 1; k < 9; ++k) {
+      const int64_t i = i0 - 1 + k;
+      if (i >= n) break;
+      const int64_t sv = v[k];
+      const bool ok = sv >= 0 && sv < num_slots && sv <= 0x7fffffff;
+      const bool begin = start >> k & 1, end = start >> (k + 1) & 1;
+      if (begin && end) {
+        dec_row[od] = i;
+        dec_slot[od] = ok ? (int32_t)sv : -1;
+        ++od;
+      } else if (begin) {
+        pre_lo[op] = ok ? i : 0;
+        pre_slot[op] = ok ? (int32_t)sv : -1;
+        s_lo[op] = ok ? (int)i : 0;
+        ++op;
+      } else if (end) {  // the last token of prefill op - 1
+        pre_hi[op - 1] = ok ? i + 1 : 0;
+        s_hi[op - 1] = ok ? (int)i + 1 : 0;
+      }
+    }
+  }
+  for (int64_t i = t; i < cap; i += PLAN_THREADS) {
+    if (i >= nd) {
+      dec_row[i] = 0;
+      dec_slot[i] = -1;
+    }
+    if (i >= np) {
+      pre_lo[i] = 0;
+      pre_hi[i] = 0;
+      pre_slot[i] = -1;
+    }
+  }
+  if (t == 0 && status) *status = over ? 1 : 0;
+  if (nwin == 0) return;
+  __syncthreads();  // s_lo, s_hi
+  const int64_t per = (np + PLAN_THREADS - 1) / PLAN_THREADS;
+  const int64_t p0 = t * per < np ? t * per : np, p1 = (p0 + per < np) ? p0 + per : np;
+  cnt = 0;
+  for (int64_t i = p0; i < p1; ++i) cnt += flat_slots(s_hi[i] - s_lo[i]);
+  int64_t acc = plan_scan(cnt, s_w, tot);
+  for (int64_t i = p0; i < p1; ++i) {
+    const int64_t c = flat_slots(s_hi[i] - s_lo[i]);
+    off[i] = acc;
+    s_lo[i] = (int)acc;  // for the search below
+    acc += c;
+  }
+  for (int64_t i = np + t; i <= cap; i += PLAN_THREADS) off[i] = tot;
+  if (t == 0) *total = tot;
+  __syncthreads();
+  for (int64_t w = t; w < nwin; w += PLAN_THREADS) {
+    const int64_t g = w * win;
+    int64_t a = 0, b = np;  // the last entry at or before slot g; past the total, the last of the list
+    while (b - a > 1) {
+      const int64_t m = (a + b) >> 1;
+      if (s_lo[m] <= g) a = m;
+      else b = m;
+    }
+    first[w] = g < tot ? a : cap - 1;
   }
 }
 
@@ -261,8 +377,8 @@ struct DecodeParams {
   void* y; int64_t ys0, ys1;
 };
 
-// Threads per (sequence, head): at least 256 and 8 per value column, so that each thread holds at most
-// 64 state elements.
+// Threads per (sequence, head): at least 256 and 8 per value column, so that each lane holds at most 64
+// state elements.
 template <int DV>
 struct DecodeThreads : std::integral_constant<int, (8 * DV > 256) ? 8 * DV : 256> {};
 
@@ -282,52 +398,84 @@ __device__ __forceinline__ float wave_sum(float v) {
 //   2. the lift, thread t computing features t, t + NT, ...: fp32 dot products with the bf16 Omega rows,
 //      c = cos(2 pi frac(x.Omega_f inv_tau / 2 pi + phase_f / 2 pi)), and the renormalisation of
 //      sqrt(2/D) c from the block's sum of squares;
-//   3. thread (g, j) holds state elements S[f][j] for its feature group g (FPT features, loaded before
-//      step 1 so that their latency overlaps the lift): partial
-//      S^T phi(k) and S^T phi(q) per group, summed in LDS in group order; y = S^T phi(q) (before the
-//      update); S[f][j] <- lambda S[f][j] + beta phi_k[f] (v_j - lambda u_j)  (delta rule), or
+//   3. a lane holds four value columns of NL features of its wave's FPW (loaded before the lift, so that
+//      their latency overlaps it): partial S^T phi(k) and S^T phi(q), summed over the lanes of a column
+//      group and then over the waves in LDS; y = S^T phi(q) (before the update);
+//      S[f][j] <- lambda S[f][j] + beta phi_k[f] (v_j - lambda u_j)  (delta rule), or
 //      lambda S[f][j] + beta phi_k[f] v_j (linear rule); written back in place.
-// One read and one write of the state: the kernel is bound by HBM.
-template <typename InT, typename OutT, int DV>
-__global__ void __launch_bounds__(DecodeThreads<DV>::value) decode_kernel(DecodeParams p) {
+// One read and one write of the state: bound by HBM, so by the bytes in flight.  VEC: the state's rows are
+// contiguous and 16-byte aligned and a slice's offsets fit 32 bits, so a lane's piece is one 16-byte access
+// at a scalar base plus one offset register; 64 scalar loads with 64-bit addresses took 242 registers (one
+// workgroup per CU) where this fits two in 128.  The accesses are streaming: a layer's states are met
+// again a whole model later.  224 x 16 states of 128 KB, split and
+// decode: 206.6 -> 170.5 us (5.5 TB/s; 191.4 with streaming accesses alone), 100 sequences 112.7 -> 86.0.
+template <typename InT, typename OutT, int DV, bool VEC>
+__global__ void __launch_bounds__(DecodeThreads<DV>::value, VEC ? 4 : 2) decode_kernel(DecodeParams p) {
   constexpr int NT = DecodeThreads<DV>::value;
-  constexpr int G = NT / DV;        // feature groups of the state pass
-  constexpr int FPT = SRV_D / G;    // features per thread in the state pass
-  constexpr int LPT = SRV_D / NT;  // lifted features per thread and input
-  __shared__ float s_x[2][SRV_DK];
-  __shared__ float s_c[2][SRV_D];
-  __shared__ float s_ss[NT / 64][2];
-  __shared__ float s_part[G][2][DV];
+  constexpr int NWV = NT / 64;
+  constexpr int LPR = DV / 4;        // lanes per state row
+  constexpr int RPI = 64 / LPR;      // rows a wave's access covers
+  constexpr int FPW = SRV_D / NWV;   // features per wave
+  constexpr int NL = FPW / RPI;      // accesses per lane
+  constexpr int LPT = SRV_D / NT;    // lifted features per thread and input
+  __shared__ __attribute__((aligned(16))) float s_x[2][SRV_DK];
+  __shared__ __attribute__((aligned(8))) float s_c[SRV_D][2];  // cosines of q, k
+  __shared__ float s_ss[NWV][2];
+  __shared__ __attribute__((aligned(16))) float s_part[NWV][2][DV];
 
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int64_t i = blockIdx.x, h = blockIdx.y, c0 = (int64_t)blockIdx.z * DV;
   const int64_t sl = p.slots[i];
   if (sl < 0) return;  // padding, an out-of-range slot or an entry the split did not fill (uniform)
   const int64_t row = p.rows[i];
 
-  // The state elements of thread (g, j) and its scalar inputs are loaded first: they do not depend on
-  // the lift, so their memory latency overlaps it.
-  const int j = t % DV, g = t / DV;
-  float* sp = p.states + sl * p.ss0 + h * p.ss1 + (int64_t)(g * FPT) * p.ss2 + (c0 + j) * p.ss3;
-  float S[FPT];
+  // The inputs, then the state elements: none depends on the lift, so their latency overlaps it.
+  float x = 0.f;
+  if (t < 2 * SRV_DK) {  // waves 0 and 1: q and k
+    const InT* src = t < SRV_DK ? (const InT*)p.q + row * p.qs0 + h * p.qs1 : (const InT*)p.k + row * p.ks0 + h * p.ks1;
+    x = (float)src[lane];
+  }
+  bf16x8 om[SRV_DK / 8];  // Omega's row of the thread's first feature
 #pragma unroll
-  for (int l = 0; l < FPT; ++l) S[l] = sp[l * p.ss2];
+  for (int c8 = 0; c8 < SRV_DK / 8; ++c8) om[c8] = reinterpret_cast<const bf16x8*>(p.omega + (int64_t)t * SRV_DK)[c8];
+  const int jc = 4 * (lane & (LPR - 1));       // this lane's first column of the slice
+  const int fr = FPW * wv + lane / LPR;        // its first feature, then every RPI-th
+  float* sp = p.states + sl * p.ss0 + h * p.ss1 + c0 * p.ss3;  // uniform
+  const unsigned voff = 4u * ((unsigned)fr * (unsigned)p.ss2 + (unsigned)jc);
+  const int64_t goff = (int64_t)fr * p.ss2 + (int64_t)jc * p.ss3;
+  // the base of access l, opaque: otherwise the lane's addresses are formed once and held in 2 NL registers
+  auto base = [&](int l) {
+    float* b = sp + l * RPI * p.ss2;
+    asm volatile("" : "+s"(b));
+    return b;
+  };
+  f32x4 S[NL];
+#pragma unroll
+  for (int l = 0; l < NL; ++l) {
+    const float* b = base(l);
+    if constexpr (VEC) {
+      S[l] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(b) + voff));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[l][e] = b[goff + e * p.ss3];
+    }
+  }
   const float be = p.beta[row * p.bs0 + h * p.bs1];
   const float la = p.decay ? fminf(fmaxf(p.decay[row * p.ds0 + h * p.ds1], 1e-5f), 1.f) : 1.f;
-  const float vin = (float)((const InT*)p.v)[row * p.vs0 + h * p.vs1 + c0 + j];
+  f32x4 vin;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) vin[e] = (float)((const InT*)p.v)[row * p.vs0 + h * p.vs1 + c0 + jc + e];
 
-  // 1. inputs (waves 0 and 1: q and k)
+  // 1. inputs
   if (t < 2 * SRV_DK) {
-    const int m = t >> 6;
-    const InT* src = m == 0 ? (const InT*)p.q + row * p.qs0 + h * p.qs1 : (const InT*)p.k + row * p.ks0 + h * p.ks1;
-    float x = (float)src[lane];
     if (p.normalize) {
       const float inv = 1.0f / fmaxf(sqrtf(wave_sum(x * x)), 1e-6f);
       x = (float)(InT)(x * inv);  // F.normalize keeps the input dtype
     }
-    s_x[m][lane] = x;
+    s_x[t >> 6][lane] = x;
   }
-  __syncthreads();
+  lds_barrier();
 
   // 2. lift
   const float ang = p.inv_tau * 0.15915494309189535f;
@@ -335,23 +483,31 @@ __global__ void __launch_bounds__(DecodeThreads<DV>::value) decode_kernel(Decode
 #pragma unroll
   for (int l = 0; l < LPT; ++l) {
     const int f = t + NT * l;
-    const bf16x8* orow = reinterpret_cast<const bf16x8*>(p.omega + (int64_t)f * SRV_DK);
     float acc[2] = {0.f, 0.f};
 #pragma unroll
     for (int c8 = 0; c8 < SRV_DK / 8; ++c8) {
-      const bf16x8 o = orow[c8];
+      // eight inputs at a time: hoisted, the 128 of them would take the registers the state is held in
+      __builtin_amdgcn_sched_barrier(0);
+      const bf16x8 o = l == 0 ? om[c8] : reinterpret_cast<const bf16x8*>(p.omega + (int64_t)f * SRV_DK)[c8];
+      f32x4 xq[2], xk[2];
+#pragma unroll
+      for (int e4 = 0; e4 < 2; ++e4) {
+        xq[e4] = *reinterpret_cast<const f32x4*>(&s_x[0][8 * c8 + 4 * e4]);
+        xk[e4] = *reinterpret_cast<const f32x4*>(&s_x[1][8 * c8 + 4 * e4]);
+      }
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float w = (float)o[e];
-        acc[0] += s_x[0][8 * c8 + e] * w;
-        acc[1] += s_x[1][8 * c8 + e] * w;
+        acc[0] += xq[e >> 2][e & 3] * w;
+        acc[1] += xk[e >> 2][e & 3] * w;
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
     const float ph = p.phase[f] * 0.15915494309189535f;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(acc[m] * ang + ph));
-      s_c[m][f] = c;
+      s_c[f][m] = c;
       ss[m] += c * c;
     }
   }
@@ -361,10 +517,10 @@ __global__ void __launch_bounds__(DecodeThreads<DV>::value) decode_kernel(Decode
     s_ss[wv][0] = ss[0];
     s_ss[wv][1] = ss[1];
   }
-  __syncthreads();
+  lds_barrier();
   float tot[2] = {0.f, 0.f};
 #pragma unroll
-  for (int w = 0; w < NT / 64; ++w) {
+  for (int w = 0; w < NWV; ++w) {
     tot[0] += s_ss[w][0];
     tot[1] += s_ss[w][1];
   }
@@ -373,37 +529,73 @@ __global__ void __launch_bounds__(DecodeThreads<DV>::value) decode_kernel(Decode
   const float sck = amp / (amp * sqrtf(tot[1]) + 1e-8f);
 
   // 3. state pass
-  float pu = 0.f, py = 0.f;
+  f32x4 pu = zero4(), py = zero4();
 #pragma unroll
-  for (int l = 0; l < FPT; ++l) {
-    pu += S[l] * s_c[1][g * FPT + l];
-    py += S[l] * s_c[0][g * FPT + l];
+  for (int l = 0; l < NL; ++l) {
+    if (l % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+    const float2 c = *reinterpret_cast<const float2*>(s_c[fr + l * RPI]);
+    py += S[l] * c.x;
+    pu += S[l] * c.y;
   }
-  s_part[g][0][j] = pu;
-  s_part[g][1][j] = py;
-  __syncthreads();
-  float u = 0.f, yv = 0.f;
 #pragma unroll
-  for (int gg = 0; gg < G; ++gg) {
-    u += s_part[gg][0][j];
-    yv += s_part[gg][1][j];
+  for (int e = 0; e < 4; ++e) {
+    if constexpr (LPR <= 4) { pu[e] += xor_shuffle<4>(pu[e]); py[e] += xor_shuffle<4>(py[e]); }
+    if constexpr (LPR <= 8) { pu[e] += xor_shuffle<8>(pu[e]); py[e] += xor_shuffle<8>(py[e]); }
+    pu[e] = sum_over_lane_groups(pu[e]);
+    py[e] = sum_over_lane_groups(py[e]);
   }
-  u *= sck;
-  yv *= scq;
-  if (g == 0) ((OutT*)p.y)[row * p.ys0 + h * p.ys1 + c0 + j] = (OutT)yv;
-  const float coef = be * sck * (p.linear ? vin : vin - la * u);  // times c_k[f]
+  if (lane < LPR) {
+    *reinterpret_cast<f32x4*>(&s_part[wv][0][jc]) = pu;
+    *reinterpret_cast<f32x4*>(&s_part[wv][1][jc]) = py;
+  }
+  lds_barrier();
+  f32x4 u = *reinterpret_cast<const f32x4*>(&s_part[0][0][jc]);
 #pragma unroll
-  for (int l = 0; l < FPT; ++l) sp[l * p.ss2] = la * S[l] + coef * s_c[1][g * FPT + l];
+  for (int w = 1; w < NWV; ++w) {
+    if (w % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+    u += *reinterpret_cast<const f32x4*>(&s_part[w][0][jc]);
+  }
+  if (t < DV) {
+    float yv = s_part[0][1][t];
+#pragma unroll
+    for (int w = 1; w < NWV; ++w) yv += s_part[w][1][t];
+    ((OutT*)p.y)[row * p.ys0 + h * p.ys1 + c0 + t] = (OutT)(yv * scq);
+  }
+  const f32x4 coef = (p.linear ? vin : vin - u * (la * sck)) * (be * sck);  // times c_k[f]
+#pragma unroll
+  for (int l = 0; l < NL; ++l) {
+    if (l % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+    const f32x4 o = S[l] * la + coef * s_c[fr + l * RPI][1];
+    float* b = base(l);
+    if constexpr (VEC) {
+      __builtin_nontemporal_store(o, reinterpret_cast<f32x4*>(reinterpret_cast<char*>(b) + voff));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) b[goff + e * p.ss3] = o[e];
+    }
+  }
+}
+
+// Whether decode_kernel may take a state row's pieces as 16-byte accesses at 32-bit offsets of the slice.
+static bool decode_vec(const DecodeParams& p) {
+  return p.ss3 == 1 && aligned(p.states, 16) && p.ss0 % 4 == 0 && p.ss1 % 4 == 0 && p.ss2 % 4 == 0 && p.ss2 >= 0 &&
+         p.ss2 < ((int64_t)1 << 20);
+}
+
+template <typename InT, typename OutT, int DV>
+static void launch_decode_dv(const DecodeParams& dp, const dim3& grid, hipStream_t st) {
+  if (decode_vec(dp)) hipLaunchKernelGGL((decode_kernel<InT, OutT, DV, true>), grid, dim3(DecodeThreads<DV>::value), 0, st, dp);
+  else hipLaunchKernelGGL((decode_kernel<InT, OutT, DV, false>), grid, dim3(DecodeThreads<DV>::value), 0, st, dp);
 }
 
 template <typename InT, typename OutT>
 static int launch_decode(const DecodeParams& dp, int64_t n, int64_t H, int dv, hipStream_t st) {
   const dim3 grid((unsigned)n, (unsigned)H, (unsigned)(dv > 64 ? dv / 64 : 1));
   switch (dv) {
-    case 16: hipLaunchKernelGGL((decode_kernel<InT, OutT, 16>), grid, dim3(DecodeThreads<16>::value), 0, st, dp); break;
-    case 32: hipLaunchKernelGGL((decode_kernel<InT, OutT, 32>), grid, dim3(DecodeThreads<32>::value), 0, st, dp); break;
+    case 16: launch_decode_dv<InT, OutT, 16>(dp, grid, st); break;
+    case 32: launch_decode_dv<InT, OutT, 32>(dp, grid, st); break;
     case 64:
-    case 128: hipLaunchKernelGGL((decode_kernel<InT, OutT, 64>), grid, dim3(DecodeThreads<64>::value), 0, st, dp); break;
+    case 128: launch_decode_dv<InT, OutT, 64>(dp, grid, st); break;
     default: return KDN_ERR_UNSUPPORTED;
   }
   return launch_status();
@@ -497,7 +689,7 @@ extern "C" int kdn_ragged_step(const kdn_ragged_args* a, void* stream, void* aux
   int32_t* dec_slot = (int32_t*)w;           w += round256(n * 8);
   int32_t* pre_slot = (int32_t*)w;           w += round256(n * 8);
   w += round256(n * 4);
-  hipLaunchKernelGGL(ragged_split_kernel, dim3(1), dim3(1024), 0, st, a->cu_seqlens, a->slots, a->num_seqs,
+  hipLaunchKernelGGL(ragged_split_kernel, dim3(1), dim3(PLAN_THREADS), 0, st, a->cu_seqlens, a->slots, a->num_seqs,
                      a->num_slots, dec_row, dec_slot, pre_lo, pre_hi, pre_slot);
   rc = launch_status();
   if (rc != KDN_OK) return rc;
@@ -560,6 +752,9 @@ namespace kdn {
 // states side by side, so a window must hold many of them: 128 slots, about two config-5 prefills per
 // window, took 5.8 ms for the config-5 step against 3.7 with host offsets), fewer when all fit.
 constexpr int64_t SLOT_WIN_MAX = 1024;
+
+// Tokens up to which a step from a slot map keeps to one stream.
+constexpr int64_t SLOT_ONE_STREAM_TOKENS = 1024;
 
 // Sizes of kdn_slot_step's workspace, all bounds from num_tokens and num_slots: `cap` runs at most (one
 // per slot, and the padding runs between them), n_pre prefills (two tokens or more each), G packed slots
@@ -652,18 +847,25 @@ extern "C" int kdn_slot_step(const kdn_slot_step_args* a, void* stream, void* au
   int64_t* fl_off = (int64_t*)w;    w += round256((c + 1) * 8);
   int64_t* fl_total = (int64_t*)w;  w += round256(8);
   int64_t* fl_first = (int64_t*)w;  w += round256((size_t)(pl.nwin > 0 ? pl.nwin : 1) * 8);
-  hipLaunchKernelGGL(slot_count_kernel, dim3((unsigned)rg.blocks), dim3(RUN_THREADS), 0, st, a->slot_mapping,
-                     a->slot_bytes, a->num_tokens, rg.span, rcnt);
-  hipLaunchKernelGGL(slot_runs_kernel, dim3((unsigned)rg.blocks), dim3(RUN_THREADS), 0, st, a->slot_mapping,
-                     a->slot_bytes, a->num_tokens, rg.span, rg.blocks, (const int64_t*)rcnt, pl.cap, cu, rslot, a->status);
-  hipLaunchKernelGGL(ragged_split_kernel, dim3(1), dim3(1024), 0, st, (const int64_t*)cu, (const int32_t*)rslot,
-                     pl.cap, a->num_slots, dec_row, dec_slot, pre_lo, pre_hi, pre_slot);
+  const bool one_plan = a->num_tokens <= SLOT_PLAN_TOKENS;
+  if (one_plan) {
+    hipLaunchKernelGGL(slot_plan_kernel, dim3(1), dim3(PLAN_THREADS), 0, st, a->slot_mapping, a->slot_bytes, a->num_tokens,
+                       pl.cap, a->num_slots, a->status, dec_row, dec_slot, pre_lo, pre_hi, pre_slot, pl.win, pl.nwin,
+                       fl_off, fl_first, fl_total);
+  } else {
+    hipLaunchKernelGGL(slot_count_kernel, dim3((unsigned)rg.blocks), dim3(RUN_THREADS), 0, st, a->slot_mapping,
+                       a->slot_bytes, a->num_tokens, rg.span, rcnt);
+    hipLaunchKernelGGL(slot_runs_kernel, dim3((unsigned)rg.blocks), dim3(RUN_THREADS), 0, st, a->slot_mapping,
+                       a->slot_bytes, a->num_tokens, rg.span, rg.blocks, (const int64_t*)rcnt, pl.cap, cu, rslot, a->status);
+    hipLaunchKernelGGL(ragged_split_kernel, dim3(1), dim3(PLAN_THREADS), 0, st, (const int64_t*)cu, (const int32_t*)rslot,
+                       pl.cap, a->num_slots, dec_row, dec_slot, pre_lo, pre_hi, pre_slot);
+  }
   rc = launch_status();
   if (rc != KDN_OK) return rc;
   // with an auxiliary stream the decode runs on it after the prefill's prep launches, as in
-  // kdn_ragged_step
+  // kdn_ragged_step; a step of few tokens has little to run side by side, and the two events cost more
   const hipStream_t aux = aux_stream ? as_stream(aux_stream) : nullptr;
-  const bool dec_aux = pl.nwin > 0 && aux && aux != st;
+  const bool dec_aux = pl.nwin > 0 && aux && aux != st && a->num_tokens > SLOT_ONE_STREAM_TOKENS;
   EventSet evs;
   if (dec_aux) {
     rc = evs.create(2);
@@ -697,10 +899,12 @@ extern "C" int kdn_slot_step(const kdn_slot_step_args* a, void* stream, void* au
   }
   if (pl.nwin == 0) return KDN_OK;
   // prefill: the packed layout, then the split scan over its windows
-  hipLaunchKernelGGL(flat_plan_kernel, dim3(1), dim3(1024), 0, st, (const int64_t*)pre_lo, (const int64_t*)pre_hi,
-                     pl.cap, pl.win, pl.nwin, fl_off, fl_first, fl_total);
-  rc = launch_status();
-  if (rc != KDN_OK) return rc;
+  if (!one_plan) {
+    hipLaunchKernelGGL(flat_plan_kernel, dim3(1), dim3(PLAN_THREADS), 0, st, (const int64_t*)pre_lo, (const int64_t*)pre_hi,
+                       pl.cap, pl.win, pl.nwin, fl_off, fl_first, fl_total);
+    rc = launch_status();
+    if (rc != KDN_OK) return rc;
+  }
   kdn_scan_args s = slot_scan_args(a, pl.seq_bound);
   s.state_slots = pre_slot;
   s.workspace = w;

@@ -382,3 +382,91 @@ def test_slot_step_rejects_maps_with_too_many_runs(proj):
     torch.cuda.synchronize()
     assert int(status[0]) == 1
     assert torch.equal(sd.cpu(), states) and (y == 3.0).all()
+
+
+# Sequence lengths whose runs meet the plan kernel's edges: 8 tokens a thread, 512 a wave, 8192 a step (one token more
+# takes the kernels for long maps); a negative entry is a padding run of that many tokens.
+PLAN_CASES = {
+    "one": [1], "two": [2], "pair": [1, 1], "eights": [8, 8, 8], "sevens": [7, 1, 8, 9, 1, 1, 15],
+    "padding": [-3, 1, -1, 5, -9, 1, -1], "wave": [511, 1, 512, 2, 510], "limit": [1] * 30 + [4000, 4162],
+    "past": [1] * 30 + [4000, 4163],
+}
+
+
+@pytest.mark.parametrize("slot_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("name", list(PLAN_CASES))
+def test_slot_plan_equals_host_offsets(proj, name, slot_dtype):
+    """The slot-map step against the same step with host offsets (fp32, H = 1, d_v = 16): decodes bit for bit,
+    prefills to 1e-5 (the two window the scan differently: fp32 sums in another order), padding rows and
+    unused slots untouched; a slot past the slab is padding too."""
+    runs = PLAN_CASES[name]
+    lens = [abs(n) for n in runs]
+    n_slots = len(runs) + 3
+    q, k, v, beta, lam, cu, slots, states = make_step(lens, 1, 16, torch.float32, n_slots, seed=3)
+    sl = slots.clone()
+    for i, n in enumerate(runs):
+        if n < 0:
+            sl[i] = -1 - i if i % 2 else n_slots + i
+    host = torch.where(sl >= n_slots, torch.full_like(sl, -1), sl)
+    sm = torch.repeat_interleave(sl.to(slot_dtype), torch.tensor(lens)).to(DEV)
+    args = [t.to(DEV) for t in (q, k, v, beta, lam)]
+    ya, yb = (torch.full((q.shape[0], 1, 16), 7.0, device=DEV) for _ in range(2))
+    sa, sb = states.to(DEV), states.to(DEV)
+    status = torch.full((1,), 9, dtype=torch.int32, device=DEV)
+    tab = (proj.device_omega(DEV), proj.device_phase(DEV), proj.tau_star_inv)
+    ops.slot_step(*args, sm, sa, *tab, y=ya, status=status)
+    ops.ragged_step(*args, cu, host, sb, *tab, y=yb)
+    torch.cuda.synchronize()
+    assert int(status) == 0
+    for i, n in enumerate(runs):
+        lo, hi = int(cu[i]), int(cu[i + 1])
+        if n == 1:
+            assert torch.equal(ya[lo:hi], yb[lo:hi]) and torch.equal(sa[sl[i]], sb[sl[i]])
+        elif n < 0:
+            assert bool((ya[lo:hi] == 7.0).all())
+    assert rel_l2(ya.cpu().numpy(), yb.cpu().numpy()) < 1e-5 and rel_l2(sa.cpu().numpy(), sb.cpu().numpy()) < 1e-5
+    rest = [s for s in range(n_slots) if s not in set(int(x) for x in sl)]
+    assert torch.equal(sa[rest].cpu(), states[rest])
+
+
+def test_slot_plan_more_runs_than_slots(proj):
+    """More runs than 2 slots + 1 (distinct runs without distinct slots): nothing runs and the status is 1."""
+    q, k, v, beta, lam, _, _, states = make_step([12], 1, 16, torch.float32, 2, seed=4)
+    sm = torch.tensor([0, 1] * 6, device=DEV)
+    sd, y = states.to(DEV), torch.full((12, 1, 16), 7.0, device=DEV)
+    status = torch.zeros(1, dtype=torch.int32, device=DEV)
+    ops.slot_step(*(t.to(DEV) for t in (q, k, v, beta, lam)), sm, sd, proj.device_omega(DEV), proj.device_phase(DEV),
+                  proj.tau_star_inv, y=y, status=status)
+    torch.cuda.synchronize()
+    assert int(status) == 1 and torch.equal(sd.cpu(), states) and bool((y == 7.0).all())
+
+
+@pytest.mark.parametrize("dv", [16, 32, 64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rule", [ops.RULE_DELTA, ops.RULE_LINEAR])
+def test_decode_state_layouts(proj, oproj, dv, dtype, rule):
+    """One decode step over the same states held with contiguous rows (16-byte accesses), as the reference's
+    [slot][h][d_v][D], and from an address and with rows that are not 16-byte aligned.  The last three take
+    the element-wise form and agree bit for bit; the 16-byte form sums in the same order but may fuse other
+    multiply-adds: up to 1e-6 in fp32, half a bf16 step (4e-3) in bf16 y.  Both match the oracle."""
+    q, k, v, beta, lam, cu, slots, states = make_step([1] * 5, 2, dv, dtype, 6, seed=dv)
+    got = []
+    for kind in ("rows", "columns", "offset", "padded"):
+        if kind == "rows":
+            sd = states.to(DEV)
+        elif kind == "columns":
+            sd = states.to(DEV).transpose(2, 3).contiguous().transpose(2, 3)
+        elif kind == "offset":
+            sd = torch.empty(states.numel() + 1, device=DEV)[1:].view_as(states).copy_(states)
+        else:
+            sd = torch.empty(6, 2, 512, dv + 1, device=DEV)[..., :dv].copy_(states)
+        y = ops.ragged_step(*(t.to(DEV) for t in (q, k, v, beta, lam)), cu, slots, sd, proj.device_omega(DEV),
+                            proj.device_phase(DEV), proj.tau_star_inv, rule=rule)
+        torch.cuda.synchronize()
+        got.append((y.float().cpu(), sd.cpu().contiguous()))
+    for y, s in got[2:]:
+        assert torch.equal(y, got[1][0]) and torch.equal(s, got[1][1])
+    assert rel_l2(got[0][0].numpy(), got[1][0].numpy()) < (1e-6 if dtype == torch.float32 else 4e-3)
+    assert rel_l2(got[0][1].numpy(), got[1][1].numpy()) < 1e-6
+    Yr, Sr = oracle_step(q, k, v, beta, lam, cu, slots, states, oproj, rule=rule)
+    assert rel_l2(got[0][0].numpy(), Yr) < TOL[dtype] and rel_l2(got[0][1].numpy(), Sr) < TOL[dtype]
