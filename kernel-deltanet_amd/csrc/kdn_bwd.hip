@@ -20,7 +20,7 @@
 // Notation per chunk (tokens i, j in 0..63): l_i = sum_{t <= i} log clamp(lambda_t, 1e-5, 1), g = e^l,
 // g_C = g_63, a_i = g_{i-1} (a_0 = 1), kappa_j = g_C / g_j; A_ij = beta_i (g_i/g_j) k_i.k_j and
 // P_ij = (g_{i-1}/g_j) q_i.k_j for j < i; Y = diag(a) Q S^T + P W; S_C^T = g_C S^T + K^T diag(kappa) W.
-// Every matrix is fp32 and row-major in a per-(head, chunk) record of the workspace.  Products use the
+// The matrices live in a per-(head, chunk) record of the workspace (struct Rec).  Products use the
 // MFMA fragment conventions of kdn_frag.hpp: the lift and the 64 x 64 chunk algebra in fp32
 // (16x16x4 f32), the contractions over the 512 features in the precision policy P (fp32 for fp32
 // inputs, bf16 operands with fp32 accumulation for bf16 inputs).
@@ -30,6 +30,7 @@
 #include <type_traits>
 #include "kdn_frag.hpp"
 #include "kdn_internal.hpp"
+#include "kdn_io.hpp"
 #include "kdn_tile.hpp"
 
 namespace kdn {
@@ -55,27 +56,35 @@ constexpr int DB_V = 0, DB_TS = 2, DB_A = 3, NDB = 5;
 __host__ __device__ constexpr int bop_dk(int m, int o, int jb) { return (m * 4 + o) * 2 + jb; }
 __host__ __device__ constexpr int bop_dq(int m, int o, int jb) { return 32 + (m * 2 + o) * 2 + jb; }
 
-// Per (head, chunk) record, offsets in floats.
+// Per (head, chunk) record, offsets in floats.  Areas that hold operands in the policy's type are sized for
+// fp32.
 struct Rec {
-  static constexpr size_t Q = 0;                // [64][512] lifted, normalised q rows (0 past T)
-  static constexpr size_t K = Q + C * D;        // [64][512] lifted, normalised k rows (0 past T)
+  static constexpr size_t Q = 0;                // SF: S^T as B fragments [n 4][jb 16][lane] for Q S^T (fp32 features:
+                                                // first the lifted q rows [64][512], until the Gram matrices)
+  static constexpr size_t K = Q + C * D;        // fp32 features: the lifted k rows, then Q in fragment order (QXF);
+                                                // bf16: Tp as A fragments [row tile 4][jb 2][lane] f32x8 (TPF)
+  static constexpr size_t TPF = K;
   static constexpr size_t AYF = K + C * D;      // a o dY as B fragments [n 4][jb 2][lane] (sized for f32x8)
-  static constexpr size_t S = AYF + 4 * 2 * 64 * 8;  // [512][64] S^T at the chunk start
-  static constexpr size_t G = S + D * DV;       // [512][64] dL/dS^T at the chunk end
+  static constexpr size_t S = AYF + 4 * 2 * 64 * 8;  // S^T at the chunk start, in 4-value pieces (piece_at)
+  static constexpr size_t G = S + D * DV;       // dL/dS^T at the chunk end, likewise
   static constexpr size_t T = G + D * DV;       // [64][64] (I + A)^-1
-  static constexpr size_t TP = T + C * C;       // [64][64] T diag(beta g)
-  static constexpr size_t P = TP + C * C;       // [64][64]
+  static constexpr size_t TPT = T + C * C;      // Tp^T = diag(beta g) T^T as A fragments [row tile 4][jb 2][lane] f32x8
+  static constexpr size_t P = TPT + C * C;      // [64][64]
   static constexpr size_t GKK = P + C * C;      // [64][64] K K^T
   static constexpr size_t U = GKK + C * C;      // U~ = T (beta o V) as tiles [m 4][n 4][lane] f32x4
   static constexpr size_t R = U + C * DV;       // P^T dY, tiles as U~
-  static constexpr size_t W = R + C * DV;       // [64][64] W = U~ - Tp X_K
-  static constexpr size_t XK = W + C * DV;      // [64][64] K S^T
-  static constexpr size_t DW = XK + C * DV;     // [64][64] dL/dW
-  static constexpr size_t X = DW + C * DV;      // [64][64] K Gamma
-  static constexpr size_t VEC = X + C * DV;     // l[64], beta[64], |phi~_q|[64], |phi~_k|[64]
+  static constexpr size_t W = R + C * DV;       // W = U~ - Tp X_K, tiles
+  static constexpr size_t XK = W + C * DV;      // K S^T, tiles
+  static constexpr size_t DW = XK + C * DV;     // dL/dW, tiles
+  static constexpr size_t X = DW + C * DV;      // K Gamma, tiles
+  // 64-vectors: l, beta, |phi~_q|, |phi~_k|, beta g (0 for the linear rule), phi_q . dphi_q and
+  // phi_k . dphi_k (from the gradient kernel), kappa
+  static constexpr size_t VEC = X + C * DV;
+  static constexpr size_t V_ELL = VEC, V_BETA = VEC + 64, V_NORM = VEC + 128, V_BG = VEC + 256, V_RD = VEC + 320, V_KAP = VEC + 448;
   // K in MFMA fragment order for the chains (one 16- or 32-byte load per lane and fragment), in the
   // precision policy's fragment type (bf16x8 or f32x8; the area is sized for f32x8):
-  static constexpr size_t KXF = VEC + 512;      // [m 4][jb 16][lane]: rows 16m.., features 32jb..
+  static constexpr size_t KXF = VEC + 512;      // [m 4][jb 16][lane]: rows 16m.., features 32jb..; with bf16 features Q
+                                                // likewise in the second half (QXF)
   static constexpr size_t KTF = KXF + C * D;    // [ft 32][jb 2][lane]: K^T rows 16ft.., tokens 32jb..
   static constexpr size_t QTF = KTF + C * D;    // [ft 32][jb 2][lane]: Q^T rows 16ft.., tokens 32jb..
   static constexpr size_t floats = QTF + C * D;
@@ -125,9 +134,9 @@ __device__ __forceinline__ float* record(const Params& p, int64_t b, int64_t h, 
   return p.ws + ((b * p.H + h) * p.cap + c) * (int64_t)Rec::floats;
 }
 
-// The lifted rows Q, K and the carried S^T, Gamma are stored in their record areas as bf16 under the bf16
-// policy (every product that reads them rounds its operands to bf16 anyway; the lift backward's
-// phi . dphi and <Gamma, S> read the rounded values) and as fp32 under the fp32 policy.
+// The features and the carried S^T, Gamma are stored in their record areas as bf16 under the bf16 policy
+// (every product that reads them rounds its operands to bf16 anyway; <Gamma, S> reads the rounded values)
+// and as fp32 under the fp32 policy.
 template <class P> struct Feat { typedef float T; };
 template <> struct Feat<PrecBF16> { typedef __bf16 T; };
 template <class P> struct IsBf16Policy : std::integral_constant<bool, std::is_same<P, PrecBF16>::value> {};
@@ -139,16 +148,26 @@ template <class P>
 __device__ __forceinline__ const typename Feat<P>::T* feat(const float* rec, size_t off) {
   return reinterpret_cast<const typename Feat<P>::T*>(rec + off);
 }
-__device__ __forceinline__ f32x8 frag_rows_t(const float* b, int ld, int r0, int k0, int lane) { return frag_rows(b, ld, r0, k0, lane); }
-__device__ __forceinline__ f32x8 frag_rows_t(const __bf16* b, int ld, int r0, int k0, int lane) { return frag_rows_bf16(b, ld, r0, k0, lane); }
-__device__ __forceinline__ f32x8 frag_cols_t(const float* b, int ld, int c0, int k0, int lane) { return frag_cols(b, ld, c0, k0, lane); }
-__device__ __forceinline__ f32x8 frag_cols_t(const __bf16* b, int ld, int c0, int k0, int lane) { return frag_cols_bf16(b, ld, c0, k0, lane); }
 __device__ __forceinline__ f32x4 ld4_t(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 __device__ __forceinline__ f32x4 ld4_t(const __bf16* p) {
   typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
   const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
   const f32x4 r = {(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
   return r;
+}
+
+// A wave-uniform pointer the compiler may not take apart: a load at uni(p)[lane] keeps its base in scalar
+// registers.  Left alone, it adds the record's large constant offsets to per-lane 64-bit addresses and holds
+// one such address per fragment (the forward carry: 242 registers against 158).
+template <class T>
+__device__ __forceinline__ T* uni(T* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+  // a pointer to global memory, and known as one: a flat load would count as an LDS access too, and every
+  // LDS-only barrier wait for it
+  auto r = (__attribute__((address_space(1))) T*)((uint64_t)hi << 32 | lo);
+  asm volatile("" : "+s"(r));
+  return (T*)r;
 }
 
 // Operand fragments straight in the policy's type (no fp32 round trip for bf16 data):
@@ -174,6 +193,24 @@ __device__ __forceinline__ typename P::frag omega_frag(const __bf16* omega, int 
   else
     return frag_rows_plain_bf16(omega, DK, r0, k0, lane);
 }
+// The carried 512 x 64 matrices in 4-value pieces: piece (ft, n, lane) holds values 16n + 4(lane >> 4) + 0..3 of
+// feature 16ft + (lane & 15), so that an A fragment of their rows is two pieces and a wave's store or load
+// of a piece is one contiguous run.
+template <class P>
+struct Piece {
+  typedef __attribute__((ext_vector_type(4))) typename Feat<P>::T type;
+};
+template <class P>
+__device__ __forceinline__ typename P::frag frag_pieces(const float* rec, size_t off, int ft, int jb, int lane) {
+  const auto* pc = uni(reinterpret_cast<const typename Piece<P>::type*>(rec + off) + (ft * 4 + 2 * jb) * 64);
+  return __builtin_shufflevector(pc[lane], pc[64 + lane], 0, 1, 2, 3, 4, 5, 6, 7);
+}
+// Q in fragment order [m 4][jb 16][lane].
+template <class P>
+__device__ __forceinline__ typename P::frag* qxf_area(float* rec) {
+  if constexpr (IsBf16Policy<P>::value) return reinterpret_cast<typename P::frag*>(rec + Rec::KXF) + 64 * 64;
+  else return reinterpret_cast<typename P::frag*>(rec + Rec::K);
+}
 template <class P>
 __device__ __forceinline__ typename P::frag bf16_frag(const bf16x8& t) {
   if constexpr (IsBf16Policy<P>::value) {
@@ -194,10 +231,13 @@ template <typename InT>
 __device__ __forceinline__ float load_x_part(const InT* x, int64_t base, bool valid, int normalize, float* part) {
   float ss = 0.f;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    part[e] = valid ? ldx(x + base + e) : 0.f;
-    ss += part[e] * part[e];
+  for (int e = 0; e < 16; ++e) part[e] = 0.f;
+  if (valid) {  // rows are 16-byte aligned (checked at the call)
+    load8<InT>(x + base, part);
+    load8<InT>(x + base + 8, part + 8);
   }
+#pragma unroll
+  for (int e = 0; e < 16; ++e) ss += part[e] * part[e];
   ss += __shfl_xor(ss, 1);
   ss += __shfl_xor(ss, 2);
   const float nrm = sqrtf(ss);
@@ -234,7 +274,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   float* bT = smem + 2 * C * LD;  // T
   float* bP = smem + 3 * C * LD;  // P
   // bT and bP are free during the lift: there each wave stages its 128 features of 32 token rows (bf16,
-  // rows padded to 272 bytes against bank conflicts) to write the record's rows 16 bytes per lane
+  // rows padded to 272 bytes against bank conflicts) to read them back as fragments
   constexpr int STG_ROW = 272, STG_WAVE = 32 * STG_ROW;
   static_assert(4 * STG_WAVE <= 2 * C * LD * (int)sizeof(float), "the lift's staging fits bT and bP");
   __shared__ float s_ell[C], s_beta[C], s_n[C], s_red[4][C];
@@ -260,8 +300,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     s_ell[lane] = l;
     s_beta[lane] = be;
-    rec[Rec::VEC + lane] = l;
-    rec[Rec::VEC + 64 + lane] = be;
+    rec[Rec::V_ELL + lane] = l;
+    rec[Rec::V_BETA + lane] = be;
+    rec[Rec::V_BG + lane] = p.linear ? 0.f : be * expf(l);
+    rec[Rec::V_KAP + lane] = expf(__shfl(l, 63) - l);
   }
   {
     float dyp[16];
@@ -291,7 +333,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     lds_barrier();
 
     // phi~ (tokens x this wave's 128 features), in two halves of 32 tokens: tile [ft][u] holds rows
-    // token 16 (2 hm + u) + .., column feature.  Normalised rows go straight to the record.
+    // token 16 (2 hm + u) + .., column feature.
     typename Feat<P>::T* phi = feat<P>(rec, which == 0 ? Rec::Q : Rec::K);
     for (int hm = 0; hm < 2; ++hm) {
       f32x4 acc[8][2];
@@ -349,12 +391,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int row = 32 * hm + tid;
         const float n = sqrtf(s_red[0][row] + s_red[1][row] + s_red[2][row] + s_red[3][row]);
         s_n[row] = n;
-        rec[Rec::VEC + 128 + 64 * which + row] = n;
+        rec[Rec::V_NORM + 64 * which + row] = n;
       }
       lds_barrier();
       // The normalised tiles: the q^T / k^T fragments of depth block hm straight from the registers (an
       // accumulator tile pair [ft][0..1] is the fragment of feature tile ft, tokens 32 hm + kappa), and
-      // the record's rows.
+      // the row fragments (fp32 features: the rows, packed below).
       {
         using frag = typename P::frag;
         frag* tf = reinterpret_cast<frag*>(rec + (which == 0 ? Rec::QTF : Rec::KTF));
@@ -373,7 +415,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
           tf[((8 * w + ft) * 2 + hm) * 64 + lane] = P::from_f32(pair_to8(acc[ft][0], acc[ft][1]));
         }
         if constexpr (IsBf16Policy<P>::value) {
-          // rows through this wave's staging area: 2-byte LDS writes, then 16-byte global stores
+          // rows through this wave's staging area, read back as fragments
           unsigned char* stg = reinterpret_cast<unsigned char*>(bT) + w * STG_WAVE;
 #pragma unroll
           for (int ft = 0; ft < 8; ++ft)
@@ -384,19 +426,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                 *reinterpret_cast<__bf16*>(stg + (16 * u + 4 * (lane >> 4) + i) * STG_ROW + 2 * (16 * ft + (lane & 15))) =
                     (__bf16)acc[ft][u][i];
           wave_lds_sync();
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {  // 32 rows x 16 pieces of 16 bytes
-            const int q = 64 * j + lane, row = q >> 4, pc = q & 15;
-            *reinterpret_cast<bf16x8*>(phi + (size_t)(32 * hm + row) * D + 128 * w + 8 * pc) =
-                *reinterpret_cast<const bf16x8*>(stg + row * STG_ROW + 16 * pc);
-          }
           {
             // K packed in fragment order for the chains, from the same staging rows: token tiles
             // 2 hm, 2 hm + 1, feature blocks 4w .. 4w + 3 (lane: row l & 15, features kappa(l, 0..7));
-            // Q likewise for the Grams below, in the second half of the area (64 fragments of 1 KB
-            // each, free until the gradient launch writes the dx operands there)
+            // Q likewise for the Grams below and the gradient launch (QXF)
             typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-            frag* kxf = reinterpret_cast<frag*>(rec + Rec::KXF) + (which == 0 ? 64 * 64 : 0);
+            frag* kxf = which == 0 ? qxf_area<P>(rec) : reinterpret_cast<frag*>(rec + Rec::KXF);
 #pragma unroll
             for (int mu = 0; mu < 2; ++mu)
 #pragma unroll
@@ -422,7 +457,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     lds_barrier();
   }
-  // The Grams below read the rows this workgroup just wrote to the record: a workgroup-scope release /
+  // The Grams below read the features this workgroup just wrote to the record: a workgroup-scope release /
   // acquire (__syncthreads) orders them.  A device-scope fence here wrote back and invalidated the whole
   // L2 in every workgroup (recompute 365 -> 213 us per segment launch without it).
   __syncthreads();
@@ -461,9 +496,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll 4
     for (int jb = 0; jb < D / 32; ++jb) {
       const typename P::frag kw = kxf[(w * 16 + jb) * 64 + lane];
-      typename P::frag qw;
-      if constexpr (IsBf16Policy<P>::value) qw = kxf[(64 + w * 16 + jb) * 64 + lane];
-      else qw = frag_rows_p<P>(Q, D, 16 * w, 32 * jb, lane);
+      typename P::frag qw, *frag_q;
+      frag_q = qxf_area<P>(rec) + (w * 16 + jb) * 64 + lane;
+      if constexpr (IsBf16Policy<P>::value) {
+        qw = *frag_q;
+      } else {  // Q's rows into fragment order over the k rows, which every wave has packed by now
+        qw = frag_rows_p<P>(Q, D, 16 * w, 32 * jb, lane);
+        *frag_q = qw;
+      }
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
         const typename P::frag kn = kxf[(n * 16 + jb) * 64 + lane];
@@ -491,11 +531,27 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   __syncthreads();
   for (int idx = tid; idx < C * C; idx += 256) {
     const int i = idx >> 6, j = idx & 63;
-    const float tij = bT[i * LD + j];
-    const float tp = p.linear ? 0.f : tij * s_beta[j] * expf(s_ell[j]);
-    rec[Rec::T + idx] = tij;
-    rec[Rec::TP + idx] = tp;
+    rec[Rec::T + idx] = bT[i * LD + j];
     rec[Rec::P + idx] = bP[i * LD + j];
+  }
+  if constexpr (IsBf16Policy<P>::value) {
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) {
+      f32x8 tp = frag_rows(bT, LD, 16 * w, 32 * jb, lane);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        const int j = 32 * jb + kappa(lane, s);
+        tp[s] = p.linear ? 0.f : tp[s] * s_beta[j] * expf(s_ell[j]);
+      }
+      reinterpret_cast<f32x8*>(rec + Rec::TPF)[(w * 2 + jb) * 64 + lane] = tp;
+    }
+  }
+  {
+    const int j = 16 * w + (lane & 15);
+    const float be = p.linear ? 0.f : s_beta[j], g = expf(s_ell[j]);
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb)
+      reinterpret_cast<f32x8*>(rec + Rec::TPT)[(w * 2 + jb) * 64 + lane] = frag_cols(bT, LD, 16 * w, 32 * jb, lane) * be * g;
   }
   {
     const InT* v = reinterpret_cast<const InT*>(p.v);
@@ -531,200 +587,319 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // --------------------------------------------------------------------------------------------- chain
-// grid: 8 * ceil(B*H / 8) * 4 workgroups of 256 threads; workgroup (head-batch hb, value tile n) with
-// the four value tiles of a head on one XCD.  Wave w keeps rows 128w .. 128w+127 of its 512 x 16 slice
-// of the carried matrix (S^T forward, Gamma backward) in registers.
+// grid: 8 * ceil(B*H / 8) * 4 workgroups of CHAIN_WAVES waves; workgroup (head-batch hb, value tile n) with
+// the four value tiles of a head on one XCD.  Wave w keeps features 64w .. 64w+63 of its 512 x 16 slice of
+// the carried matrix (S^T forward, Gamma backward) in registers.
 //
 // Per chunk: store the slice (chunk start S^T / chunk end Gamma); X = K Sigma (partial over the wave's
-// features, reduced through LDS); forward W = U~ - Tp X_K and Z = kappa o W, reverse dW = R + kappa o X
-// and Z = -Tp^T dW; Sigma <- g_C Sigma (+ H) + K^T Z.  With bf16 fragments the K-row fragments of the
-// next chunk are loaded one iteration ahead (two register sets); every other operand is issued at the
-// top of its own iteration, ahead of the first barrier, and the next chunk's lines are prefetched to L2.
+// features, reduced through LDS by waves 0..3, one token tile each); forward W = U~ - Tp X_K and
+// Z = kappa o W, reverse dW = R + kappa o X and Z = -Tp^T dW; Sigma <- g_C Sigma (+ H) + K^T Z.
+//
+// What bounds a step: the CU takes one 128-byte line from L2 every four to six cycles, so the lines a step
+// loads (K 64 KB, in reverse Q^T 64 KB; K^T is formed from K on the matrix cores, 16 products with the
+// identity) and the latency of those that miss L2; then the chain of its three barriers with the 64-deep
+// fp32 product of Tp (512 cycles) between them.  Loads of a wave complete in issue order, so every operand
+// of chunk c + 1 is issued where its registers come free in step c, a step ahead of its use, and waves 4..7,
+// which wait for the reduction and the Tp product, pull chunk c + CHAIN_AHEAD's lines into L2.  Eight waves
+// of 64 features put two on a SIMD; the slice goes out as 8-byte pieces (transposed exactly, again by
+// products with the identity) and whole fragments.  16 heads, 256 chunks, us per carry, forward / reverse:
+// 706 / 948; without the prefetch 856 / 1111; K^T loaded 896 / 899; loads at the top of the step 1175 / 1115;
+// four waves of 128 features with 32 two-byte stores a lane 1051 / 1351.  With L2 always hit: 644 / 645.
 // The barriers order the LDS exchange only (no wave reads another's global writes within a step), so
 // the loads issued ahead and the stores of the step stay in flight across them.
-template <class P>
-struct ChainK {
-  typename P::frag kx[4][4];  // K rows 16m .., features 128w + 32jj ..
-};
-
-template <class P>
-__device__ __forceinline__ void chain_load_kx(ChainK<P>& o, const float* rec, int w, int lane) {
-  const typename P::frag* kx = reinterpret_cast<const typename P::frag*>(rec + Rec::KXF);
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) o.kx[m][jj] = kx[(m * 16 + 4 * w + jj) * 64 + lane];
-}
-
+constexpr int CHAIN_WAVES = 8;
+constexpr int CHAIN_AHEAD = 3;  // chunks between a step and the operands it pulls into L2
 struct ChainShared {
-  f32x4 xp[4][4][64];
+  f32x4 xp[CHAIN_WAVES][4][64];
   f32x4 x[4][64];
   f32x4 z[4][64];
 };
 
-template <class P, bool REV, bool PIPE>
-__device__ __forceinline__ bool chain_step(const Params& p, ChainShared& sh, int64_t b, int64_t h, int64_t step,
-                                           ChainK<P>& cur, ChainK<P>& nxt, f32x4 (&Sg)[8], int w, int lane, int n,
-                                           unsigned& sink) {
+// A chunk's operands of one wave, in registers.
+template <class P, bool REV>
+struct ChainOps {
   using frag = typename P::frag;
-  const int vc = 16 * n + (lane & 15);
-  const int64_t c = REV ? p.nseg - 1 - step : step;
-  const bool more = step + 1 < p.nseg;
-  const int64_t cn = REV ? c - 1 : c + 1;
-  float* rec = record(p, b, h, c);
-  if constexpr (!PIPE) chain_load_kx<P>(cur, rec, w, lane);
-  // operands used later in this iteration
-  // Tp rows (forward) or Tp^T rows, i.e. Tp columns (reverse)
-  const f32x8 tp0 = REV ? frag_cols(rec + Rec::TP, C, 16 * w, 0, lane) : frag_rows(rec + Rec::TP, C, 16 * w, 0, lane);
-  const f32x8 tp1 = REV ? frag_cols(rec + Rec::TP, C, 16 * w, 32, lane) : frag_rows(rec + Rec::TP, C, 16 * w, 32, lane);
-  const f32x4 ur = reinterpret_cast<const f32x4*>(rec + (REV ? Rec::R : Rec::U))[(w * 4 + n) * 64 + lane];
-  const f32x4 lr = *reinterpret_cast<const f32x4*>(rec + Rec::VEC + 16 * w + 4 * (lane >> 4));
-  const float l63 = rec[Rec::VEC + 63];
-  unsigned pf = 0;  // L2-prefetch loads, folded into `sink` at the end of the step (no early wait)
-  if (more) {
-    const float* nrec = record(p, b, h, cn);
-    if constexpr (PIPE) chain_load_kx<P>(nxt, nrec, w, lane);
-    // L2 prefetch of the next chunk: one dword per 128-byte line, spread over the head's 4 workgroups
-    const unsigned* nr = reinterpret_cast<const unsigned*>(nrec);
-    const int idx = n * 256 + (int)threadIdx.x;
-    if (idx < 512 * (int)sizeof(frag) / 16) pf += nr[Rec::KTF + 32 * idx];
-    if (idx < 128) pf += nr[Rec::TP + 32 * idx];
-    else if (idx < 256) pf += nr[(REV ? Rec::R : Rec::U) + 32 * (idx - 128)];
-    else if (idx < 272) pf += nr[Rec::VEC + 32 * (idx - 256)];
-    if constexpr (!PIPE) pf += nr[Rec::KXF + 32 * idx];
-    if constexpr (REV) {
-      if (idx < 512 * (int)sizeof(frag) / 16) pf += nr[Rec::QTF + 32 * idx];
-      if (idx < 8 * (int)sizeof(frag) / 2) pf += nr[Rec::AYF + 32 * idx];
+  // fp32 fragments take twice the registers: K's and Q^T's then share theirs, each loaded where the other is
+  // used up, the Q^T of a chunk inside its step
+  static constexpr bool SHARE = REV && !IsBf16Policy<P>::value;
+  frag kx[4][2];              // K rows 16m .., features 64w + 32jj ..
+  frag kt[4][2];              // K^T rows 64w + 16t .., tokens 32jb ..
+  frag qt[REV ? 4 : 1][2];    // Q^T likewise, and a o dY (reverse)
+  frag y[2];
+  // waves 0..3: row tile w of Tp or Tp^T; with fp32 features, whose record has no room for Tp's fragments, the
+  // forward carry takes T's rows and scales them by beta g
+  static constexpr bool SCALE = !REV && !IsBf16Policy<P>::value;
+  f32x8 tp[2];
+  f32x4 bg[SCALE ? 4 : 1];    // beta g
+  f32x4 ur, kap;              // U~ or R, kappa
+  float l63;
+
+  __device__ __forceinline__ void load_kx(const float* rec, int w, int lane) {
+    const frag* f = reinterpret_cast<const frag*>(rec + Rec::KXF);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj) kx[m][jj] = uni(f + (m * 16 + 2 * w + jj) * 64)[lane];
+  }
+  __device__ __forceinline__ void load_kt(const float* rec, int w, int lane) {
+    const frag* f = reinterpret_cast<const frag*>(rec + Rec::KTF);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) kt[t][jb] = uni(f + ((4 * w + t) * 2 + jb) * 64)[lane];
+  }
+  // The same from kx with bf16 features: a K fragment times the identity has the accumulator layout of K^T
+  // columns, two token tiles of it are a K^T fragment (the values exactly).
+  __device__ __forceinline__ void transpose_k(const frag (&eye)[2]) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      __builtin_amdgcn_sched_barrier(0);  // four products' results at a time
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) {
+        kt[t][jb] = P::from_f32(pair_to8(P::mma(zero4(), kx[2 * jb][t >> 1], eye[t & 1]), P::mma(zero4(), kx[2 * jb + 1][t >> 1], eye[t & 1])));
+        asm volatile("" : "+v"(kt[t][jb]));  // packed here, not at its use
+      }
     }
   }
-
-  // K^T fragments (the update) and, in reverse, Q^T and a o dY fragments (H): with bf16 fragments
-  // issued here and used after the first barrier, so that their latency hides behind the products of the
-  // carried slice (fp32 fragments, twice the registers, are loaded after the barrier)
-  constexpr bool HOIST = IsBf16Policy<P>::value;
-  frag kt[8][2], qt[REV ? 8 : 1][2], y0, y1;
-  auto load_kq = [&]() {
-    const frag* ktf = reinterpret_cast<const frag*>(rec + Rec::KTF);
-#pragma unroll
-    for (int t = 0; t < 8; ++t)
-#pragma unroll
-      for (int jb = 0; jb < 2; ++jb) kt[t][jb] = ktf[((8 * w + t) * 2 + jb) * 64 + lane];
+  __device__ __forceinline__ void load_q(const float* rec, int w, int n, int lane) {
     if constexpr (REV) {
-      const frag* qtf = reinterpret_cast<const frag*>(rec + Rec::QTF);
-      const frag* ayf = reinterpret_cast<const frag*>(rec + Rec::AYF);
-      y0 = ayf[(n * 2) * 64 + lane];
-      y1 = ayf[(n * 2 + 1) * 64 + lane];
+      const frag* fy = reinterpret_cast<const frag*>(rec + Rec::AYF);
+      const frag* f = reinterpret_cast<const frag*>(rec + Rec::QTF);
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+      for (int jb = 0; jb < 2; ++jb) y[jb] = uni(fy + (n * 2 + jb) * 64)[lane];
 #pragma unroll
-        for (int jb = 0; jb < 2; ++jb) qt[t][jb] = qtf[((8 * w + t) * 2 + jb) * 64 + lane];
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb) qt[t][jb] = uni(f + ((4 * w + t) * 2 + jb) * 64)[lane];
     }
-  };
-  if constexpr (HOIST) load_kq();
-
-  typename Feat<P>::T* dst = feat<P>(rec, REV ? Rec::G : Rec::S);
+  }
+  __device__ __forceinline__ void load_lead(const float* rec, int w, int n, int lane) {
+    if constexpr (!SCALE) {
+      const f32x8* f = reinterpret_cast<const f32x8*>(rec + (REV ? Rec::TPT : Rec::TPF));
 #pragma unroll
-  for (int t = 0; t < 8; ++t)
+      for (int jb = 0; jb < 2; ++jb) tp[jb] = uni(f + (w * 2 + jb) * 64)[lane];
+    } else {
+      const float* t = uni(rec + Rec::T + 16 * w * C);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dst[(size_t)(128 * w + 16 * t + 4 * (lane >> 4) + i) * DV + vc] = Sg[t][i];
+      for (int jb = 0; jb < 2; ++jb) tp[jb] = frag_rows(t, C, 0, 32 * jb, lane);
+      const f32x4* vb = reinterpret_cast<const f32x4*>(uni(rec + Rec::V_BG));
+#pragma unroll
+      for (int k = 0; k < 4; ++k) bg[k] = vb[4 * k + (lane >> 4)];
+    }
+    ur = uni(reinterpret_cast<const f32x4*>(rec + (REV ? Rec::R : Rec::U)) + (w * 4 + n) * 64)[lane];
+    kap = reinterpret_cast<const f32x4*>(uni(rec + Rec::V_KAP + 16 * w))[lane >> 4];
+  }
+  __device__ __forceinline__ void load_l63(const float* rec) { l63 = uni(rec + Rec::V_ELL + 63)[0]; }
+};
 
+// One dword of each 128-byte line of a later chunk's operands, shared out over waves 4..7 of the head's four
+// workgroups (1024 lanes): pulls them into the XCD's L2.
+template <class P, bool REV>
+struct ChainPrefetch {
+  static constexpr int AREA = 4096 * (int)sizeof(typename P::frag) / 128;  // lines of a K, K^T or Q^T area
+  static constexpr int KT = IsBf16Policy<P>::value ? 0 : AREA;             // K^T is loaded with fp32 features only
+  static constexpr int E0 = AREA, E1 = E0 + KT, E2 = E1 + (REV ? AREA : 0), E3 = E2 + 128, E4 = E3 + 128, E5 = E4 + 16;
+  static constexpr int LINES = E5 + (REV ? 4 * (int)sizeof(typename P::frag) : 0);
+  static constexpr int PER = (LINES + 1023) / 1024;
+  unsigned v[PER];  // the loaded words: used, and so waited for, only where the next step replaces them
+  __device__ __forceinline__ void load(const float* rec, int n, int w, int lane) {
+    const unsigned* r = reinterpret_cast<const unsigned*>(uni(rec));
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int i = (n * 4 + (w - 4)) * 64 + lane + 1024 * k;
+      unsigned at = Rec::VEC;
+      if (i < E0) at = Rec::KXF + 32 * i;
+      else if (i < E1) at = Rec::KTF + 32 * (i - E0);
+      else if (i < E2) at = Rec::QTF + 32 * (i - E1);
+      else if (i < E3) at = (REV ? Rec::TPT : ChainOps<P, REV>::SCALE ? Rec::T : Rec::TPF) + 32 * (i - E2);
+      else if (i < E4) at = (REV ? Rec::R : Rec::U) + 32 * (i - E3);
+      else if (i < E5) at = Rec::VEC + 32 * (i - E4);
+      else if (REV && i < LINES) at = Rec::AYF + 32 * (i - E5);
+      v[k] = r[at];
+    }
+  }
+};
+
+template <class P, bool REV>
+__device__ __forceinline__ void chain_step(ChainShared& sh, float* rec, const float* nrec, const float* frec, ChainOps<P, REV>& o,
+                                           ChainPrefetch<P, REV>& pf, unsigned& sink,
+                                           f32x4 (&Sg)[4], const typename P::frag (&eye)[2], int w, int lane, int n) {
+  using frag = typename P::frag;
+  using piece = typename Piece<P>::type;
+  const bool lead = w < 4;
+  constexpr bool SHARE = ChainOps<P, REV>::SHARE;
   // K times the carried slice, partial over this wave's features
+  frag sb[2];
+#pragma unroll
+  for (int jj = 0; jj < 2; ++jj) sb[jj] = P::from_f32(pair_to8(Sg[2 * jj], Sg[2 * jj + 1]));
   f32x4 xp[4];
 #pragma unroll
-  for (int m = 0; m < 4; ++m) xp[m] = zero4();
+  for (int m = 0; m < 4; ++m) xp[m] = P::mma(zero4(), o.kx[m][0], sb[0]);
 #pragma unroll
-  for (int jj = 0; jj < 4; ++jj) {
-    const frag sb = P::from_f32(pair_to8(Sg[2 * jj], Sg[2 * jj + 1]));
-#pragma unroll
-    for (int m = 0; m < 4; ++m) xp[m] = P::mma(xp[m], cur.kx[m][jj], sb);
-  }
+  for (int m = 0; m < 4; ++m) xp[m] = P::mma(xp[m], o.kx[m][1], sb[1]);
 #pragma unroll
   for (int m = 0; m < 4; ++m) sh.xp[w][m][lane] = xp[m];
-  // the old slice is dead past the products above: apply g_C now
-  const float gC = expf(l63);
+  // the old slice is dead past the products above (sb holds what is stored): apply g_C now
+  const float gC = expf(o.l63);
+  f32x4 old[IsBf16Policy<P>::value ? 1 : 4];
+  if constexpr (!IsBf16Policy<P>::value) {
 #pragma unroll
-  for (int t = 0; t < 8; ++t) Sg[t] = Sg[t] * gC;
-  lds_barrier();
-  if constexpr (!HOIST) load_kq();
-  f32x4 hh[8];
-  if constexpr (REV) {
-    // this wave's rows of H = Q^T (a o dY) for value tile n
-#pragma unroll
-    for (int t = 0; t < 8; ++t) hh[t] = P::mma(P::mma(zero4(), qt[t][0], y0), qt[t][1], y1);
+    for (int t = 0; t < 4; ++t) old[t] = Sg[t];
   }
-  const f32x4 X = sh.xp[0][w][lane] + sh.xp[1][w][lane] + sh.xp[2][w][lane] + sh.xp[3][w][lane];
-  f32x4 kap;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) kap[i] = expf(l63 - lr[i]);
-  if constexpr (!REV) {
-    sh.x[w][lane] = X;
+  for (int t = 0; t < 4; ++t) Sg[t] = Sg[t] * gC;
+  __builtin_amdgcn_sched_barrier(0);
+  if (IsBf16Policy<P>::value && lead) {
+    o.transpose_k(eye);
+    __builtin_amdgcn_sched_barrier(0);
+    o.load_kx(nrec, w, lane);
+  }
+  if constexpr (!IsBf16Policy<P>::value) {
+    if constexpr (SHARE) o.load_q(rec, w, n, lane);
+    else o.load_kx(nrec, w, lane);
+  }
+  o.load_l63(nrec);
+
+  // the slice to the record: pieces of its rows (both carries), B fragments (forward)
+  {
+    piece* dst = reinterpret_cast<piece*>(rec + (REV ? Rec::G : Rec::S));
+    if constexpr (IsBf16Policy<P>::value) {
+      // D = Sigma^T-tile x identity: lane (feature l & 15, values 4 (l >> 4) + i), the bf16 values exactly
 #pragma unroll
-    for (int i = 0; i < 4; ++i) rec[Rec::XK + (16 * w + 4 * (lane >> 4) + i) * DV + vc] = X[i];
-    lds_barrier();
-    f32x4 tx = mm<PrecF32>(zero4(), tp0, pair_to8(sh.x[0][lane], sh.x[1][lane]));
-    tx = mm<PrecF32>(tx, tp1, pair_to8(sh.x[2][lane], sh.x[3][lane]));
-    const f32x4 Wt = ur - tx;
+      for (int t = 0; t < 4; ++t) {
+        const f32x4 d = P::mma(zero4(), sb[t >> 1], eye[t & 1]);
+        piece v;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) rec[Rec::W + (16 * w + 4 * (lane >> 4) + i) * DV + vc] = Wt[i];
-    sh.z[w][lane] = kap * Wt;
-  } else {
-    const f32x4 dW = ur + kap * X;
+        for (int i = 0; i < 4; ++i) v[i] = (typename Feat<P>::T)d[i];
+        uni(dst + ((4 * w + t) * 4 + n) * 64)[lane] = v;
+      }
+    } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ri = 16 * w + 4 * (lane >> 4) + i;
-      rec[Rec::X + ri * DV + vc] = X[i];
-      rec[Rec::DW + ri * DV + vc] = dW[i];
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          reinterpret_cast<typename Feat<P>::T*>(uni(dst + ((4 * w + t) * 4 + n) * 64))[(4 * (lane >> 4) + i + 16 * ((lane & 15) >> 2)) * 4 + (lane & 3)] = old[t][i];
     }
-    sh.x[w][lane] = dW;
-    lds_barrier();
-    f32x4 zt = mm<PrecF32>(zero4(), tp0, pair_to8(sh.x[0][lane], sh.x[1][lane]));
-    zt = mm<PrecF32>(zt, tp1, pair_to8(sh.x[2][lane], sh.x[3][lane]));
-    sh.z[w][lane] = -zt;
+    if constexpr (!REV) {
+      frag* sf = reinterpret_cast<frag*>(rec + Rec::Q);
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj) uni(sf + (n * 16 + 2 * w + jj) * 64)[lane] = sb[jj];
+    }
+  }
+  lds_barrier();
+  if (lead) {
+    f32x4 X = sh.xp[0][w][lane];
+#pragma unroll
+    for (int v = 1; v < CHAIN_WAVES; ++v) X += sh.xp[v][w][lane];
+    if constexpr (!REV) {
+      sh.x[w][lane] = X;
+      uni(reinterpret_cast<f32x4*>(rec + Rec::XK) + (w * 4 + n) * 64)[lane] = X;
+    } else {
+      const f32x4 dW = o.ur + o.kap * X;
+      sh.x[w][lane] = dW;
+      uni(reinterpret_cast<f32x4*>(rec + Rec::X) + (w * 4 + n) * 64)[lane] = X;
+      uni(reinterpret_cast<f32x4*>(rec + Rec::DW) + (w * 4 + n) * 64)[lane] = dW;
+    }
+  } else if constexpr (IsBf16Policy<P>::value) {
+    o.transpose_k(eye);
+    __builtin_amdgcn_sched_barrier(0);
+    o.load_kx(nrec, w, lane);
+  }
+  lds_barrier();
+  if (lead) {
+    const f32x8 x0 = pair_to8(sh.x[0][lane], sh.x[1][lane]), x1 = pair_to8(sh.x[2][lane], sh.x[3][lane]);
+    if constexpr (ChainOps<P, REV>::SCALE) {
+      o.tp[0] = o.tp[0] * pair_to8(o.bg[0], o.bg[1]);
+      o.tp[1] = o.tp[1] * pair_to8(o.bg[2], o.bg[3]);
+    }
+    const f32x4 t = mm<PrecF32>(mm<PrecF32>(zero4(), o.tp[0], x0), o.tp[1], x1);
+    if constexpr (!REV) {
+      const f32x4 Wt = o.ur - t;
+      sh.z[w][lane] = o.kap * Wt;
+      uni(reinterpret_cast<f32x4*>(rec + Rec::W) + (w * 4 + n) * 64)[lane] = Wt;
+    } else {
+      sh.z[w][lane] = -t;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    o.load_lead(nrec, w, n, lane);
+  } else if (frec) {
+#pragma unroll
+    for (int k = 0; k < ChainPrefetch<P, REV>::PER; ++k) sink ^= pf.v[k];
+    pf.load(frec, n, w, lane);
+  }
+  if constexpr (REV) {
+    // this wave's rows of H = Q^T (a o dY) for value tile n, added to the carry
+#pragma unroll
+    for (int t = 0; t < 4; ++t) Sg[t] = Sg[t] + P::mma(P::mma(zero4(), o.qt[t][0], o.y[0]), o.qt[t][1], o.y[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (SHARE) o.load_kx(nrec, w, lane);
+    else o.load_q(nrec, w, n, lane);
   }
   lds_barrier();
   const frag zb0 = P::from_f32(pair_to8(sh.z[0][lane], sh.z[1][lane]));
   const frag zb1 = P::from_f32(pair_to8(sh.z[2][lane], sh.z[3][lane]));
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    f32x4 acc = Sg[t];
-    if constexpr (REV) acc += hh[t];
-    Sg[t] = P::mma(P::mma(acc, kt[t][0], zb0), kt[t][1], zb1);
+  for (int t = 0; t < 4; ++t) Sg[t] = P::mma(P::mma(Sg[t], o.kt[t][0], zb0), o.kt[t][1], zb1);
+  if constexpr (!IsBf16Policy<P>::value) {
+    __builtin_amdgcn_sched_barrier(0);
+    o.load_kt(nrec, w, lane);
   }
-  sink += pf;
-  return more;
 }
 
 // The carry of workgroup `id` of a chain grid.
 template <class P, bool REV>
 __device__ __forceinline__ void chain_body(const Params& p, ChainShared& sh, int64_t id) {
-  constexpr bool PIPE = std::is_same<P, PrecBF16>::value && !REV;  // two register sets of K fragments fit only as bf16 (forward carry)
+  using frag = typename P::frag;
   const int64_t xcd = id & 7, jdx = id >> 3;
   const int n = (int)(jdx & 3);
   const int64_t hb = (jdx >> 2) * 8 + xcd;
   if (hb >= p.B * p.H) return;
-  const int64_t b = hb / p.H, h = hb % p.H;
+  // the division is done in vector registers: back to scalars, so that every record address is one
+  const int b = __builtin_amdgcn_readfirstlane((int)(hb / p.H));
+  const int h = (int)hb - b * (int)p.H;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int vc = 16 * n + (lane & 15);
 
-  f32x4 Sg[8];
+  f32x4 Sg[4];
   {
     const float* src = REV ? p.dfin : p.init;
     const int64_t s0 = REV ? p.fs0 : p.is0, s1 = REV ? p.fs1 : p.is1, s2 = REV ? p.fs2 : p.is2, s3 = REV ? p.fs3 : p.is3;
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int f = 128 * w + 16 * t + 4 * (lane >> 4) + i;
+        const int f = 64 * w + 16 * t + 4 * (lane >> 4) + i;
         Sg[t][i] = src ? src[b * s0 + h * s1 + f * s2 + vc * s3] : 0.f;
       }
   }
-  unsigned sink = 0;  // keeps the L2 prefetch loads alive (never stored: nseg is positive)
-  ChainK<P> ka, kb;
-  if constexpr (PIPE) chain_load_kx<P>(ka, record(p, b, h, REV ? p.nseg - 1 : 0), w, lane);
-  for (int64_t step = 0;; step += 2) {
-    if (!chain_step<P, REV, PIPE>(p, sh, b, h, step, ka, kb, Sg, w, lane, n, sink)) break;
-    if (!chain_step<P, REV, PIPE>(p, sh, b, h, step + 1, kb, ka, Sg, w, lane, n, sink)) break;
+  // the two halves of a 32 x 32 identity as B fragments: depth kappa(l, s), column 16 k + (l & 15)
+  frag eye[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    f32x8 e;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) e[s] = kappa(lane, s) == 16 * k + (lane & 15) ? 1.f : 0.f;
+    eye[k] = P::from_f32(e);
+  }
+  const int nseg = (int)p.nseg;
+  ChainOps<P, REV> o;
+  {
+    const float* rec = record(p, b, h, REV ? nseg - 1 : 0);
+    o.load_kx(rec, w, lane);
+    o.load_l63(rec);
+    if (w < 4) o.load_lead(rec, w, n, lane);
+    if constexpr (!ChainOps<P, REV>::SHARE) o.load_q(rec, w, n, lane);
+    if constexpr (!IsBf16Policy<P>::value) o.load_kt(rec, w, lane);
+  }
+  ChainPrefetch<P, REV> pf = {};
+  unsigned sink = 0;  // keeps the prefetch loads alive (never stored: nseg is positive)
+  for (int step = 0; step < nseg; ++step) {
+    const int c = REV ? nseg - 1 - step : step;
+    const int cn = step + 1 < nseg ? (REV ? c - 1 : c + 1) : c;  // the last step loads its own chunk again
+    const int cf = REV ? c - CHAIN_AHEAD : c + CHAIN_AHEAD;
+    chain_step<P, REV>(sh, record(p, b, h, c), record(p, b, h, cn), cf >= 0 && cf < nseg ? record(p, b, h, cf) : nullptr, o,
+                       pf, sink, Sg, eye, w, lane, n);
   }
   if (p.nseg < 0) p.ws[0] = (float)sink;
   if constexpr (REV) {
@@ -732,10 +907,10 @@ __device__ __forceinline__ void chain_body(const Params& p, ChainShared& sh, int
     // thread rewrites exactly the elements it read at the top when both are the segment carry
     if (p.gout) {
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int f = 128 * w + 16 * t + 4 * (lane >> 4) + i;
+          const int f = 64 * w + 16 * t + 4 * (lane >> 4) + i;
           p.gout[b * p.gos0 + h * p.gos1 + f * p.gos2 + vc * p.gos3] = Sg[t][i];
         }
     }
@@ -743,7 +918,7 @@ __device__ __forceinline__ void chain_body(const Params& p, ChainShared& sh, int
 }
 
 template <class P, bool REV>
-__global__ void __launch_bounds__(256) bwd_chain_kernel(Params p) {
+__global__ void __launch_bounds__(64 * CHAIN_WAVES) bwd_chain_kernel(Params p) {
   __shared__ ChainShared sh;
   chain_body<P, REV>(p, sh, blockIdx.x);
 }
@@ -752,167 +927,23 @@ __global__ void __launch_bounds__(256) bwd_chain_kernel(Params p) {
 // backward (each reads only what the recompute wrote and they write disjoint fields).  `half` is a
 // multiple of 8, so both halves keep the XCD mapping of a single carry.
 template <class P>
-__global__ void __launch_bounds__(256) bwd_chains_kernel(Params p, unsigned half) {
+__global__ void __launch_bounds__(64 * CHAIN_WAVES) bwd_chains_kernel(Params p, unsigned half) {
   __shared__ ChainShared sh;
   if (blockIdx.x < half) chain_body<P, false>(p, sh, blockIdx.x);
   else chain_body<P, true>(p, sh, blockIdx.x - half);
 }
 
 // ---------------------------------------------------------------------------------------------- grad
-// The lift backward of one of q / k for this wave's NFT = 32 / NW feature tiles (16 features each,
-// features [16 NFT w, 16 NFT (w + 1))) and the 32 tokens of half hm, given dPhi^T in acc[ft][u] (rows
-// feature 16 NFT w + 16 ft + .., column token 16(2hm + u) + ..):
-// ds = -sqrt(2/D) sin(s) (dphi / (n + 1e-8) - phi (phi . dphi) / n), then dx^ = ds Omega reduced over
-// the waves into `dx` (LDS [64][LD], zeroed by the caller).  `xh` holds the normalised
-// input rows; s_rd[w] receives wave w's part of phi . dphi per token (summed in wave order).
-// GEN: the general feature map (per-head or hi + lo Omega, per-head phases and 1/tau, optional
-// renormalisation, dL/d(1/tau)); without it the one shared structured Omega, renormalised, in the
-// registers the path needs alone.  LO (with GEN): Omega has low parts.
-template <class P, int NW, bool LO, bool GEN>
-__device__ __forceinline__ void lift_backward_half(const Params& p, const typename Feat<P>::T* phi, const float* nrm,
-                                                   float (*s_rd)[C], const float* xh, float* dx,
-                                                   f32x4 (&acc)[32 / NW][2], int hm, int w, int lane, int64_t h,
-                                                   float& dit) {
-  constexpr int NFT = 32 / NW;
-  const int fb = 16 * NFT * w;  // the wave's first feature
-  // Omega (and its low parts), the phases and the Omega^T tables of head h, opaque per call: their load
-  // addresses do not depend on the half, and hoisted out of the caller's loop they would hold registers
-  // through it.
-  const __bf16* omega = GEN ? p.omega + h * p.oms : p.omega;
-  const __bf16* omega_lo = LO ? p.omega_lo + h * p.oms : nullptr;
-  const float* phase = GEN ? p.phase + h * p.phs : p.phase;
-  const bf16x8* omt = GEN ? p.omt + h * p.omt_hs : p.omt;
-  asm volatile("" : "+s"(omega), "+s"(omega_lo), "+s"(phase), "+s"(omt));
-  const float itau = GEN ? head_inv_tau(p, h) : p.inv_tau;
-  const bool renorm = GEN ? !p.no_renorm : true;
-  // per token of the half: 1 / (n + 1e-8) and (phi . dphi) / n (without renormalisation dphi~ = dphi)
-  float inv_n[2] = {1.f, 1.f}, rd_n[2] = {0.f, 0.f};
-  if (renorm) {  // uniform over the workgroup
-    float rd[2] = {0.f, 0.f};
-#pragma unroll
-    for (int ft = 0; ft < NFT; ++ft)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int tok = 16 * (2 * hm + u) + (lane & 15);
-        const f32x4 ph = ld4_t(phi + (size_t)tok * D + fb + 16 * ft + 4 * (lane >> 4));
-        rd[u] += ph[0] * acc[ft][u][0] + ph[1] * acc[ft][u][1] + ph[2] * acc[ft][u][2] + ph[3] * acc[ft][u][3];
-      }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const float v = sum_col4(rd[u]);
-      if (lane < 16) s_rd[w][16 * (2 * hm + u) + lane] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int tok = 16 * (2 * hm + u) + (lane & 15);
-      inv_n[u] = 1.f / (nrm[tok] + 1e-8f);
-      float rs = s_rd[0][tok];
-#pragma unroll
-      for (int v = 1; v < NW; ++v) rs += s_rd[v][tok];
-      rd_n[u] = rs / nrm[tok];
-    }
-  }
-  const float amp = sqrtf(2.f / D);
-  typename P::frag xb[2][2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-#pragma unroll
-    for (int jb = 0; jb < 2; ++jb) xb[u][jb] = P::from_f32(frag_rows_plain(xh, LD, 16 * (2 * hm + u), 32 * jb, lane));
-  typename P::frag on0 = omega_frag<P>(omega, fb, 0, lane), on1 = omega_frag<P>(omega, fb, 32, lane);
-  f32x4 phn = *reinterpret_cast<const f32x4*>(phase + fb + 4 * (lane >> 4));
-  float dsv = 0.f;  // sum of dL/d(angle) * (Omega x^) over this lane's elements: dL/d(1/tau)
-#pragma unroll
-  for (int ft = 0; ft < NFT; ++ft) {
-    const int f0 = fb + 16 * ft;
-    const typename P::frag o0 = on0, o1 = on1;
-    const f32x4 ph4 = phn;
-    if (ft + 1 < NFT) {  // the next feature tile's Omega rows and phases, issued one region ahead
-      on0 = omega_frag<P>(omega, f0 + 16, 0, lane);
-      on1 = omega_frag<P>(omega, f0 + 16, 32, lane);
-      phn = *reinterpret_cast<const f32x4*>(phase + f0 + 16 + 4 * (lane >> 4));
-    }
-    typename P::frag l0{}, l1{};
-    if constexpr (LO) {
-      l0 = omega_frag<P>(omega_lo, f0, 0, lane);
-      l1 = omega_frag<P>(omega_lo, f0, 32, lane);
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      f32x4 sv = P::mma(P::mma(zero4(), o0, xb[u][0]), o1, xb[u][1]);
-      if constexpr (LO) sv = P::mma(P::mma(sv, l0, xb[u][0]), l1, xb[u][1]);
-      f32x4 ph = zero4();
-      if (renorm) ph = ld4_t(phi + (size_t)(16 * (2 * hm + u) + (lane & 15)) * D + f0 + 4 * (lane >> 4));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float dphit = acc[ft][u][i] * inv_n[u] - ph[i] * rd_n[u];
-        const float da = -amp * sin_rad(sv[i] * itau + ph4[i]) * dphit;
-        acc[ft][u][i] = da;
-        if constexpr (GEN) dsv += da * sv[i];
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  dit += dsv;
-  f32x4 d[4][2];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int u = 0; u < 2; ++u) d[a][u] = zero4();
-#pragma unroll
-  for (int jj = 0; jj < NFT / 2; ++jj) {
-    typename P::frag ob[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) ob[a] = bf16_frag<P>(omt[(a * 16 + fb / 32 + jj) * 64 + lane]);
-    typename P::frag bs[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      bs[u] = P::from_f32(pair_to8(acc[2 * jj][u], acc[2 * jj + 1][u]));
-#pragma unroll
-      for (int a = 0; a < 4; ++a) d[a][u] = P::mma(d[a][u], ob[a], bs[u]);
-    }
-    if constexpr (LO) {  // dx^ through the low parts of Omega (their table follows the head's)
-#pragma unroll
-      for (int a = 0; a < 4; ++a) ob[a] = bf16_frag<P>(omt[OMT_ENTRIES + (a * 16 + fb / 32 + jj) * 64 + lane]);
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) d[a][u] = P::mma(d[a][u], ob[a], bs[u]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  // Reduce over the waves into dx: groups of four waves in turn, and in turn t of a group wave w adds its
-  // partial of input columns 16a .. 16a+15, a = (w + t) & 3, with 16-byte read-modify-writes; within a
-  // turn the active waves touch disjoint columns.  (Per-element LDS atomics here cost ~15 % of the
-  // kernel: four waves adding to the same addresses.)
-#pragma unroll
-  for (int t = 0; t < NW; ++t) {
-    const bool mine = (w >> 2) == (t >> 2);  // uniform over the wave
-    const int a = (w + t) & 3;
-#pragma unroll
-    for (int aa = 0; aa < 4; ++aa) {
-      if (mine && aa == a) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          f32x4* px = reinterpret_cast<f32x4*>(&dx[(16 * (2 * hm + u) + (lane & 15)) * LD + 16 * aa + 4 * (lane >> 4)]);
-          *px = *px + d[aa][u];
-        }
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// Thread (row tid >> 2, features (tid & 3) * 16 ..): dx = inv_tau * dx^ through the input normalisation,
-// written for tokens before T.
+// Thread (row r, features c0 .. c0 + 15): dx = inv_tau * dx^ through the input normalisation, dx^ the sum of
+// two partials, written for tokens before T.
 template <typename InT>
 __device__ __forceinline__ void write_dx(const Params& p, const InT* x, int64_t xbase, float* out, int64_t obase,
-                                         const float* dx, int r, int c0, bool valid, float itau) {
+                                         const float* dx0, const float* dx1, int r, int c0, bool valid, float itau) {
   float part[16];
   const float nrm = load_x_part<InT>(x, xbase, valid, p.normalize, part);
   float g[16];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) g[e] = itau * dx[r * LD + c0 + e];
+  for (int e = 0; e < 16; ++e) g[e] = itau * (dx0[r * LD + c0 + e] + dx1[r * LD + c0 + e]);
   if (p.normalize) {
     float dot = 0.f;
 #pragma unroll
@@ -929,8 +960,17 @@ __device__ __forceinline__ void write_dx(const Params& p, const InT* x, int64_t 
     }
   }
   if (valid) {
+    float* o = out + obase;
+    if ((reinterpret_cast<uintptr_t>(o) & 15) == 0) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) out[obase + e] = g[e];
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 v = {g[4 * e], g[4 * e + 1], g[4 * e + 2], g[4 * e + 3]};
+        reinterpret_cast<f32x4*>(o)[e] = v;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[e] = g[e];
+    }
   }
 }
 
@@ -951,7 +991,8 @@ __global__ void __launch_bounds__(64 * GRAD_WAVES) bwd_grad_kernel(Params p) {
   //   s_dlp: contributions to dl_i = dL/dl_i (rows DL_*); s_dbp: to dbeta_i (rows DB_*);
   //   s_tsp: column sums of T o dTp per row tile;
   //   s_w63: sums that land on dl_63: the dkappa term per row tile [0..3], <Gamma, S> per wave [4..11]
-  __shared__ float s_dlp[NDL][C], s_dbp[NDB][C], s_tsp[4][C], s_w63[4 + GRAD_WAVES];
+  //   s_da0: the a o dY . Q S^T term of row 0 (a_0 = 1 is no decay: only phi . dphi takes it)
+  __shared__ float s_dlp[NDL][C], s_dbp[NDB][C], s_tsp[4][C], s_w63[4 + GRAD_WAVES], s_da0[2];
 
   const int64_t h = blockIdx.y, b = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -963,8 +1004,8 @@ __global__ void __launch_bounds__(64 * GRAD_WAVES) bwd_grad_kernel(Params p) {
   const bool rvalid = t0 + r < p.T;
 
   if (tid < C) {
-    s_ell[tid] = rec[Rec::VEC + tid];
-    s_beta[tid] = rec[Rec::VEC + 64 + tid];
+    s_ell[tid] = rec[Rec::V_ELL + tid];
+    s_beta[tid] = rec[Rec::V_BETA + tid];
   }
   if (tid == 0)  // the only slots no source writes
     s_dlp[DL_RP][63] = s_dlp[DL_RP + 1][63] = s_dlp[DL_DA][63] = s_dlp[DL_DA + 1][63] = 0.f;
@@ -972,22 +1013,29 @@ __global__ void __launch_bounds__(64 * GRAD_WAVES) bwd_grad_kernel(Params p) {
     const InT* v = reinterpret_cast<const InT*>(p.v);
     const int64_t vb = b * p.vs0 + (t0 + r) * p.vs1 + h * p.vs2 + c0;
     const int64_t yb = b * p.ys0 + (t0 + r) * p.ys1 + h * p.ys2 + c0;
-    // the record's rows as 16-byte pieces (16 contiguous floats per thread, 64-byte aligned)
 #pragma unroll
-    for (int e4 = 0; e4 < 4; ++e4) {
-      const int o = r * LD + c0 + 4 * e4, q = r * DV + c0 + 4 * e4;
-      *reinterpret_cast<f32x4*>(&bW[o]) = *reinterpret_cast<const f32x4*>(rec + Rec::W + q);
-      *reinterpret_cast<f32x4*>(&bdW[o]) = rvalid ? *reinterpret_cast<const f32x4*>(rec + Rec::DW + q) : zero4();
-      *reinterpret_cast<f32x4*>(&bXK[o]) = *reinterpret_cast<const f32x4*>(rec + Rec::XK + q);
-      *reinterpret_cast<f32x4*>(&bX[o]) = *reinterpret_cast<const f32x4*>(rec + Rec::X + q);
-      *reinterpret_cast<f32x4*>(&bT[o]) = *reinterpret_cast<const f32x4*>(rec + Rec::T + r * C + c0 + 4 * e4);
-    }
+    for (int e4 = 0; e4 < 4; ++e4)
+      *reinterpret_cast<f32x4*>(&bT[r * LD + c0 + 4 * e4]) = *reinterpret_cast<const f32x4*>(rec + Rec::T + r * C + c0 + 4 * e4);
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int o = r * LD + c0 + e;
       bY[o] = rvalid ? p.dy[yb + e] : 0.f;
       bV[o] = rvalid ? ldx(v + vb + e) : 0.f;
     }
+  }
+  // W, dW, X_K, X: tiles of the chains (row tile rt, column tiles 2 ch, 2 ch + 1) into rows
+#pragma unroll
+  for (int nn = 0; nn < 2; ++nn) {
+    const int n = 2 * ch + nn;
+    auto tile = [&](size_t off, float* dst) {
+      const f32x4 v = reinterpret_cast<const f32x4*>(rec + off)[(rt * 4 + n) * 64 + lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dst[(16 * rt + 4 * (lane >> 4) + i) * LD + 16 * n + (lane & 15)] = v[i];
+    };
+    tile(Rec::W, bW);
+    tile(Rec::DW, bdW);
+    tile(Rec::XK, bXK);
+    tile(Rec::X, bX);
   }
   __syncthreads();
   const float l63 = s_ell[63], gC = expf(l63);
@@ -1076,15 +1124,16 @@ __global__ void __launch_bounds__(64 * GRAD_WAVES) bwd_grad_kernel(Params p) {
     s_dlp[DL_TS][tid] = s_beta[tid] * g * ts;
   }
   {
+    const typename P::frag* qxf = qxf_area<P>(rec);
+    const typename P::frag* sf = reinterpret_cast<const typename P::frag*>(rec + Rec::Q);
     f32x4 qs[2];
 #pragma unroll
     for (int nn = 0; nn < 2; ++nn) qs[nn] = zero4();
 #pragma unroll 4
     for (int jb = 0; jb < D / 32; ++jb) {
-      const typename P::frag qa = frag_rows_p<P>(feat<P>(rec, Rec::Q), D, 16 * rt, 32 * jb, lane);
+      const typename P::frag qa = qxf[(rt * 16 + jb) * 64 + lane];
 #pragma unroll
-      for (int nn = 0; nn < 2; ++nn)
-        qs[nn] = P::mma(qs[nn], qa, P::from_f32(frag_cols_t(feat<P>(rec, Rec::S), DV, 16 * (2 * ch + nn), 32 * jb, lane)));
+      for (int nn = 0; nn < 2; ++nn) qs[nn] = P::mma(qs[nn], qa, sf[((2 * ch + nn) * 16 + jb) * 64 + lane]);
     }
     float dap[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1096,7 +1145,10 @@ __global__ void __launch_bounds__(64 * GRAD_WAVES) bwd_grad_kernel(Params p) {
     for (int i = 0; i < 4; ++i) {
       const int ri = 16 * rt + 4 * (lane >> 4) + i;
       const float da = sum_row16(dap[i]);
-      if ((lane & 15) == 0 && ri > 0) s_dlp[DL_DA + ch][ri - 1] = da * expf(s_ell[ri - 1]);
+      if ((lane & 15) == 0) {
+        if (ri > 0) s_dlp[DL_DA + ch][ri - 1] = da * expf(s_ell[ri - 1]);
+        else s_da0[ch] = da;
+      }
     }
     // scale this wave's block only (no other wave reads it in this phase)
     for (int e = lane; e < 16 * 32; e += 64) {
@@ -1124,7 +1176,8 @@ __global__ void __launch_bounds__(64 * GRAD_WAVES) bwd_grad_kernel(Params p) {
   f32x4 y1[2], zn[2];
   {
     const f32x8 a0 = frag_rows(bX, LD, 16 * rt, 0, lane), a1 = frag_rows(bX, LD, 16 * rt, 32, lane);
-    const f32x8 p0 = frag_cols(rec + Rec::TP, C, 16 * rt, 0, lane), p1 = frag_cols(rec + Rec::TP, C, 16 * rt, 32, lane);
+    const f32x8* tpt = reinterpret_cast<const f32x8*>(rec + Rec::TPT);
+    const f32x8 p0 = tpt[(rt * 2) * 64 + lane], p1 = tpt[(rt * 2 + 1) * 64 + lane];
 #pragma unroll
     for (int nn = 0; nn < 2; ++nn) {
       const int n = 2 * ch + nn;
@@ -1185,7 +1238,22 @@ __global__ void __launch_bounds__(64 * GRAD_WAVES) bwd_grad_kernel(Params p) {
   }
   __syncthreads();
 
-  // ---- phase 5: dbeta and dlambda (dlog lambda_t = sum_{i >= t} dl_i)
+  // ---- phase 5: dbeta and dlambda (dlog lambda_t = sum_{i >= t} dl_i); phi . dphi per token, which the
+  // renormalisation's backward needs over all features: every term of dphi is a product with Q, K rows or
+  // the carries, so phi . dphi is a sum of terms already here:
+  //   phi_q[i] . dphi_q[i] = a_i dY_i . (Q S)_i + sum_j P_ij dP_ij
+  //   phi_k[j] . dphi_k[j] = (kappa o W)_j . X_j + sum_i P_ij dP_ij + sum_i Tp_ij dTp_ij (X_K . Zn)
+  //                          + row and column sums of A o dA (M + M^T)
+  if (w == 1) {
+    float rq = lane > 0 ? s_dlp[DL_DA][lane - 1] + s_dlp[DL_DA + 1][lane - 1] : s_da0[0] + s_da0[1];
+    if (lane > 0) rq += s_dlp[DL_RP][lane - 1] + s_dlp[DL_RP + 1][lane - 1];
+    float rk = s_dlp[DL_TS][lane] - s_dlp[DL_KAPPA][lane];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) rk -= s_dlp[DL_COLP + v][lane] + s_dlp[DL_DLC + v][lane];
+    rk += s_dlp[DL_A][lane] + s_dlp[DL_A + 1][lane];
+    rec[Rec::V_RD + lane] = rq;
+    rec[Rec::V_RD + 64 + lane] = rk;
+  }
   if (w == 0) {
     float dl = 0.f;
 #pragma unroll
@@ -1233,139 +1301,248 @@ __global__ void __launch_bounds__(64 * GRAD_WAVES) bwd_grad_kernel(Params p) {
 }
 
 // ---------------------------------------------------------------------------------------------- dx
-// One of the two passes of the dx kernel (NW waves, each 512 / NW features): WHICH 1 (k: dK^T and the
-// lift backward of k) or 0 (q).  The first four waves load the input rows and write dx.
-template <class P, typename InT, int WHICH, int NW, bool LO, bool GEN>
-__device__ __forceinline__ void dx_pass(const Params& p, const float* rec, const typename P::frag* bop, float* bT,
-                                        float* bDX, float* s_n, float (*s_rdp)[C], int64_t b, int64_t h, int64_t t0,
-                                        int tid, int w, int lane, int r, int c0, bool rvalid, float& dit) {
-  constexpr int which = WHICH;
-  constexpr int NFT = 32 / NW;  // 16-feature tiles per wave
-  const InT* x = reinterpret_cast<const InT*>(which == 0 ? p.q : p.k);
-  const int64_t xb = which == 0 ? b * p.qs0 + (t0 + r) * p.qs1 + h * p.qs2 + c0 : b * p.ks0 + (t0 + r) * p.ks1 + h * p.ks2 + c0;
-  if (tid < 256) {
-    float part[16];
-    load_x_part<InT>(x, xb, rvalid, p.normalize, part);
-    round_like_input<InT>(p.normalize, part);
+// grid (nseg, H, B), DX_WAVES waves of 64 features each.
+//   dK^T = Gamma (kappa o W)^T + S^T Zn^T + Q^T N + K^T (M + M^T)      dQ^T = S^T (a o dY)^T + K^T N^T
+// for all 64 tokens, 32 features at a time, each followed by their lift backward: with theta = inv_tau (Omega x^) + b recomputed,
+//   dphi~ = dphi / (n + 1e-8) - phi (phi . dphi) / n,  ds = -sqrt(2/D) sin(theta) dphi~,  dx^ = ds Omega
+// (phi . dphi from the gradient kernel, phi from the cosine of the same angle), and the input
+// normalisation's backward to dk, dq.  GEN: the general feature map (per-head or hi + lo Omega, per-head
+// phases and 1/tau, optional renormalisation, dL/d(1/tau)); LO (with GEN): Omega has low parts.
+//
+// The kernel is bound by the record's bytes: each A operand (Gamma, S^T, Q^T, K^T rows, 64 KB each with
+// bf16 features) is read once, for both gradients and all four token tiles;
+// the token-side operands of the gradient kernel (48 fragments) are staged in LDS, one read feeding two
+// feature tiles.  Two halves of 32 tokens and k before q, with the rows of phi read again for phi . dphi,
+// took 1 MB of HBM reads per chunk and head: 4096 chunks 1328 us, this form 426.
+constexpr int DX_WAVES = 8;
+
+template <class P>
+struct DxShared {
+  static constexpr int NBOP = IsBf16Policy<P>::value ? 48 : 0;  // fp32 operands (96 KB) are read from L2: the fp32
+                                                                // products take longer than that
+  static constexpr size_t BOP_BYTES = (size_t)NBOP * 64 * sizeof(typename P::frag), RED_BYTES = 4 * C * LD * sizeof(float);
+  // the token-side operands (bop_dk, bop_dq), then dx^ partials [wave group 2][q, k][64][LD]
+  __attribute__((aligned(16))) unsigned char big[BOP_BYTES > RED_BYTES ? BOP_BYTES : RED_BYTES];
+  typename P::frag x[2][4][2][64];  // normalised q, k rows as B fragments (plain depth order)
+  // per input and token: 1 / (n + 1e-8) and (phi . dphi) / n (without renormalisation dphi~ = dphi: 1, 0)
+  float inv[2][C], rdn[2][C], dit[DX_WAVES];
+};
+
+// dx^ of the inputs W0 .. W0 + NWH - 1 (0 q, 1 k) into the shared partials: with bf16 features both at once,
+// so that S^T and K^T are read once; with fp32 features, whose fragments take twice the registers, k, then q.
+template <class P, bool LO, bool GEN, int W0, int NWH>
+__device__ __forceinline__ void dx_features(const Params& p, DxShared<P>& sh, const float* rec, int64_t h, int w, int lane,
+                                            float itau, float& dit) {
+  using frag = typename P::frag;
+  constexpr int NFT = 32 / DX_WAVES;                   // 16-feature tiles per wave
+  constexpr int PF = IsBf16Policy<P>::value ? 2 : 1;   // feature tiles whose A operands are held at once
+  constexpr bool HASQ = W0 == 0, HASK = W0 + NWH == 2;
+  const frag* bop = DxShared<P>::NBOP ? reinterpret_cast<const frag*>(sh.big) : reinterpret_cast<const frag*>(rec + Rec::KXF);
+  const int fb = 64 * w;
+  const __bf16* omega = GEN ? p.omega + h * p.oms : p.omega;
+  const __bf16* omega_lo = LO ? p.omega_lo + h * p.oms : nullptr;
+  const float* phase = GEN ? p.phase + h * p.phs : p.phase;
+  const bf16x8* omt = GEN ? p.omt + h * p.omt_hs : p.omt;
+  const float amp = sqrtf(2.f / D);
+  // dL/dtheta by input, 32-feature block, token tile, as the B fragments of dx^^T = Omega^T dtheta^T
+  frag bs[NWH][NFT / 2][4];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      bT[r * LD + c0 + e] = part[e];
-      bDX[r * LD + c0 + e] = 0.f;
-    }
-  }
-  if (tid < C) s_n[tid] = rec[Rec::VEC + 128 + 64 * which + tid];
-  __syncthreads();
-#pragma nounroll
-  for (int hm = 0; hm < 2; ++hm) {
-    // The record pointer, opaque to the compiler in each half: the addresses of the A-operand loads below
-    // (a few hundred, 64-bit) do not depend on hm, and hoisted out of the loop they would hold more
-    // registers than the wave has.
-    const float* rec_h = rec;
-    asm volatile("" : "+s"(rec_h));
-    f32x4 acc[NFT][2];
-    // dPhi^T of the half's two token tiles as sums of products of A operands over this wave's features
-    // and B operands from the record (the same for every feature tile):
-    //   dK^T = Gamma (kappa o W)^T + S^T Zn^T + Q^T N + K^T (M + M^T)    (in two passes of two products,
-    //          the accumulators carried, so that only four B fragments per token tile are live)
-    //   dQ^T = S^T (a o dY)^T + K^T N^T
-    constexpr int NPASS = which == 1 ? 2 : 1;
+  for (int fp = 0; fp < NFT / 2; ++fp) {
+    f32x4 acc[NWH][2][4];  // features 32 fp + 16 f + 4 (lane >> 4) + i, token 16u + (lane & 15)
 #pragma unroll
-    for (int ps = 0; ps < NPASS; ++ps) {
-      typename P::frag bo[2][2][2];  // [token tile u][product][depth block jb]
+    for (int fs0 = 0; fs0 < 2; fs0 += PF) {
+      frag fg[PF][2], fs[PF][2], fq[PF][2], fk[PF][2];
+      const frag* qtf = reinterpret_cast<const frag*>(rec + Rec::QTF);
+      const frag* ktf = reinterpret_cast<const frag*>(rec + Rec::KTF);
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int f = 0; f < PF; ++f)
 #pragma unroll
-        for (int oo = 0; oo < 2; ++oo)
-#pragma unroll
-          for (int jb = 0; jb < 2; ++jb)
-            bo[u][oo][jb] = bop[(which == 1 ? bop_dk(2 * hm + u, 2 * ps + oo, jb) : bop_dq(2 * hm + u, oo, jb)) * 64 + lane];
-#pragma unroll
-      for (int ft = 0; ft < NFT; ++ft) {
-        const int f0 = 16 * NFT * w + 16 * ft;
-        // the pass's two A operands (depth blocks 0, 1): Gamma and S^T rows from the record, Q^T and K^T as
-        // the fragments prep stored (one 16- or 32-byte load each)
-        using frag = typename P::frag;
-        const frag* qtf = reinterpret_cast<const frag*>(rec_h + Rec::QTF);
-        const frag* ktf = reinterpret_cast<const frag*>(rec_h + Rec::KTF);
-        const int fi = (f0 >> 4) * 2;  // fragment index of feature tile f0 / 16, depth block 0
-        frag a[2][2];
-        if (which == 1 && ps == 0) {
-          const auto* fG = feat<P>(rec_h, Rec::G);
-          const auto* fS = feat<P>(rec_h, Rec::S);
-          a[0][0] = frag_rows_p<P>(fG, DV, f0, 0, lane); a[0][1] = frag_rows_p<P>(fG, DV, f0, 32, lane);
-          a[1][0] = frag_rows_p<P>(fS, DV, f0, 0, lane); a[1][1] = frag_rows_p<P>(fS, DV, f0, 32, lane);
-        } else if (which == 1) {
-          a[0][0] = qtf[fi * 64 + lane]; a[0][1] = qtf[(fi + 1) * 64 + lane];
-          a[1][0] = ktf[fi * 64 + lane]; a[1][1] = ktf[(fi + 1) * 64 + lane];
-        } else {
-          const auto* fS = feat<P>(rec_h, Rec::S);
-          a[0][0] = frag_rows_p<P>(fS, DV, f0, 0, lane); a[0][1] = frag_rows_p<P>(fS, DV, f0, 32, lane);
-          a[1][0] = ktf[fi * 64 + lane]; a[1][1] = ktf[(fi + 1) * 64 + lane];
+        for (int jb = 0; jb < 2; ++jb) {
+          const int ft = NFT * w + 2 * fp + fs0 + f;
+          if constexpr (HASK) {
+            fg[f][jb] = frag_pieces<P>(rec, Rec::G, ft, jb, lane);
+            fq[f][jb] = uni(qtf + (ft * 2 + jb) * 64)[lane];
+          }
+          fs[f][jb] = frag_pieces<P>(rec, Rec::S, ft, jb, lane);
+          fk[f][jb] = uni(ktf + (ft * 2 + jb) * 64)[lane];
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          f32x4 t = ps == 0 ? zero4() : acc[ft][u];
+      for (int u = 0; u < 4; ++u) {
+        f32x4 tk[PF], tq[PF];
 #pragma unroll
-          for (int oo = 0; oo < 2; ++oo)
+        for (int f = 0; f < PF; ++f) tk[f] = tq[f] = zero4();
 #pragma unroll
-            for (int jb = 0; jb < 2; ++jb) t = P::mma(t, a[oo][jb], bo[u][oo][jb]);
-          acc[ft][u] = t;
+        for (int jb = 0; jb < 2; ++jb) {
+          __builtin_amdgcn_sched_barrier(0);  // at most six fragments of the token side at a time
+          frag k0, k1, k2, k3, q0, q1;
+          if constexpr (HASK) {
+            k0 = bop[bop_dk(u, 0, jb) * 64 + lane]; k1 = bop[bop_dk(u, 1, jb) * 64 + lane];
+            k2 = bop[bop_dk(u, 2, jb) * 64 + lane]; k3 = bop[bop_dk(u, 3, jb) * 64 + lane];
+          }
+          if constexpr (HASQ) { q0 = bop[bop_dq(u, 0, jb) * 64 + lane]; q1 = bop[bop_dq(u, 1, jb) * 64 + lane]; }
+#pragma unroll
+          for (int f = 0; f < PF; ++f) {
+            if constexpr (HASK) tk[f] = P::mma(tk[f], fg[f][jb], k0);
+            if constexpr (HASQ) tq[f] = P::mma(tq[f], fs[f][jb], q0);
+            if constexpr (HASK) tk[f] = P::mma(tk[f], fs[f][jb], k1);
+            if constexpr (HASQ) tq[f] = P::mma(tq[f], fk[f][jb], q1);
+            if constexpr (HASK) tk[f] = P::mma(P::mma(tk[f], fq[f][jb], k2), fk[f][jb], k3);
+          }
         }
-        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int f = 0; f < PF; ++f) {
+          if constexpr (HASQ) acc[0][fs0 + f][u] = tq[f];
+          if constexpr (HASK) acc[NWH - 1][fs0 + f][u] = tk[f];
+        }
       }
     }
-    lift_backward_half<P, NW, LO, GEN>(p, feat<P>(rec_h, which == 0 ? Rec::Q : Rec::K), s_n, s_rdp, bT, bDX, acc,
-                                       hm, w, lane, h, dit);
+    // the lift backward of these 32 features, in place: acc <- dL/dtheta
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      const int f0 = fb + 32 * fp + 16 * f;
+      const frag o0 = omega_frag<P>(omega, f0, 0, lane), o1 = omega_frag<P>(omega, f0, 32, lane);
+      const f32x4 ph4 = *reinterpret_cast<const f32x4*>(phase + f0 + 4 * (lane >> 4));
+      frag l0{}, l1{};
+      if constexpr (LO) {
+        l0 = omega_frag<P>(omega_lo, f0, 0, lane);
+        l1 = omega_frag<P>(omega_lo, f0, 32, lane);
+      }
+#pragma unroll
+      for (int wi = 0; wi < NWH; ++wi)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (u % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+          const frag x0 = sh.x[W0 + wi][u][0][lane], x1 = sh.x[W0 + wi][u][1][lane];
+          const float inv_n = sh.inv[W0 + wi][16 * u + (lane & 15)], rd_n = sh.rdn[W0 + wi][16 * u + (lane & 15)];
+          f32x4 sv = P::mma(P::mma(zero4(), o0, x0), o1, x1);
+          if constexpr (LO) sv = P::mma(P::mma(sv, l0, x0), l1, x1);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float rv = (sv[i] * itau + ph4[i]) * 0.15915494309189535f;
+            rv -= __builtin_rintf(rv);
+            const float cs = amp * __builtin_amdgcn_cosf(rv), sn = amp * __builtin_amdgcn_sinf(rv);
+            const float da = -sn * ((acc[wi][f][u][i] - cs * rd_n) * inv_n);
+            acc[wi][f][u][i] = da;
+            if constexpr (GEN) dit += da * sv[i];
+          }
+          if constexpr (GEN) asm volatile("" : "+v"(dit));  // summed here, not from held terms at the end
+        }
+    }
+#pragma unroll
+    for (int wi = 0; wi < NWH; ++wi)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        bs[wi][fp][u] = P::from_f32(pair_to8(acc[wi][0][u], acc[wi][1][u]));
+        // in its packed form from here on: sunk to the use, the conversion would keep the fp32 values live
+        asm volatile("" : "+v"(bs[wi][fp][u]));
+      }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __syncthreads();
-  if (tid < 256) {
-    const float itau = GEN ? head_inv_tau(p, h) : p.inv_tau;
-    if (which == 0) {
-      write_dx<InT>(p, x, xb, p.dq, b * p.dqs0 + (t0 + r) * p.dqs1 + h * p.dqs2 + c0, bDX, r, c0, rvalid, itau);
-    } else {
-      write_dx<InT>(p, x, xb, p.dk, b * p.dks0 + (t0 + r) * p.dks1 + h * p.dks2 + c0, bDX, r, c0, rvalid, itau);
+  if constexpr (DxShared<P>::NBOP > 0) __syncthreads();  // the token-side operands' LDS takes the dx^ partials
+
+  // dx^^T = Omega^T ds^T over this wave's features, then the waves' partials: two groups of four waves, each
+  // into its own buffer, in turns (turn t: wave w takes input columns 16a .. 16a + 15, a = (w + t) & 3; the
+  // first turn writes) so that the sums have a fixed order.
+#pragma unroll
+  for (int wi = 0; wi < NWH; ++wi) {
+    f32x4 d[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) d[a][u] = zero4();
+#pragma unroll
+    for (int jj = 0; jj < NFT / 2; ++jj)
+#pragma unroll
+      for (int part = 0; part < (LO ? 2 : 1); ++part) {
+        __builtin_amdgcn_sched_barrier(0);
+        frag ob[4];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) ob[a] = bf16_frag<P>(omt[part * OMT_ENTRIES + (a * 16 + fb / 32 + jj) * 64 + lane]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int a = 0; a < 4; ++a) d[a][u] = P::mma(d[a][u], ob[a], bs[wi][jj][u]);
+      }
+    float* red = reinterpret_cast<float*>(sh.big) + ((w >> 2) * 2 + W0 + wi) * C * LD;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int a = (w + t) & 3;
+#pragma unroll
+      for (int aa = 0; aa < 4; ++aa) {
+        if (aa == a) {  // uniform over the wave
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            f32x4* px = reinterpret_cast<f32x4*>(&red[(16 * u + (lane & 15)) * LD + 16 * aa + 4 * (lane >> 4)]);
+            *px = t == 0 ? d[aa][u] : *px + d[aa][u];
+          }
+        }
+      }
+      lds_barrier();
     }
   }
-  __syncthreads();
 }
 
-// grid (nseg, H, B), DX_WAVES waves.  dK^T = Gamma (kappa o W)^T + S^T Zn^T + Q^T N + K^T (M + M^T) and
-// dQ^T = S^T (a o dY)^T + K^T N^T over each wave's 512 / DX_WAVES features, then the lift backward of k
-// and q to dk, dq, each in two halves of 32 tokens.  The small B operands come from the gradient kernel
-// through the record; LDS holds only the input rows and dx^ (36 KB).  Eight waves (64 features each)
-// halve each wave's accumulators and loops, so that two waves share each SIMD.  With Omega's low parts the
-// lift backward reads twice the Omega fragments, which two waves per SIMD (256 registers each) cannot
-// hold without spilling: that variant runs four waves of 128 features.
-constexpr int DX_WAVES = 8;
-template <bool LO>
-struct DxWaves : std::integral_constant<int, LO ? 4 : DX_WAVES> {};
-template <class P, typename InT, bool LO, bool GEN, int NW = DxWaves<LO>::value>
-__global__ void __launch_bounds__(64 * NW) bwd_dx_kernel(Params p) {
-  __shared__ __attribute__((aligned(16))) float bT[C * LD];   // normalised k / q rows
-  __shared__ __attribute__((aligned(16))) float bDX[C * LD];  // dx^ of k / q
-  __shared__ float s_n[C], s_rdp[NW][C], s_dit[NW];
-
+template <class P, typename InT, bool LO, bool GEN>
+__global__ void __launch_bounds__(64 * DX_WAVES) bwd_dx_kernel(Params p) {
+  using frag = typename P::frag;
+  __shared__ DxShared<P> sh;
   const int64_t h = blockIdx.y, b = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t t0 = (p.c0 + blockIdx.x) * C;
   const float* rec = record(p, b, h, blockIdx.x);
-  const int r = tid >> 2, c0 = (tid & 3) * 16;
+  // loaders: input `which` (0 q, 1 k), row r, features c0 .. c0 + 15
+  const int which = tid >> 8, r = (tid >> 2) & 63, c0 = (tid & 3) * 16;
   const bool rvalid = t0 + r < p.T;
-  const typename P::frag* bop = reinterpret_cast<const typename P::frag*>(rec + Rec::KXF);
-
-  float dit = 0.f;  // this lane's share of dL/d(1/tau) over k, then q
-  dx_pass<P, InT, 1, NW, LO, GEN>(p, rec, bop, bT, bDX, s_n, s_rdp, b, h, t0, tid, w, lane, r, c0, rvalid, dit);
-  dx_pass<P, InT, 0, NW, LO, GEN>(p, rec, bop, bT, bDX, s_n, s_rdp, b, h, t0, tid, w, lane, r, c0, rvalid, dit);
+  const InT* x = reinterpret_cast<const InT*>(which == 0 ? p.q : p.k);
+  const int64_t xb = which == 0 ? b * p.qs0 + (t0 + r) * p.qs1 + h * p.qs2 + c0 : b * p.ks0 + (t0 + r) * p.ks1 + h * p.ks2 + c0;
+  {
+    const frag* bop = reinterpret_cast<const frag*>(rec + Rec::KXF);
+    frag* s_bop = reinterpret_cast<frag*>(sh.big);
+#pragma unroll
+    for (int e = 0; e < DxShared<P>::NBOP / DX_WAVES; ++e) s_bop[e * 64 * DX_WAVES + tid] = bop[e * 64 * DX_WAVES + tid];
+    if (tid < 2 * C) {
+      const bool renorm = GEN ? !p.no_renorm : true;
+      const float n = rec[Rec::V_NORM + tid];
+      sh.inv[tid >> 6][tid & 63] = renorm ? 1.f / (n + 1e-8f) : 1.f;
+      sh.rdn[tid >> 6][tid & 63] = renorm ? rec[Rec::V_RD + tid] / n : 0.f;
+    }
+    float part[16];
+    load_x_part<InT>(x, xb, rvalid, p.normalize, part);
+    round_like_input<InT>(p.normalize, part);
+#pragma unroll
+    for (int e8 = 0; e8 < 2; ++e8) {
+      f32x8 v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = part[8 * e8 + e];
+      const int cc = c0 + 8 * e8;
+      sh.x[which][r >> 4][cc >> 5][(r & 15) + 16 * ((cc & 31) >> 3)] = P::from_f32(v);
+    }
+  }
+  __syncthreads();
+  const float itau = GEN ? head_inv_tau(p, h) : p.inv_tau;
+  float dit = 0.f;  // this lane's share of dL/d(1/tau)
+  if constexpr (IsBf16Policy<P>::value) {
+    dx_features<P, LO, GEN, 0, 2>(p, sh, rec, h, w, lane, itau, dit);
+  } else {
+    dx_features<P, LO, GEN, 1, 1>(p, sh, rec, h, w, lane, itau, dit);
+    dx_features<P, LO, GEN, 0, 1>(p, sh, rec, h, w, lane, itau, dit);
+  }
+  {
+    const float* d0 = reinterpret_cast<const float*>(sh.big) + which * C * LD;
+    const float* d1 = d0 + 2 * C * LD;
+    if (which == 0) write_dx<InT>(p, x, xb, p.dq, b * p.dqs0 + (t0 + r) * p.dqs1 + h * p.dqs2 + c0, d0, d1, r, c0, rvalid, itau);
+    else write_dx<InT>(p, x, xb, p.dk, b * p.dks0 + (t0 + r) * p.dks1 + h * p.dks2 + c0, d0, d1, r, c0, rvalid, itau);
+  }
   if (GEN && p.dit) {  // fixed order: lanes by a shuffle tree, then the waves in order
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) dit += __shfl_xor(dit, o);
-    if (lane == 0) s_dit[w] = dit;
+    if (lane == 0) sh.dit[w] = dit;
     __syncthreads();
     if (tid == 0) {
-      float t = s_dit[0];
+      float t = sh.dit[0];
 #pragma unroll
-      for (int v = 1; v < NW; ++v) t += s_dit[v];
+      for (int v = 1; v < DX_WAVES; ++v) t += sh.dit[v];
       p.dit[(b * p.H + h) * p.nch + p.c0 + blockIdx.x] = t;
     }
   }
@@ -1564,20 +1741,20 @@ static int segment_phase(const Params& p, int phase, hipStream_t st) {
     if (p.omega_lo) hipLaunchKernelGGL((bwd_prep_kernel<P, InT, true>), chunk_grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((bwd_prep_kernel<P, InT, false>), chunk_grid, dim3(256), 0, st, p);
   }
-  if (phase == 2) hipLaunchKernelGGL((bwd_chain_kernel<P, false>), dim3(chain_wgs), dim3(256), 0, st, p);
-  if (phase == 3) hipLaunchKernelGGL((bwd_chain_kernel<P, true>), dim3(chain_wgs), dim3(256), 0, st, p);
+  if (phase == 2) hipLaunchKernelGGL((bwd_chain_kernel<P, false>), dim3(chain_wgs), dim3(64 * CHAIN_WAVES), 0, st, p);
+  if (phase == 3) hipLaunchKernelGGL((bwd_chain_kernel<P, true>), dim3(chain_wgs), dim3(64 * CHAIN_WAVES), 0, st, p);
   if (phase == 4 || phase == PH_GRAD)
     hipLaunchKernelGGL((bwd_grad_kernel<P, InT>), chunk_grid, dim3(64 * GRAD_WAVES), 0, st, p);
   if (phase == 4 || phase == PH_DX) {
     const bool gen = p.omega_lo || p.oms || p.phs || p.inv_tau_head || p.no_renorm || p.dit;
-    if (p.omega_lo) hipLaunchKernelGGL((bwd_dx_kernel<P, InT, true, true>), chunk_grid, dim3(64 * DxWaves<true>::value), 0, st, p);
+    if (p.omega_lo) hipLaunchKernelGGL((bwd_dx_kernel<P, InT, true, true>), chunk_grid, dim3(64 * DX_WAVES), 0, st, p);
     else if (gen) hipLaunchKernelGGL((bwd_dx_kernel<P, InT, false, true>), chunk_grid, dim3(64 * DX_WAVES), 0, st, p);
     else hipLaunchKernelGGL((bwd_dx_kernel<P, InT, false, false>), chunk_grid, dim3(64 * DX_WAVES), 0, st, p);
     // segment 0 is the last one processed: every partial of dL/d(1/tau) is written
     if (p.dit && p.c0 == 0)
       hipLaunchKernelGGL(bwd_dit_reduce_kernel, dim3((unsigned)p.H), dim3(64), 0, st, p.dit, p.B, p.H, p.nch, p.dinv_tau);
   }
-  if (phase == PH_CARRIES) hipLaunchKernelGGL((bwd_chains_kernel<P>), dim3(2 * chain_wgs), dim3(256), 0, st, p, chain_wgs);
+  if (phase == PH_CARRIES) hipLaunchKernelGGL((bwd_chains_kernel<P>), dim3(2 * chain_wgs), dim3(64 * CHAIN_WAVES), 0, st, p, chain_wgs);
   return launch_status();
 }
 
