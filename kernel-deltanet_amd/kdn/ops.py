@@ -28,8 +28,51 @@ def require_device(t: torch.Tensor, what: str) -> None:
         raise RuntimeError(f"{what}: kernel-deltanet_amd runs on gfx950 device tensors only (got {t.device})")
 
 
+def _index(dev: torch.device) -> int:
+    return dev.index if dev.index is not None else torch.cuda.current_device()
+
+
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The raw handle of the current stream of `dev` (without a Stream object around it)."""
+    return torch._C._cuda_getCurrentRawStream(_index(dev))
+
+
+class _Here:
+    """The context of work on the device that is current already."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def _on(dev: torch.device):
+    """torch.cuda.device(dev), or nothing when dev is the current device (it usually is, and switching to
+    it and back costs more than the check)."""
+    return _HERE if _index(dev) == torch.cuda.current_device() else torch.cuda.device(dev)
+
+
+def _table(t: torch.Tensor, dev: torch.device, dtype: torch.dtype) -> torch.Tensor:
+    """t contiguous on dev in dtype: t itself when it is that already."""
+    if t.dtype is dtype and t.device == dev and t.is_contiguous():
+        return t
+    return t.to(device=dev, dtype=dtype).contiguous()
+
+
+def _aux_failed(status: int, streams, tensors) -> None:
+    """A call that runs work on auxiliary streams ends with the caller's stream waiting for all of it, so memory
+    freed afterwards is reused only by work ordered behind it, and the tensors need no record_stream (which
+    would hold every call's workspace back until its events have been seen, and grow a queue of calls by a
+    workspace each).  A call that failed half-way may not have joined: mark its tensors then."""
+    if status != N.KDN_OK:
+        for t in tensors:
+            if t is not None:
+                for st in streams:
+                    t.record_stream(st)
 
 
 def _rows(x: torch.Tensor, n: int) -> torch.Tensor:
@@ -48,7 +91,7 @@ def build_omega(sign_bits: torch.Tensor, d_k: int, D: int, device, dtype=torch.b
     bits = sign_bits.to(device=device, dtype=torch.int64).contiguous()
     require_device(bits, "build_omega")
     out = torch.empty(D, d_k, dtype=dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         N.check(N.lib().kdn_build_omega(ctypes.c_void_p(bits.data_ptr()), d_k, D, ctypes.c_void_p(out.data_ptr()),
                                         _tag(dtype, "build_omega"), ctypes.c_void_p(_stream(device))),
                 "kdn_build_omega")
@@ -61,7 +104,7 @@ def fwht(x: torch.Tensor) -> torch.Tensor:
     n = x.shape[-1]
     x2 = _rows(x, n)
     out = torch.empty_like(x2)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         N.check(N.lib().kdn_fwht(ctypes.c_void_p(x2.data_ptr()), x2.shape[0], x2.stride(0), n,
                                  _tag(x.dtype, "fwht"), ctypes.c_void_p(out.data_ptr()), out.stride(0),
                                  ctypes.c_void_p(_stream(x.device))), "kdn_fwht")
@@ -79,16 +122,14 @@ def lift(x: torch.Tensor, omega_bf16: torch.Tensor, phase: torch.Tensor, inv_tau
     x2 = _rows(x, d_k)
     if (x2.stride(0) * x2.element_size()) % 16 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
-    ph = phase.to(device=x.device, dtype=torch.float32).contiguous()
-    om = omega_bf16.to(device=x.device).contiguous()
+    ph = _table(phase, x.device, torch.float32)
+    om = _table(omega_bf16, x.device, omega_bf16.dtype)
     out = torch.empty(x2.shape[0], D, dtype=out_dtype, device=x.device)
-    with torch.cuda.device(x.device):
-        N.check(N.lib().kdn_fwht_lift(ctypes.c_void_p(x2.data_ptr()), x2.shape[0], x2.stride(0),
-                                      _tag(x.dtype, "lift"), 1 if normalize else 0,
-                                      ctypes.c_void_p(om.data_ptr()), ctypes.c_void_p(ph.data_ptr()),
-                                      d_k, D, float(inv_tau), ctypes.c_void_p(out.data_ptr()), out.stride(0),
-                                      _tag(out_dtype, "lift output"), ctypes.c_void_p(_stream(x.device))),
-                "kdn_fwht_lift")
+    with _on(x.device):
+        N.check(N.lib().kdn_fwht_lift(x2.data_ptr(), x2.shape[0], x2.stride(0), _tag(x.dtype, "lift"),
+                                      1 if normalize else 0, om.data_ptr(), ph.data_ptr(), d_k, D, float(inv_tau),
+                                      out.data_ptr(), out.stride(0), _tag(out_dtype, "lift output"),
+                                      _stream(x.device)), "kdn_fwht_lift")
     return out.view(*x.shape[:-1], D)
 
 
@@ -109,17 +150,15 @@ def lift_bits(x: torch.Tensor, rademacher_bits: torch.Tensor, phase: torch.Tenso
     x2 = _rows(x, d_k)
     if (x2.stride(0) * x2.element_size()) % 16 or x2.data_ptr() % 16:
         x2 = x2.contiguous()
-    bits = rademacher_bits.to(device=x.device, dtype=torch.int64).contiguous()
-    ph = phase.to(device=x.device, dtype=torch.float32).contiguous()
+    bits = _table(rademacher_bits, x.device, torch.int64)
+    ph = _table(phase, x.device, torch.float32)
     out = torch.empty(x2.shape[0], D, dtype=out_dtype, device=x.device)
     name = "kdn_fwht_lift_bits_butterfly" if butterfly else "kdn_fwht_lift_bits"
-    with torch.cuda.device(x.device):
-        N.check(getattr(N.lib(), name)(ctypes.c_void_p(x2.data_ptr()), x2.shape[0], x2.stride(0),
-                                       _tag(x.dtype, "lift_bits"), d_k, ctypes.c_void_p(bits.data_ptr()), D,
-                                       float(inv_tau), ctypes.c_void_p(ph.data_ptr()), 1 if normalize else 0,
-                                       ctypes.c_void_p(out.data_ptr()), out.stride(0),
-                                       _tag(out_dtype, "lift_bits output"), ctypes.c_void_p(_stream(x.device))),
-                name)
+    with _on(x.device):
+        N.check(getattr(N.lib(), name)(x2.data_ptr(), x2.shape[0], x2.stride(0), _tag(x.dtype, "lift_bits"), d_k,
+                                       bits.data_ptr(), D, float(inv_tau), ph.data_ptr(), 1 if normalize else 0,
+                                       out.data_ptr(), out.stride(0), _tag(out_dtype, "lift_bits output"),
+                                       _stream(x.device)), name)
     return out.view(*x.shape[:-1], D)
 
 
@@ -139,7 +178,7 @@ def lift_factored(x: torch.Tensor, omega1: torch.Tensor, phase1: torch.Tensor, o
     p1 = phase1.to(device=dev, dtype=torch.float32).contiguous()
     p2 = phase2.to(device=dev, dtype=torch.float32).contiguous()
     out = torch.empty(x2.shape[0], 1024, dtype=out_dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(N.lib().kdn_fwht_lift_factored(
             ctypes.c_void_p(x2.data_ptr()), x2.shape[0], x2.stride(0), _tag(x.dtype, "lift_factored"),
             ctypes.c_void_p(o1.data_ptr()), ctypes.c_void_p(p1.data_ptr()), ctypes.c_void_p(o2.data_ptr()),
@@ -165,7 +204,7 @@ def lift_factored_backward(x: torch.Tensor, dphi: torch.Tensor, omega1: torch.Te
     p1 = phase1.to(device=dev, dtype=torch.float32).contiguous()
     p2 = phase2.to(device=dev, dtype=torch.float32).contiguous()
     dx = torch.empty(x2.shape[0], 128, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         N.check(N.lib().kdn_fwht_lift_factored_bwd(
             ctypes.c_void_p(x2.data_ptr()), x2.shape[0], x2.stride(0), _tag(x.dtype, "lift_factored_backward"),
             ctypes.c_void_p(o1.data_ptr()), ctypes.c_void_p(p1.data_ptr()), ctypes.c_void_p(o2.data_ptr()),
@@ -294,20 +333,15 @@ def aux_stream(dev: torch.device, which: int = 0) -> torch.cuda.Stream:
 
 def _launch_scan(a, dev: torch.device, pipelined: bool, keep=()):
     """kdn_delta_scan_fwd, or the pipelined three-stream variant (kdn_delta_scan_fwd_streams: prep and
-    output on two auxiliary streams).  Tensors the auxiliary streams read or write are marked with
-    record_stream so the caching allocator does not hand their memory out again before that work ends."""
-    st = torch.cuda.current_stream(dev)
+    output on two auxiliary streams, joined back into the current one); `keep`: the tensors the auxiliary
+    streams read or write (_aux_failed)."""
     if pipelined:
         aux_p, aux_o = aux_stream(dev, 0), aux_stream(dev, 1)
-        for t in keep:
-            if t is not None:
-                t.record_stream(aux_p)
-                t.record_stream(aux_o)
-        N.check(N.lib().kdn_delta_scan_fwd_streams(ctypes.byref(a), ctypes.c_void_p(st.cuda_stream),
-                                                   ctypes.c_void_p(aux_p.cuda_stream),
-                                                   ctypes.c_void_p(aux_o.cuda_stream)), "kdn_delta_scan_fwd_streams")
+        rc = N.lib().kdn_delta_scan_fwd_streams(ctypes.byref(a), _stream(dev), aux_p.cuda_stream, aux_o.cuda_stream)
+        _aux_failed(rc, (aux_p, aux_o), keep)
+        N.check(rc, "kdn_delta_scan_fwd_streams")
     else:
-        N.check(N.lib().kdn_delta_scan_fwd(ctypes.byref(a), ctypes.c_void_p(st.cuda_stream)), "kdn_delta_scan_fwd")
+        N.check(N.lib().kdn_delta_scan_fwd(ctypes.byref(a), _stream(dev)), "kdn_delta_scan_fwd")
 
 
 def scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, decay: Optional[torch.Tensor],
@@ -360,7 +394,7 @@ def scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, 
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     a = scan_args(q, k, v, beta, decay, None, None, inv_tau, normalize, initial_state, final_state, y,
                   workspace, segment_chunks, features, rule)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _launch_scan(a, dev, pipelined, (q, k, v, beta, decay, initial_state, final_state, y, workspace)
                      + features.keep())
     return y, final_state
@@ -475,14 +509,16 @@ class ScanBackwardPlan:
         stream 0 runs the other launches around them (kdn_delta_scan_bwd_streams), else every launch runs
         in order on `stream` (kdn_delta_scan_bwd).  The results are the same bit for bit."""
         st = self._st(stream)
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             if concurrent_carries:
                 aux = aux_stream(self.device, 0)
-                for t in self._tensors():
-                    t.record_stream(aux)
-                N.check(N.lib().kdn_delta_scan_bwd_streams(ctypes.byref(self.args), ctypes.c_void_p(st.cuda_stream),
-                                                           ctypes.c_void_p(aux.cuda_stream)),
-                        "kdn_delta_scan_bwd_streams")
+                rc = N.lib().kdn_delta_scan_bwd_streams(ctypes.byref(self.args), st.cuda_stream, aux.cuda_stream)
+                if rc != N.KDN_OK:
+                    _aux_failed(rc, (aux,), self._tensors())
+                elif stream is not None and stream != torch.cuda.current_stream(self.device):
+                    for t in self._tensors():  # the plan's memory belongs to the current stream, not to `stream`
+                        t.record_stream(st)
+                N.check(rc, "kdn_delta_scan_bwd_streams")
             else:
                 N.check(N.lib().kdn_delta_scan_bwd(ctypes.byref(self.args), ctypes.c_void_p(st.cuda_stream)),
                         "kdn_delta_scan_bwd")
@@ -490,7 +526,7 @@ class ScanBackwardPlan:
 
     def phase(self, i: int, segment: int = 0, stream=None):
         st = self._st(stream)
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             N.check(N.lib().kdn_scan_bwd_phase(ctypes.byref(self.args), int(i), int(segment),
                                                ctypes.c_void_p(st.cuda_stream)), "kdn_scan_bwd_phase")
 
@@ -620,10 +656,9 @@ def _features_on(fm: FeatureMap, dev: torch.device, H: int) -> FeatureMap:
     itau = fm.inv_tau_head
     if itau is not None and tuple(itau.shape) != (H,):
         raise ValueError(f"scan: inv_tau_head must be ({H},)")
-    return FeatureMap(fm.omega.to(dev).contiguous(), fm.phase.to(device=dev, dtype=torch.float32).contiguous(),
-                      None if fm.omega_lo is None else fm.omega_lo.to(dev).contiguous(),
-                      None if itau is None else itau.to(device=dev, dtype=torch.float32).contiguous(),
-                      fm.no_renorm, False)
+    return FeatureMap(_table(fm.omega, dev, torch.bfloat16), _table(fm.phase, dev, torch.float32),
+                      None if fm.omega_lo is None else _table(fm.omega_lo, dev, torch.bfloat16),
+                      None if itau is None else _table(itau, dev, torch.float32), fm.no_renorm, False)
 
 
 SCHEDULE_SPLIT, SCHEDULE_FUSED, SCHEDULE_GENERAL = 0, 1, 2  # kdn_scan_schedule (include/kdn.h)
@@ -657,7 +692,7 @@ class ScanPlan:
         # the library's segment length for this shape (its default when segment_chunks is 0)
         probe = scan_args(self.q, self.k, self.v, self.beta, self.decay, self.omega, self.phase, inv_tau, normalize,
                           initial_state, self.final_state, self.y, None, segment_chunks)
-        with torch.cuda.device(dev):
+        with _on(dev):
             self.segment_chunks = int(N.lib().kdn_scan_segment_chunks(ctypes.byref(probe), 1 if pipelined else 0))
             self.schedule = int(N.lib().kdn_scan_schedule(ctypes.byref(probe)))
         if self.segment_chunks <= 0 or self.schedule < 0:
@@ -783,8 +818,8 @@ def _ragged_args(q, k, v, beta, decay, cu_seqlens, slots, states, omega_bf16, ph
     d_v = v.shape[-1]
     if y is None:
         y = torch.empty(T, H, d_v, device=dev, dtype=q.dtype if out_dtype is None else out_dtype)
-    om = omega_bf16.to(dev).contiguous()
-    ph = phase.to(device=dev, dtype=torch.float32).contiguous()
+    om = _table(omega_bf16, dev, omega_bf16.dtype)
+    ph = _table(phase, dev, torch.float32)
     a = N.RaggedArgs()
     a.num_seqs, a.H = n, H
     a.d_k, a.D, a.d_v = q.shape[-1], om.shape[0], d_v
@@ -851,17 +886,12 @@ def ragged_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.T
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    st = torch.cuda.current_stream(dev)
-    with torch.cuda.device(dev):
-        aux = None
-        if pipelined:
-            aux = aux_stream(dev)
-            for t in keep[:11] + (workspace,):
-                if t is not None:
-                    t.record_stream(aux)
-        N.check(N.lib().kdn_ragged_step(ctypes.byref(a), ctypes.c_void_p(st.cuda_stream),
-                                        ctypes.c_void_p(aux.cuda_stream) if aux is not None else None),
-                "kdn_ragged_step")
+    aux = aux_stream(dev) if pipelined else None
+    with _on(dev):
+        rc = N.lib().kdn_ragged_step(ctypes.byref(a), _stream(dev), None if aux is None else aux.cuda_stream)
+    if aux is not None:
+        _aux_failed(rc, (aux,), keep[:11] + (workspace,))
+    N.check(rc, "kdn_ragged_step")
     return y
 
 
@@ -896,8 +926,8 @@ def slot_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Ten
     d_v = v.shape[-1]
     if y is None:
         y = torch.empty(T, H, d_v, device=dev, dtype=q.dtype if out_dtype is None else out_dtype)
-    om = omega_bf16.to(dev).contiguous()
-    ph = phase.to(device=dev, dtype=torch.float32).contiguous()
+    om = _table(omega_bf16, dev, omega_bf16.dtype)
+    ph = _table(phase, dev, torch.float32)
     a = N.SlotStepArgs()
     a.num_tokens, a.H = T, H
     a.d_k, a.D, a.d_v = q.shape[-1], om.shape[0], d_v
@@ -921,17 +951,12 @@ def slot_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Ten
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    st = torch.cuda.current_stream(dev)
-    with torch.cuda.device(dev):
-        aux = None
-        if pipelined:
-            aux = aux_stream(dev)
-            for t in (q, k, v, beta, decay, om, ph, states, y, sm, workspace, status):
-                if t is not None:
-                    t.record_stream(aux)
-        N.check(N.lib().kdn_slot_step(ctypes.byref(a), ctypes.c_void_p(st.cuda_stream),
-                                      ctypes.c_void_p(aux.cuda_stream) if aux is not None else None),
-                "kdn_slot_step")
+    aux = aux_stream(dev) if pipelined else None
+    with _on(dev):
+        rc = N.lib().kdn_slot_step(ctypes.byref(a), _stream(dev), None if aux is None else aux.cuda_stream)
+    if aux is not None:
+        _aux_failed(rc, (aux,), (q, k, v, beta, decay, om, ph, states, y, sm, workspace, status))
+    N.check(rc, "kdn_slot_step")
     return y
 
 

@@ -88,7 +88,9 @@ class MultiHeadRKHSKernel(nn.Module):
             om2 = torch.cat([om, om], dim=1)
             hi = om2.to(torch.bfloat16)
             lo = (om2 - hi.to(torch.float32)).to(torch.bfloat16)
-            phase = torch.cat([torch.zeros(self.m), torch.full((self.m,), -math.pi / 2)]).to(device)
+            # filled on the device: a host tensor's copy would make every call wait for the queue
+            phase = torch.zeros(2 * self.m, device=device)
+            phase[self.m:] = -math.pi / 2
             inv_tau = torch.sqrt(2.0 * torch.exp(self.log_gamma.detach().to(device=device, dtype=torch.float32)))
         return ops.FeatureMap(omega=hi.contiguous(), phase=phase, omega_lo=lo.contiguous(),
                               inv_tau_head=inv_tau.contiguous(), no_renorm=True)
