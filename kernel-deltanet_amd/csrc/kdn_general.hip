@@ -31,40 +31,63 @@ namespace gen {
 constexpr int C = 64;
 constexpr int LD = 68;
 
+// Record fields that hold operands in the precision policy's type are sized for fp32.
+//
+// Feature order.  A fragment read straight from a feature row takes eight consecutive features per lane (one
+// 16- or 32-byte load): lane (g = l >> 4) slot s holds feature 8g + s of a 32-feature block.  A pair of
+// accumulator tiles (2j, 2j + 1) over the block's features then holds feature 8g + 4a + i in row 4g + i of
+// tile 2j + a, so that a lane's eight values of the pair are again eight consecutive features.
+__device__ __forceinline__ int feature_of(int tile, int row) { return 32 * (tile >> 1) + 8 * (row >> 2) + 4 * (tile & 1) + (row & 3); }
+
 template <int D, int DV>
 struct Rec {
   static constexpr int NV = DV / 16;
-  static constexpr size_t KXF = 0;            // K-row fragments [m 4][jb D/32][lane], sized for f32x8
-  static constexpr size_t KTF = KXF + C * D;  // K^T-row fragments [ft D/16][jb 2][lane]
-  static constexpr size_t S = KTF + C * D;    // S^T at the chunk start as output B fragments [jb D/32][n NV][lane]
-  static constexpr size_t TP = S + D * DV;    // [64][64] T diag(beta g)
-  static constexpr size_t P = TP + C * C;     // [64][64]
+  static constexpr size_t KXF = 0;            // K-row fragments [m 4][jb D/32][lane]; backward with bf16 fragments: Q's
+                                              // likewise in the second half (QXF)
+  static constexpr size_t KTF = KXF + C * D;  // fp32: K^T-row fragments [tile D/16][jb 2][lane]
+  static constexpr size_t S = KTF + C * D;    // S^T at the chunk start as output fragments [jb D/32][n NV][lane]
+  static constexpr size_t TPF = S + D * DV;   // Tp = T diag(beta g) as A fragments [row tile 4][jb 2][lane] f32x8
+  static constexpr size_t P = TPF + C * C;    // forward: as A fragments, likewise; backward: rows [64][64]
   static constexpr size_t U = P + C * C;      // U~ as tiles [m 4][n NV][lane] f32x4
-  static constexpr size_t W = U + C * DV;     // [64][DV]
-  static constexpr size_t VEC = W + C * DV;   // l[64], beta[64]
-  static constexpr size_t floats = (VEC + 128 + 63) / 64 * 64;
+  static constexpr size_t W = U + C * DV;     // forward: tiles, likewise; backward: rows [64][DV]
+  static constexpr size_t VEC = W + C * DV;   // 64-vectors: l, kappa
+  static constexpr size_t V_L = VEC, V_KAP = VEC + 64;
+  static constexpr size_t floats = VEC + 128;
 };
 
-// The backward's record (kdn_delta_scan_bwd at D = 1024): the forward's record followed by the
-// fields of the gradient (offsets in floats).
+// The backward's record (kdn_delta_scan_bwd at D = 1024): the forward's record (its S field unused) followed
+// by the fields of the gradient (offsets in floats).  D x DV matrices in accumulator tiles [n NV][tile D/16][lane]
+// f32x4: lane (g, v = l & 15) holds features feature_of(tile, 4g + i) of value 16n + v.
 template <int D, int DV>
 struct BRec {
-  static constexpr size_t T = Rec<D, DV>::floats;  // [64][64] (I + A)^-1
-  static constexpr size_t G = T + C * C;            // [64][64] K K^T
-  static constexpr size_t XK = G + C * C;           // [64][DV] K S^T
-  static constexpr size_t SR = XK + C * DV;         // [DV][D] the chunk-start state (S, not S^T), fp32
-  static constexpr size_t H1 = SR + D * DV;         // [DV][D] (Q^T (a o dY))^T
-  static constexpr size_t RR = H1 + D * DV;         // [64][DV] P^T dY
-  static constexpr size_t GR = RR + C * DV;         // [DV][D] (dL/dS^T)^T at the chunk end
+  static constexpr size_t SR = Rec<D, DV>::S;       // S^T at the chunk start, fp32 tiles
+  static constexpr size_t T = Rec<D, DV>::floats;   // [64][64] (I + A)^-1
+  static constexpr size_t G = T + C * C;            // [64][64] K K^T (on and below the diagonal tiles)
+  static constexpr size_t TPT = G + C * C;          // Tp^T as A fragments, as TPF
+  static constexpr size_t XK = TPT + C * C;         // [64][DV] K S^T
+  static constexpr size_t QTF = XK + C * DV;        // fp32: Q^T-row fragments, as KTF
+  static constexpr size_t RR = QTF + C * D;         // P^T dY, tiles as U~
+  static constexpr size_t GR = RR + C * DV;         // dL/dS^T at the chunk end, fp32 tiles
   static constexpr size_t X = GR + D * DV;          // [64][DV] K Gamma
   static constexpr size_t DW = X + C * DV;          // [64][DV] dL/dW
-  static constexpr size_t ZN = DW + C * DV;         // [64][DV] -Tp^T dW (= dL/dX_K)
+  static constexpr size_t DWT = DW + C * DV;        // the same as tiles, as U~
+  static constexpr size_t ZN = DWT + C * DV;        // [64][DV] -Tp^T dW (= dL/dX_K)
   static constexpr size_t AY = ZN + C * DV;         // [64][DV] a o dY
-  static constexpr size_t KW = AY + C * DV;         // [64][DV] kappa o W
-  static constexpr size_t NN = KW + C * DV;         // [64][64] N
-  static constexpr size_t MM = NN + C * C;          // [64][64] M + M^T
-  static constexpr size_t floats = (MM + C * C + 63) / 64 * 64;
+  static constexpr size_t AYF = AY + C * DV;        // a o dY as B fragments over tokens [n NV][jb 2][lane]
+  static constexpr size_t OPS = AYF + C * DV;       // right operands of the feature gradients (bop_*), fragments
+  static constexpr size_t PART = OPS + 3 * C * DV + 3 * C * C;  // [D/32][64] a o dY . Q S^T by 32-feature block, then
+                                                                // [D/32] <Gamma, S> likewise
+  static constexpr size_t V_BETA = PART + (D / 32 * 65 + 63) / 64 * 64;  // 64-vectors: beta, dl without the terms of S
+  static constexpr size_t V_DL = V_BETA + 64;
+  // The size of a record is what callers have sized workspaces by: kept, though the fields no longer fill it.
+  static constexpr size_t floats = T + 3 * D * DV + 7 * C * DV + 4 * C * C;
+  static_assert(V_DL + 64 <= floats, "the fields fit the record");
 };
+// Fragment index in OPS: token tile m, 32-deep block of the value columns (AY, KW, ZN) or of the tokens
+// (N, M + M^T, N^T).
+template <int DV> __host__ __device__ constexpr int bop_v(int o, int m, int kb) { return (o * 4 + m) * (DV / 32) + kb; }
+template <int DV> __host__ __device__ constexpr int bop_t(int o, int m, int jb) { return 3 * 4 * (DV / 32) + (o * 4 + m) * 2 + jb; }
+template <int DV> __host__ __device__ constexpr int bop_count() { return 3 * 4 * (DV / 32) + 3 * 4 * 2; }
 
 struct Params {
   int64_t B, T, H, nch;
@@ -77,6 +100,19 @@ struct Params {
   float* fin; int64_t fs0, fs1, fs2, fs3;
   void* y; int64_t ys0, ys1, ys2;
   float* ws;
+  int qkvec, vvec, yvec;  // rows of q and k / of v / of y start on 16 bytes (4 elements for y), whatever the token
+};
+
+struct BwdP {
+  const float* dy; int64_t ys0, ys1, ys2;         // NULL in the checkpoint pass
+  const float* dfin; int64_t fs0, fs1, fs2, fs3;  // dL/dS^T at the end (NULL: zero)
+  float* dq; int64_t dqs0, dqs1, dqs2;
+  float* dk; int64_t dks0, dks1, dks2;
+  float* dv; int64_t dvs0, dvs1, dvs2;
+  float* dbeta; int64_t dbs0, dbs1, dbs2;
+  float* ddecay; int64_t dds0, dds1, dds2;        // NULL: not wanted
+  float* dinit; int64_t gis0, gis1, gis2, gis3;   // dL/dS^T at the start (NULL: not wanted)
+  int yvec, gvec;                                 // rows of dy / of dq and dk start on 16 bytes
 };
 
 // Record of (b, h, c): the forward's layout, or the backward's longer one.
@@ -86,54 +122,141 @@ __device__ __forceinline__ float* record(const Params& p, int64_t b, int64_t h, 
   return p.ws + ((b * p.H + h) * p.nch + c) * F;
 }
 
-// Fragments read straight from the input feature rows of one chunk (row i = token t0 + i, stride rs
-// elements; rows at or past `nrows` read as zero).  rows: element (r0 + l%16, k0 + kappa);
-// cols: element (c0 + l%16, k0 + kappa) = row k0 + kappa, column c0 + l%16.
-template <typename InT>
-__device__ __forceinline__ f32x8 frag_rows_in(const InT* base, int64_t rs, int r0, int k0, int lane, int nrows) {
-  const int row = r0 + (lane & 15);
-  f32x8 r;
-  if (row < nrows) {
-    const InT* q = base + row * rs + k0 + 4 * (lane >> 4);
+// Eight consecutive elements as a fragment of policy PB.
+template <class PB, typename InT, bool VEC>
+__device__ __forceinline__ typename PB::frag load8(const InT* x) {
+  typedef __attribute__((ext_vector_type(8))) InT in8;
+  if constexpr (VEC) {
+    const in8 t = *reinterpret_cast<const in8*>(x);
+    if constexpr (std::is_same<typename PB::frag, in8>::value) {
+      return t;
+    } else {
+      f32x8 r;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      r[s] = ldx(q + s);
-      r[4 + s] = ldx(q + 16 + s);
+      for (int s = 0; s < 8; ++s) r[s] = (float)t[s];
+      return PB::from_f32(r);
     }
   } else {
+    f32x8 r;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) r[s] = 0.f;
+    for (int s = 0; s < 8; ++s) r[s] = ldx(x + s);
+    return PB::from_f32(r);
   }
-  return r;
 }
+template <class PB>
+__device__ __forceinline__ typename PB::frag zero_frag() {
+  f32x8 z;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) z[s] = 0.f;
+  return PB::from_f32(z);
+}
+// Fragment of the input's rows r0 .. r0 + 15, features k0 .. k0 + 31 (rows at or past `nrows` read as zero;
+// their loads go to the last row).
+template <class PB, typename InT, bool VEC>
+__device__ __forceinline__ typename PB::frag row_frag(const InT* base, int64_t rs, int r0, int k0, int lane, int nrows) {
+  const int row = r0 + (lane & 15);
+  const typename PB::frag f = load8<PB, InT, VEC>(base + (row < nrows ? row : nrows - 1) * rs + k0 + 8 * (lane >> 4));
+  return row < nrows ? f : zero_frag<PB>();
+}
+// Row tile `tile`, tokens k0 + kappa of the transposed input (fp32 fragments).
 template <typename InT>
-__device__ __forceinline__ f32x8 frag_cols_in(const InT* base, int64_t rs, int c0, int k0, int lane, int nrows) {
+__device__ __forceinline__ f32x8 col_frag(const InT* base, int64_t rs, int tile, int k0, int lane, int nrows) {
   f32x8 r;
+  const int f = feature_of(tile, lane & 15);
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
     const int row = k0 + kappa(lane, s);
-    r[s] = row < nrows ? ldx(base + row * rs + c0 + (lane & 15)) : 0.f;
+    r[s] = row < nrows ? ldx(base + row * rs + f) : 0.f;
   }
   return r;
 }
+// B fragments that pick row tile a of a 32-feature block: a row fragment times selector(a) has the
+// accumulator layout of that tile's transpose (the values exactly: one product with 1, the rest with 0).
+template <class PB>
+__device__ __forceinline__ typename PB::frag selector(int a, int lane) {
+  f32x8 e;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) e[s] = ((lane & 15) >> 2) == (lane >> 4) && s == 4 * a + (lane & 3) ? 1.f : 0.f;
+  return PB::from_f32(e);
+}
 
 // ---------------------------------------------------------------------------------------------- prep
-template <class PB, typename InT, int D, int DV, bool BWD = false>
-__global__ void __launch_bounds__(256) gen_prep_kernel(Params p) {
+// grid (nch, H, B), 256 threads.  The features are split over the waves: wave w reads blocks [w D/128,
+// (w+1) D/128) of every row of K and Q once, multiplies what it read (the tiles on and below the
+// diagonal), packs it, and the four waves' partial Grams are added in LDS; reading rows 16w .. instead,
+// every wave read all of K, element by element.  The bound is the traffic: 256 KB in and 128 KB (backward
+// 256 KB) of fragments out per chunk.  2016 chunks, bf16, d_v = 128: 668 -> 284 us, backward 676 -> 442 us (which now
+// also forms R and packs a o dY and Q).
+template <class PB, typename InT, int D, int DV, bool BWD, bool VEC>
+__device__ __forceinline__ void prep_grams(const Params& p, float* rec, const InT* Kin, const InT* Qin, int w, int lane,
+                                           int nrows, f32x4 (&gkk)[10], f32x4 (&gqk)[10]) {
   using R = Rec<D, DV>;
-  constexpr int LDV = DV + 4;
-  __shared__ __attribute__((aligned(16))) float bA[C * LD];
-  __shared__ __attribute__((aligned(16))) float bT[C * LD];
-  __shared__ __attribute__((aligned(16))) float bV[C * LDV];
+  using frag = typename PB::frag;
+  frag* kxf = reinterpret_cast<frag*>(rec + R::KXF);
+  frag* qxf = kxf + 4 * (D / 32) * 64;
+  constexpr int NJ = D / 128;
+  constexpr bool PACKQ = BWD && std::is_same<PB, PrecBF16>::value;
+#pragma unroll
+  for (int t = 0; t < 10; ++t) gkk[t] = gqk[t] = zero4();
+  const InT* kr[4];
+  const InT* qr[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const int row = 16 * m + (lane & 15), rc = row < nrows ? row : nrows - 1;
+    kr[m] = Kin + rc * p.ks1 + 32 * NJ * w + 8 * (lane >> 4);
+    qr[m] = Qin + rc * p.qs1 + 32 * NJ * w + 8 * (lane >> 4);
+  }
+  frag kn[4], qn[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    kn[m] = load8<PB, InT, VEC>(kr[m]);
+    qn[m] = load8<PB, InT, VEC>(qr[m]);
+  }
+#pragma unroll
+  for (int jj = 0; jj < NJ; ++jj) {
+    frag kf[4], qf[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      kf[m] = kn[m];
+      qf[m] = qn[m];
+      if (16 * m + (lane & 15) >= nrows) kf[m] = qf[m] = zero_frag<PB>();
+      if (jj + 1 < NJ) {
+        kn[m] = load8<PB, InT, VEC>(kr[m] + 32 * (jj + 1));
+        qn[m] = load8<PB, InT, VEC>(qr[m] + 32 * (jj + 1));
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      kxf[(m * (D / 32) + NJ * w + jj) * 64 + lane] = kf[m];
+      if constexpr (PACKQ) qxf[(m * (D / 32) + NJ * w + jj) * 64 + lane] = qf[m];
+#pragma unroll
+      for (int n = 0; n <= m; ++n) {
+        gkk[m * (m + 1) / 2 + n] = PB::mma(gkk[m * (m + 1) / 2 + n], kf[m], kf[n]);
+        gqk[m * (m + 1) / 2 + n] = PB::mma(gqk[m * (m + 1) / 2 + n], qf[m], kf[n]);
+      }
+    }
+  }
+}
+
+template <class PB, typename InT, int D, int DV, bool BWD = false>
+__global__ void __launch_bounds__(256) gen_prep_kernel(Params p, BwdP g) {
+  using R = Rec<D, DV>;
+  using BR = BRec<D, DV>;
+  using frag = typename PB::frag;
+  constexpr int LDV = DV + 4, NV = R::NV;
+  constexpr int BUF = C * LD + C * LDV > 40 * 256 ? C * LD + C * LDV : 40 * 256;
+  __shared__ __attribute__((aligned(16))) float bA[C * LD];  // A (as the inverse reads it), then P
+  __shared__ __attribute__((aligned(16))) float buf[BUF];    // partial Grams [wave][tile][lane], then T and the value rows
   __shared__ float s_ell[C], s_beta[C];
+  float* bT = buf;
+  float* bV = buf + C * LD;
 
   const int64_t c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t t0 = c * C;
   float* rec = record<D, DV, BWD>(p, b, h, c);
-  const int r = tid >> 2, part = tid & 3;
-  const bool rvalid = t0 + r < p.T;
+  const int nrows = (int)(p.T - t0 < C ? p.T - t0 : C);
 
   if (w == 0) {
     const int64_t t = t0 + lane;
@@ -148,227 +271,440 @@ __global__ void __launch_bounds__(256) gen_prep_kernel(Params p) {
     }
     s_ell[lane] = l;
     s_beta[lane] = be;
-    rec[R::VEC + lane] = l;
-    rec[R::VEC + 64 + lane] = be;
+    rec[R::V_L + lane] = l;
+    rec[R::V_KAP + lane] = expf(__shfl(l, 63) - l);
+    if constexpr (BWD) rec[BR::V_BETA + lane] = be;
   }
   // the chunk's feature rows, read in place (rows past T read as zero)
-  const int nrows = (int)(p.T - t0 < C ? p.T - t0 : C);
   const InT* Kin = reinterpret_cast<const InT*>(p.k) + b * p.ks0 + t0 * p.ks1 + h * p.ks2;
   const InT* Qin = reinterpret_cast<const InT*>(p.q) + b * p.qs0 + t0 * p.qs1 + h * p.qs2;
-  __syncthreads();
-  // beta o V in LDS
+  f32x4 pt[3];  // this wave's tiles of P (tiles w, w + 4, w + 8 of the ten)
   {
-    const InT* vi = reinterpret_cast<const InT*>(p.v) + b * p.vs0 + (t0 + r) * p.vs1 + h * p.vs2 + part * (DV / 4);
-    const float be = s_beta[r];
+    f32x4 gkk[10], gqk[10];
+    if (p.qkvec) prep_grams<PB, InT, D, DV, BWD, true>(p, rec, Kin, Qin, w, lane, nrows, gkk, gqk);
+    else prep_grams<PB, InT, D, DV, BWD, false>(p, rec, Kin, Qin, w, lane, nrows, gkk, gqk);
+    f32x4* part = reinterpret_cast<f32x4*>(buf);
 #pragma unroll
-    for (int e = 0; e < DV / 4; ++e) bV[r * LDV + part * (DV / 4) + e] = rvalid ? be * ldx(vi + e) : 0.f;
-  }
-  // Grams (row tile w) -> A and P
-  {
-    f32x4 gkk[4], gqk[4];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) gkk[n] = gqk[n] = zero4();
-    for (int jb = 0; jb < D / 32; ++jb) {
-      const f32x8 kw = frag_rows_in(Kin, p.ks1, 16 * w, 32 * jb, lane, nrows);
-      const f32x8 qw = frag_rows_in(Qin, p.qs1, 16 * w, 32 * jb, lane, nrows);
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        const f32x8 kn = frag_rows_in(Kin, p.ks1, 16 * n, 32 * jb, lane, nrows);
-        gkk[n] = mm<PB>(gkk[n], kw, kn);
-        gqk[n] = mm<PB>(gqk[n], qw, kn);
-      }
-    }
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
+    for (int t = 0; t < 10; ++t) part[(w * 10 + t) * 64 + lane] = gkk[t];
+    for (int idx = tid; idx < C * C; idx += 256) bA[idx] = 0.f;
+    __syncthreads();
+    auto reduced = [&](int t) {
+      return ((part[t * 64 + lane] + part[(10 + t) * 64 + lane]) + part[(20 + t) * 64 + lane]) + part[(30 + t) * 64 + lane];
+    };
+    for (int t = w; t < 10; t += 4) {
+      const int m = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3, n = t - m * (m + 1) / 2;
+      const f32x4 s = reduced(t);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int ri = 16 * w + 4 * (lane >> 4) + i, cj = 16 * n + (lane & 15);
-        const float li = s_ell[ri], lj = s_ell[cj], lim1 = ri > 0 ? s_ell[ri - 1] : 0.f;
+        const int ri = 16 * m + 4 * (lane >> 4) + i, cj = 16 * n + (lane & 15);
         // A transposed for the column-oriented inverse: [j][p][s] = A[4s+p][j]
-        bA[(cj * 4 + (ri & 3)) * 16 + (ri >> 2)] = cj < ri ? s_beta[ri] * expf(fminf(li - lj, 0.f)) * gkk[n][i] : 0.f;
-        rec[R::P + ri * C + cj] = cj < ri ? expf(fminf(lim1 - lj, 0.f)) * gqk[n][i] : 0.f;
-        if constexpr (BWD) rec[BRec<D, DV>::G + ri * C + cj] = gkk[n][i];
+        if (cj < ri) bA[(cj * 4 + (ri & 3)) * 16 + (ri >> 2)] = s_beta[ri] * expf(fminf(s_ell[ri] - s_ell[cj], 0.f)) * s[i];
+        if constexpr (BWD) rec[BR::G + ri * C + cj] = s[i];
       }
-  }
-  // K packed in fragment order: wave w the row fragments of feature blocks [w D/128, (w+1) D/128) and
-  // the transposed fragments of feature tiles [w D/64, (w+1) D/64)
-  {
-    using frag = typename PB::frag;
-    frag* kxf = reinterpret_cast<frag*>(rec + R::KXF);
-    frag* ktf = reinterpret_cast<frag*>(rec + R::KTF);
-    for (int jj = 0; jj < D / 128; ++jj) {
-      const int jb = w * (D / 128) + jj;
-#pragma unroll
-      for (int m = 0; m < 4; ++m)
-        kxf[(m * (D / 32) + jb) * 64 + lane] = PB::from_f32(frag_rows_in(Kin, p.ks1, 16 * m, 32 * jb, lane, nrows));
     }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 10; ++t) part[(w * 10 + t) * 64 + lane] = gqk[t];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) pt[k] = w + 4 * k < 10 ? reduced(w + 4 * k) : zero4();
+    __syncthreads();
+  }
+  if constexpr (!std::is_same<PB, PrecBF16>::value) {
+    // fp32 fragments: the transposed operands packed too (wave w the feature tiles [w D/64, (w+1) D/64))
+    frag* ktf = reinterpret_cast<frag*>(rec + R::KTF);
     for (int tt = 0; tt < D / 64; ++tt) {
       const int ft = w * (D / 64) + tt;
 #pragma unroll
-      for (int jb = 0; jb < 2; ++jb)
-        ktf[(ft * 2 + jb) * 64 + lane] = PB::from_f32(frag_cols_in(Kin, p.ks1, 16 * ft, 32 * jb, lane, nrows));
+      for (int jb = 0; jb < 2; ++jb) {
+        ktf[(ft * 2 + jb) * 64 + lane] = PB::from_f32(col_frag(Kin, p.ks1, ft, 32 * jb, lane, nrows));
+        if constexpr (BWD)
+          reinterpret_cast<frag*>(rec + BR::QTF)[(ft * 2 + jb) * 64 + lane] = PB::from_f32(col_frag(Qin, p.qs1, ft, 32 * jb, lane, nrows));
+      }
     }
   }
-  __syncthreads();
-  // T = (I + A)^-1 (column-oriented substitution over lane quads)
+  // beta o V in LDS; T = (I + A)^-1 (column-oriented substitution over lane quads)
+  {
+    const InT* Vin = reinterpret_cast<const InT*>(p.v) + b * p.vs0 + t0 * p.vs1 + h * p.vs2;
+#pragma unroll 8
+    for (int idx = tid; idx < C * DV; idx += 256) {
+      const int r = idx / DV, e = idx % DV;
+      bV[r * LDV + e] = r < nrows ? s_beta[r] * ldx(Vin + r * p.vs1 + e) : 0.f;
+    }
+  }
   unit_lower_inverse(bA, bT, LD, w, lane);
   __syncthreads();
-  for (int idx = tid; idx < C * C; idx += 256) {
-    const int i = idx >> 6, j = idx & 63;
-    rec[R::TP + idx] = bT[i * LD + j] * s_beta[j] * expf(s_ell[j]);
-    if constexpr (BWD) rec[BRec<D, DV>::T + idx] = bT[i * LD + j];
+  // P to LDS (A is used up), zero above its diagonal
+  for (int idx = tid; idx < C * LD; idx += 256) bA[idx] = 0.f;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int t = w + 4 * k;
+    const int m = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3, n = t - m * (m + 1) / 2;
+    if (t < 10) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int ri = 16 * m + 4 * (lane >> 4) + i, cj = 16 * n + (lane & 15);
+        if (cj < ri) bA[ri * LD + cj] = expf(fminf((ri > 0 ? s_ell[ri - 1] : 0.f) - s_ell[cj], 0.f)) * pt[k][i];
+      }
+    }
+  }
+  // Tp (and its transpose) as fragments, T
+#pragma unroll
+  for (int jb = 0; jb < 2; ++jb) {
+    f32x8 f = frag_rows(bT, LD, 16 * w, 32 * jb, lane);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int j = 32 * jb + kappa(lane, s);
+      f[s] = f[s] * s_beta[j] * expf(s_ell[j]);
+    }
+    reinterpret_cast<f32x8*>(rec + R::TPF)[(w * 2 + jb) * 64 + lane] = f;
+    if constexpr (BWD) {
+      const int j = 16 * w + (lane & 15);
+      f32x8 ft = frag_cols(bT, LD, 16 * w, 32 * jb, lane);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) ft[s] = ft[s] * s_beta[j] * expf(s_ell[j]);
+      reinterpret_cast<f32x8*>(rec + BR::TPT)[(w * 2 + jb) * 64 + lane] = ft;
+    }
+  }
+  if constexpr (BWD) {
+    for (int idx = tid; idx < C * C; idx += 256) rec[BR::T + idx] = bT[(idx >> 6) * LD + (idx & 63)];
   }
   // U~ = T (beta o V), row tile w
   {
     const f32x8 ta0 = frag_rows(bT, LD, 16 * w, 0, lane), ta1 = frag_rows(bT, LD, 16 * w, 32, lane);
 #pragma unroll
-    for (int n = 0; n < R::NV; ++n) {
+    for (int n = 0; n < NV; ++n) {
       const f32x4 u = mm<PrecF32>(mm<PrecF32>(zero4(), ta0, frag_cols(bV, LDV, 16 * n, 0, lane)), ta1,
                                   frag_cols(bV, LDV, 16 * n, 32, lane));
-      reinterpret_cast<f32x4*>(rec + R::U)[(w * R::NV + n) * 64 + lane] = u;
+      reinterpret_cast<f32x4*>(rec + R::U)[(w * NV + n) * 64 + lane] = u;
     }
+  }
+  __syncthreads();
+  if constexpr (!BWD) {
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) reinterpret_cast<f32x8*>(rec + R::P)[(w * 2 + jb) * 64 + lane] = frag_rows(bA, LD, 16 * w, 32 * jb, lane);
+  } else {
+    for (int idx = tid; idx < C * C; idx += 256) rec[R::P + idx] = bA[(idx >> 6) * LD + (idx & 63)];
+    if (!g.dy) return;  // the checkpoint pass
+    // R = P^T dY; a o dY as rows and as fragments over tokens and over values
+    const float* Yin = g.dy + b * g.ys0 + t0 * g.ys1 + h * g.ys2;
+#pragma unroll 8
+    for (int idx = tid; idx < C * DV; idx += 256) {
+      const int r = idx / DV, e = idx % DV;
+      bV[r * LDV + e] = r < nrows ? Yin[r * g.ys1 + e] : 0.f;
+    }
+    __syncthreads();
+    const f32x8 pa0 = frag_cols(bA, LD, 16 * w, 0, lane), pa1 = frag_cols(bA, LD, 16 * w, 32, lane);
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      reinterpret_cast<f32x4*>(rec + BR::RR)[(w * NV + n) * 64 + lane] =
+          mm<PrecF32>(mm<PrecF32>(zero4(), pa0, frag_cols(bV, LDV, 16 * n, 0, lane)), pa1, frag_cols(bV, LDV, 16 * n, 32, lane));
+    __syncthreads();
+    for (int idx = tid; idx < C * DV; idx += 256) {
+      const int r = idx / DV, e = idx % DV;
+      const float ay = (r > 0 ? expf(s_ell[r - 1]) : 1.f) * bV[r * LDV + e];
+      bV[r * LDV + e] = ay;
+      rec[BR::AY + idx] = ay;
+    }
+    __syncthreads();
+    frag* ayf = reinterpret_cast<frag*>(rec + BR::AYF);
+    frag* ops = reinterpret_cast<frag*>(rec + BR::OPS);
+#pragma unroll
+    for (int k = 0; k < NV / 2; ++k) {  // NV 2 fragments over tokens: four waves
+      const int f = w * (NV / 2) + k;
+      ayf[f * 64 + lane] = PB::from_f32(frag_cols(bV, LDV, 16 * (f >> 1), 32 * (f & 1), lane));
+    }
+#pragma unroll
+    for (int kb = 0; kb < DV / 32; ++kb) ops[bop_v<DV>(0, w, kb) * 64 + lane] = PB::from_f32(frag_rows(bV, LDV, 16 * w, 32 * kb, lane));
   }
 }
 
 // --------------------------------------------------------------------------------------------- carry
-// grid: 8 * ceil(B*H / 8) * NV workgroups of 256 threads; workgroup (head-batch hb, value tile n), the
-// NV value tiles of a head on one XCD.  Wave w keeps features [w D/4, (w+1) D/4) of its D x 16 slice of
-// S^T in registers.  The chunk-start slice is stored as the B fragments of the output's Q S^T product
-// (the pairs of 16-feature tiles, kdn_frag.hpp) in the policy's fragment type.  With bf16 fragments the
-// next chunk's K-row fragments are loaded one iteration ahead (two register sets).
+// grid: 8 * ceil(B*H / 8) * NV workgroups of CARRY_WAVES waves; workgroup (head-batch hb, value tile n), the
+// NV value tiles of a head on one XCD.  Wave w keeps features [w D/8, (w+1) D/8) of its D x 16 slice of the
+// carried matrix in registers: S^T forward, Gamma = dL/dS^T in reverse (REV, chunks last to first).
+//
+// Per chunk: store the slice; X = K Sigma (partial over the wave's features, reduced through LDS by waves 0..3,
+// one token tile each); forward W = U~ - Tp X and Z = kappa o W, reverse dW = R + kappa o X and Z = -Tp^T dW;
+// Sigma <- g_C Sigma (+ H = Q^T (a o dY)) + K^T Z.
+//
+// What bounds a step: the lines the CU takes from L2 (K 128 KB, in reverse Q likewise) and its three barriers with
+// the 64-deep fp32 product of Tp between them.  With bf16 fragments K^T and Q^T are formed from the rows on
+// the matrix cores, the next chunk's rows are loaded as soon as their registers come free, and waves 4..7 pull
+// later chunks into L2 (as the D = 512 backward's carries do); fp32 fragments, twice the registers, are read
+// where they are used.  32 heads, 63 chunks, bf16, d_v = 128, us per carry: forward 669 -> 280, in the backward
+// (fp32 tiles of S written) 750 -> 359, reverse 1233 -> 534 against four waves that loaded K and K^T where they
+// used them, K^T from memory and, in reverse, H (512 KB a chunk, another 502 us to form) in fp32.
+constexpr int CARRY_WAVES = 8;
+constexpr int CARRY_AHEAD = 3;  // chunks between a step and the operands it pulls into L2
 struct CarryShared {
-  f32x4 xp[4][4][64];
+  f32x4 xp[CARRY_WAVES][4][64];
   f32x4 x[4][64];
   f32x4 z[4][64];
 };
 
-template <class PB, int D>
-struct CarryK {
-  typename PB::frag kx[4][D / 128];
+template <class PB, int D, int DV, bool BWD, bool REV>
+struct CarryOps {
+  using R = Rec<D, DV>;
+  using BR = BRec<D, DV>;
+  using frag = typename PB::frag;
+  static constexpr int NV = DV / 16, JPW = D / 32 / CARRY_WAVES, TPW = 2 * JPW;
+  static constexpr bool KEEP = std::is_same<PB, PrecBF16>::value;
+  frag kx[4][KEEP ? JPW : 1];    // K rows 16m .., features of block JPW w + jj; in reverse then Q's
+  frag kt[KEEP ? TPW : 1][2];    // K^T tile TPW w + t, tokens 32jb ..
+  frag y[2];                     // a o dY (reverse)
+  f32x8 tp[2];                   // waves 0..3: row tile w of Tp or Tp^T
+  f32x4 ur, kap;                 // U~ or R, kappa
+  float l63;
+
+  __device__ __forceinline__ static frag k_frag(const float* rec, int w, int m, int jj, int lane) {
+    return uni(reinterpret_cast<const frag*>(rec + R::KXF) + (m * (D / 32) + JPW * w + jj) * 64)[lane];
+  }
+  __device__ __forceinline__ void load_rows(const float* rec, bool q, int w, int lane) {
+    const frag* f = reinterpret_cast<const frag*>(rec + R::KXF) + (q ? 4 * (D / 32) * 64 : 0);
+#pragma unroll
+    for (int jj = 0; jj < JPW; ++jj)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) kx[m][jj] = uni(f + (m * (D / 32) + JPW * w + jj) * 64)[lane];
+  }
+  // Tile t of the transpose of the rows in kx, tokens 32jb ..
+  __device__ __forceinline__ frag transposed(int t, int jb, const frag (&sel)[2]) const {
+    return PB::from_f32(pair_to8(PB::mma(zero4(), kx[2 * jb][t >> 1], sel[t & 1]), PB::mma(zero4(), kx[2 * jb + 1][t >> 1], sel[t & 1])));
+  }
+  __device__ __forceinline__ void transpose_k(const frag (&sel)[2]) {
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      __builtin_amdgcn_sched_barrier(0);  // four products' results at a time
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) {
+        kt[t][jb] = transposed(t, jb, sel);
+        asm volatile("" : "+v"(kt[t][jb]));  // packed here, not at its use
+      }
+    }
+  }
+  __device__ __forceinline__ void load_y(const float* rec, int n, int lane) {
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) y[jb] = uni(reinterpret_cast<const frag*>(rec + BR::AYF) + (n * 2 + jb) * 64)[lane];
+  }
+  __device__ __forceinline__ void load_lead(const float* rec, int w, int n, int lane) {
+    const f32x8* f = reinterpret_cast<const f32x8*>(rec + (REV ? BR::TPT : R::TPF));
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) tp[jb] = uni(f + (w * 2 + jb) * 64)[lane];
+    ur = uni(reinterpret_cast<const f32x4*>(rec + (REV ? BR::RR : R::U)) + (w * NV + n) * 64)[lane];
+    kap = reinterpret_cast<const f32x4*>(uni(rec + R::V_KAP + 16 * w))[lane >> 4];
+  }
+  __device__ __forceinline__ void load_l63(const float* rec) { l63 = uni(rec + R::V_L + 63)[0]; }
 };
 
-template <class PB, int D, int DV>
-__device__ __forceinline__ void carry_load_kx(CarryK<PB, D>& o, const float* rec, int w, int lane) {
+// One dword of each 128-byte line of a later chunk's operands, shared out over waves 4..7 of the head's NV
+// workgroups: pulls them into the XCD's L2.
+template <class PB, int D, int DV, bool REV>
+struct CarryPrefetch {
   using R = Rec<D, DV>;
-  constexpr int JPW = D / 128;
-  const typename PB::frag* kxf = reinterpret_cast<const typename PB::frag*>(rec + R::KXF);
+  using BR = BRec<D, DV>;
+  static constexpr int LANES = 256 * (DV / 16);
+  static constexpr int AREA = C * D * (int)sizeof(typename PB::frag) / 8 / 128;  // lines of K
+  static constexpr bool BF = std::is_same<PB, PrecBF16>::value;
+  // K rows (bf16, reverse: and Q's behind them; fp32: K^T and in reverse Q^T), Tp, U~ or R, the vectors, a o dY
+  static constexpr int E0 = BF && REV ? 2 * AREA : AREA, E1 = E0 + (BF ? 0 : AREA), E2 = E1 + (!BF && REV ? AREA : 0);
+  static constexpr int E3 = E2 + 128, E4 = E3 + 2 * DV, E5 = E4 + 4;
+  static constexpr int LINES = E5 + (REV ? C * DV * (int)sizeof(typename PB::frag) / 8 / 128 : 0);
+  static constexpr int PER = (LINES + LANES - 1) / LANES;
+  unsigned v[PER];  // the loaded words: used, and so waited for, only where the next step replaces them
+  __device__ __forceinline__ void load(const float* rec, int n, int w, int lane) {
+    const unsigned* r = reinterpret_cast<const unsigned*>(uni(rec));
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
-#pragma unroll
-    for (int jj = 0; jj < JPW; ++jj) o.kx[m][jj] = kxf[(m * (D / 32) + w * JPW + jj) * 64 + lane];
-}
-
-template <class PB, int D, int DV, bool PIPE, bool BWD>
-__device__ __forceinline__ bool carry_step(const Params& p, CarryShared& sh, int64_t b, int64_t h, int64_t c,
-                                           CarryK<PB, D>& cur, CarryK<PB, D>& nxt, f32x4 (&Sg)[D / 64], int w,
-                                           int lane, int n, unsigned& sink) {
-  using R = Rec<D, DV>;
-  using frag = typename PB::frag;
-  constexpr int NV = R::NV, TPW = D / 64, JPW = D / 128;
-  const bool more = c + 1 < p.nch;
-  float* rec = record<D, DV, BWD>(p, b, h, c);
-  const frag* kxf = reinterpret_cast<const frag*>(rec + R::KXF);
-  const f32x8 tp0 = frag_rows(rec + R::TP, C, 16 * w, 0, lane), tp1 = frag_rows(rec + R::TP, C, 16 * w, 32, lane);
-  const f32x4 ur = reinterpret_cast<const f32x4*>(rec + R::U)[(w * NV + n) * 64 + lane];
-  const f32x4 lr = *reinterpret_cast<const f32x4*>(rec + R::VEC + 16 * w + 4 * (lane >> 4));
-  const float l63 = rec[R::VEC + 63];
-  unsigned pf = 0;  // L2-prefetch loads, folded into `sink` at the end of the step
-  if (more) {
-    const float* nrec = record<D, DV, BWD>(p, b, h, c + 1);
-    if constexpr (PIPE) carry_load_kx<PB, D, DV>(nxt, nrec, w, lane);
-    const unsigned* nr = reinterpret_cast<const unsigned*>(nrec);
-    const int idx = n * 256 + (int)threadIdx.x;  // 0 .. 256 NV - 1
-    constexpr int KLINES = D * (int)sizeof(frag) / 16;  // 128-byte lines of one packed K (D/8 fragments)
-    for (int l = idx; l < KLINES; l += 256 * NV) {
-      pf += nr[R::KTF + 32 * l];
-      if constexpr (!PIPE) pf += nr[R::KXF + 32 * l];
+    for (int k = 0; k < PER; ++k) {
+      const int i = (n * 4 + (w - 4)) * 64 + lane + LANES * k;
+      unsigned at = R::VEC;
+      if (i < E0) at = R::KXF + 32 * i;
+      else if (i < E1) at = R::KTF + 32 * (i - E0);
+      else if (i < E2) at = BR::QTF + 32 * (i - E1);
+      else if (i < E3) at = (REV ? BR::TPT : R::TPF) + 32 * (i - E2);
+      else if (i < E4) at = (REV ? BR::RR : R::U) + 32 * (i - E3);
+      else if (i < E5) at = R::VEC + 32 * (i - E4);
+      else if (REV && i < LINES) at = BR::AYF + 32 * (i - E5);
+      v[k] = r[at];
     }
-    if (idx < 128) pf += nr[R::TP + 32 * idx];                       // 128 lines of Tp
-    else if (idx < 128 + 2 * DV) pf += nr[R::U + 32 * (idx - 128)];  // 2 DV lines of U~
   }
+};
 
-  // store the chunk-start slice (as output fragments) and form K times it, partial over this wave's features
-  // (the backward's recompute keeps the slice in fp32 rows instead: no output kernel reads the fragments)
-  if constexpr (BWD) {  // value-major rows: a lane's four features are one 16-byte store
-    float* srow = rec + BRec<D, DV>::SR + (int64_t)(16 * n + (lane & 15)) * D + (D / 4) * w + 4 * (lane >> 4);
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) *reinterpret_cast<f32x4*>(srow + 16 * t) = Sg[t];
-  }
-  frag* sf = reinterpret_cast<frag*>(rec + R::S);
+// `lead`: waves 0..3, which reduce X and take the Tp product, and so transpose K before the first barrier; the others
+// transpose it while those work.  The two run their own loops (one loop with both paths does not fit the registers).
+template <class PB, int D, int DV, bool BWD, bool REV, bool lead>
+__device__ __forceinline__ void carry_step(CarryShared& sh, float* rec, const float* nrec, const float* frec,
+                                           CarryOps<PB, D, DV, BWD, REV>& o, CarryPrefetch<PB, D, DV, REV>& pf, unsigned& sink,
+                                           f32x4 (&Sg)[D / 16 / CARRY_WAVES], const typename PB::frag (&sel)[2], int w,
+                                           int lane, int n) {
+  using O = CarryOps<PB, D, DV, BWD, REV>;
+  using R = Rec<D, DV>;
+  using BR = BRec<D, DV>;
+  using frag = typename PB::frag;
+  constexpr int NV = O::NV, JPW = O::JPW, TPW = O::TPW;
+  constexpr bool KEEP = O::KEEP;
+  const int row0 = 16 * w + 4 * (lane >> 4), vc = 16 * n + (lane & 15);  // a lead wave's rows and column
+  // K times the carried slice, partial over this wave's features
   f32x4 xp[4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m) xp[m] = zero4();
+  frag sb[JPW];
 #pragma unroll
   for (int jj = 0; jj < JPW; ++jj) {
-    const frag sb = PB::from_f32(pair_to8(Sg[2 * jj], Sg[2 * jj + 1]));
-    if constexpr (!BWD) sf[((w * JPW + jj) * NV + n) * 64 + lane] = sb;
+    sb[jj] = PB::from_f32(pair_to8(Sg[2 * jj], Sg[2 * jj + 1]));
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
-      xp[m] = PB::mma(xp[m], PIPE ? cur.kx[m][jj] : kxf[(m * (D / 32) + w * JPW + jj) * 64 + lane], sb);
+    for (int m = 0; m < 4; ++m) {
+      if constexpr (KEEP) xp[m] = PB::mma(jj ? xp[m] : zero4(), o.kx[m][jj], sb[jj]);
+      else xp[m] = PB::mma(jj ? xp[m] : zero4(), O::k_frag(rec, w, m, jj, lane), sb[jj]);
+    }
   }
 #pragma unroll
   for (int m = 0; m < 4; ++m) sh.xp[w][m][lane] = xp[m];
-  const float gC = expf(l63);
+  __builtin_amdgcn_sched_barrier(0);
+  // the slice to the record: fp32 tiles (backward), output fragments (forward)
+  if constexpr (BWD) {
+    f32x4* dst = reinterpret_cast<f32x4*>(rec + (REV ? BR::GR : BR::SR));
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) uni(dst + (n * (D / 16) + TPW * w + t) * 64)[lane] = Sg[t];
+  } else {
+    frag* sf = reinterpret_cast<frag*>(rec + R::S);
+#pragma unroll
+    for (int jj = 0; jj < JPW; ++jj) uni(sf + ((JPW * w + jj) * NV + n) * 64)[lane] = sb[jj];
+  }
+  const float gC = expf(o.l63);
 #pragma unroll
   for (int t = 0; t < TPW; ++t) Sg[t] = Sg[t] * gC;
-  __syncthreads();
-  // K^T fragments for the update, issued now (bf16: 128 registers) so that they arrive during the W / Z
-  // phase; fp32 fragments are read where the update consumes them
-  constexpr bool EARLY = std::is_same<PB, PrecBF16>::value;
-  const frag* ktf = reinterpret_cast<const frag*>(rec + R::KTF);
-  frag kt[EARLY ? TPW : 1][2];
-  if constexpr (EARLY) {
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-      for (int jb = 0; jb < 2; ++jb) kt[t][jb] = ktf[((w * TPW + t) * 2 + jb) * 64 + lane];
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (KEEP && lead) {
+    o.transpose_k(sel);
+    __builtin_amdgcn_sched_barrier(0);
+    o.load_rows(REV ? rec : nrec, REV, w, lane);
   }
-  const f32x4 X = sh.xp[0][w][lane] + sh.xp[1][w][lane] + sh.xp[2][w][lane] + sh.xp[3][w][lane];
-  sh.x[w][lane] = X;
-  if constexpr (BWD) {
+  o.load_l63(nrec);
+  lds_barrier();
+  if constexpr (lead) {
+    f32x4 X = sh.xp[0][w][lane];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) rec[BRec<D, DV>::XK + (16 * w + 4 * (lane >> 4) + i) * DV + 16 * n + (lane & 15)] = X[i];
-  }
-  __syncthreads();
-  f32x4 tx = mm<PrecF32>(zero4(), tp0, pair_to8(sh.x[0][lane], sh.x[1][lane]));
-  tx = mm<PrecF32>(tx, tp1, pair_to8(sh.x[2][lane], sh.x[3][lane]));
-  const f32x4 Wt = ur - tx;
-  const int vc = 16 * n + (lane & 15);
-  f32x4 kap;
+    for (int v = 1; v < CARRY_WAVES; ++v) X += sh.xp[v][w][lane];
+    if constexpr (!REV) {
+      sh.x[w][lane] = X;
+      if constexpr (BWD) {
+        float* d = uni(rec + BR::XK);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    rec[R::W + (16 * w + 4 * (lane >> 4) + i) * DV + vc] = Wt[i];
-    kap[i] = expf(l63 - lr[i]);
+        for (int i = 0; i < 4; ++i) d[(row0 + i) * DV + vc] = X[i];
+      }
+    } else {
+      const f32x4 dW = o.ur + o.kap * X;
+      sh.x[w][lane] = dW;
+      float* dx = uni(rec + BR::X);
+      float* dd = uni(rec + BR::DW);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dx[(row0 + i) * DV + vc] = X[i];
+        dd[(row0 + i) * DV + vc] = dW[i];
+      }
+      uni(reinterpret_cast<f32x4*>(rec + BR::DWT) + (w * NV + n) * 64)[lane] = dW;
+    }
+  } else if constexpr (KEEP) {
+    o.transpose_k(sel);
+    __builtin_amdgcn_sched_barrier(0);
+    o.load_rows(REV ? rec : nrec, REV, w, lane);
   }
-  sh.z[w][lane] = kap * Wt;
-  __syncthreads();
+  lds_barrier();
+  if constexpr (lead) {
+    const f32x4 t = mm<PrecF32>(mm<PrecF32>(zero4(), o.tp[0], pair_to8(sh.x[0][lane], sh.x[1][lane])), o.tp[1],
+                                pair_to8(sh.x[2][lane], sh.x[3][lane]));
+    if constexpr (!REV) {
+      const f32x4 Wt = o.ur - t;
+      sh.z[w][lane] = o.kap * Wt;
+      if constexpr (BWD) {
+        float* d = uni(rec + R::W);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[(row0 + i) * DV + vc] = Wt[i];
+      } else {
+        uni(reinterpret_cast<f32x4*>(rec + R::W) + (w * NV + n) * 64)[lane] = Wt;
+      }
+    } else {
+      sh.z[w][lane] = -t;
+      float* d = uni(rec + BR::ZN);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) d[(row0 + i) * DV + vc] = -t[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    o.load_lead(nrec, w, n, lane);
+  } else if (frec) {
+#pragma unroll
+    for (int k = 0; k < CarryPrefetch<PB, D, DV, REV>::PER; ++k) sink ^= pf.v[k];
+    pf.load(frec, n, w, lane);
+  }
+  if constexpr (REV) {
+    // this wave's rows of H = Q^T (a o dY) for value tile n
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      if constexpr (KEEP) {
+        __builtin_amdgcn_sched_barrier(0);
+        Sg[t] = PB::mma(PB::mma(Sg[t], o.transposed(t, 0, sel), o.y[0]), o.transposed(t, 1, sel), o.y[1]);
+      } else {
+        const frag* qtf = reinterpret_cast<const frag*>(rec + BR::QTF) + (TPW * w + t) * 2 * 64;
+        Sg[t] = PB::mma(PB::mma(Sg[t], uni(qtf)[lane], o.y[0]), uni(qtf + 64)[lane], o.y[1]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    o.load_y(nrec, n, lane);
+    if constexpr (KEEP) o.load_rows(nrec, false, w, lane);
+  }
+  lds_barrier();
   const frag zb0 = PB::from_f32(pair_to8(sh.z[0][lane], sh.z[1][lane]));
   const frag zb1 = PB::from_f32(pair_to8(sh.z[2][lane], sh.z[3][lane]));
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
-    if constexpr (EARLY) {
-      Sg[t] = PB::mma(PB::mma(Sg[t], kt[t][0], zb0), kt[t][1], zb1);
+    if constexpr (KEEP) {
+      Sg[t] = PB::mma(PB::mma(Sg[t], o.kt[t][0], zb0), o.kt[t][1], zb1);
     } else {
-      Sg[t] = PB::mma(PB::mma(Sg[t], ktf[((w * TPW + t) * 2) * 64 + lane], zb0), ktf[((w * TPW + t) * 2 + 1) * 64 + lane],
-                      zb1);
+      const frag* ktf = reinterpret_cast<const frag*>(rec + R::KTF) + (TPW * w + t) * 2 * 64;
+      Sg[t] = PB::mma(PB::mma(Sg[t], uni(ktf)[lane], zb0), uni(ktf + 64)[lane], zb1);
     }
   }
-  sink += pf;
-  return more;
 }
 
-template <class PB, int D, int DV, bool BWD = false>
-__global__ void __launch_bounds__(256) gen_carry_kernel(Params p) {
-  using R = Rec<D, DV>;
-  constexpr int NV = R::NV, FPW = D / 4, TPW = FPW / 16;
-  constexpr bool PIPE = false;  // two register sets of 32 K fragments do not fit beside the D = 1024 slice
+template <class PB, int D, int DV, bool BWD, bool REV, bool lead>
+__device__ __forceinline__ void carry_loop(CarryShared& sh, const Params& p, int b, int h, int nch, f32x4 (&Sg)[D / 16 / CARRY_WAVES],
+                                           const typename PB::frag (&sel)[2], int w, int lane, int n, unsigned& sink) {
+  using O = CarryOps<PB, D, DV, BWD, REV>;
+  O o;
+  {
+    const float* rec = record<D, DV, BWD>(p, b, h, REV ? nch - 1 : 0);
+    if constexpr (O::KEEP) o.load_rows(rec, false, w, lane);
+    o.load_l63(rec);
+    if constexpr (lead) o.load_lead(rec, w, n, lane);
+    if constexpr (REV) o.load_y(rec, n, lane);
+  }
+  CarryPrefetch<PB, D, DV, REV> pf = {};
+  for (int step = 0; step < nch; ++step) {
+    const int c = REV ? nch - 1 - step : step;
+    const int cn = step + 1 < nch ? (REV ? c - 1 : c + 1) : c;  // the last step loads its own chunk again
+    const int cf = REV ? c - CARRY_AHEAD : c + CARRY_AHEAD;
+    carry_step<PB, D, DV, BWD, REV, lead>(sh, record<D, DV, BWD>(p, b, h, c), record<D, DV, BWD>(p, b, h, cn),
+                                          cf >= 0 && cf < nch ? record<D, DV, BWD>(p, b, h, cf) : nullptr, o, pf, sink, Sg, sel, w,
+                                          lane, n);
+  }
+}
+
+// The carried slice from / to a caller's state (NULL: zero / nothing).  In reverse over segments source and
+// destination may be the same buffer: a thread rewrites exactly the elements it read.
+template <class PB, int D, int DV, bool BWD, bool REV>
+__global__ void __launch_bounds__(64 * CARRY_WAVES) gen_carry_kernel(Params p, const float* src, int64_t s0, int64_t s1, int64_t s2,
+                                                                   int64_t s3, float* dst, int64_t o0, int64_t o1, int64_t o2,
+                                                                   int64_t o3) {
+  using O = CarryOps<PB, D, DV, BWD, REV>;
+  constexpr int NV = O::NV, TPW = O::TPW;
   __shared__ CarryShared sh;
   const int64_t id = blockIdx.x;
   const int64_t xcd = id & 7, jdx = id >> 3;
   const int n = (int)(jdx % NV);
   const int64_t hb = (jdx / NV) * 8 + xcd;
   if (hb >= p.B * p.H) return;
-  const int64_t b = hb / p.H, h = hb % p.H;
+  // the division is done in vector registers: back to scalars, so that every record address is one
+  const int b = __builtin_amdgcn_readfirstlane((int)(hb / p.H));
+  const int h = (int)hb - b * (int)p.H;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int vc = 16 * n + (lane & 15);
@@ -377,35 +713,51 @@ __global__ void __launch_bounds__(256) gen_carry_kernel(Params p) {
 #pragma unroll
   for (int t = 0; t < TPW; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int f = FPW * w + 16 * t + 4 * (lane >> 4) + i;
-      Sg[t][i] = p.init ? p.init[b * p.is0 + h * p.is1 + f * p.is2 + vc * p.is3] : 0.f;
-    }
-  unsigned sink = 0;  // keeps the L2 prefetch loads alive (never stored: nch is positive)
-  CarryK<PB, D> ka, kb;
-  if constexpr (PIPE) carry_load_kx<PB, D, DV>(ka, record<D, DV, BWD>(p, b, h, 0), w, lane);
-  for (int64_t c = 0;; c += 2) {
-    if (!carry_step<PB, D, DV, PIPE, BWD>(p, sh, b, h, c, ka, kb, Sg, w, lane, n, sink)) break;
-    if (!carry_step<PB, D, DV, PIPE, BWD>(p, sh, b, h, c + 1, kb, ka, Sg, w, lane, n, sink)) break;
-  }
+    for (int i = 0; i < 4; ++i)
+      Sg[t][i] = src ? src[b * s0 + h * s1 + feature_of(TPW * w + t, 4 * (lane >> 4) + i) * s2 + vc * s3] : 0.f;
+  const typename PB::frag sel[2] = {selector<PB>(0, lane), selector<PB>(1, lane)};
+  const int nch = (int)p.nch;
+  unsigned sink = 0;  // keeps the prefetch loads alive (never stored: nch is positive)
+  if (w < 4) carry_loop<PB, D, DV, BWD, REV, true>(sh, p, b, h, nch, Sg, sel, w, lane, n, sink);
+  else carry_loop<PB, D, DV, BWD, REV, false>(sh, p, b, h, nch, Sg, sel, w, lane, n, sink);
   if (p.nch < 0) p.ws[0] = (float)sink;
+  if (dst) {
 #pragma unroll
-  for (int t = 0; t < TPW; ++t)
+    for (int t = 0; t < TPW; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int f = FPW * w + 16 * t + 4 * (lane >> 4) + i;
-      p.fin[b * p.fs0 + h * p.fs1 + f * p.fs2 + vc * p.fs3] = Sg[t][i];
-    }
+      for (int i = 0; i < 4; ++i) dst[b * o0 + h * o1 + feature_of(TPW * w + t, 4 * (lane >> 4) + i) * o2 + vc * o3] = Sg[t][i];
+  }
 }
 
 // -------------------------------------------------------------------------------------------- output
-// grid (nch, H, B), 256 threads; wave w the 16 tokens of tile w, every value tile.
+// grid (nch, H, B), 256 threads; wave w the token tiles 2 (w & 1), 2 (w & 1) + 1 and half the value tiles, so that
+// both operands are read twice (token tile w with every value tile: S four times).  Computed transposed
+// (values in the rows), which puts four consecutive values of a token in a lane.
 template <typename T>
 __device__ __forceinline__ void store_el(T* p, float v);
 template <>
 __device__ __forceinline__ void store_el<float>(float* p, float v) { *p = v; }
 template <>
 __device__ __forceinline__ void store_el<__bf16>(__bf16* p, float v) { *p = (__bf16)v; }
+
+template <class PB, typename InT, int D, int DV, bool VEC>
+__device__ __forceinline__ void output_qs(const Params& p, const float* rec, const InT* Qin, int m0, int n0, int lane, int nrows,
+                                          f32x4 (&acc)[DV / 32][2]) {
+  constexpr int NV = DV / 16;
+  const typename PB::frag* sf = reinterpret_cast<const typename PB::frag*>(rec + Rec<D, DV>::S);
+#pragma unroll 4
+  for (int jb = 0; jb < D / 32; ++jb) {
+    typename PB::frag q[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) q[k] = row_frag<PB, InT, VEC>(Qin, p.qs1, 16 * (m0 + k), 32 * jb, lane, nrows);
+#pragma unroll
+    for (int n = 0; n < NV / 2; ++n) {
+      const typename PB::frag s = sf[(jb * NV + n0 + n) * 64 + lane];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) acc[n][k] = PB::mma(acc[n][k], s, q[k]);
+    }
+  }
+}
 
 template <class PB, typename InT, typename OutT, int D, int DV>
 __global__ void __launch_bounds__(256) gen_output_kernel(Params p) {
@@ -414,45 +766,59 @@ __global__ void __launch_bounds__(256) gen_output_kernel(Params p) {
   const int64_t c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = 2 * (w & 1), n0 = (w >> 1) * (NV / 2);
   const int64_t t0 = c * C;
   const float* rec = record<D, DV>(p, b, h, c);
   const int nrows = (int)(p.T - t0 < C ? p.T - t0 : C);
   const InT* Qin = reinterpret_cast<const InT*>(p.q) + b * p.qs0 + t0 * p.qs1 + h * p.qs2;
-  f32x4 qs[NV];
+  f32x4 acc[NV / 2][2];
 #pragma unroll
-  for (int n = 0; n < NV; ++n) qs[n] = zero4();
-  const typename PB::frag* sf = reinterpret_cast<const typename PB::frag*>(rec + R::S);
-  for (int jb = 0; jb < D / 32; ++jb) {
-    const typename PB::frag qa = PB::from_f32(frag_rows_in(Qin, p.qs1, 16 * w, 32 * jb, lane, nrows));
+  for (int n = 0; n < NV / 2; ++n) acc[n][0] = acc[n][1] = zero4();
+  if (p.qkvec) output_qs<PB, InT, D, DV, true>(p, rec, Qin, m0, n0, lane, nrows, acc);
+  else output_qs<PB, InT, D, DV, false>(p, rec, Qin, m0, n0, lane, nrows, acc);
+  const f32x8* pf = reinterpret_cast<const f32x8*>(rec + R::P);
+  const f32x4* wt = reinterpret_cast<const f32x4*>(rec + R::W);
+  OutT* y = reinterpret_cast<OutT*>(p.y) + b * p.ys0 + h * p.ys2;
 #pragma unroll
-    for (int n = 0; n < NV; ++n) qs[n] = PB::mma(qs[n], qa, sf[(jb * NV + n) * 64 + lane]);
-  }
-  const f32x8 p0 = frag_rows(rec + R::P, C, 16 * w, 0, lane), p1 = frag_rows(rec + R::P, C, 16 * w, 32, lane);
-  f32x4 a;
+  for (int k = 0; k < 2; ++k) {
+    const f32x8 p0 = pf[((m0 + k) * 2) * 64 + lane], p1 = pf[((m0 + k) * 2 + 1) * 64 + lane];
+    const int64_t t = t0 + 16 * (m0 + k) + (lane & 15);
+    const int ri = 16 * (m0 + k) + (lane & 15);
+    const float a = ri > 0 ? expf(rec[R::V_L + ri - 1]) : 1.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int ri = 16 * w + 4 * (lane >> 4) + i;
-    a[i] = ri > 0 ? expf(rec[R::VEC + ri - 1]) : 1.f;
-  }
-  OutT* y = reinterpret_cast<OutT*>(p.y);
+    for (int n = 0; n < NV / 2; ++n) {
+      auto tile = [&](int m) { return wt[(m * NV + n0 + n) * 64 + lane]; };
+      const f32x4 pw = mm<PrecF32>(mm<PrecF32>(zero4(), pair_to8(tile(0), tile(1)), p0), pair_to8(tile(2), tile(3)), p1);
+      const f32x4 r = a * acc[n][k] + pw;
+      if (t < p.T) {
+        OutT* d = y + t * p.ys1 + 16 * (n0 + n) + 4 * (lane >> 4);
+        if (p.yvec) {
+          typedef __attribute__((ext_vector_type(4))) OutT out4;
+          out4 o;
 #pragma unroll
-  for (int n = 0; n < NV; ++n) {
-    const f32x4 pw = mm<PrecF32>(mm<PrecF32>(zero4(), p0, frag_cols(rec + R::W, DV, 16 * n, 0, lane)), p1,
-                                 frag_cols(rec + R::W, DV, 16 * n, 32, lane));
+          for (int i = 0; i < 4; ++i) o[i] = (OutT)r[i];
+          *reinterpret_cast<out4*>(d) = o;
+        } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t t = t0 + 16 * w + 4 * (lane >> 4) + i;
-      if (t < p.T) store_el<OutT>(y + b * p.ys0 + t * p.ys1 + h * p.ys2 + 16 * n + (lane & 15), a[i] * qs[n][i] + pw[i]);
+          for (int i = 0; i < 4; ++i) store_el<OutT>(d + i, r[i]);
+        }
+      }
     }
   }
+}
+
+template <class PB, int D, int DV, bool BWD>
+static void launch_carry(const Params& p, hipStream_t st) {
+  const unsigned wgs = (unsigned)(((p.B * p.H + 7) / 8) * 8 * (DV / 16));
+  hipLaunchKernelGGL((gen_carry_kernel<PB, D, DV, BWD, false>), dim3(wgs), dim3(64 * CARRY_WAVES), 0, st, p, p.init, p.is0, p.is1,
+                     p.is2, p.is3, p.fin, p.fs0, p.fs1, p.fs2, p.fs3);
 }
 
 template <class PB, typename InT, typename OutT, int D, int DV>
 static int launch(const Params& p, hipStream_t st) {
   const dim3 chunk_grid((unsigned)p.nch, (unsigned)p.H, (unsigned)p.B);
-  const unsigned carry_wgs = (unsigned)(((p.B * p.H + 7) / 8) * 8 * (DV / 16));
-  hipLaunchKernelGGL((gen_prep_kernel<PB, InT, D, DV>), chunk_grid, dim3(256), 0, st, p);
-  hipLaunchKernelGGL((gen_carry_kernel<PB, D, DV>), dim3(carry_wgs), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((gen_prep_kernel<PB, InT, D, DV>), chunk_grid, dim3(256), 0, st, p, BwdP{});
+  launch_carry<PB, D, DV, false>(p, st);
   hipLaunchKernelGGL((gen_output_kernel<PB, InT, OutT, D, DV>), chunk_grid, dim3(256), 0, st, p);
   return launch_status();
 }
@@ -478,202 +844,32 @@ static size_t record_floats(int D, int DV) {
 // gradients of a loss with respect to phi_q, phi_k, v, beta, lambda and the initial state, given dL/dy
 // and dL/d(final state).  The closed form per chunk is that of the D = 512 backward (kdn_bwd.hip), with
 // one record per (batch, head, chunk) for the whole sequence:
-//   prep, carry (the forward's kernels)  T, K K^T, Tp, P, U~, W; S^T at every chunk start, X_K = K S^T
-//   rh      (parallel)                   R = P^T dY, H = Q^T (a o dY)
-//   rchain  (sequential, reversed)       Gamma = dL/dS^T at every chunk end, X = K Gamma,
+//   prep, carry (the forward's kernels)  T, K K^T, Tp, P, U~, W; S^T at every chunk start, X_K = K S^T; and
+//                                        R = P^T dY, a o dY
+//   reverse carry (sequential)           Gamma = dL/dS^T at every chunk end, X = K Gamma, H = Q^T (a o dY),
 //                                        dW = R + kappa o X, Z = Tp^T dW, Gamma <- g_C Gamma + H - K^T Z
-//   grad    (parallel)                   dv, dbeta, dlambda; the left operands of the feature gradients
+//   grad    (parallel)                   dv, dbeta, the terms of dlambda without S; the right operands of the
+//                                        feature gradients
 //   dphi    (parallel, 256 features per workgroup)
-//                                        dphi_q = (a o dY) S + N K
-//                                        dphi_k = (kappa o W) Gamma^T - Z S + (M + M^T) K + N^T Q
+//                                        dphi_q^T = S^T (a o dY)^T + K^T N^T
+//                                        dphi_k^T = Gamma (kappa o W)^T - S^T Z^T + K^T (M + M^T) + Q^T N
+//                                        and the terms of dlambda with S, a o dY . Q S^T and <Gamma, S>, in partial sums
+//   decay   (parallel)                   dlambda, where it is wanted
 // with S the chunk-start state as the recurrence's d_v x D matrix (the carries hold S^T, D x d_v),
 // N_ij = dP_ij g_{i-1}/g_j and M_ij = dA_ij beta_i g_i/g_j below the diagonal, dP = dY W^T and
-// dA = -T^T dT T^T.
+// dA = -T^T dT T^T.  S and Gamma, 512 KB each per chunk in fp32, are most of the backward's traffic: each is
+// written once, in the accumulators' own tiles, and read once.
 // The contractions that involve the features (the carries, H, Q S^T and the feature gradients) take the
 // forward's precision policy (bf16 operands with fp32 accumulation for bf16 inputs, as the D = 512
 // backward); the 64 x 64 chunk algebra runs on fp32 MFMA.  Every reduction has a fixed order (no
 // atomics).
 
-struct BwdP {
-  const float* dy; int64_t ys0, ys1, ys2;
-  const float* dfin; int64_t fs0, fs1, fs2, fs3;  // dL/dS^T at the end (NULL: zero)
-  float* dq; int64_t dqs0, dqs1, dqs2;
-  float* dk; int64_t dks0, dks1, dks2;
-  float* dv; int64_t dvs0, dvs1, dvs2;
-  float* dbeta; int64_t dbs0, dbs1, dbs2;
-  float* ddecay; int64_t dds0, dds1, dds2;        // NULL: not wanted
-  float* dinit; int64_t gis0, gis1, gis2, gis3;   // dL/dS^T at the start (NULL: not wanted)
-};
-
-// ------------------------------------------------------------------------------------------------ rh
-// grid (nch, H, B), 256 threads.  Wave w: rows 16w .. of R, feature tiles [w D/64, (w+1) D/64) of H.
-template <class PB, typename InT, int D, int DV>
-__global__ void __launch_bounds__(256) gbwd_rh_kernel(Params p, BwdP g) {
-  using F = Rec<D, DV>;
-  using R = BRec<D, DV>;
-  constexpr int LDV = DV + 4, NV = DV / 16;
-  __shared__ __attribute__((aligned(16))) float bY[C * LDV];   // dY
-  __shared__ __attribute__((aligned(16))) float bAY[C * LDV];  // a o dY
-  const int64_t c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t t0 = c * C;
-  float* rec = record<D, DV, true>(p, b, h, c);
-  const int nrows = (int)(p.T - t0 < C ? p.T - t0 : C);
-  for (int idx = tid; idx < C * DV; idx += 256) {
-    const int r = idx / DV, v = idx % DV;
-    const float y = r < nrows ? g.dy[b * g.ys0 + (t0 + r) * g.ys1 + h * g.ys2 + v] : 0.f;
-    const float ay = (r > 0 ? expf(rec[F::VEC + r - 1]) : 1.f) * y;
-    bY[r * LDV + v] = y;
-    bAY[r * LDV + v] = ay;
-    rec[R::AY + idx] = ay;
-  }
-  __syncthreads();
-  const f32x8 pa0 = frag_cols(rec + F::P, C, 16 * w, 0, lane), pa1 = frag_cols(rec + F::P, C, 16 * w, 32, lane);
-#pragma unroll
-  for (int n = 0; n < NV; ++n) {
-    const f32x4 rr = mm<PrecF32>(mm<PrecF32>(zero4(), pa0, frag_cols(bY, LDV, 16 * n, 0, lane)), pa1,
-                                 frag_cols(bY, LDV, 16 * n, 32, lane));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rec[R::RR + (16 * w + 4 * (lane >> 4) + i) * DV + 16 * n + (lane & 15)] = rr[i];
-  }
-  const InT* Qin = reinterpret_cast<const InT*>(p.q) + b * p.qs0 + t0 * p.qs1 + h * p.qs2;
-  for (int tt = 0; tt < D / 64; ++tt) {
-    const int ft = w * (D / 64) + tt;
-    const typename PB::frag q0 = PB::from_f32(frag_cols_in(Qin, p.qs1, 16 * ft, 0, lane, nrows));
-    const typename PB::frag q1 = PB::from_f32(frag_cols_in(Qin, p.qs1, 16 * ft, 32, lane, nrows));
-#pragma unroll
-    for (int n = 0; n < NV; ++n) {
-      const f32x4 hv = PB::mma(PB::mma(zero4(), q0, PB::from_f32(frag_cols(bAY, LDV, 16 * n, 0, lane))), q1,
-                               PB::from_f32(frag_cols(bAY, LDV, 16 * n, 32, lane)));
-      *reinterpret_cast<f32x4*>(rec + R::H1 + (int64_t)(16 * n + (lane & 15)) * D + 16 * ft + 4 * (lane >> 4)) = hv;
-    }
-  }
-}
-
-// -------------------------------------------------------------------------------------------- rchain
-// grid as gen_carry_kernel: workgroup (head-batch hb, value tile n); wave w keeps features
-// [w D/4, (w+1) D/4) of its D x 16 slice of Gamma = dL/dS^T in registers, chunks last to first.
-template <class PB, int D, int DV>
-__global__ void __launch_bounds__(256) gbwd_rchain_kernel(Params p, BwdP g) {
-  using F = Rec<D, DV>;
-  using R = BRec<D, DV>;
-  using frag = typename PB::frag;
-  constexpr int NV = DV / 16, FPW = D / 4, TPW = FPW / 16, JPW = D / 128;
-  __shared__ CarryShared sh;
-  const int64_t id = blockIdx.x;
-  const int64_t xcd = id & 7, jdx = id >> 3;
-  const int n = (int)(jdx % NV);
-  const int64_t hb = (jdx / NV) * 8 + xcd;
-  if (hb >= p.B * p.H) return;
-  const int64_t b = hb / p.H, h = hb % p.H;
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int vc = 16 * n + (lane & 15);
-
-  f32x4 Gg[TPW];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int f = FPW * w + 16 * t + 4 * (lane >> 4) + i;
-      Gg[t][i] = g.dfin ? g.dfin[b * g.fs0 + h * g.fs1 + f * g.fs2 + vc * g.fs3] : 0.f;
-    }
-  unsigned sink = 0;  // keeps the L2-prefetch loads alive (never stored: nch is positive)
-  for (int64_t c = p.nch - 1; c >= 0; --c) {
-    float* rec = record<D, DV, true>(p, b, h, c);
-    const frag* kxf = reinterpret_cast<const frag*>(rec + F::KXF);
-    const frag* ktf = reinterpret_cast<const frag*>(rec + F::KTF);
-    const float l63 = rec[F::VEC + 63];
-    if (c > 0) {
-      // touch the previous chunk's operands so that its loads hit L2: the packed K (lines shared by the
-      // head's NV workgroups), Tp, P^T dY and this workgroup's 16 rows of H (one dword per 128-byte line)
-      const unsigned* pr = reinterpret_cast<const unsigned*>(record<D, DV, true>(p, b, h, c - 1));
-      const int idx = n * 256 + (int)threadIdx.x;
-      constexpr int KLINES = D * (int)sizeof(frag) / 16;
-      for (int l = idx; l < KLINES; l += 256 * NV) sink += pr[F::KXF + 32 * l] + pr[F::KTF + 32 * l];
-      if (idx < 128) sink += pr[F::TP + 32 * idx];
-      else if (idx < 128 + 2 * DV) sink += pr[R::RR + 32 * (idx - 128)];
-      for (int l = (int)threadIdx.x; l < 16 * D / 32; l += 256)
-        sink += pr[R::H1 + (int64_t)(16 * n + l / (D / 32)) * D + 32 * (l % (D / 32))];
-    }
-    const f32x4 lr = *reinterpret_cast<const f32x4*>(rec + F::VEC + 16 * w + 4 * (lane >> 4));
-    // the step's small operands and this wave's rows of H, issued first so that their latency overlaps
-    // the K Gamma products instead of following the last barrier
-    float* grow = rec + R::GR + (int64_t)vc * D + FPW * w + 4 * (lane >> 4);
-    const float* hrow = rec + R::H1 + (int64_t)vc * D + FPW * w + 4 * (lane >> 4);
-    f32x4 hv[TPW];
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) hv[t] = *reinterpret_cast<const f32x4*>(hrow + 16 * t);
-    const f32x8 ta0 = frag_cols(rec + F::TP, C, 16 * w, 0, lane), ta1 = frag_cols(rec + F::TP, C, 16 * w, 32, lane);
-    f32x4 rr;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rr[i] = rec[R::RR + (16 * w + 4 * (lane >> 4) + i) * DV + vc];
-    // Gamma at the chunk end; K Gamma, partial over this wave's features
-    f32x4 xp[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) xp[m] = zero4();
-#pragma unroll
-    for (int jj = 0; jj < JPW; ++jj) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) *reinterpret_cast<f32x4*>(grow + 16 * (2 * jj + u)) = Gg[2 * jj + u];
-      const frag gb = PB::from_f32(pair_to8(Gg[2 * jj], Gg[2 * jj + 1]));
-#pragma unroll
-      for (int m = 0; m < 4; ++m) xp[m] = PB::mma(xp[m], kxf[(m * (D / 32) + w * JPW + jj) * 64 + lane], gb);
-    }
-#pragma unroll
-    for (int m = 0; m < 4; ++m) sh.xp[w][m][lane] = xp[m];
-    __syncthreads();
-    // token tile w: X, dW = R + kappa o X
-    const f32x4 X = sh.xp[0][w][lane] + sh.xp[1][w][lane] + sh.xp[2][w][lane] + sh.xp[3][w][lane];
-    f32x4 dw;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ri = 16 * w + 4 * (lane >> 4) + i;
-      dw[i] = rr[i] + expf(l63 - lr[i]) * X[i];
-      rec[R::X + ri * DV + vc] = X[i];
-      rec[R::DW + ri * DV + vc] = dw[i];
-    }
-    sh.z[w][lane] = dw;
-    __syncthreads();
-    // token tile w of Z = Tp^T dW (stored negated: dL/dX_K)
-    const f32x4 Z = mm<PrecF32>(mm<PrecF32>(zero4(), ta0, pair_to8(sh.z[0][lane], sh.z[1][lane])), ta1,
-                                pair_to8(sh.z[2][lane], sh.z[3][lane]));
-    const f32x4 zn = -Z;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rec[R::ZN + (16 * w + 4 * (lane >> 4) + i) * DV + vc] = zn[i];
-    sh.x[w][lane] = zn;
-    __syncthreads();
-    // Gamma <- g_C Gamma + H - K^T Z over this wave's features
-    const frag zb0 = PB::from_f32(pair_to8(sh.x[0][lane], sh.x[1][lane]));
-    const frag zb1 = PB::from_f32(pair_to8(sh.x[2][lane], sh.x[3][lane]));
-    const float gC = expf(l63);
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const f32x4 acc = gC * Gg[t] + hv[t];
-      Gg[t] = PB::mma(PB::mma(acc, ktf[((w * TPW + t) * 2) * 64 + lane], zb0), ktf[((w * TPW + t) * 2 + 1) * 64 + lane],
-                      zb1);
-    }
-  }
-  if (p.nch < 0) p.ws[0] = (float)sink;
-  if (g.dinit) {
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int f = FPW * w + 16 * t + 4 * (lane >> 4) + i;
-        g.dinit[b * g.gis0 + h * g.gis1 + f * g.gis2 + vc * g.gis3] = Gg[t][i];
-      }
-  }
-}
-
 // ---------------------------------------------------------------------------------------------- grad
 // grid (nch, H, B), 256 threads; wave w owns row tile w of the 64 x 64 chunk algebra.  Rows of the
 // fixed-order partial-sum tables: dl_i from the kappa term, the column sums of P o dP per row tile (4),
-// the row sums of P o dP (at i - 1), beta g (T o dTp) column sums, the a o dY . Q S^T term (at i - 1),
-// the column sums of beta o A o dA per row tile (4), its row sums; dbeta_i from the V . T^T dW row sums,
-// the Tp column sums and the A o dA row sums.
-constexpr int GDL_K = 0, GDL_COLP = 1, GDL_RP = 5, GDL_TS = 6, GDL_DA = 7, GDL_DLC = 8, GDL_A = 12, GNDL = 13;
+// the row sums of P o dP (at i - 1), beta g (T o dTp) column sums, the column sums of beta o A o dA per row
+// tile (4), its row sums; dbeta_i from the V . T^T dW row sums, the Tp column sums and the A o dA row sums.
+constexpr int GDL_K = 0, GDL_COLP = 1, GDL_RP = 5, GDL_TS = 6, GDL_DLC = 7, GDL_A = 11, GNDL = 12;
 constexpr int GDB_V = 0, GDB_TS = 1, GDB_A = 2, GNDB = 3;
 
 // Sum over the 64 lanes of a wave in a fixed order (the result in every lane).
@@ -683,16 +879,39 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// The products over the value columns (phase 1 of grad), VV: V's rows and dY's start on 16 bytes.
+template <typename InT, int D, int DV, bool VV>
+__device__ __forceinline__ void grad_products(const float* rec, const InT* Vin, int64_t vs, const float* Yin, int64_t ys, int rt,
+                                              int lane, int nrows, f32x4 (&dtp)[4], f32x4 (&e1)[4], f32x4 (&dp)[4]) {
+  using F = Rec<D, DV>;
+  using R = BRec<D, DV>;
+#pragma unroll
+  for (int n4 = 0; n4 < 4; ++n4) dtp[n4] = e1[n4] = dp[n4] = zero4();
+#pragma unroll 2
+  for (int kb = 0; kb < DV / 32; ++kb) {
+    const f32x8 da = frag_rows_plain(rec + R::DW, DV, 16 * rt, 32 * kb, lane);
+    const f32x8 ya = row_frag<PrecF32, float, VV>(Yin, ys, 16 * rt, 32 * kb, lane, nrows);
+#pragma unroll
+    for (int n4 = 0; n4 < 4; ++n4) {
+      dtp[n4] = mm<PrecF32>(dtp[n4], da, frag_rows_plain(rec + R::XK, DV, 16 * n4, 32 * kb, lane));
+      e1[n4] = mm<PrecF32>(e1[n4], da, row_frag<PrecF32, InT, VV>(Vin, vs, 16 * n4, 32 * kb, lane, nrows));
+      dp[n4] = mm<PrecF32>(dp[n4], ya, frag_rows_plain(rec + F::W, DV, 16 * n4, 32 * kb, lane));
+    }
+  }
+}
+
 template <class PB, typename InT, int D, int DV>
 __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
   using F = Rec<D, DV>;
   using R = BRec<D, DV>;
+  using frag = typename PB::frag;
   constexpr int NV = DV / 16;
   __shared__ __attribute__((aligned(16))) float bT[C * LD];   // T
-  __shared__ __attribute__((aligned(16))) float bD[C * LD];   // dT
+  __shared__ __attribute__((aligned(16))) float bD[C * LD];   // dT, then M + M^T
   __shared__ __attribute__((aligned(16))) float bY1[C * LD];  // dT T^T
-  __shared__ float s_ell[C], s_beta[C];
-  __shared__ float s_dl[GNDL][C], s_db[GNDB][C], s_ts[4][C], s_kt[C], s_63[5];
+  __shared__ __attribute__((aligned(16))) float bN[C * LD];   // N
+  __shared__ float s_ell[C], s_beta[C], s_kap[C];
+  __shared__ float s_dl[GNDL][C], s_db[GNDB][C], s_ts[4][C], s_kt[C], s_63;
 
   const int64_t c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -700,38 +919,28 @@ __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
   const int rt = w;
   const int64_t t0 = c * C;
   float* rec = record<D, DV, true>(p, b, h, c);
+  frag* ops = reinterpret_cast<frag*>(rec + R::OPS);
   const int nrows = (int)(p.T - t0 < C ? p.T - t0 : C);
   const InT* Vin = reinterpret_cast<const InT*>(p.v) + b * p.vs0 + t0 * p.vs1 + h * p.vs2;
-  const InT* Qin = reinterpret_cast<const InT*>(p.q) + b * p.qs0 + t0 * p.qs1 + h * p.qs2;
   const float* Yin = g.dy + b * g.ys0 + t0 * g.ys1 + h * g.ys2;
 
   if (tid < C) {
-    s_ell[tid] = rec[F::VEC + tid];
-    s_beta[tid] = rec[F::VEC + 64 + tid];
+    s_ell[tid] = rec[F::V_L + tid];
+    s_beta[tid] = rec[R::V_BETA + tid];
+    s_kap[tid] = rec[F::V_KAP + tid];
   }
   for (int idx = tid; idx < GNDL * C; idx += 256) (&s_dl[0][0])[idx] = 0.f;
   for (int idx = tid; idx < GNDB * C; idx += 256) (&s_db[0][0])[idx] = 0.f;
-  for (int idx = tid; idx < C * C; idx += 256) bT[(idx >> 6) * LD + (idx & 63)] = rec[R::T + idx];
+  for (int idx = 4 * tid; idx < C * C; idx += 1024)
+    *reinterpret_cast<f32x4*>(bT + (idx >> 6) * LD + (idx & 63)) = *reinterpret_cast<const f32x4*>(rec + R::T + idx);
   __syncthreads();
-  const float l63 = s_ell[63], gC = expf(l63);
 
   // ---- phase 1: dTp = -dW X_K^T, dW V^T, dP = dY W^T -> dT, N, the Tp and P o dP sums; T^T dW -> dv, dbeta;
-  //      the kappa term and kappa o W
+  //      the kappa term; kappa o W and Z as operands of the feature gradients
   {
     f32x4 dtp[4], e1[4], dp[4];
-#pragma unroll
-    for (int n4 = 0; n4 < 4; ++n4) dtp[n4] = e1[n4] = dp[n4] = zero4();
-#pragma unroll
-    for (int kb = 0; kb < DV / 32; ++kb) {
-      const f32x8 da = frag_rows(rec + R::DW, DV, 16 * rt, 32 * kb, lane);
-      const f32x8 ya = frag_rows_in(Yin, g.ys1, 16 * rt, 32 * kb, lane, nrows);
-#pragma unroll
-      for (int n4 = 0; n4 < 4; ++n4) {
-        dtp[n4] = mm<PrecF32>(dtp[n4], da, frag_rows(rec + R::XK, DV, 16 * n4, 32 * kb, lane));
-        e1[n4] = mm<PrecF32>(e1[n4], da, frag_rows_in(Vin, p.vs1, 16 * n4, 32 * kb, lane, nrows));
-        dp[n4] = mm<PrecF32>(dp[n4], ya, frag_rows(rec + F::W, DV, 16 * n4, 32 * kb, lane));
-      }
-    }
+    if (p.vvec && g.yvec) grad_products<InT, D, DV, true>(rec, Vin, p.vs1, Yin, g.ys1, rt, lane, nrows, dtp, e1, dp);
+    else grad_products<InT, D, DV, false>(rec, Vin, p.vs1, Yin, g.ys1, rt, lane, nrows, dtp, e1, dp);
     float rowp[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int n4 = 0; n4 < 4; ++n4) {
@@ -751,7 +960,7 @@ __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
           colp += pb;
           nv = dp[n4][i] * expf(fminf(s_ell[ri - 1] - s_ell[cj], 0.f));
         }
-        rec[R::NN + ri * C + cj] = nv;
+        bN[ri * LD + cj] = nv;
       }
       ts = sum_col4(ts);
       colp = sum_col4(colp);
@@ -768,11 +977,12 @@ __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
     }
     // T^T dW, rows 16 rt ..: dv and the V . (T^T dW) row sums
     const f32x8 ta0 = frag_cols(bT, LD, 16 * rt, 0, lane), ta1 = frag_cols(bT, LD, 16 * rt, 32, lane);
+    const f32x4* dwt = reinterpret_cast<const f32x4*>(rec + R::DWT);
     float dbv[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int nv = 0; nv < NV; ++nv) {
-      const f32x4 td = mm<PrecF32>(mm<PrecF32>(zero4(), ta0, frag_cols(rec + R::DW, DV, 16 * nv, 0, lane)), ta1,
-                                   frag_cols(rec + R::DW, DV, 16 * nv, 32, lane));
+      auto tile = [&](int m) { return dwt[(m * NV + nv) * 64 + lane]; };
+      const f32x4 td = mm<PrecF32>(mm<PrecF32>(zero4(), ta0, pair_to8(tile(0), tile(1))), ta1, pair_to8(tile(2), tile(3)));
       const int vcol = 16 * nv + (lane & 15);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -791,21 +1001,21 @@ __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
     }
   }
   {
-    // the kappa term: dkappa_i = W_i . X_i (row tid / 4, a quarter of the columns per thread, the quad's
-    // four partials added in a fixed order); and kappa o W for the feature gradients
-    const int r = tid >> 2, q0 = (tid & 3) * (DV / 4);
-    const float kap = expf(l63 - s_ell[r]);
+    // the kappa term: dkappa_i = W_i . X_i (token 16w + (l & 15), a quarter of the columns per lane group, the
+    // four partials added in a fixed order); kappa o W and -Z as fragments
+    const int r = 16 * w + (lane & 15);
+    const float kap = s_kap[r];
     float dk = 0.f;
-#pragma unroll 4
-    for (int v = q0; v < q0 + DV / 4; v += 4) {
-      const f32x4 wv = *reinterpret_cast<const f32x4*>(rec + F::W + r * DV + v);
-      const f32x4 xv = *reinterpret_cast<const f32x4*>(rec + R::X + r * DV + v);
-      dk += wv[0] * xv[0] + wv[1] * xv[1] + wv[2] * xv[2] + wv[3] * xv[3];
-      *reinterpret_cast<f32x4*>(rec + R::KW + r * DV + v) = kap * wv;
+#pragma unroll
+    for (int kb = 0; kb < DV / 32; ++kb) {
+      const f32x8 wv = frag_rows(rec + F::W, DV, 16 * w, 32 * kb, lane), xv = frag_rows(rec + R::X, DV, 16 * w, 32 * kb, lane);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) dk += wv[s] * xv[s];
+      ops[bop_v<DV>(1, w, kb) * 64 + lane] = PB::from_f32(kap * wv);
+      ops[bop_v<DV>(2, w, kb) * 64 + lane] = PB::from_f32(frag_rows(rec + R::ZN, DV, 16 * w, 32 * kb, lane));
     }
-    dk += __shfl_xor(dk, 1);
-    dk += __shfl_xor(dk, 2);
-    if ((tid & 3) == 0) {
+    dk = sum_col4(dk);
+    if (lane < 16) {
       s_dl[GDL_K][r] = -dk * kap;
       s_kt[r] = dk * kap;
     }
@@ -813,55 +1023,19 @@ __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
   __syncthreads();
   if (w == 0) {
     const float tot = wave_sum(s_kt[lane]);
-    if (lane == 0) s_63[0] = tot;
+    if (lane == 0) s_63 = tot;
   }
-
-  // ---- phase 2: the Tp sums; Q S^T -> da; <Gamma, S>
+  // ---- phase 2: the Tp sums; Y1 = dT T^T; N and N^T as fragments
   if (tid < C) {
     const float gj = expf(s_ell[tid]), ts = ((s_ts[0][tid] + s_ts[1][tid]) + s_ts[2][tid]) + s_ts[3][tid];
     s_db[GDB_TS][tid] = gj * ts;
     s_dl[GDL_TS][tid] = s_beta[tid] * gj * ts;
   }
-  {
-    float dap[4] = {0.f, 0.f, 0.f, 0.f};
-    f32x4 qs[NV];
 #pragma unroll
-    for (int nv = 0; nv < NV; ++nv) qs[nv] = zero4();
-    for (int jb = 0; jb < D / 32; ++jb) {
-      const typename PB::frag qa = PB::from_f32(frag_rows_in(Qin, p.qs1, 16 * rt, 32 * jb, lane, nrows));
-#pragma unroll
-      for (int nv = 0; nv < NV; ++nv)
-        qs[nv] = PB::mma(qs[nv], qa, PB::from_f32(frag_rows(rec + R::SR, D, 16 * nv, 32 * jb, lane)));
-    }
-#pragma unroll
-    for (int nv = 0; nv < NV; ++nv) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int ri = 16 * rt + 4 * (lane >> 4) + i;
-        if (ri < nrows) dap[i] += Yin[ri * g.ys1 + 16 * nv + (lane & 15)] * qs[nv][i];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ri = 16 * rt + 4 * (lane >> 4) + i;
-      const float da = sum_row16(dap[i]);
-      if ((lane & 15) == 0 && ri > 0) s_dl[GDL_DA][ri - 1] = da * expf(s_ell[ri - 1]);
-    }
+  for (int jb = 0; jb < 2; ++jb) {
+    ops[bop_t<DV>(0, w, jb) * 64 + lane] = PB::from_f32(frag_rows(bN, LD, 16 * w, 32 * jb, lane));
+    ops[bop_t<DV>(2, w, jb) * 64 + lane] = PB::from_f32(frag_cols(bN, LD, 16 * w, 32 * jb, lane));
   }
-  {
-    float gs = 0.f;
-    const f32x4* G4 = reinterpret_cast<const f32x4*>(rec + R::GR);
-    const f32x4* S4 = reinterpret_cast<const f32x4*>(rec + R::SR);
-    for (int e = tid; e < D * DV / 4; e += 256) {
-      const f32x4 gg = G4[e], ss = S4[e];
-      gs += gg[0] * ss[0] + gg[1] * ss[1] + gg[2] * ss[2] + gg[3] * ss[3];
-    }
-    gs = wave_sum(gs);
-    if (lane == 0) s_63[1 + w] = gs;
-  }
-  __syncthreads();
-
-  // ---- phase 3: Y1 = dT T^T
   {
     const f32x8 a0 = frag_rows(bD, LD, 16 * rt, 0, lane), a1 = frag_rows(bD, LD, 16 * rt, 32, lane);
 #pragma unroll
@@ -874,7 +1048,7 @@ __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
   }
   __syncthreads();
 
-  // ---- phase 4: dA = -T^T Y1 (strictly lower); M + M^T; dbeta and dl from A
+  // ---- phase 3: dA = -T^T Y1 (strictly lower); M + M^T (over dT); dbeta and dl from A
   {
     const f32x8 ta0 = frag_cols(bT, LD, 16 * rt, 0, lane), ta1 = frag_cols(bT, LD, 16 * rt, 32, lane);
     float dbr[4] = {0.f, 0.f, 0.f, 0.f}, dlr[4] = {0.f, 0.f, 0.f, 0.f};
@@ -895,10 +1069,10 @@ __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
           dlr[i] += ab;
           dlc += ab;
           const float mv = dA[i] * s_beta[ri] * ex;
-          rec[R::MM + ri * C + cj] = mv;
-          rec[R::MM + cj * C + ri] = mv;
+          bD[ri * LD + cj] = mv;
+          bD[cj * LD + ri] = mv;
         } else if (cj == ri) {
-          rec[R::MM + ri * C + cj] = 0.f;
+          bD[ri * LD + cj] = 0.f;
         }
       }
       dlc = sum_col4(dlc);
@@ -915,121 +1089,207 @@ __global__ void __launch_bounds__(256) gbwd_grad_kernel(Params p, BwdP g) {
     }
   }
   __syncthreads();
+#pragma unroll
+  for (int jb = 0; jb < 2; ++jb) ops[bop_t<DV>(1, w, jb) * 64 + lane] = PB::from_f32(frag_rows(bD, LD, 16 * w, 32 * jb, lane));
 
-  // ---- phase 5: dbeta and dlambda (dlog lambda_t = sum_{i >= t} dl_i)
+  // ---- phase 4: dbeta, and dl without the terms of S
   if (w == 0) {
     float dl = 0.f;
 #pragma unroll
     for (int k = 0; k < GNDL; ++k) dl += s_dl[k][lane];
-    if (lane == 63) dl += s_63[0] + gC * (((s_63[1] + s_63[2]) + s_63[3]) + s_63[4]);
+    if (lane == 63) dl += s_63;
     float dbeta = 0.f;
 #pragma unroll
     for (int k = 0; k < GNDB; ++k) dbeta += s_db[k][lane];
+    rec[R::V_DL + lane] = dl;
+    if (lane < nrows) g.dbeta[b * g.dbs0 + (t0 + lane) * g.dbs1 + h * g.dbs2] = dbeta;
+  }
+}
+
+// dlambda: one wave per chunk adds the partial sums over the feature blocks in their order, then
+// dlog lambda_t = sum_{i >= t} dl_i.
+template <int D, int DV>
+__global__ void __launch_bounds__(64) gbwd_decay_kernel(Params p, BwdP g) {
+  using F = Rec<D, DV>;
+  using R = BRec<D, DV>;
+  const int64_t c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int lane = threadIdx.x;
+  const float* rec = record<D, DV, true>(p, b, h, c);
+  const float* part = rec + R::PART;
+  float da = 0.f, gs = 0.f;
+#pragma unroll 8
+  for (int k = 0; k < D / 32; ++k) {
+    da += part[k * 64 + lane];
+    gs += part[D / 32 * 64 + k];
+  }
+  // dl_{i-1} takes row i's a o dY . Q S^T, dl_63 takes g_C <Gamma, S>
+  const float up = __shfl_down(da, 1);
+  float dl = rec[R::V_DL + lane] + (lane < 63 ? up : expf(rec[F::V_L + 63]) * gs);
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const float u = __shfl_down(dl, o);
-      if (lane + o < 64) dl += u;
-    }
-    const int64_t t = t0 + lane;
-    if (lane < nrows) {
-      g.dbeta[b * g.dbs0 + t * g.dbs1 + h * g.dbs2] = dbeta;
-      if (g.ddecay) {
-        const float la = p.decay ? p.decay[b * p.ds0 + t * p.ds1 + h * p.ds2] : 1.f;
-        g.ddecay[b * g.dds0 + t * g.dds1 + h * g.dds2] = (la >= 1e-5f && la <= 1.f) ? dl / la : 0.f;
-      }
-    }
+  for (int o = 1; o < 64; o <<= 1) {
+    const float u = __shfl_down(dl, o);
+    if (lane + o < 64) dl += u;
+  }
+  const int64_t t = c * C + lane;
+  if (t < p.T) {
+    const float la = p.decay ? p.decay[b * p.ds0 + t * p.ds1 + h * p.ds2] : 1.f;
+    g.ddecay[b * g.dds0 + t * g.dds1 + h * g.dds2] = (la >= 1e-5f && la <= 1.f) ? dl / la : 0.f;
   }
 }
 
 // ---------------------------------------------------------------------------------------------- dphi
-// grid (nch * D / 256, H, B), 256 threads; workgroup (chunk, block of 256 features), wave w features
-// [64 w, 64 w + 64) of the block for all 64 tokens (each wave loads only its own features' operands).
+// grid (nch * D / 256, H, B), DPHI_WAVES waves; workgroup (chunk, block of 256 features), wave w features
+// [32 w, 32 w + 32) of the block for all 64 tokens.  The gradients are formed transposed (features in the
+// rows): a lane's pair of accumulator tiles is eight consecutive features of a token.  The bound is the
+// traffic, 1.9 MB a chunk, of which S and Gamma are 1 MB: both are read once, as coalesced tiles that serve as
+// the operand of Q S^T as they are, and of the gradients after an exact transpose on the matrix cores (products
+// with selector()).  With bf16 fragments the right operands, the same for every wave, are staged in LDS.
+// 2016 chunks, bf16, d_v = 128: 1316 -> 919 us (4.2 TB/s) with the sums over S taken over from the gradient kernel
+// (1319 -> 343 us), which read S and Gamma a second time.
+constexpr int DPHI_WAVES = 8;
 template <class PB, typename InT, int D, int DV>
-__global__ void __launch_bounds__(256) gbwd_dphi_kernel(Params p, BwdP g) {
+__global__ void __launch_bounds__(64 * DPHI_WAVES) gbwd_dphi_kernel(Params p, BwdP g) {
+  using F = Rec<D, DV>;
   using R = BRec<D, DV>;
-  constexpr int FB = 256;
+  using frag = typename PB::frag;
+  constexpr bool BF = std::is_same<PB, PrecBF16>::value;
+  constexpr int FB = 32 * DPHI_WAVES, NOP = bop_count<DV>();
+  __shared__ frag s_ops[BF ? NOP * 64 : 1];
   const int64_t c = blockIdx.x / (D / FB), h = blockIdx.y, b = blockIdx.z;
   const int fb = (int)(blockIdx.x % (D / FB));
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t t0 = c * C;
-  const float* rec = record<D, DV, true>(p, b, h, c);
+  float* rec = record<D, DV, true>(p, b, h, c);
   const int nrows = (int)(p.T - t0 < C ? p.T - t0 : C);
-  const InT* Qin = reinterpret_cast<const InT*>(p.q) + b * p.qs0 + t0 * p.qs1 + h * p.qs2;
-  const InT* Kin = reinterpret_cast<const InT*>(p.k) + b * p.ks0 + t0 * p.ks1 + h * p.ks2;
-  const int f0 = fb * FB + 64 * w;
-  f32x4 aq[4][4], ak[4][4];  // [token tile][feature tile]
+  const frag* ops = reinterpret_cast<const frag*>(rec + R::OPS);
+  if constexpr (BF) {
+#pragma unroll
+    for (int k = 0; k < NOP / DPHI_WAVES; ++k) s_ops[(k * DPHI_WAVES + w) * 64 + lane] = ops[(k * DPHI_WAVES + w) * 64 + lane];
+  }
+  auto op = [&](int i) { return BF ? s_ops[i * 64 + lane] : ops[i * 64 + lane]; };
+  const int jf = fb * DPHI_WAVES + w;  // the wave's 32-feature block
+  const frag sel[2] = {selector<PB>(0, lane), selector<PB>(1, lane)};
+  // token rows of Q and K (fragments [m][jb]): packed by prep with bf16 fragments, else from the input
+  frag qf[4];
+  if constexpr (BF) {
+    const frag* qxf = reinterpret_cast<const frag*>(rec + F::KXF) + 4 * (D / 32) * 64;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) qf[m] = qxf[(m * (D / 32) + jf) * 64 + lane];
+  } else {
+    const InT* Qin = reinterpret_cast<const InT*>(p.q) + b * p.qs0 + t0 * p.qs1 + h * p.qs2;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) qf[m] = row_frag<PB, InT, false>(Qin, p.qs1, 16 * m, 32 * jf, lane, nrows);
+  }
+  if constexpr (BF) __syncthreads();
+  f32x4 aq[4][2], ak[4][2];  // [token tile][feature tile]
 #pragma unroll
   for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int ft = 0; ft < 4; ++ft) aq[m][ft] = ak[m][ft] = zero4();
-  // contractions over the value columns: (a o dY) S, (kappa o W) Gamma^T, -Z S
+    for (int t = 0; t < 2; ++t) aq[m][t] = ak[m][t] = zero4();
+  float dap[4] = {0.f, 0.f, 0.f, 0.f}, gs = 0.f;
+  const bool want = g.ddecay != nullptr;
+  const f32x4* st = reinterpret_cast<const f32x4*>(rec + R::SR) + 2 * jf * 64 + lane;
+  const f32x4* gt = reinterpret_cast<const f32x4*>(rec + R::GR) + 2 * jf * 64 + lane;
+  // contractions over the value columns: S^T (a o dY)^T, Gamma (kappa o W)^T, -S^T Z^T
+#pragma unroll 1
   for (int kb = 0; kb < DV / 32; ++kb) {
-    f32x8 sb[4], gb[4];
+    frag sb[2], gb[2];
 #pragma unroll
-    for (int ft = 0; ft < 4; ++ft) {
-      sb[ft] = frag_cols(rec + R::SR, D, f0 + 16 * ft, 32 * kb, lane);
-      gb[ft] = frag_cols(rec + R::GR, D, f0 + 16 * ft, 32 * kb, lane);
+    for (int nn = 0; nn < 2; ++nn) {
+      const size_t at = (size_t)(2 * kb + nn) * (D / 16) * 64;
+      const f32x8 sv = pair_to8(st[at], st[at + 64]), gv = pair_to8(gt[at], gt[at + 64]);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) gs += sv[s] * gv[s];
+      sb[nn] = PB::from_f32(sv);
+      gb[nn] = PB::from_f32(gv);
+    }
+    if (want) {
+#pragma unroll
+      for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          const f32x4 qs = PB::mma(zero4(), sb[nn], qf[m]);
+          const f32x4 ay = *reinterpret_cast<const f32x4*>(rec + R::AY + (16 * m + (lane & 15)) * DV + 32 * kb + 16 * nn + 4 * (lane >> 4));
+          dap[m] += ((ay[0] * qs[0] + ay[1] * qs[1]) + ay[2] * qs[2]) + ay[3] * qs[3];
+        }
     }
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const f32x8 ay = frag_rows(rec + R::AY, DV, 16 * m, 32 * kb, lane);
-      const f32x8 kw = frag_rows(rec + R::KW, DV, 16 * m, 32 * kb, lane);
-      const f32x8 zn = frag_rows(rec + R::ZN, DV, 16 * m, 32 * kb, lane);
+    for (int t = 0; t < 2; ++t) {
+      const frag sf = PB::from_f32(pair_to8(PB::mma(zero4(), sb[0], sel[t]), PB::mma(zero4(), sb[1], sel[t])));
+      const frag gf = PB::from_f32(pair_to8(PB::mma(zero4(), gb[0], sel[t]), PB::mma(zero4(), gb[1], sel[t])));
 #pragma unroll
-      for (int ft = 0; ft < 4; ++ft) {
-        aq[m][ft] = mm<PB>(aq[m][ft], ay, sb[ft]);
-        ak[m][ft] = mm<PB>(mm<PB>(ak[m][ft], kw, gb[ft]), zn, sb[ft]);
+      for (int m = 0; m < 4; ++m) {
+        aq[m][t] = PB::mma(aq[m][t], sf, op(bop_v<DV>(0, m, kb)));
+        ak[m][t] = PB::mma(PB::mma(ak[m][t], gf, op(bop_v<DV>(1, m, kb))), sf, op(bop_v<DV>(2, m, kb)));
       }
     }
   }
-  // contractions over the chunk's tokens: N K, (M + M^T) K, N^T Q
-  for (int kb = 0; kb < 2; ++kb) {
-    f32x8 kf[4], qf[4];
+  // contractions over the chunk's tokens: K^T N^T, K^T (M + M^T), Q^T N
+  {
+    frag kf[4];
+    const frag* kxf = reinterpret_cast<const frag*>(rec + F::KXF);
 #pragma unroll
-    for (int ft = 0; ft < 4; ++ft) {
-      kf[ft] = frag_cols_in(Kin, p.ks1, f0 + 16 * ft, 32 * kb, lane, nrows);
-      qf[ft] = frag_cols_in(Qin, p.qs1, f0 + 16 * ft, 32 * kb, lane, nrows);
-    }
+    for (int m = 0; m < 4; ++m) kf[m] = kxf[(m * (D / 32) + jf) * 64 + lane];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const f32x8 nr = frag_rows(rec + R::NN, C, 16 * m, 32 * kb, lane);
-      const f32x8 mr = frag_rows(rec + R::MM, C, 16 * m, 32 * kb, lane);
-      const f32x8 nt = frag_cols(rec + R::NN, C, 16 * m, 32 * kb, lane);
+    for (int jb = 0; jb < 2; ++jb)
 #pragma unroll
-      for (int ft = 0; ft < 4; ++ft) {
-        aq[m][ft] = mm<PB>(aq[m][ft], nr, kf[ft]);
-        ak[m][ft] = mm<PB>(mm<PB>(ak[m][ft], mr, kf[ft]), nt, qf[ft]);
-      }
-    }
-  }
+      for (int t = 0; t < 2; ++t) {
+        const frag kt = PB::from_f32(pair_to8(PB::mma(zero4(), kf[2 * jb], sel[t]), PB::mma(zero4(), kf[2 * jb + 1], sel[t])));
+        const frag qt = PB::from_f32(pair_to8(PB::mma(zero4(), qf[2 * jb], sel[t]), PB::mma(zero4(), qf[2 * jb + 1], sel[t])));
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
-#pragma unroll
-    for (int ft = 0; ft < 4; ++ft)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int ri = 16 * m + 4 * (lane >> 4) + i;
-        if (ri < nrows) {
-          const int64_t t = t0 + ri;
-          const int f = f0 + 16 * ft + (lane & 15);
-          g.dq[b * g.dqs0 + t * g.dqs1 + h * g.dqs2 + f] = aq[m][ft][i];
-          g.dk[b * g.dks0 + t * g.dks1 + h * g.dks2 + f] = ak[m][ft][i];
+        for (int m = 0; m < 4; ++m) {
+          aq[m][t] = PB::mma(aq[m][t], kt, op(bop_t<DV>(0, m, jb)));
+          ak[m][t] = PB::mma(PB::mma(ak[m][t], kt, op(bop_t<DV>(1, m, jb))), qt, op(bop_t<DV>(2, m, jb)));
         }
       }
+  }
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const int ri = 16 * m + (lane & 15);
+    if (ri >= nrows) continue;
+    const int64_t t = t0 + ri;
+    const int f = 32 * jf + 8 * (lane >> 4);
+    float* dq = g.dq + b * g.dqs0 + t * g.dqs1 + h * g.dqs2 + f;
+    float* dk = g.dk + b * g.dks0 + t * g.dks1 + h * g.dks2 + f;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      if (g.gvec) {
+        *reinterpret_cast<f32x4*>(dq + 4 * a) = aq[m][a];
+        *reinterpret_cast<f32x4*>(dk + 4 * a) = ak[m][a];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          dq[4 * a + i] = aq[m][a][i];
+          dk[4 * a + i] = ak[m][a][i];
+        }
+      }
+    }
+  }
+  if (want) {
+    float* part = rec + R::PART;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const float s = sum_col4(dap[m]);
+      if (lane < 16) part[jf * 64 + 16 * m + lane] = s;
+    }
+    gs = wave_sum(gs);
+    if (lane == 0) part[D / 32 * 64 + jf] = gs;
+  }
 }
 
 template <class PB, typename InT, int D, int DV>
 static int launch_bwd(const Params& p, const BwdP& g, hipStream_t st) {
   const dim3 chunk_grid((unsigned)p.nch, (unsigned)p.H, (unsigned)p.B);
-  const unsigned carry_wgs = (unsigned)(((p.B * p.H + 7) / 8) * 8 * (DV / 16));
-  hipLaunchKernelGGL((gen_prep_kernel<PB, InT, D, DV, true>), chunk_grid, dim3(256), 0, st, p);
-  hipLaunchKernelGGL((gen_carry_kernel<PB, D, DV, true>), dim3(carry_wgs), dim3(256), 0, st, p);
-  hipLaunchKernelGGL((gbwd_rh_kernel<PB, InT, D, DV>), chunk_grid, dim3(256), 0, st, p, g);
-  hipLaunchKernelGGL((gbwd_rchain_kernel<PB, D, DV>), dim3(carry_wgs), dim3(256), 0, st, p, g);
+  const unsigned wgs = (unsigned)(((p.B * p.H + 7) / 8) * 8 * (DV / 16));
+  hipLaunchKernelGGL((gen_prep_kernel<PB, InT, D, DV, true>), chunk_grid, dim3(256), 0, st, p, g);
+  launch_carry<PB, D, DV, true>(p, st);
+  hipLaunchKernelGGL((gen_carry_kernel<PB, D, DV, true, true>), dim3(wgs), dim3(64 * CARRY_WAVES), 0, st, p, g.dfin, g.fs0, g.fs1,
+                     g.fs2, g.fs3, g.dinit, g.gis0, g.gis1, g.gis2, g.gis3);
   hipLaunchKernelGGL((gbwd_grad_kernel<PB, InT, D, DV>), chunk_grid, dim3(256), 0, st, p, g);
-  hipLaunchKernelGGL((gbwd_dphi_kernel<PB, InT, D, DV>), dim3((unsigned)(p.nch * (D / 256)), (unsigned)p.H, (unsigned)p.B),
-                     dim3(256), 0, st, p, g);
+  hipLaunchKernelGGL((gbwd_dphi_kernel<PB, InT, D, DV>), dim3((unsigned)(p.nch * (D / (32 * DPHI_WAVES))), (unsigned)p.H, (unsigned)p.B),
+                     dim3(64 * DPHI_WAVES), 0, st, p, g);
+  if (g.ddecay) hipLaunchKernelGGL((gbwd_decay_kernel<D, DV>), chunk_grid, dim3(64), 0, st, p, g);
   return launch_status();
 }
 
@@ -1038,9 +1298,8 @@ static int launch_bwd(const Params& p, const BwdP& g, hipStream_t st) {
 template <class PB, typename InT, int D, int DV>
 static int launch_ckpt(const Params& p, hipStream_t st) {
   const dim3 chunk_grid((unsigned)p.nch, (unsigned)p.H, (unsigned)p.B);
-  const unsigned carry_wgs = (unsigned)(((p.B * p.H + 7) / 8) * 8 * (DV / 16));
-  hipLaunchKernelGGL((gen_prep_kernel<PB, InT, D, DV, true>), chunk_grid, dim3(256), 0, st, p);
-  hipLaunchKernelGGL((gen_carry_kernel<PB, D, DV, true>), dim3(carry_wgs), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((gen_prep_kernel<PB, InT, D, DV, true>), chunk_grid, dim3(256), 0, st, p, BwdP{});
+  launch_carry<PB, D, DV, true>(p, st);
   return launch_status();
 }
 
@@ -1084,6 +1343,16 @@ static BwdPlan bwd_plan(const kdn_scan_args* f) {
   return L;
 }
 
+// Whether every row of a (B, T, H, d) view starts on `bytes` (strides of dimensions of one are not used).
+static bool rows_aligned(const Params& p, const void* x, int64_t s0, int64_t s1, int64_t s2, size_t elem, size_t bytes) {
+  const int64_t n = (int64_t)(bytes / elem);
+  return aligned(x, bytes) && (p.B == 1 || s0 % n == 0) && (p.T == 1 || s1 % n == 0) && (p.H == 1 || s2 % n == 0);
+}
+static void set_row_flags(Params& p, size_t isz) {
+  p.qkvec = rows_aligned(p, p.q, p.qs0, p.qs1, p.qs2, isz, 16) && rows_aligned(p, p.k, p.ks0, p.ks1, p.ks2, isz, 16);
+  p.vvec = rows_aligned(p, p.v, p.vs0, p.vs1, p.vs2, isz, 16);
+}
+
 }  // namespace gen
 
 bool general_scan_applies(const kdn_scan_args* a) { return a && a->D == 1024; }
@@ -1116,6 +1385,9 @@ int general_scan(const kdn_scan_args* a, void* stream) {
   p.fs0 = a->final_stride[0]; p.fs1 = a->final_stride[1]; p.fs2 = a->final_stride[2]; p.fs3 = a->final_stride[3];
   p.y = a->y; p.ys0 = a->y_stride[0]; p.ys1 = a->y_stride[1]; p.ys2 = a->y_stride[2];
   p.ws = reinterpret_cast<float*>(a->workspace);
+  gen::set_row_flags(p, dtype_size(a->in_dtype));
+  const size_t osz = dtype_size(a->out_dtype);
+  p.yvec = gen::rows_aligned(p, p.y, p.ys0, p.ys1, p.ys2, osz, 4 * osz);
   const hipStream_t st = as_stream(stream);
   if (a->d_v == 64) return gen::launch_dtypes<1024, 64>(p, a->in_dtype, a->out_dtype, st);
   return gen::launch_dtypes<1024, 128>(p, a->in_dtype, a->out_dtype, st);
@@ -1266,6 +1538,9 @@ int general_bwd(const kdn_scan_bwd_args* a, void* stream) {
   g.gis0 = a->dinit_stride[0]; g.gis1 = a->dinit_stride[1]; g.gis2 = a->dinit_stride[2]; g.gis3 = a->dinit_stride[3];
   const hipStream_t st = as_stream(stream);
   const size_t isz = dtype_size(f->in_dtype);
+  gen::set_row_flags(p, isz);
+  g.yvec = gen::rows_aligned(p, g.dy, g.ys0, g.ys1, g.ys2, 4, 16);
+  g.gvec = gen::rows_aligned(p, g.dq, g.dqs0, g.dqs1, g.dqs2, 4, 16) && gen::rows_aligned(p, g.dk, g.dks0, g.dks1, g.dks2, 4, 16);
   if (DV == 64) {
     if (f->in_dtype == KDN_DTYPE_BF16) return general_bwd_run<PrecBF16, __bf16, 1024, 64>(p, g, L, isz, st);
     return general_bwd_run<PrecF32, float, 1024, 64>(p, g, L, isz, st);

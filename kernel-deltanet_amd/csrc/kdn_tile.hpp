@@ -6,6 +6,20 @@
 
 namespace kdn {
 
+// A wave-uniform pointer the compiler may not take apart: a load at uni(p)[lane] keeps its base in scalar
+// registers.  Left alone, it adds the record's large constant offsets to per-lane 64-bit addresses and holds
+// one such address per fragment (the forward carry: 242 registers against 158).
+template <class T>
+__device__ __forceinline__ T* uni(T* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+  // a pointer to global memory, and known as one: a flat load would count as an LDS access too, and every
+  // LDS-only barrier wait for it
+  auto r = (__attribute__((address_space(1))) T*)((uint64_t)hi << 32 | lo);
+  asm volatile("" : "+s"(r));
+  return (T*)r;
+}
+
 template <typename T>
 __device__ __forceinline__ float ldx(const T* p) { return (float)*p; }
 

@@ -25,7 +25,8 @@ HIP_FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
 # VALU work on them needs no v_accvgpr_read copies: faster for the prep and backward kernels, which
 # post-process nearly every MFMA result (measured); slower for the state kernel, so not global.
 SOURCE_FLAGS = {"kdn_prep.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-                "kdn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+                "kdn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                "kdn_general.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def hipcc() -> str:

@@ -298,3 +298,32 @@ def test_d1024_scan_backward_two_heads_without_decay(oprojs):
         (Y * dy[:, :, h].double()).sum().backward()
         for name, a, r in zip(("dphi_q", "dphi_k", "dv", "dbeta"), (dq, dk, dvv, dbeta), leaves):
             assert rel(a[:, :, h].cpu().numpy(), r.grad.numpy()) < 1e-4, (h, name)
+
+
+@pytest.mark.parametrize("dtype,dv,T", [(torch.bfloat16, 128, 130), (torch.bfloat16, 64, 64), (torch.float32, 128, 65)])
+def test_d1024_scan_backward_rows_off_16_bytes(oprojs, dtype, dv, T):
+    # rows of q, k, v and dy that do not start on 16 bytes are read element by element: the same values in the
+    # same products, so every gradient is the same bit for bit; T one chunk, one token and two past a chunk
+    pq, pk, v, beta, decay, s0, dy, ds = _prelifted_case(2, T, dv, dtype, oprojs, 9)
+
+    def off(t):
+        wide = torch.zeros(*t.shape[:-1], t.shape[-1] + 1, device=DEV, dtype=t.dtype)
+        wide[..., 1:] = t.to(DEV)
+        return wide[..., 1:].unsqueeze(2)
+
+    outs = []
+    for view in (lambda t: t.to(DEV).unsqueeze(2), off):
+        plan = ops.ScanBackwardPlan(view(pq), view(pk), view(v), beta.to(DEV).unsqueeze(-1), decay.to(DEV).unsqueeze(-1),
+                                    None, None, 1.0, view(dy), ds.to(DEV).unsqueeze(1).transpose(2, 3),
+                                    initial_state=s0.to(DEV).unsqueeze(1).transpose(2, 3),
+                                    features=ops.FeatureMap(lifted=True))
+        outs.append([t.clone() for t in plan.run()])
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dphi_q", "dphi_k", "dv", "dbeta", "ddecay", "dS0"), *outs):
+        assert torch.equal(a, b), name
+    ref = _oracle_scan_grads(pq, pk, v, beta, decay, s0, dy, ds)
+    dq, dk, dvv, dbeta, ddecay, dinit = outs[1]
+    tol = 1e-4 if dtype == torch.float32 else 2e-2
+    got = [dq[:, :, 0], dk[:, :, 0], dvv[:, :, 0], dbeta[:, :, 0], ddecay[:, :, 0], dinit[:, 0].transpose(1, 2)]
+    for name, a, r in zip(("dphi_q", "dphi_k", "dv", "dbeta", "ddecay", "dS0"), got, ref):
+        assert rel(a.cpu().numpy(), r) < tol, name
