@@ -905,151 +905,179 @@ extern "C" int kdn_fwht_lift_factored(const void* x, int64_t rows, int64_t x_row
 }
 
 namespace kdn {
-constexpr int FLB_TILES = 2;
-// Backward of the factored lift: dx = (d out / d x)^T dout, one wave per 16 x FLB_TILES rows.  Each wave forms the
-// transposed angles theta^T = Omega_h x_h^T (features x rows) on MFMA, feature tile by feature tile, so
-// that a lane holds four consecutive features of one row (16-byte loads of the phases and of dout), and
-// needs two passes over them:
-//   1. per half h and row: n_h^2 = sum cs^2 and t_h = sum cs g (cs = sqrt(2/512) cos theta, g = dout);
-//      the renormalisations' backward needs only these four sums per row:
+// Backward of the factored lift: dx = (d out / d x)^T dout.  A workgroup takes 16 rows at a time; wave w forms the
+// transposed angles theta^T = Omega_h x_h^T (features x rows) of its 128 of the 1024 features (h = w / 4) on MFMA,
+// so that a lane holds four consecutive features of one row (16-byte loads of dout), and keeps what the
+// second half needs of them in registers:
+//   1. per half h and row: n_h^2 = sum cs^2 and t_h = sum cs g (cs = sqrt(2/512) cos theta, g = dout), added
+//      over the waves in LDS; the renormalisations' backward needs only these four sums per row:
 //        E = |c| + 1e-7 with |c|^2 = sum_h n_h^2 / e_h^2, e_h = n_h + 1e-8, c = cs / e_h;
 //        dc = g / E - c (c . g) / (E^2 |c|);  s_h = cs . dc = t_h / E - (c . g) / (E^2 |c|) n_h^2 / e_h;
 //        dphi~ = dc / e_h - cs s_h / (e_h^2 n_h)
 //   2. dL/dtheta = -sqrt(2/512) sin(theta) dphi~, and dx_h^T += Omega_h^T dtheta^T: the accumulator
-//      tiles of two feature tiles are the B operand of that product as they stand (kappa order).
-// A wave takes FLB_TILES row tiles, so that each Omega fragment it loads feeds that many products.
-// Per-row sums run over the four lane groups in a fixed order.  Products take the precision policy P
-// (bf16 operands for bf16 inputs: x and Omega are exact in bf16, so the angles equal the forward's).
+//      tiles of two feature tiles are the B operand of that product as they stand (kappa order); the four
+//      waves of a half add their parts in LDS.
+// The workgroup is persistent (one per CU): its Omega rows stay in registers and Omega^T, formed from them once on
+// the matrix cores (products with the identity, exact), in LDS as fragments.  The bounds are dout, read once, and
+// the sines and cosines, one each per feature.
+// Per-row sums have a fixed order.  Products take the precision policy P (bf16 operands for bf16 inputs: x and
+// Omega are exact in bf16, so the angles equal the forward's).
+struct LiftBwdShared {
+  bf16x8 ot[8][16][64];  // [wave][32-feature block, 16-column tile of Omega][lane]
+  f32x4 dx[2][3][4][64];
+  float ph[1024];
+  float n2[8][16], tg[8][16];
+};
+template <class P>
+__device__ __forceinline__ typename P::frag frag_of_bf16(const bf16x8& t) {
+  if constexpr (std::is_same<typename P::frag, bf16x8>::value) {
+    return t;
+  } else {
+    bf16x8 u = t;
+    asm volatile("" : "+v"(u));  // converted at its use: sixteen held fragments would not fit the registers
+    f32x8 r;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) r[s] = (float)u[s];
+    return r;
+  }
+}
 template <class P, typename InT>
-__global__ void __launch_bounds__(256) lift_factored_bwd_kernel(const InT* x, int64_t rows, int64_t xs,
+__global__ void __launch_bounds__(512) lift_factored_bwd_kernel(const InT* x, int64_t rows, int64_t xs, int xvec,
                                                                 const __bf16* om1, const float* ph1,
                                                                 const __bf16* om2, const float* ph2, float inv_tau,
                                                                 const float* dout, int64_t ds, float* dx,
                                                                 int64_t dxs) {
   using frag = typename P::frag;
-  constexpr int RT = FLB_TILES;  // 16-row tiles per wave: each Omega fragment feeds RT products
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t r0 = ((int64_t)blockIdx.x * 4 + w) * 16 * RT;
-  if (r0 >= rows) return;  // wave-uniform; the kernel has no barriers
-  const int fq = 4 * (lane >> 4);  // this lane's first feature inside a 16-feature tile
-  int64_t row[RT];
-  bool valid[RT];
-  frag xb[RT][2][2];  // x^T as B fragments: row tile, half h, 32-deep block kb
+  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+  typedef __attribute__((ext_vector_type(8))) InT in8;
+  __shared__ LiftBwdShared sh;
+  const int lane = threadIdx.x & 63, g = lane >> 4, fq = 4 * g;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = w >> 2, f0 = 128 * (w & 3);
+  bf16x8 oa[8][2];  // Omega rows f0 + 16 ft .., columns 32 kb + 8 g + s
+  {
+    const __bf16* om = (h ? om2 : om1) + (size_t)(f0 + (lane & 15)) * 64 + 8 * g;
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    row[rt] = r0 + 16 * rt + (lane & 15);
-    valid[rt] = row[rt] < rows;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int ft = 0; ft < 8; ++ft)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
-        f32x8 v;
-#pragma unroll
-        for (int s = 0; s < 8; ++s)
-          v[s] = valid[rt] ? (float)x[row[rt] * xs + 64 * h + 32 * kb + kappa(lane, s)] : 0.f;
-        xb[rt][h][kb] = P::from_f32(v);
+        const bf16x4* q = reinterpret_cast<const bf16x4*>(om + 16 * 64 * ft + 32 * kb);
+        oa[ft][kb] = __builtin_shufflevector(q[0], q[1], 0, 1, 2, 3, 4, 5, 6, 7);
       }
   }
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    f32x8 e;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) e[s] = 8 * g + s == 16 * a + (lane & 15) ? 1.f : 0.f;
+    const bf16x8 eye = PrecBF16::from_f32(e);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int fb = 0; fb < 4; ++fb)
+        sh.ot[w][fb * 4 + 2 * kb + a][lane] =
+            PrecBF16::from_f32(pair_to8(PrecBF16::mma(zero4(), oa[2 * fb][kb], eye), PrecBF16::mma(zero4(), oa[2 * fb + 1][kb], eye)));
+  }
+  for (int i = threadIdx.x; i < 1024; i += 512) sh.ph[i] = i < 512 ? ph1[i] : ph2[i - 512];
+  __syncthreads();
+
   const float amp = sqrtf(2.f / 512.f);
-  // pass 1
-  float n2[RT][2], tg[RT][2];
+  const int64_t ntiles = (rows + 15) / 16;
+  frag xb[2];  // x_h^T as B fragments
+  f32x4 gv[8];
+  auto load = [&](int64_t tile) {
+    const int64_t row = tile * 16 + (lane & 15);
+    const bool valid = row < rows;
+    const InT* xr = x + (valid ? row : rows - 1) * xs + 64 * h + 8 * g;
+    const float* gr = dout + (valid ? row : rows - 1) * ds + 512 * h + f0 + fq;
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) n2[rt][0] = n2[rt][1] = tg[rt][0] = tg[rt][1] = 0.f;
+    for (int kb = 0; kb < 2; ++kb) {
+      f32x8 v;
+      if (xvec) {
+        const in8 t = *reinterpret_cast<const in8*>(xr + 32 * kb);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const __bf16* om = h ? om2 : om1;
-    const float* ph = h ? ph2 : ph1;
-    for (int ft = 0; ft < 32; ++ft) {
-      const int f0 = 16 * ft;
-      const frag oa0 = P::from_f32(frag_rows_bf16(om, 64, f0, 0, lane));
-      const frag oa1 = P::from_f32(frag_rows_bf16(om, 64, f0, 32, lane));
-      const f32x4 b4 = *reinterpret_cast<const f32x4*>(ph + f0 + fq);
+        for (int s = 0; s < 8; ++s) v[s] = (float)t[s];
+      } else {
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        const f32x4 acc = P::mma(P::mma(zero4(), oa0, xb[rt][h][0]), oa1, xb[rt][h][1]);
-        const f32x4 g4 =
-            valid[rt] ? *reinterpret_cast<const f32x4*>(dout + row[rt] * ds + 512 * h + f0 + fq) : zero4();
+        for (int s = 0; s < 8; ++s) v[s] = (float)xr[32 * kb + s];
+      }
+      xb[kb] = P::from_f32(v);
+    }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float cs = amp * cos_rad(acc[i] * inv_tau + b4[i]);
-          n2[rt][h] += cs * cs;
-          tg[rt][h] += cs * g4[i];
-        }
+    for (int ft = 0; ft < 8; ++ft) gv[ft] = *reinterpret_cast<const f32x4*>(gr + 16 * ft);
+  };
+  // the next rows are loaded while these are worked on (bf16; fp32 fragments leave no registers for it)
+  constexpr bool AHEAD = std::is_same<P, PrecBF16>::value;
+  if constexpr (AHEAD) load(blockIdx.x);
+  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    if constexpr (!AHEAD) load(tile);
+    f32x4 sg[8], sc[8];  // sin times g, sin times cos (each with its amplitude)
+    float n2 = 0.f, tg = 0.f;
+#pragma unroll
+    for (int ft = 0; ft < 8; ++ft) {
+      const f32x4 acc = P::mma(P::mma(zero4(), frag_of_bf16<P>(oa[ft][0]), xb[0]), frag_of_bf16<P>(oa[ft][1]), xb[1]);
+      const f32x4 b4 = *reinterpret_cast<const f32x4*>(sh.ph + 512 * h + f0 + 16 * ft + fq);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float th = acc[i] * inv_tau + b4[i];
+        const float cs = amp * cos_rad(th), sn = amp * sin_rad(th);
+        n2 += cs * cs;
+        tg += cs * gv[ft][i];
+        sg[ft][i] = sn * gv[ft][i];
+        sc[ft][i] = sn * cs;
       }
     }
-  }
-  // per row: 1/e_h, 1/E, and the coefficients of dphi~ = g / (E e_h) - cs (corr / e_h^2 + k_h)
-  float ie[RT][2], ca[RT][2], cb[RT][2];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    float nn[2], e[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      n2[rt][h] = sum_over_lane_groups(n2[rt][h]);
-      tg[rt][h] = sum_over_lane_groups(tg[rt][h]);
-      nn[h] = sqrtf(n2[rt][h]);
-      e[h] = nn[h] + 1e-8f;
-      ie[rt][h] = 1.f / e[h];
+    if (AHEAD && tile + gridDim.x < ntiles) load(tile + gridDim.x);
+    n2 = sum_over_lane_groups(n2);
+    tg = sum_over_lane_groups(tg);
+    if (lane < 16) {
+      sh.n2[w][lane] = n2;
+      sh.tg[w][lane] = tg;
     }
-    const float cn = sqrtf(n2[rt][0] * ie[rt][0] * ie[rt][0] + n2[rt][1] * ie[rt][1] * ie[rt][1]);
-    const float iE = 1.f / (cn + 1e-7f);
-    const float sc = tg[rt][0] * ie[rt][0] + tg[rt][1] * ie[rt][1];
-    const float corr = cn > 0.f ? sc * iE * iE / cn : 0.f;
+    lds_barrier();
+    // 1/e_h, 1/E, and the coefficients of dphi~ = g / (E e_h) - cs (corr / e_h^2 + k_h)
+    float ca, cb;
+    {
+      float ns[2], ts[2], nn[2], ie[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const float sh = tg[rt][h] * iE - corr * n2[rt][h] * ie[rt][h];
-      const float kh = nn[h] > 0.f ? sh * ie[rt][h] * ie[rt][h] / nn[h] : 0.f;
-      ca[rt][h] = iE * ie[rt][h];                   // times g
-      cb[rt][h] = corr * ie[rt][h] * ie[rt][h] + kh;  // times cs
-    }
-  }
-  // pass 2
-  f32x4 dxt[RT][2][4];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const __bf16* om = h ? om2 : om1;
-    const float* ph = h ? ph2 : ph1;
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt) dxt[rt][h][jt] = zero4();
-    for (int fb = 0; fb < 16; ++fb) {
-      f32x4 dth[RT][2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int f0 = 32 * fb + 16 * u;
-        const frag oa0 = P::from_f32(frag_rows_bf16(om, 64, f0, 0, lane));
-        const frag oa1 = P::from_f32(frag_rows_bf16(om, 64, f0, 32, lane));
-        const f32x4 b4 = *reinterpret_cast<const f32x4*>(ph + f0 + fq);
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          const f32x4 acc = P::mma(P::mma(zero4(), oa0, xb[rt][h][0]), oa1, xb[rt][h][1]);
-          const f32x4 g4 =
-              valid[rt] ? *reinterpret_cast<const f32x4*>(dout + row[rt] * ds + 512 * h + f0 + fq) : zero4();
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float th = acc[i] * inv_tau + b4[i];
-            const float cs = amp * cos_rad(th), sn = amp * sin_rad(th);
-            dth[rt][u][i] = -sn * (g4[i] * ca[rt][h] - cs * cb[rt][h]);
-          }
-        }
+      for (int k = 0; k < 2; ++k) {
+        const int r = lane & 15;
+        ns[k] = ((sh.n2[4 * k][r] + sh.n2[4 * k + 1][r]) + sh.n2[4 * k + 2][r]) + sh.n2[4 * k + 3][r];
+        ts[k] = ((sh.tg[4 * k][r] + sh.tg[4 * k + 1][r]) + sh.tg[4 * k + 2][r]) + sh.tg[4 * k + 3][r];
+        nn[k] = sqrtf(ns[k]);
+        ie[k] = 1.f / (nn[k] + 1e-8f);
       }
+      const float cn = sqrtf(ns[0] * ie[0] * ie[0] + ns[1] * ie[1] * ie[1]);
+      const float iE = 1.f / (cn + 1e-7f);
+      const float s = ts[0] * ie[0] + ts[1] * ie[1];
+      const float corr = cn > 0.f ? s * iE * iE / cn : 0.f;
+      const float ieh = h ? ie[1] : ie[0], nh = h ? nn[1] : nn[0];
+      const float sh_ = (h ? ts[1] : ts[0]) * iE - corr * (h ? ns[1] : ns[0]) * ieh;
+      const float kh = nh > 0.f ? sh_ * ieh * ieh / nh : 0.f;
+      ca = iE * ieh;                 // times g
+      cb = corr * ieh * ieh + kh;    // times cs
+    }
+    f32x4 dxt[4];
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) dxt[jt] = zero4();
+#pragma unroll
+    for (int fb = 0; fb < 4; ++fb) {
+      const frag dth = P::from_f32(pair_to8(cb * sc[2 * fb] - ca * sg[2 * fb], cb * sc[2 * fb + 1] - ca * sg[2 * fb + 1]));
+#pragma unroll
+      for (int jt = 0; jt < 4; ++jt) dxt[jt] = P::mma(dxt[jt], frag_of_bf16<P>(sh.ot[w][fb * 4 + jt][lane]), dth);
+    }
+    if ((w & 3) != 0) {
+#pragma unroll
+      for (int jt = 0; jt < 4; ++jt) sh.dx[h][(w & 3) - 1][jt][lane] = dxt[jt];
+    }
+    lds_barrier();
+    const int64_t row = tile * 16 + (lane & 15);
+    if ((w & 3) == 0 && row < rows) {
 #pragma unroll
       for (int jt = 0; jt < 4; ++jt) {
-        const frag ot = P::from_f32(frag_cols_bf16(om, 64, 16 * jt, 32 * fb, lane));
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) dxt[rt][h][jt] = P::mma(dxt[rt][h][jt], ot, P::from_f32(pair_to8(dth[rt][0], dth[rt][1])));
+        const f32x4 t = ((dxt[jt] + sh.dx[h][0][jt][lane]) + sh.dx[h][1][jt][lane]) + sh.dx[h][2][jt][lane];
+        *reinterpret_cast<f32x4*>(dx + row * dxs + 64 * h + 16 * jt + fq) = inv_tau * t;
       }
-    }
-  }
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    if (valid[rt]) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt)
-          *reinterpret_cast<f32x4*>(dx + row[rt] * dxs + 64 * h + 16 * jt + fq) = inv_tau * dxt[rt][h][jt];
     }
   }
 }
@@ -1070,18 +1098,21 @@ extern "C" int kdn_fwht_lift_factored_bwd(const void* x, int64_t rows, int64_t x
       dx_row_stride % 4)
     return KDN_ERR_MISALIGNED;
   if (rows == 0) return KDN_OK;
-  const int64_t wgs = (rows + 64 * FLB_TILES - 1) / (64 * FLB_TILES);
-  if (wgs > 0x7fffffff) return KDN_ERR_UNSUPPORTED;
+  if ((rows + 127) / 128 > 0x7fffffff) return KDN_ERR_UNSUPPORTED;
+  int64_t wgs = (rows + 15) / 16;
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  if (wgs > cus) wgs = cus;
+  const int xvec = aligned(x, 16) && (rows == 1 || (x_row_stride * (int64_t)dtype_size(x_dtype)) % 16 == 0);
   const hipStream_t st = as_stream(stream);
   const __bf16* o1 = static_cast<const __bf16*>(omega1_bf16);
   const __bf16* o2 = static_cast<const __bf16*>(omega2_bf16);
   if (x_dtype == KDN_DTYPE_BF16)
-    hipLaunchKernelGGL((lift_factored_bwd_kernel<PrecBF16, __bf16>), dim3((unsigned)wgs), dim3(256), 0, st,
-                       static_cast<const __bf16*>(x), rows, x_row_stride, o1, phase1, o2, phase2, inv_tau, dout,
+    hipLaunchKernelGGL((lift_factored_bwd_kernel<PrecBF16, __bf16>), dim3((unsigned)wgs), dim3(512), 0, st,
+                       static_cast<const __bf16*>(x), rows, x_row_stride, xvec, o1, phase1, o2, phase2, inv_tau, dout,
                        dout_row_stride, dx, dx_row_stride);
   else
-    hipLaunchKernelGGL((lift_factored_bwd_kernel<PrecF32, float>), dim3((unsigned)wgs), dim3(256), 0, st,
-                       static_cast<const float*>(x), rows, x_row_stride, o1, phase1, o2, phase2, inv_tau, dout,
+    hipLaunchKernelGGL((lift_factored_bwd_kernel<PrecF32, float>), dim3((unsigned)wgs), dim3(512), 0, st,
+                       static_cast<const float*>(x), rows, x_row_stride, xvec, o1, phase1, o2, phase2, inv_tau, dout,
                        dout_row_stride, dx, dx_row_stride);
   return launch_status();
 }

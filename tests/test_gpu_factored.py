@@ -327,3 +327,20 @@ def test_d1024_scan_backward_rows_off_16_bytes(oprojs, dtype, dv, T):
     got = [dq[:, :, 0], dk[:, :, 0], dvv[:, :, 0], dbeta[:, :, 0], ddecay[:, :, 0], dinit[:, 0].transpose(1, 2)]
     for name, a, r in zip(("dphi_q", "dphi_k", "dv", "dbeta", "ddecay", "dS0"), got, ref):
         assert rel(a.cpu().numpy(), r) < tol, name
+
+
+@pytest.mark.parametrize("rows,offset", [(1, 0), (17, 1), (16 * 256 + 3, 0), (2 * 16 * 256 + 16, 1)])
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 5e-3)])
+def test_factored_lift_backward_row_counts(fproj, oprojs, dtype, tol, rows, offset):
+    # sixteen rows a workgroup and one workgroup per CU: one row, a second tile of one row, one tile more than the
+    # CUs take in their first turn, three turns; x rows off 16 bytes.  Tolerances as above.
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, 128 + offset, generator=g).to(dtype)
+    dphi = torch.randn(rows, 1024, generator=g)
+    p1, p2 = fproj.proj1, fproj.proj2
+    dx = ops.lift_factored_backward(x.to(DEV)[:, offset:], dphi.to(DEV), p1.device_omega(DEV), p1.device_phase(DEV),
+                                    p2.device_omega(DEV), p2.device_phase(DEV), p1.tau_star_inv)
+    torch.cuda.synchronize()
+    xr = x[:, offset:].double().requires_grad_(True)
+    (osc.factored_lift_torch(xr, *oprojs) * dphi.double()).sum().backward()
+    assert rel(dx.cpu().numpy(), xr.grad.numpy()) < tol
