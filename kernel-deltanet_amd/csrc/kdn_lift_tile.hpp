@@ -35,6 +35,9 @@ struct RawRow {
   }
 };
 
+// Slot of piece pc (16 bytes, columns 8 pc .. + 7) of row r of a 16-row tile of Omega in LDS.
+__device__ __forceinline__ int omega_slot(int r, int pc) { return r * 8 + (pc ^ ((r >> 1) & 7)); }
+
 // Lift of one 16-row tile per wave, for NX inputs at once (each Omega fragment feeds NX MFMAs).
 // Projection in the transposed orientation Phi^T = Omega X^T: accumulator tile t holds, in lane l,
 // feature 16t + 4(l>>4) + i of row (l & 15), which is slot (t & 1) * 4 + i of X fragment t / 2.
@@ -85,11 +88,12 @@ __device__ __forceinline__ void lift_tile(const RawRow<InT> (&raw)[NX], int norm
   // issued in the scheduling region of the cosines of tile t, with Omega's fragments for them read one
   // tile earlier still (so that the read's latency is covered by a tile's cosines, not waited on by the
   // MFMAs that follow it).
+  const int om_at = omega_slot(lane & 15, lane >> 4);
   auto fetch = [&](int t, bf16x8 (&a)[2]) {
     const int tg = tile0 + t;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
-      if constexpr (OMEGA_LDS) a[kb] = s_omega[(tg * 2 + kb) * 64 + lane];
+      if constexpr (OMEGA_LDS) a[kb] = s_omega[tg * 128 + (om_at ^ (4 * kb))];
       else a[kb] = *reinterpret_cast<const bf16x8*>(omega + (int64_t)(16 * tg + (lane & 15)) * 64 + 32 * kb + 8 * (lane >> 4));
     }
   };
@@ -158,24 +162,26 @@ __device__ __forceinline__ void lift_tile(const RawRow<InT> (&raw)[NX], int norm
   for (int x = 0; x < NX; ++x) ss[x] = sum_over_lane_groups(ss[x]);
 }
 
-// Omega as A fragments in LDS (lane l of fragment (t, kb): Omega[16t + (l&15)][32kb + 8(l>>4) .. +8])
-// and phase / (2 pi), by a workgroup of NTHREADS threads.  The fragment loop has a fixed trip count, so
-// that every load is issued before the first LDS store waits for one (a loop bounded by blockDim is not
-// unrolled and pays one L2 round trip per iteration).
+// Omega in LDS as its rows, and phase / (2 pi), by a workgroup of NTHREADS threads.  The rows (128 bytes, eight
+// pieces of 16) are copied by the load unit itself (global_load_lds), whole lines at a time: as fragments in
+// registers a load took half a line of each of 16 rows, and the CU takes one line every four to six cycles whatever
+// is used of it (the first 12 k cycles of a prep8 workgroup's 47 k; with the loads of q and k issued first).  A row's
+// pieces are permuted (omega_slot) so that the sixteen rows of a fragment read fall on distinct banks.  Ends with
+// the copies complete for this wave; the caller's barrier completes them for the workgroup.
 template <int D, bool OMEGA_LDS, int NTHREADS = 256>
 __device__ __forceinline__ void stage_omega(const __bf16* omega, const float* phase, bf16x8* s_omega, float* s_phrev) {
   if constexpr (OMEGA_LDS) {
-    constexpr int NF = (D / 16) * 2 * 64;
-    static_assert(NF % NTHREADS == 0, "fragment slots per thread");
-    bf16x8 v[NF / NTHREADS];
+    constexpr int NW = NTHREADS / 64, NB = D / 8;  // blocks of eight rows, 1 KB
+    static_assert(NB % NW == 0, "blocks per wave");
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-    for (int i = 0; i < NF / NTHREADS; ++i) {
-      const int idx = (int)threadIdx.x + NTHREADS * i;
-      const int l = idx & 63, tk = idx >> 6, t = tk >> 1, kb = tk & 1;
-      v[i] = *reinterpret_cast<const bf16x8*>(omega + (int64_t)(16 * t + (l & 15)) * 64 + 32 * kb + 8 * (l >> 4));
+    for (int i = 0; i < NB / NW; ++i) {
+      const int blk = i * NW + w;
+      const int row = 8 * blk + (lane >> 3);
+      __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(omega + row * 64 + 8 * ((lane & 7) ^ ((row >> 1) & 7))),
+                                       (__attribute__((address_space(3))) void*)(s_omega + blk * 64), 16, 0, 0);
     }
-#pragma unroll
-    for (int i = 0; i < NF / NTHREADS; ++i) s_omega[(int)threadIdx.x + NTHREADS * i] = v[i];
   }
   static_assert(D % NTHREADS == 0, "phases per thread");
   float ph[D / NTHREADS];
@@ -183,6 +189,7 @@ __device__ __forceinline__ void stage_omega(const __bf16* omega, const float* ph
   for (int i = 0; i < D / NTHREADS; ++i) ph[i] = phase[(int)threadIdx.x + NTHREADS * i];
 #pragma unroll
   for (int i = 0; i < D / NTHREADS; ++i) s_phrev[(int)threadIdx.x + NTHREADS * i] = ph[i] * 0.15915494309189535f;
+  if constexpr (OMEGA_LDS) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
 }
 
 }  // namespace kdn

@@ -145,8 +145,8 @@ __global__ void __launch_bounds__(256, (PrepWaves<P, FM>::value)) prep_kernel(Sc
     else store_frag_nt<P>(base, lane, f);
   };
   if constexpr (FM != FM_PRELIFTED) {
-    stage_omega<D, OMEGA_LDS>(omega_h, p.phase + h * p.phs, s_omega, s_phrev);
     in.template load_qk<NOQ>(p, sq, h, (p.chunk0 + cl0) * CH, w, lane);
+    stage_omega<D, OMEGA_LDS>(omega_h, p.phase + h * p.phs, s_omega, s_phrev);
   } else {
     // no lift: only beta / decay come through the prefetch
     const int64_t t = (p.chunk0 + cl0) * CH + lane;
@@ -426,7 +426,6 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
     else store_frag_nt<P>(base, lane, f);
   };
 
-  stage_omega<D, true, 512>(omega_h, p.phase + h * p.phs, s_omega, s_phrev);
   RawRow<InT> qk[2];
   {
     const int64_t trow = t0 + 16 * m + (lane & 15);
@@ -441,6 +440,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
     be = valid ? p.beta[sq.be + t * p.bs1 + h * p.bs2] : 0.f;
     la = (valid && p.decay) ? p.decay[sq.de + t * p.ds1 + h * p.ds2] : 1.f;
   }
+  stage_omega<D, true, 512>(omega_h, p.phase + h * p.phs, s_omega, s_phrev);
   lds_barrier();  // Omega staged
 
   // ---- beta and the in-chunk log-decay prefix (wave 0)
@@ -508,6 +508,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   for (int jl = 0; jl < NJH; ++jl) {
 #pragma unroll
     for (int mm = 0; mm < 4; ++mm) {
+      if (mm > m) break;  // above the diagonal: neither A nor P uses it
       const frag a = s_phik[(mm * NJ + NJH * hf + jl) * 64 + lane];
       gkk[mm] = P::mma(gkk[mm], a, cqk[1][jl]);
       gqk[mm] = P::mma(gqk[mm], a, cqk[0][jl]);
@@ -516,6 +517,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   lds_barrier();  // K fragments in LDS are dead from here on
 #pragma unroll
   for (int mm = 0; mm < 4; ++mm) {
+    if (mm > m) break;
     if (hf == 0) s_part[(m * 4 + mm) * 64 + lane] = gqk[mm];
     else s_part[((4 + m) * 4 + mm) * 64 + lane] = gkk[mm];
   }
@@ -530,6 +532,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
       const float bt = p.linear ? 0.f : s_beta[t], skt = s_sk[t];
 #pragma unroll
       for (int mm = 0; mm < 4; ++mm) {
+        if (mm > m) break;  // the inverse reads no block above the diagonal
         const f32x4 gk = gkk[mm] + s_part[((4 + m) * 4 + mm) * 64 + lane];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -543,6 +546,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
       f32x4 pt[4];
 #pragma unroll
       for (int mm = 0; mm < 4; ++mm) {
+        pt[mm] = zero4();
+        if (mm > m) continue;
         const f32x4 gq = s_part[(m * 4 + mm) * 64 + lane] + gqk[mm];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
