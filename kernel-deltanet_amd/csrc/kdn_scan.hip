@@ -33,114 +33,241 @@
 #include "kdn_io.hpp"
 #include "kdn_scan_common.hpp"
 #include "kdn_lift_tile.hpp"
+#include "kdn_tile.hpp"
 
 namespace kdn {
 
 // ------------------------------------------------------------------------------------------------
-// state: one workgroup of 4 waves per (head, 16 value components = 16 state rows), sequential over the
-// chunks of the segment.  Wave w owns features [128w, 128w + 128) of those rows: S^T tiles (feature
+// state (fp32 inputs): one workgroup of eight waves per (head, 16 value components = 16 state rows), sequential
+// over the chunks of the segment.  Wave w owns features [64w, 64w + 64) of those rows: S^T tiles (feature
 // tile, row tile) in accumulator layout, lane l holds S^T[16tt + 4(l>>4) + i][r0 + (l&15)].  Per chunk:
-//   checkpoint the chunk-start S^T (B fragments in the operand precision) for the output kernel
-//   X_K partial over the wave's features -> LDS -> barrier -> wave w reduces token tile w -> LDS -> barrier
-//   E tile w = U~ - Tp X_K (checkpointed) -> LDS -> barrier
-//   S^T <- gammaC S^T + K^T (kscale o E) on the wave's feature tiles, with the K^T operand read back
-//   transposed (ds_read_b64_tr_b16) from a wave-private LDS copy of the wave's K fragments.
-// Three workgroup barriers per chunk.  bf16: the K fragments and small operands of chunk c+1 are loaded
-// at the start of chunk c (a two-slot register ring) while an L2 prefetch runs L2_AHEAD chunks ahead;
-// the refill is unconditional (its chunk index is clamped to the segment) so that the compiler's
-// memory-counter waits stay static and only wait for the slot that is about to be used.
+//   checkpoint the chunk-start S^T (B fragments) for the output kernel; X_K partial over the wave's
+//   features -> LDS; the wave's K fragments -> a wave-private LDS copy               | A
+//   waves 0-3: X_K token tile w reduced -> LDS                                      | B
+//   waves 0-3: E tile w = U~ - Tp X_K (checkpointed) -> LDS, scaled by kscale         | C
+//   S^T <- gammaC S^T + K^T (kscale o E) on the wave's feature tiles, the K^T operand read back from the LDS copy
+// The bound is the fp32 matrix rate: 256 products of 32 cycles per SIMD and chunk, of which a step with its three
+// barriers took two and a half times that with four waves: one wave a SIMD waits for every LDS and memory
+// latency, each K^T operand was eight 4-byte reads with eight-fold bank conflicts, and the second of a lane's two
+// L2-prefetch loads was waited for where it was added to the first.  Now two waves share a SIMD, the copy is
+// permuted (f32_slot) so that neither its writes nor its reads conflict, K of the next chunk is loaded as soon as its
+// registers are free, and waves 4-7, idle during the reduction, read their K^T operands and prefetch into L2.
+// 4 heads, 16 chunks: 153 -> 101 us (9.6 -> 6.3 us a chunk).
 //
 // Workgroups are dispatched round-robin over the 8 XCDs (linear id % 8); the value tiles of one head
 // get ids with equal residue so that they share one XCD's L2 for the K fragments they all read.
-template <class P, int D, int DV>
-struct StateOps {
-  using L = WsLayout<P, D, DV>;
-  using frag = typename P::frag;
-  static constexpr int NJ = D / 32;
-  static constexpr int TPW = D / 64;   // feature tiles per wave
-  static constexpr int JPW = D / 128;  // 32-deep feature blocks per wave
+template <int DV>
+struct StateF32 {
+  using P = PrecF32;
+  using L = WsLayout<P, 512, DV>;
+  using frag = P::frag;
   static constexpr int NV = DV / 16;
-  static constexpr int L2_AHEAD = 3;  // chunks ahead of the current one that the L2 prefetch touches (3 measured best of 1, 3, 6)
-  // dword loads per wave that cover the operand area [0, Sfr) of one chunk record at one per line
-  static constexpr int L2_LOADS = (int)((L::Sfr / 128 + 4 * NV * 64 - 1) / (4 * NV * 64));
-  struct Small {
-    frag tp[2];  // Tp fragments of row tile w
-    f32x4 u;     // U~ tile (w, n)
-    f32x4 ks;    // kscale of the rows of token tile w, accumulator order
+  static constexpr int L2_AHEAD = 3;                // chunks ahead of the current one that the L2 prefetch touches
+  static constexpr int LINES = (int)(L::Sfr / 128);  // of the operand area
+  static constexpr int L2_LOADS = (LINES + 256 * NV - 1) / (256 * NV);
+  // The partial X_K tiles: tile m of wave v in part[m][v - (v > m)], except wave m's own (it adds it from its
+  // registers); part[m][0] takes the reduced tile.  160 KB with the K copies: the whole CU.
+  struct Shared {
+    frag k[8][8 * 64];   // wave-private K fragments [4 token tiles x 2 blocks], eight floats per f32_slot
+    f32x4 part[4][7][64];
+    f32x4 e[4][64];
+  };
+  struct Ops {
+    frag kx[4][2];
+    frag tp[2];   // waves 0-3: Tp row tile w, U~ tile, kscale (accumulator order)
+    f32x4 u, ks;
     float gC;
   };
-  // The operands of one chunk in four parts (token tile m of K plus one small operand each), so that
-  // the refill of a slot can be spread over the four barrier-separated phases of a step instead of
-  // queueing ~20 KB of loads per wave at once behind the texture unit.
-  template <int PART>
-  __device__ static void load_part(const unsigned char* ws, int w, int lane, int n, frag (&ak)[4][JPW], Small& sm) {
+  __device__ static void load_k(const unsigned char* ws, int w, int lane, Ops& o) {
 #pragma unroll
-    for (int jj = 0; jj < JPW; ++jj) ak[PART][jj] = load_frag<P>(ws + L::phiK + (size_t)(PART * NJ + JPW * w + jj) * 64 * L::FB, lane);
-    if constexpr (PART == 0) {
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
-      for (int jb = 0; jb < 2; ++jb) sm.tp[jb] = load_frag<P>(ws + L::Tp + (size_t)(w * 2 + jb) * 64 * L::FB, lane);
-    } else if constexpr (PART == 1) {
-      sm.u = *reinterpret_cast<const f32x4*>(ws + L::U + ((size_t)(w * NV + n) * 64 + lane) * 16);
-    } else if constexpr (PART == 2) {
-      sm.ks = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(ws + L::VEC) + 64 + 16 * w + 4 * (lane >> 4));
+      for (int jj = 0; jj < 2; ++jj) o.kx[m][jj] = load_frag<P>(uni(ws + L::phiK + (size_t)(m * 16 + 2 * w + jj) * 64 * L::FB), lane);
+  }
+  __device__ static void load_lead(const unsigned char* ws, int w, int n, int lane, Ops& o) {
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) o.tp[jb] = load_frag<P>(uni(ws + L::Tp + (size_t)(w * 2 + jb) * 64 * L::FB), lane);
+    o.u = reinterpret_cast<const f32x4*>(uni(ws + L::U + (size_t)(w * NV + n) * 64 * 16))[lane];
+    o.ks = reinterpret_cast<const f32x4*>(uni(ws + L::VEC + (64 + 16 * w) * 4))[lane >> 4];
+  }
+  __device__ static void load_g(const unsigned char* ws, Ops& o) { o.gC = reinterpret_cast<const float*>(uni(ws + L::VEC))[128]; }
+};
+
+// Slot (of 64, eight floats each) of the values of token c = 4g + e and features 4q .. 4q + 3 (+ 16) of a K fragment in
+// its LDS copy; the two halves of a slot change places where g >= 2.  The sixteen 16-byte writes of a lane group (16
+// tokens) and the 64 four-byte reads of a K^T operand (fixed e, all g, q and feature & 3) fall on distinct banks.
+__device__ __forceinline__ int f32_slot(int g, int e, int q) { return ((q ^ e) | ((g & 1) << 2)) + 8 * (e | ((g >> 1) << 2)); }
+
+template <int DV, bool DECAY, bool lead>
+__device__ __forceinline__ void state_f32_loop(const ScanParams& p, typename StateF32<DV>::Shared& sh, unsigned char* wsh, int nloc,
+                                               int w, int lane, int n, f32x4 (&S)[4]) {
+  using O = StateF32<DV>;
+  using P = PrecF32;
+  using L = typename O::L;
+  using frag = typename O::frag;
+  constexpr int NV = O::NV;
+  float* kl = reinterpret_cast<float*>(sh.k[w]);
+  const int kw = 8 * f32_slot((lane & 15) >> 2, lane & 3, lane >> 4);  // written: token lane & 15, features of lane >> 4
+  const int kflip = 4 * ((lane & 15) >> 3);
+  int kr[4];  // read: feature lane & 15, token 4 (lane >> 4) + e
+#pragma unroll
+  for (int e = 0; e < 4; ++e) kr[e] = 8 * f32_slot(lane >> 4, e, (lane & 15) >> 2) + 4 * (lane >> 5) + (lane & 3);
+  // K^T operand of feature tile tl (of the wave's four), tokens 32jb + kappa
+  auto kt_frag = [&](int tl, int jb) {
+    frag f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) f[s] = kl[(2 * (2 * jb + (s >> 2)) + (tl >> 1)) * 512 + (kr[s & 3] ^ (4 * (tl & 1)))];
+    return f;
+  };
+  typename O::Ops o;
+  O::load_k(wsh, w, lane, o);
+  O::load_g(wsh, o);
+  if constexpr (lead) O::load_lead(wsh, w, n, lane, o);
+  unsigned touch[O::L2_LOADS] = {}, sink = 0;  // the prefetched words, folded a chunk later, which keeps the loads
+  for (int cl = 0; cl < nloc; ++cl) {
+    unsigned char* cur = wsh + (int64_t)cl * L::bytes;
+    const unsigned char* nxt = wsh + (int64_t)(cl + 1 < nloc ? cl + 1 : cl) * L::bytes;
+    // X_K partial; checkpoint and K copy
+    frag sf[2];
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) sf[jj] = pair_to8(S[2 * jj], S[2 * jj + 1]);
+    f32x4 xp[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) xp[m] = zero4();
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) xp[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kx[m][jj][s], sf[jj][s], xp[m], 0, 0, 0);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          const frag& f = o.kx[m][jj];
+          const f32x4 v = {f[4 * hh], f[4 * hh + 1], f[4 * hh + 2], f[4 * hh + 3]};
+          *reinterpret_cast<f32x4*>(kl + (2 * m + jj) * 512 + kw + ((4 * hh) ^ kflip)) = v;
+        }
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) store_frag<P>(uni(cur + L::Sfr + (size_t)((2 * w + jj) * NV + n) * 64 * L::FB), lane, sf[jj]);
+    const float gC = o.gC;
+    __builtin_amdgcn_sched_barrier(0);
+    O::load_k(nxt, w, lane, o);
+    O::load_g(nxt, o);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      if (lead && m == w) continue;
+      sh.part[m][w - (w > m ? 1 : 0)][lane] = xp[m];
+    }
+    if constexpr (DECAY) {  // without decay gammaC is exactly 1
+#pragma unroll
+      for (int tl = 0; tl < 4; ++tl) S[tl] = S[tl] * gC;
+    }
+    lds_barrier();  // A
+    frag kt[lead ? 1 : 4][2];
+    if constexpr (lead) {
+      // wave w's own partial of tile w in its place of the order
+      f32x4 own = xp[0];
+#pragma unroll
+      for (int m = 1; m < 4; ++m) own = w == m ? xp[m] : own;
+      f32x4 X = w == 0 ? own : sh.part[w][0][lane];
+#pragma unroll
+      for (int v = 1; v < 8; ++v) X += v == w ? own : sh.part[w][v - (v > w ? 1 : 0)][lane];
+      sh.part[w][0][lane] = X;
+      lds_barrier();  // B
+      f32x4 ek = zero4();
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) ek = P::mma(ek, o.tp[jb], pair_to8(sh.part[2 * jb][0][lane], sh.part[2 * jb + 1][0][lane]));
+      const f32x4 e = o.u - ek;
+      sh.e[w][lane] = e * o.ks;
+      store_e_tile<P>(cur + L::Eck, (size_t)(w * NV + n), lane, e);
+      __builtin_amdgcn_sched_barrier(0);
+      O::load_lead(nxt, w, n, lane, o);
     } else {
-      sm.gC = reinterpret_cast<const float*>(ws + L::VEC)[128];
+#pragma unroll
+      for (int tl = 0; tl < 4; ++tl)
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb) kt[tl][jb] = kt_frag(tl, jb);
+      lds_barrier();  // B
+      const unsigned char* base = uni(wsh + (int64_t)(cl + O::L2_AHEAD < nloc ? cl + O::L2_AHEAD : nloc - 1) * L::bytes);
+#pragma unroll
+      for (int i = 0; i < O::L2_LOADS; ++i) {
+        const int li = ((n + i * NV) * 4 + (w - 4)) * 64 + lane;
+        sink ^= touch[i];
+        touch[i] = *reinterpret_cast<const unsigned*>(base + 128 * (li < O::LINES ? li : 0));
+      }
+    }
+    lds_barrier();  // C
+    frag eb[2];
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) eb[jb] = pair_to8(sh.e[2 * jb][lane], sh.e[2 * jb + 1][lane]);
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb) {
+      frag k4[4];
+#pragma unroll
+      for (int tl = 0; tl < 4; ++tl) {
+        if constexpr (lead) k4[tl] = kt_frag(tl, jb);
+        else k4[tl] = kt[tl][jb];
+      }
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int tl = 0; tl < 4; ++tl) S[tl] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[tl][s], eb[jb][s], S[tl], 0, 0, 0);
     }
   }
-  __device__ static void load_all(const unsigned char* ws, int w, int lane, int n, frag (&ak)[4][JPW], Small& sm) {
-    load_part<0>(ws, w, lane, n, ak, sm);
-    load_part<1>(ws, w, lane, n, ak, sm);
-    load_part<2>(ws, w, lane, n, ak, sm);
-    load_part<3>(ws, w, lane, n, ak, sm);
+  if (p.nseg < 0) p.state_out[0] = (float)sink;  // never: nseg is at least 1
+}
+
+template <int DV, bool DECAY>
+__global__ void __launch_bounds__(512) state_kernel(ScanParams p) {
+  using O = StateF32<DV>;
+  using L = typename O::L;
+  constexpr int NV = O::NV;
+  __shared__ typename O::Shared sh;
+
+  // XCD-aware decomposition of the 1-D grid: id = xcd + 8 * (rank * NV + n), head-batch pair
+  // hb = rank * 8 + xcd.  Ids that land past B*H exit at once.
+  const int64_t id = blockIdx.x;
+  const int64_t xcd = id & 7, jdx = id >> 3;
+  const int n = (int)(jdx % NV);
+  const int64_t hb = (jdx / NV) * 8 + xcd;
+  if (hb >= p.B * p.H) return;
+  int64_t b, h, nloc, cfirst;
+  size_t woff;
+  if (!state_item<L::bytes>(p, hb, b, h, nloc, woff, cfirst)) return;
+  const int64_t sl = p.slots ? (int64_t)p.slots[b] : b;
+  if (sl < 0) return;  // a skipped sequence of a ragged step (its state is not touched)
+
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = 16 * n + (lane & 15);
+  f32x4 S[4];
+  const float* si = p.state_in ? p.state_in + sl * p.is0 + h * p.is1 + r * p.is3 : nullptr;
+#pragma unroll
+  for (int tl = 0; tl < 4; ++tl)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[tl][i] = si ? si[(int64_t)(64 * w + 16 * tl + 4 * (lane >> 4) + i) * p.is2] : 0.f;
+  if (nloc > 0) {  // an empty sequence (uniform across the workgroup) runs no chunk
+    unsigned char* wsh = uni(p.ws + woff);
+    const int nc = __builtin_amdgcn_readfirstlane((int)nloc);
+    if (w < 4) state_f32_loop<DV, DECAY, true>(p, sh, wsh, nc, w, lane, n, S);
+    else state_f32_loop<DV, DECAY, false>(p, sh, wsh, nc, w, lane, n, S);
   }
-};
-
-struct StateShared {
-  f32x4 xp[4][4][64];  // per-wave partial X_K tiles [wave][token tile][lane]
-  f32x4 x[4][64];      // reduced X_K [token tile][lane]
-  f32x4 e[4][64];      // E tiles [token tile][lane]
-};
-
-// Wave-private LDS copy of the wave's 16 K fragments (token tile m, local 32-feature block jj), from
-// which the K^T operand of the state update is read back transposed.
-//   bf16: two planes of 8 KB; plane h holds bytes [8h, 8h+8) of every lane's 16-byte fragment slot
-//         (features 16h .. 16h+15 of the 32-block) at (fragment * 64 + kimg_swizzle(lane)) * 8, the
-//         layout of the record's K image (bank-conflict-free for the plain and the transposed read).
-//   fp32: fragments in lane order, 32 bytes per lane.
-template <class P>
-__device__ __forceinline__ void stage_k(typename P::frag* kl, int lane, const typename P::frag (&ak)[4][4]);
-
-template <>
-__device__ __forceinline__ void stage_k<PrecBF16>(PrecBF16::frag* kl, int lane, const PrecBF16::frag (&ak)[4][4]) {
-  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-  unsigned char* base = reinterpret_cast<unsigned char*>(kl);
+  float* so = p.state_out + sl * p.os0 + h * p.os1 + r * p.os3;
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
+  for (int tl = 0; tl < 4; ++tl)
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int fi = m * 4 + jj;
-      *reinterpret_cast<bf16x4*>(base + (size_t)(fi * 64 + kimg_swizzle(lane)) * 8) =
-          __builtin_shufflevector(ak[m][jj], ak[m][jj], 0, 1, 2, 3);
-      *reinterpret_cast<bf16x4*>(base + 8192 + (size_t)(fi * 64 + kimg_swizzle(lane)) * 8) =
-          __builtin_shufflevector(ak[m][jj], ak[m][jj], 4, 5, 6, 7);
-    }
+    for (int i = 0; i < 4; ++i) so[(int64_t)(64 * w + 16 * tl + 4 * (lane >> 4) + i) * p.os2] = S[tl][i];
 }
 
-template <>
-__device__ __forceinline__ void stage_k<PrecF32>(PrecF32::frag* kl, int lane, const PrecF32::frag (&ak)[4][4]) {
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) kl[(m * 4 + jj) * 64 + lane] = ak[m][jj];
-}
-
-// K^T operand (wave-local feature tile tl, chunk block jb) from the staged copy:
+// The bf16 state kernel's K^T operand (wave-local feature tile tl, chunk block jb) from its slice of a chunk's K image:
 // lane l slot s = K[32jb + kappa(l,s)][16tl + (l&15)].
-template <class P>
-__device__ __forceinline__ typename P::frag kt_frag(const typename P::frag* kl, int lane, int tl, int jb);
-
-template <>
-__device__ __forceinline__ PrecBF16::frag kt_frag<PrecBF16>(const PrecBF16::frag* kl, int lane, int tl, int jb) {
+//   Two planes of 8 KB; plane h holds bytes [8h, 8h+8) of every lane's 16-byte fragment slot
+//   (features 16h .. 16h+15 of the 32-block) at (fragment * 64 + kimg_swizzle(lane)) * 8, the
+//   layout of the record's K image (bank-conflict-free for the plain and the transposed read).
+__device__ __forceinline__ PrecBF16::frag kt_frag(const PrecBF16::frag* kl, int lane, int tl, int jb) {
   // ds_read_b64_tr_b16: in each 16-lane group, output lane i slot v = element (i & 3) of the 8-byte run
   // addressed by lane 4v + (i >> 2).  Source lane (group g, j = l & 15) addresses the 4 features
   // 16tl + 4(j & 3) .. +3 of chunk row c = 32jb + 16 half + 4g + (j >> 2); in X-fragment order that run
@@ -162,213 +289,15 @@ __device__ __forceinline__ PrecBF16::frag kt_frag<PrecBF16>(const PrecBF16::frag
   return __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-template <>
-__device__ __forceinline__ PrecF32::frag kt_frag<PrecF32>(const PrecF32::frag* kl, int lane, int tl, int jb) {
-  const float* e = reinterpret_cast<const float*>(kl);
-  PrecF32::frag f;
-  const int d = 16 * tl + (lane & 15);  // wave-local feature
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const int c = 32 * jb + kappa(lane, s);
-    const int fi = (c >> 4) * 4 + (d >> 5);
-    f[s] = e[((size_t)fi * 64 + (c & 15) + 16 * ((d >> 2) & 3)) * 8 + 4 * ((d >> 4) & 1) + (d & 3)];
-  }
-  return f;
-}
-
-// The sequential loop is rotated so that one scheduling region (between the third barrier of chunk c
-// and the first barrier of chunk c+1) holds the state update of chunk c, the refill loads, the
-// checkpoint stores and the X_K product of chunk c+1.  Per CU each chunk moves ~100 KB through the
-// texture unit (64 KB of K, the checkpoint and the small operands) at ~64 B/clk, so these memory
-// instructions are interleaved one-for-one with the MFMAs of the region (sched_group_barrier) instead
-// of being issued in a burst that would block the in-order wave for ~1500 cycles.
-
-// Phase 1 of chunk cl (region ending at barrier A): checkpoint S^T, X_K partial from the K fragments
-// in `ak`, stage `ak` for the transposed read, publish the partial.
-template <class P, int D, int DV>
-__device__ __forceinline__ void state_phase1(StateShared& sh, typename P::frag* kl, unsigned char* cur, int w, int lane,
-                                             int n, const f32x4 (&S)[D / 64], const typename P::frag (&ak)[4][D / 128]) {
-  using O = StateOps<P, D, DV>;
-  using L = typename O::L;
-  using frag = typename P::frag;
-  constexpr int JPW = O::JPW, NV = O::NV;
-  frag sf[JPW];
-#pragma unroll
-  for (int jj = 0; jj < JPW; ++jj) {
-    sf[jj] = P::from_f32(pair_to8(S[2 * jj], S[2 * jj + 1]));
-    store_frag<P>(cur + L::Sfr + (size_t)((JPW * w + jj) * NV + n) * 64 * L::FB, lane, sf[jj]);
-  }
-  f32x4 xp[4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    xp[m] = zero4();
-#pragma unroll
-    for (int jj = 0; jj < JPW; ++jj) xp[m] = P::mma(xp[m], ak[m][jj], sf[jj]);
-  }
-  stage_k<P>(kl, lane, ak);
-#pragma unroll
-  for (int m = 0; m < 4; ++m) sh.xp[w][m][lane] = xp[m];
-}
-
-// Phase 2 of chunk cl (after barrier A, through barrier C): reduce X_K tile w, E tile w = U~ - Tp X_K
-// (checkpointed; shared scaled by kscale).
-template <class P, int D, int DV>
-__device__ __forceinline__ void state_phase2(StateShared& sh, unsigned char* cur, int w, int lane, int n,
-                                             const typename StateOps<P, D, DV>::Small& sm) {
-  using O = StateOps<P, D, DV>;
-  using L = typename O::L;
-  constexpr int NV = O::NV;
-  sh.x[w][lane] = sh.xp[0][w][lane] + sh.xp[1][w][lane] + sh.xp[2][w][lane] + sh.xp[3][w][lane];
-  __syncthreads();
-  f32x4 ek = zero4();
-#pragma unroll
-  for (int jb = 0; jb < 2; ++jb) ek = P::mma(ek, sm.tp[jb], P::from_f32(pair_to8(sh.x[2 * jb][lane], sh.x[2 * jb + 1][lane])));
-  const f32x4 e = sm.u - ek;
-  sh.e[w][lane] = e * sm.ks;
-  store_e_tile<P>(cur + L::Eck, (size_t)(w * NV + n), lane, e);
-  __syncthreads();
-}
-
-// Phase 3 of chunk cl: S^T = gammaC S^T + K^T (kscale o E) on the wave's feature tiles.
-template <class P, int D, int DV, bool DECAY>
-__device__ __forceinline__ void state_phase3(StateShared& sh, const typename P::frag* kl, int lane, f32x4 (&S)[D / 64],
-                                             float gC) {
-  using frag = typename P::frag;
-  constexpr int TPW = D / 64;
-  frag eb[2];
-#pragma unroll
-  for (int jb = 0; jb < 2; ++jb) eb[jb] = P::from_f32(pair_to8(sh.e[2 * jb][lane], sh.e[2 * jb + 1][lane]));
-#pragma unroll
-  for (int tl = 0; tl < TPW; ++tl) {
-    f32x4 acc = S[tl];
-    if constexpr (DECAY) acc = acc * gC;  // without decay gammaC is exactly 1
-#pragma unroll
-    for (int jb = 0; jb < 2; ++jb) acc = P::mma(acc, kt_frag<P>(kl, lane, tl, jb), eb[jb]);
-    S[tl] = acc;
-  }
-}
-
-// L2 prefetch of the operands of chunk cp: the 4 NV waves of a head touch one dword per 128-byte line
-// of its K / Tp / P / U~ / scale area.  The dword loaded one iteration earlier is folded into l2acc so
-// that the load is kept; it has long completed by then.
-template <class P, int D, int DV>
-__device__ __forceinline__ void l2_prefetch(const unsigned char* base, int w, int lane, int n, unsigned& slot, unsigned& acc) {
-  using O = StateOps<P, D, DV>;
-  using L = typename O::L;
-  acc += slot;
-  unsigned v = 0;
-#pragma unroll
-  for (int i = 0; i < O::L2_LOADS; ++i) {
-    const size_t off = ((size_t)((i * 4 * O::NV + n * 4 + w) * 64 + lane)) * 128;
-    if (off < L::Sfr) v += *reinterpret_cast<const unsigned*>(base + off);
-  }
-  slot = v;
-}
-
-// One iteration of the rotated loop for chunk cl, whose operands are in (ak_c, sm_c) and whose K is
-// staged in LDS; (ak_n, sm_n) hold chunk cl+1.  Phase 2 and 3 of chunk cl, then -- if cl+1 exists --
-// the refill of (ak_c, sm_c) with chunk min(cl+2, last) and phase 1 of chunk cl+1, then barrier A.
-template <class P, int D, int DV, bool DECAY>
-__device__ __forceinline__ bool state_iter(const ScanParams& p, StateShared& sh, typename P::frag* kl, unsigned char* wsh,
-                                           int64_t cl, int w, int lane, int n, f32x4 (&S)[D / 64],
-                                           typename P::frag (&ak_c)[4][D / 128], typename StateOps<P, D, DV>::Small& sm_c,
-                                           typename P::frag (&ak_n)[4][D / 128], typename StateOps<P, D, DV>::Small& sm_n,
-                                           unsigned& l2slot, unsigned& l2acc, int64_t nloc) {
-  using O = StateOps<P, D, DV>;
-  using L = typename O::L;
-  unsigned char* cur = wsh + cl * L::bytes;
-  state_phase2<P, D, DV>(sh, cur, w, lane, n, sm_c);
-  const float gC = sm_c.gC;
-  state_phase3<P, D, DV, DECAY>(sh, kl, lane, S, gC);
-  // Unconditional (no branch splits the region): after the last chunk, phase 1 runs on the clamped
-  // operands of the last chunk and writes its checkpoint into the record after the last chunk (the
-  // spare record nseg of the head, or an unused record of a ragged sequence that ends earlier).
-  const int64_t cr = (cl + 2 < nloc) ? cl + 2 : nloc - 1;
-  O::load_all(wsh + cr * L::bytes, w, lane, n, ak_c, sm_c);
-  const int64_t cp = (cl + 1 + O::L2_AHEAD < nloc) ? cl + 1 + O::L2_AHEAD : nloc - 1;
-  l2_prefetch<P, D, DV>(wsh + cp * L::bytes, w, lane, n, l2slot, l2acc);
-  state_phase1<P, D, DV>(sh, kl, cur + L::bytes, w, lane, n, S, ak_n);
-  // 32 MFMAs (16 update, 16 X_K) and ~26 memory instructions: alternate them.
-#pragma unroll
-  for (int i = 0; i < 26; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-    __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);  // one vector-memory instruction
-  }
-  __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
-  __syncthreads();
-  return cl + 1 < nloc;
-}
-
-template <class P, int D, int DV, bool DECAY>
-__global__ void __launch_bounds__(256) state_kernel(ScanParams p) {
-  using O = StateOps<P, D, DV>;
-  using L = typename O::L;
-  using frag = typename P::frag;
-  constexpr int TPW = O::TPW, JPW = O::JPW, NV = O::NV;
-  __shared__ StateShared sh;
-  __shared__ frag s_kl[4][4 * JPW * 64];  // wave-private K fragments
-
-  // XCD-aware decomposition of the 1-D grid: id = xcd + 8 * (rank * NV + n), head-batch pair
-  // hb = rank * 8 + xcd.  Ids that land past B*H exit at once.
-  const int64_t id = blockIdx.x;
-  const int64_t xcd = id & 7, jdx = id >> 3;
-  const int n = (int)(jdx % NV);
-  const int64_t hb = (jdx / NV) * 8 + xcd;
-  if (hb >= p.B * p.H) return;
-  int64_t b, h, nloc, cfirst;
-  size_t woff;
-  if (!state_item<L::bytes>(p, hb, b, h, nloc, woff, cfirst)) return;
-  const int64_t sl = p.slots ? (int64_t)p.slots[b] : b;
-  if (sl < 0) return;  // a skipped sequence of a ragged step (its state is not touched)
-
-  const int lane = threadIdx.x & 63;
-  // The wave index is uniform across the wave; reading it into a scalar register lets every
-  // fragment address be a scalar base plus the per-lane offset.
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = 16 * n + (lane & 15);
-  frag* kl = s_kl[w];
-
-  f32x4 S[TPW];
-  if (p.state_in) {
-    const float* si = p.state_in + sl * p.is0 + h * p.is1 + r * p.is3;
-#pragma unroll
-    for (int tl = 0; tl < TPW; ++tl)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) S[tl][i] = si[(int64_t)(16 * (TPW * w + tl) + 4 * (lane >> 4) + i) * p.is2];
-  } else {
-#pragma unroll
-    for (int tl = 0; tl < TPW; ++tl) S[tl] = zero4();
-  }
-
-  unsigned char* wsh = p.ws + woff;
-  frag k0[4][JPW], k1[4][JPW];
-  typename O::Small s0, s1;
-  unsigned l2acc = 0, l2s0 = 0, l2s1 = 0;  // sink of the L2-prefetch loads (never stored; see below)
-  if (nloc > 0) {  // an empty sequence (uniform across the workgroup) runs no chunk
-    // Prologue: chunk 0 in slot 0, chunk min(1, last) in slot 1, phase 1 of chunk 0.
-    O::load_all(wsh, w, lane, n, k0, s0);
-    O::load_all(wsh + (nloc > 1 ? L::bytes : 0), w, lane, n, k1, s1);
-    state_phase1<P, D, DV>(sh, kl, wsh, w, lane, n, S, k0);
-    __syncthreads();
-    for (int64_t cl = 0;; cl += 2) {
-      if (!state_iter<P, D, DV, DECAY>(p, sh, kl, wsh, cl, w, lane, n, S, k0, s0, k1, s1, l2s0, l2acc, nloc)) break;
-      if (!state_iter<P, D, DV, DECAY>(p, sh, kl, wsh, cl + 1, w, lane, n, S, k1, s1, k0, s0, l2s1, l2acc, nloc)) break;
-    }
-    l2acc += l2s0 + l2s1;
-  }
-
-  float* so = p.state_out + sl * p.os0 + h * p.os1 + r * p.os3;
-#pragma unroll
-  for (int tl = 0; tl < TPW; ++tl)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) so[(int64_t)(16 * (TPW * w + tl) + 4 * (lane >> 4) + i) * p.os2] = S[tl][i];
-  // Keeps the prefetch loads alive: nseg is at least 1, so this branch never runs.
-  if (p.nseg < 0) so[0] = (float)l2acc;
-}
+struct StateShared {
+  f32x4 xp[4][4][64];  // per-wave partial X_K tiles [wave][token tile][lane]
+  f32x4 x[4][64];      // reduced X_K [token tile][lane]
+  f32x4 e[4][64];      // E tiles [token tile][lane]
+};
 
 // ------------------------------------------------------------------------------------------------
 // state (bf16, D = 512): the carry of state_kernel with each chunk's lifted keys streamed by a fifth
-// wave.  Waves 0-3 carry the state as state_kernel does (wave w owns features [128w, 128w + 128) of the
+// wave.  Waves 0-3 carry the state (wave w owns features [128w, 128w + 128) of the
 // workgroup's 16 state rows; the same products in the same order, so the results are identical).  Wave 4
 // copies each chunk's K image (64 KB, written by prep in the LDS layout, store_k_image) into a two-slot
 // LDS ring with global_load_lds_dwordx4 one chunk ahead, and touches the records L2_AHEAD chunks ahead
@@ -398,14 +327,20 @@ __device__ __forceinline__ void wait_vmcnt() {
 
 template <int DV>
 struct DmaState {
-  using O = StateOps<PrecBF16, 512, DV>;
-  using L = typename O::L;
+  using L = WsLayout<PrecBF16, 512, DV>;
   static constexpr int NV = DV / 16;
+  static constexpr int L2_AHEAD = 3;  // chunks ahead of the current one that the L2 prefetch covers (best of 1, 3, 6)
+  struct Small {
+    PrecBF16::frag tp[2];  // Tp fragments of row tile w
+    f32x4 u;               // U~ tile (w, n)
+    f32x4 ks;              // kscale of the rows of token tile w, accumulator order
+    float gC;
+  };
   static constexpr int KIMG = 4 * KIMG_SLICE;  // bytes of a chunk's K image
   // dword loads of the L2 prefetch per loader wave: one per 128-byte line of the operand area [0, Sfr),
   // shared by the NV workgroups of a head
   static constexpr int L2_LOADS = (int)((L::Sfr / 128 + 64 * NV - 1) / (64 * NV));
-  __device__ static void load_small(const unsigned char* ws, int w, int lane, int n, typename O::Small& sm) {
+  __device__ static void load_small(const unsigned char* ws, int w, int lane, int n, Small& sm) {
 #pragma unroll
     for (int jb = 0; jb < 2; ++jb) sm.tp[jb] = load_frag<PrecBF16>(ws + L::Tp + (size_t)(w * 2 + jb) * 64 * L::FB, lane);
     sm.u = *reinterpret_cast<const f32x4*>(ws + L::U + ((size_t)(w * NV + n) * 64 + lane) * 16);
@@ -425,7 +360,7 @@ struct DmaState {
 // sm its small operands, refilled here with those of chunk min(cl + 2, last).
 template <int DV, bool DECAY>
 __device__ __forceinline__ void dma_step(StateShared& sh, const unsigned char* kw, unsigned char* wsh, int64_t cl,
-                                         int w, int lane, int n, f32x4 (&S)[8], typename StateOps<PrecBF16, 512, DV>::Small& sm,
+                                         int w, int lane, int n, f32x4 (&S)[8], typename DmaState<DV>::Small& sm,
                                          int64_t nloc) {
   using P = PrecBF16;
   using Dm = DmaState<DV>;
@@ -470,7 +405,7 @@ __device__ __forceinline__ void dma_step(StateShared& sh, const unsigned char* k
     f32x4 acc = S[tl];
     if constexpr (DECAY) acc = acc * gC;  // without decay gammaC is exactly 1
 #pragma unroll
-    for (int jb = 0; jb < 2; ++jb) acc = P::mma(acc, kt_frag<P>(kl, lane, tl, jb), eb[jb]);
+    for (int jb = 0; jb < 2; ++jb) acc = P::mma(acc, kt_frag(kl, lane, tl, jb), eb[jb]);
     S[tl] = acc;
   }
   __syncthreads();  // D
@@ -480,7 +415,6 @@ template <int DV, bool DECAY>
 __global__ void __launch_bounds__(320) state_kernel_dma(ScanParams p) {
   using P = PrecBF16;
   using Dm = DmaState<DV>;
-  using O = typename Dm::O;
   using L = typename Dm::L;
   constexpr int NV = Dm::NV;
   __shared__ StateShared sh;
@@ -518,7 +452,7 @@ __global__ void __launch_bounds__(320) state_kernel_dma(ScanParams p) {
       if (cl + 1 < nloc) Dm::copy_k(wsh + (cl + 1) * L::bytes, ((cl + 1) & 1) ? s_ring1 : s_ring0, lane);
       // L2 prefetch: one dword per 128-byte line of the operand area of chunk cl + 1 + L2_AHEAD, each lane
       // its own line, copied into a scratch LDS word (no register result, so nothing waits for it)
-      const int64_t cp = (cl + 1 + O::L2_AHEAD < nloc) ? cl + 1 + O::L2_AHEAD : nloc - 1;
+      const int64_t cp = (cl + 1 + Dm::L2_AHEAD < nloc) ? cl + 1 + Dm::L2_AHEAD : nloc - 1;
       const unsigned char* pb = wsh + cp * L::bytes;
 #pragma unroll
       for (int i = 0; i < Dm::L2_LOADS; ++i) {
@@ -548,7 +482,7 @@ __global__ void __launch_bounds__(320) state_kernel_dma(ScanParams p) {
     for (int tl = 0; tl < 8; ++tl) S[tl] = zero4();
   }
   if (nloc > 0) {
-    typename O::Small sm0, sm1;
+    typename Dm::Small sm0, sm1;
     Dm::load_small(wsh, w, lane, n, sm0);
     Dm::load_small(wsh + (nloc > 1 ? L::bytes : 0), w, lane, n, sm1);
     __syncthreads();  // P: slot 0 holds chunk 0
@@ -837,11 +771,6 @@ static ScanParams flat_params(const kdn_scan_args* a, const RunSpec& r, int64_t 
   return p;
 }
 
-// The state kernel keeps its CU to itself: 40 KB of unused dynamic LDS raise its request to 128 KB, so
-// that neither a prep workgroup (~131 KB) nor an output workgroup (~49 KB) fits beside it in the CU's
-// 160 KB and takes issue slots from the sequential chain.
-constexpr int STATE_EXCLUSIVE_LDS = 40 * 1024;
-
 template <class P, typename InT, typename OutT, int D, int DV>
 static int launch_phase(const ScanParams& p, int phase, hipStream_t st) {
   if (phase == PHASE_PREP) {
@@ -850,16 +779,15 @@ static int launch_phase(const ScanParams& p, int phase, hipStream_t st) {
     if constexpr (Fused<P, D>::value) return launch_chain<OutT, DV>(p, st);
     return KDN_ERR_UNSUPPORTED;
   } else if (phase == PHASE_STATE) {
-    // The state workgroups are the sequential critical path: reserve enough LDS that no prep or output
-    // workgroup can share their CU (a CU has 160 KB; the bf16 state kernel uses 88 KB statically).
-    // (bf16: the streaming kernel's 152 KB of LDS keep its CU exclusive by themselves.)
+    // The state workgroups are the sequential critical path: their LDS (152 and 160 KB) keeps prep and output
+    // workgroups off their CUs.
     if constexpr (IsBF16<P>::value && D == 512) {
       if (p.decay) hipLaunchKernelGGL((state_kernel_dma<DV, true>), dim3(state_grid(p.B, p.H, DV / 16)), dim3(320), 0, st, p);
       else hipLaunchKernelGGL((state_kernel_dma<DV, false>), dim3(state_grid(p.B, p.H, DV / 16)), dim3(320), 0, st, p);
     } else {
-      const size_t excl = IsBF16<P>::value ? (size_t)STATE_EXCLUSIVE_LDS : 0;
-      if (p.decay) hipLaunchKernelGGL((state_kernel<P, D, DV, true>), dim3(state_grid(p.B, p.H, DV / 16)), dim3(256), excl, st, p);
-      else hipLaunchKernelGGL((state_kernel<P, D, DV, false>), dim3(state_grid(p.B, p.H, DV / 16)), dim3(256), excl, st, p);
+      static_assert(!IsBF16<P>::value && D == 512, "the fp32 carry");
+      if (p.decay) hipLaunchKernelGGL((state_kernel<DV, true>), dim3(state_grid(p.B, p.H, DV / 16)), dim3(512), 0, st, p);
+      else hipLaunchKernelGGL((state_kernel<DV, false>), dim3(state_grid(p.B, p.H, DV / 16)), dim3(512), 0, st, p);
     }
   } else {
     // Beside the state kernel (p.out_wgs > 0): at most one workgroup per CU it leaves free, each CU held
