@@ -210,6 +210,14 @@ __device__ __forceinline__ typename P::frag bf16_frag(const bf16x8& t) {
 }
 
 
+// A fragment of Omega held in registers, converted at its use (held converted, fp32's would take twice as many).
+template <class P>
+__device__ __forceinline__ typename P::frag omega_reg(const bf16x8& t) {
+  bf16x8 u = t;
+  if constexpr (!IsBf16Policy<P>::value) asm volatile("" : "+v"(u));
+  return bf16_frag<P>(u);
+}
+
 // Thread `tid` of 256 holds 16 consecutive features (tid & 3) * 16 .. of token row tid >> 2: loads the
 // raw row part of x (zero past T), its L2 norm over the 64 features (shared by the four threads of the
 // row), and the normalised part (x / max(|x|, 1e-6), or x itself without normalisation).
@@ -306,6 +314,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const __bf16* oml = LO ? p.omega_lo + h * p.oms : nullptr;
   const float* phs = p.phase + h * p.phs;
   const float itau = head_inv_tau(p, h);
+  // This wave's 128 rows of Omega and its phases, kept in registers for the four lifts below (q and k, two halves
+  // of the tokens), instead of read in each of them, half a line of sixteen rows per load.  With the Grams below:
+  // 4096 chunks, bf16, 586 -> 573 us; fp32 with low parts, 1024 chunks, 238 -> 216 us.  What bounds the kernel is the
+  // record it writes, 380 KB a chunk in bf16.
+  bf16x8 og[8][2];
+  float phg[8];
+#pragma unroll
+  for (int ft = 0; ft < 8; ++ft) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+      og[ft][kb] = *reinterpret_cast<const bf16x8*>(om + (size_t)(128 * w + 16 * ft + (lane & 15)) * DK + 32 * kb + 8 * (lane >> 4));
+    phg[ft] = phs[128 * w + 16 * ft + (lane & 15)];
+  }
   for (int which = 0; which < 2; ++which) {  // 0: q, 1: k
     const InT* x = reinterpret_cast<const InT*>(which == 0 ? p.q : p.k);
     const int64_t xb = which == 0 ? b * p.qs0 + (t0 + r) * p.qs1 + h * p.qs2 : b * p.ks0 + (t0 + r) * p.ks1 + h * p.ks2;
@@ -323,29 +344,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     typename Feat<P>::T* phi = feat<P>(rec, which == 0 ? Rec::Q : Rec::K);
     for (int hm = 0; hm < 2; ++hm) {
       f32x4 acc[8][2];
-      f32x8 xa[2][2];
+      typename P::frag xa[2][2];
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int jb = 0; jb < 2; ++jb) xa[u][jb] = frag_rows_plain(xs, LD, 16 * (2 * hm + u), 32 * jb, lane);
+        for (int jb = 0; jb < 2; ++jb) xa[u][jb] = P::from_f32(frag_rows_plain(xs, LD, 16 * (2 * hm + u), 32 * jb, lane));
       float ss[2][4];
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int i = 0; i < 4; ++i) ss[u][i] = 0.f;
-      // Omega rows and phases of feature tile ft + 1 are issued in the region of tile ft
-      f32x8 on0 = frag_rows_plain_bf16(om, DK, 128 * w, 0, lane), on1 = frag_rows_plain_bf16(om, DK, 128 * w, 32, lane);
-      float phn = phs[128 * w + (lane & 15)];
 #pragma unroll
       for (int ft = 0; ft < 8; ++ft) {
         const int f0 = 128 * w + 16 * ft;
-        const f32x8 o0 = on0, o1 = on1;
-        const float ph = phn;
-        if (ft + 1 < 8) {
-          on0 = frag_rows_plain_bf16(om, DK, f0 + 16, 0, lane);
-          on1 = frag_rows_plain_bf16(om, DK, f0 + 16, 32, lane);
-          phn = phs[f0 + 16 + (lane & 15)];
-        }
+        const typename P::frag o0 = omega_reg<P>(og[ft][0]), o1 = omega_reg<P>(og[ft][1]);
+        const float ph = phg[ft];
         f32x8 l0 = {}, l1 = {};
         if constexpr (LO) {  // the low parts: their products are added like the forward's
           l0 = frag_rows_plain_bf16(oml, DK, f0, 0, lane);
@@ -353,8 +366,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          f32x4 sv = mm<P>(mm<P>(zero4(), xa[u][0], o0), xa[u][1], o1);
-          if constexpr (LO) sv = mm<P>(mm<P>(sv, xa[u][0], l0), xa[u][1], l1);
+          f32x4 sv = P::mma(P::mma(zero4(), xa[u][0], o0), xa[u][1], o1);
+          if constexpr (LO) sv = P::mma(P::mma(sv, xa[u][0], P::from_f32(l0)), xa[u][1], P::from_f32(l1));
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float v = amp * cos_rad(sv[i] * itau + ph);
@@ -471,45 +484,84 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
   __syncthreads();  // a o dY in bA is dead from here on (bA becomes A below)
 
-  // Gram matrices (row tile w) from the features just written, in fragment order (one contiguous 16- or
-  // 32-byte piece per lane; Q from its rows with fp32 features); A and P into LDS.
+  // Gram matrices: each wave the products over its 128 features of the tiles on and below the diagonal, from the
+  // fragments it has just written (one contiguous 16- or 32-byte piece per lane; Q from its rows with fp32
+  // features), the four waves' parts added in LDS; A and P into LDS.  A row tile per wave over all features read
+  // every fragment of K in every wave, 384 KB a chunk.
   {
+    using frag = typename P::frag;
     const typename Feat<P>::T* Q = feat<P>(rec, Rec::Q);
-    const typename P::frag* kxf = reinterpret_cast<const typename P::frag*>(rec + Rec::KXF);
-    f32x4 gkk[4], gqk[4];
+    const frag* kxf = reinterpret_cast<const frag*>(rec + Rec::KXF);
+    f32x4 gkk[10], gqk[10];
 #pragma unroll
-    for (int n = 0; n < 4; ++n) gkk[n] = gqk[n] = zero4();
-#pragma unroll 4
-    for (int jb = 0; jb < D / 32; ++jb) {
-      const typename P::frag kw = kxf[(w * 16 + jb) * 64 + lane];
-      typename P::frag qw, *frag_q;
-      frag_q = qxf_area<P>(rec) + (w * 16 + jb) * 64 + lane;
-      if constexpr (IsBf16Policy<P>::value) {
-        qw = *frag_q;
-      } else {  // Q's rows into fragment order over the k rows, which every wave has packed by now
-        qw = frag_rows_p<P>(Q, D, 16 * w, 32 * jb, lane);
-        *frag_q = qw;
-      }
+    for (int t = 0; t < 10; ++t) gkk[t] = gqk[t] = zero4();
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        const typename P::frag kn = kxf[(n * 16 + jb) * 64 + lane];
-        gkk[n] = P::mma(gkk[n], kw, kn);
-        gqk[n] = P::mma(gqk[n], qw, kn);
+    for (int jj = 0; jj < 4; ++jj) {
+      const int jb = 4 * w + jj;
+      frag kf[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) kf[m] = kxf[(m * 16 + jb) * 64 + lane];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        frag qf, *fq = qxf_area<P>(rec) + (m * 16 + jb) * 64 + lane;
+        if constexpr (IsBf16Policy<P>::value) {
+          qf = *fq;
+        } else {  // Q's rows into fragment order over the k rows, which every wave has packed by now
+          qf = frag_rows_p<P>(Q, D, 16 * m, 32 * jb, lane);
+          *fq = qf;
+        }
+#pragma unroll
+        for (int n = 0; n <= m; ++n) {
+          gkk[m * (m + 1) / 2 + n] = P::mma(gkk[m * (m + 1) / 2 + n], kf[m], kf[n]);
+          gqk[m * (m + 1) / 2 + n] = P::mma(gqk[m * (m + 1) / 2 + n], qf, kf[n]);
+        }
       }
     }
+    // 40 partial tiles of 1 KB: 17 fit xs, the rest bT and bP
+    static_assert(17 * 256 <= C * LD && 23 * 256 <= 2 * C * LD, "the partial Grams fit");
+    auto part = [&](int t, int v) {
+      const int u = v * 10 + t;
+      return reinterpret_cast<f32x4*>(u < 17 ? xs + u * 256 : bT + (u - 17) * 256) + lane;
+    };
+    auto total = [&](int t) { return ((*part(t, 0) + *part(t, 1)) + *part(t, 2)) + *part(t, 3); };
+    auto tile_m = [](int t) { return t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3; };
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
+    for (int t = 0; t < 10; ++t) *part(t, w) = gkk[t];
+    for (int idx = tid; idx < C * C; idx += 256) bA[idx] = 0.f;
+    lds_barrier();
+    for (int t = w; t < 10; t += 4) {
+      const int m = tile_m(t), n = t - m * (m + 1) / 2;
+      const f32x4 g = total(t);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int ri = 16 * w + 4 * (lane >> 4) + i, cj = 16 * n + (lane & 15);
-        rec[Rec::GKK + ri * C + cj] = gkk[n][i];
-        const float li = s_ell[ri], lj = s_ell[cj], lim1 = ri > 0 ? s_ell[ri - 1] : 0.f;
+        const int ri = 16 * m + 4 * (lane >> 4) + i, cj = 16 * n + (lane & 15);
+        rec[Rec::GKK + ri * C + cj] = g[i];
         // A transposed for the column-oriented inverse below: [j][p][s] = A[4s+p][j]
         // (the linear rule has no erasure coupling: A = 0, so T = I and Tp = 0 below)
-        bA[(cj * 4 + (ri & 3)) * 16 + (ri >> 2)] =
-            (cj < ri && !p.linear) ? s_beta[ri] * expf(fminf(li - lj, 0.f)) * gkk[n][i] : 0.f;
-        bP[ri * LD + cj] = cj < ri ? expf(fminf(lim1 - lj, 0.f)) * gqk[n][i] : 0.f;
+        if (cj < ri && !p.linear) bA[(cj * 4 + (ri & 3)) * 16 + (ri >> 2)] = s_beta[ri] * expf(fminf(s_ell[ri] - s_ell[cj], 0.f)) * g[i];
       }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int t = 0; t < 10; ++t) *part(t, w) = gqk[t];
+    lds_barrier();
+    f32x4 pt[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) pt[k] = w + 4 * k < 10 ? total(w + 4 * k) : zero4();
+    lds_barrier();
+    for (int idx = tid; idx < C * LD; idx += 256) bP[idx] = 0.f;
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int t = w + 4 * k, m = tile_m(t), n = t - m * (m + 1) / 2;
+      if (t < 10) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int ri = 16 * m + 4 * (lane >> 4) + i, cj = 16 * n + (lane & 15);
+          if (cj < ri) bP[ri * LD + cj] = expf(fminf((ri > 0 ? s_ell[ri - 1] : 0.f) - s_ell[cj], 0.f)) * pt[k][i];
+        }
+      }
+    }
   }
   __syncthreads();
   // T = (I + A)^-1 (column-oriented substitution over lane quads)
