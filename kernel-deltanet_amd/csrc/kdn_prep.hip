@@ -18,9 +18,10 @@ namespace kdn {
 // bf16 lifts (exact or hi + lo projection): one chunk per workgroup, two workgroups per CU (67 KB of LDS,
 // at most 256 registers per wave), each hiding the other's latencies.  The exact projection's Omega is
 // staged in LDS in the area the K fragments take later; the hi + lo parts are read from L2.  The exact
-// projection with queries runs the eight-wave form below (prep8_kernel) instead: four waves per SIMD.
+// projection with queries, and with fp32 inputs the hi + lo one, run the eight-wave form below (prep8_kernel).
 // Given features (bf16): runs of `run` chunks chosen at launch (ScanParams::prep_run), the next chunk's
-// beta / decay prefetched.  fp32: one chunk, one workgroup per CU (its fragments are twice as wide).
+// beta / decay prefetched.  fp32 given features and keys alone: one chunk, one workgroup per CU (its fragments are
+// twice as wide).
 template <class P, int FM>
 struct PrepRun : std::integral_constant<int, (IsBF16<P>::value && FM == FM_PRELIFTED) ? 0 : 1> {};
 template <class P, int FM>
@@ -80,7 +81,7 @@ __device__ __forceinline__ void load_lifted(const InT* row, bool valid, int lane
 // the query scales are formed.
 template <class P, typename InT, int D, int DV, int FM, bool NOQ = false>
 __global__ void __launch_bounds__(256, (PrepWaves<P, FM>::value)) prep_kernel(ScanParams p) {
-  static_assert(!NOQ || FM == FM_EXACT, "the key-only prep is the exact projection's");
+  static_assert(NOQ ? FM == FM_EXACT : FM == FM_PRELIFTED || (FM == FM_HILO && IsBF16<P>::value), "the rest is prep8_kernel's");
   using L = WsLayout<P, D, DV>;
   using frag = typename P::frag;
   using In = PrepInputs<InT, DV>;
@@ -359,22 +360,22 @@ __global__ void __launch_bounds__(256, (PrepWaves<P, FM>::value)) prep_kernel(Sc
 }
 
 // ------------------------------------------------------------------------------------------------
-// prep8: the bf16 exact-projection prep (no ScanParams::prep_no_q) with eight waves per workgroup, 512
-// threads, one chunk per workgroup and two workgroups per CU at <= 128 registers: four waves per SIMD to
-// hide each phase's latencies instead of two.  Wave w = 4 hf + m owns token tile m (rows 16m .. 16m + 15)
+// prep8: the exact-projection prep (no ScanParams::prep_no_q), and with fp32 inputs the hi + lo projection's too, with
+// eight waves per workgroup, 512 threads, one chunk per workgroup.  bf16: two workgroups per CU at <= 128
+// registers, four waves per SIMD to hide each phase's latencies instead of two.  fp32: one workgroup (132 KB), two
+// waves per SIMD instead of one, and the products of the Grams, which bound it, spread evenly over the waves: 64
+// chunks 39 -> 32 us.  Wave w = 4 hf + m owns token tile m (rows 16m .. 16m + 15)
 // and feature half hf (features 256 hf .. + 255, 32-feature blocks 8 hf .. 8 hf + 7): it lifts its rows
 // of q and k on that half only (64 fragment registers instead of 128), stores those record fragments and
 // forms the half's partial Gram tiles.  The halves meet in LDS: the rows' sums of squares, then the
 // partial Grams (hf = 0 hands over its K Q^T part, hf = 1 its K K^T part), after which the hf = 0 waves
 // form A and the hf = 1 waves P; waves 0-3 invert the diagonal blocks and 0-2 walk the block columns;
-// the Tp tiles are hf = 0's and the U~ tiles are split between the halves.  It writes the record
-// prep_kernel<PrecBF16, __bf16, 512, DV, FM_EXACT> writes: the same K and Q features bit for bit; the
-// scales and Grams summed in two halves (rounding order only).
-template <int DV>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) prep8_kernel(ScanParams p) {
-  using P = PrecBF16;
-  using InT = __bf16;
+// the Tp tiles are hf = 0's and the U~ tiles are split between the halves.  It writes prep_kernel's record.
+template <class P, typename InT, int DV, int FM>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(IsBF16<P>::value ? 4 : 2, IsBF16<P>::value ? 4 : 2))) prep8_kernel(ScanParams p) {
+  static_assert(FM == FM_EXACT || (FM == FM_HILO && !IsBF16<P>::value), "the forms launch_prep sends here");
   constexpr int D = 512;
+  constexpr bool OMEGA_LDS = FM == FM_EXACT;
   using L = WsLayout<P, D, DV>;
   using frag = typename P::frag;
   constexpr int NJ = D / 32, NJH = NJ / 2, NV = DV / 16;
@@ -419,6 +420,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   const Seq sq = seq_of(p, b);
   const int64_t t0 = (p.chunk0 + cl) * CH;
   const __bf16* omega_h = p.omega + h * p.oms;
+  const __bf16* omega_lo_h = FM == FM_HILO ? p.omega_lo + h * p.oms : nullptr;
   const float ang = (p.inv_tau_head ? p.inv_tau_head[h] : p.inv_tau) * 0.15915494309189535f;
   const bool cached = p.k_plain != 0;
   auto put = [&](void* base, const frag& f) {
@@ -440,7 +442,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
     be = valid ? p.beta[sq.be + t * p.bs1 + h * p.bs2] : 0.f;
     la = (valid && p.decay) ? p.decay[sq.de + t * p.ds1 + h * p.ds2] : 1.f;
   }
-  stage_omega<D, true, 512>(omega_h, p.phase + h * p.phs, s_omega, s_phrev);
+  stage_omega<D, OMEGA_LDS, 512>(omega_h, p.phase + h * p.phs, s_omega, s_phrev);
   lds_barrier();  // Omega staged
 
   // ---- beta and the in-chunk log-decay prefix (wave 0)
@@ -458,8 +460,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   // ---- lift q and k of tile m on feature half hf: fragment jl holds features 32 (8 hf + jl) .. + 31
   frag cqk[2][NJH];
   float ss[2];
-  lift_tile<P, InT, D, true, 2, false, NJ>(qk, p.normalize, s_omega, omega_h, s_phrev, ang, lane, cqk, ss, nullptr,
-                                           NJ * hf);
+  lift_tile<P, InT, D, OMEGA_LDS, 2, FM == FM_HILO, NJ>(qk, p.normalize, s_omega, omega_h, s_phrev, ang, lane, cqk, ss,
+                                                        omega_lo_h, NJ * hf);
   if (lane < 16) {
     s_ss[hf][0][16 * m + lane] = ss[0];
     s_ss[hf][1][16 * m + lane] = ss[1];
@@ -493,14 +495,19 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
 #pragma unroll
   for (int jl = 0; jl < NJH; ++jl) {
     const int jg = NJH * hf + jl;
-    if (p.k_plain) put(ws + L::phiK + (size_t)(m * NJ + jg) * 64 * L::FB, cqk[1][jl]);
-    else store_k_image(ws + L::phiK, m, jg, lane, cqk[1][jl]);
+    if constexpr (IsBF16<P>::value) {
+      if (p.k_plain) put(ws + L::phiK + (size_t)(m * NJ + jg) * 64 * L::FB, cqk[1][jl]);
+      else store_k_image(ws + L::phiK, m, jg, lane, cqk[1][jl]);
+    } else {
+      put(ws + L::phiK + (size_t)(m * NJ + jg) * 64 * L::FB, cqk[1][jl]);
+    }
     if (!p.q_relift) put(ws + L::phiQ + (size_t)(m * NJ + jg) * 64 * L::FB, cqk[0][jl]);
     s_phik[(m * NJ + jg) * 64 + lane] = cqk[1][jl];
   }
   lds_barrier();
 
-  // ---- partial Gram tiles over feature half hf: Gkk[mm][m] = K_mm K_m^T, GqkT[mm][m] = K_mm Q_m^T
+  // ---- partial Gram tiles over feature half hf: Gkk[mm][m] = K_mm K_m^T for mm >= m, GqkT[mm][m] = K_mm Q_m^T for
+  // mm <= m (what A and P use): five tiles a wave
   f32x4 gkk[4], gqk[4];
 #pragma unroll
   for (int mm = 0; mm < 4; ++mm) { gkk[mm] = zero4(); gqk[mm] = zero4(); }
@@ -508,52 +515,50 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
   for (int jl = 0; jl < NJH; ++jl) {
 #pragma unroll
     for (int mm = 0; mm < 4; ++mm) {
-      if (mm > m) break;  // above the diagonal: neither A nor P uses it
       const frag a = s_phik[(mm * NJ + NJH * hf + jl) * 64 + lane];
-      gkk[mm] = P::mma(gkk[mm], a, cqk[1][jl]);
-      gqk[mm] = P::mma(gqk[mm], a, cqk[0][jl]);
+      if (mm >= m) gkk[mm] = P::mma(gkk[mm], a, cqk[1][jl]);
+      if (mm <= m) gqk[mm] = P::mma(gqk[mm], a, cqk[0][jl]);
     }
   }
   lds_barrier();  // K fragments in LDS are dead from here on
 #pragma unroll
   for (int mm = 0; mm < 4; ++mm) {
-    if (mm > m) break;
-    if (hf == 0) s_part[(m * 4 + mm) * 64 + lane] = gqk[mm];
-    else s_part[((4 + m) * 4 + mm) * 64 + lane] = gkk[mm];
+    if (hf == 0 && mm <= m) s_part[(m * 4 + mm) * 64 + lane] = gqk[mm];
+    if (hf == 1 && mm >= m) s_part[((4 + m) * 4 + mm) * 64 + lane] = gkk[mm];
   }
   lds_barrier();
 
-  // ---- A (hf = 0) and P (hf = 1) of rows 16m .. 16m + 15, scale vectors (wave 5)
+  // ---- A (hf = 0, columns 16m .. 16m + 15) and P (hf = 1, rows 16m ..), scale vectors (wave 5)
   {
     const int t = 16 * m + (lane & 15);
-    const float gt = s_g[t], gtm1 = t > 0 ? s_g[t - 1] : 0.f;
     if (hf == 0) {
-      // the linear rule has no erasure coupling: A = 0, so T = I below
-      const float bt = p.linear ? 0.f : s_beta[t], skt = s_sk[t];
+      const float gt = s_g[t], skt = s_sk[t];
 #pragma unroll
       for (int mm = 0; mm < 4; ++mm) {
-        if (mm > m) break;  // the inverse reads no block above the diagonal
+        if (mm < m) continue;  // the inverse reads no block above the diagonal
         const f32x4 gk = gkk[mm] + s_part[((4 + m) * 4 + mm) * 64 + lane];
+        const int r0 = 16 * mm + 4 * (lane >> 4);
+        const f32x4 gr = *reinterpret_cast<const f32x4*>(s_g + r0), skr = *reinterpret_cast<const f32x4*>(s_sk + r0);
+        const f32x4 br = *reinterpret_cast<const f32x4*>(s_beta + r0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int j = 16 * mm + 4 * (lane >> 4) + i;
-          const float a = (j < t) ? bt * __expf(fminf(gt - s_g[j], 0.f)) * gk[i] * skt * s_sk[j] : 0.f;
-          s_A[(j * 4 + (t & 3)) * 16 + a_swizzle(j, t >> 2, t & 3)] = a;
+          // the linear rule has no erasure coupling: A = 0, so T = I below
+          const float a = (t < r0 + i && !p.linear) ? br[i] * __expf(fminf(gr[i] - gt, 0.f)) * gk[i] * skr[i] * skt : 0.f;
+          s_A[(t * 4 + i) * 16 + a_swizzle(t, (r0 >> 2), i)] = a;
         }
       }
     } else {
-      const float sqt = s_sq[t];
+      const float sqt = s_sq[t], gtm1 = t > 0 ? s_g[t - 1] : 0.f;
       f32x4 pt[4];
 #pragma unroll
       for (int mm = 0; mm < 4; ++mm) {
         pt[mm] = zero4();
         if (mm > m) continue;
         const f32x4 gq = s_part[(m * 4 + mm) * 64 + lane] + gqk[mm];
+        const int j0 = 16 * mm + 4 * (lane >> 4);
+        const f32x4 gj = *reinterpret_cast<const f32x4*>(s_g + j0), skj = *reinterpret_cast<const f32x4*>(s_sk + j0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int j = 16 * mm + 4 * (lane >> 4) + i;
-          pt[mm][i] = (j < t) ? __expf(fminf(gtm1 - s_g[j], 0.f)) * gq[i] * sqt * s_sk[j] : 0.f;
-        }
+        for (int i = 0; i < 4; ++i) pt[mm][i] = (j0 + i < t) ? __expf(fminf(gtm1 - gj[i], 0.f)) * gq[i] * sqt * skj[i] : 0.f;
       }
 #pragma unroll
       for (int jb = 0; jb < 2; ++jb)
@@ -614,16 +619,22 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
       f32x4 acc = zero4();
 #pragma unroll
       for (int jb = 0; jb < 2; ++jb) {
-        // hi + lo split of T diag(beta): V is exact in bf16, so U~ keeps ~16 bits
-        bf16x8 hi, lo, vb;
+        frag vb;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-          hi[s] = (__bf16)tb[jb][s];
-          lo[s] = (__bf16)(tb[jb][s] - (float)hi[s]);
-          vb[s] = s_V[(32 * jb + kappa(lane, s)) * DVP + 16 * n + (lane & 15)];
+        for (int s = 0; s < 8; ++s) vb[s] = s_V[(32 * jb + kappa(lane, s)) * DVP + 16 * n + (lane & 15)];
+        if constexpr (IsBF16<P>::value) {
+          // hi + lo split of T diag(beta): V is exact in bf16, so U~ keeps ~16 bits
+          bf16x8 hi, lo;
+#pragma unroll
+          for (int s = 0; s < 8; ++s) {
+            hi[s] = (__bf16)tb[jb][s];
+            lo[s] = (__bf16)(tb[jb][s] - (float)hi[s]);
+          }
+          acc = P::mma(acc, hi, vb);
+          acc = P::mma(acc, lo, vb);
+        } else {
+          acc = P::mma(acc, tb[jb], vb);
         }
-        acc = PrecBF16::mma(acc, hi, vb);
-        acc = PrecBF16::mma(acc, lo, vb);
       }
       f32x4* ud = reinterpret_cast<f32x4*>(ws + L::U + ((size_t)(m * NV + n) * 64 + lane) * 16);
       if (cached) *ud = acc;
@@ -641,10 +652,10 @@ int launch_prep(const ScanParams& p, hipStream_t st) {
   const dim3 prep_grid = p.fl_off ? dim3((unsigned)p.nseg, (unsigned)p.H, 1u)
                                   : dim3((unsigned)((p.nseg + run - 1) / run), (unsigned)p.H, (unsigned)p.B);
   if (fm == FM_PRELIFTED) hipLaunchKernelGGL((prep_kernel<P, InT, D, DV, FM_PRELIFTED>), prep_grid, dim3(256), 0, st, p);
-  else if (fm == FM_HILO) hipLaunchKernelGGL((prep_kernel<P, InT, D, DV, FM_HILO>), prep_grid, dim3(256), 0, st, p);
+  else if (fm == FM_HILO && IsBF16<P>::value) hipLaunchKernelGGL((prep_kernel<PrecBF16, __bf16, D, DV, FM_HILO>), prep_grid, dim3(256), 0, st, p);
+  else if (fm == FM_HILO) hipLaunchKernelGGL((prep8_kernel<PrecF32, float, DV, FM_HILO>), prep_grid, dim3(512), 0, st, p);
   else if (p.prep_no_q) hipLaunchKernelGGL((prep_kernel<P, InT, D, DV, FM_EXACT, true>), prep_grid, dim3(256), 0, st, p);
-  else if constexpr (IsBF16<P>::value && D == 512) hipLaunchKernelGGL((prep8_kernel<DV>), prep_grid, dim3(512), 0, st, p);
-  else hipLaunchKernelGGL((prep_kernel<P, InT, D, DV, FM_EXACT>), prep_grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((prep8_kernel<P, InT, DV, FM_EXACT>), prep_grid, dim3(512), 0, st, p);
   return hipGetLastError() == hipSuccess ? KDN_OK : KDN_ERR_DEVICE;
 }
 
