@@ -6,9 +6,9 @@
 // D = 512 scan: y_t = S_{t-1} phi_q(t), S_t = lambda_t S_{t-1} (I - beta_t phi_k phi_k^T) + beta_t v_t phi_k^T.
 //
 // Three launches per call, with one fp32 record per (batch, head, 64-token chunk):
-//   prep   (parallel)   Grams K K^T and Q K^T from the feature rows in place, A, T = (I + A)^-1 (column-
-//                       oriented substitution), Tp = T diag(beta g), P, U~ = T (beta o V); K packed in MFMA
-//                       fragment order (rows and transposed)
+//   prep   (parallel)   Grams K K^T and Q K^T from the feature rows, A, T = (I + A)^-1 (column-oriented
+//                       substitution), Tp = T diag(beta g), P, U~ = T (beta o V); K packed in MFMA fragment
+//                       order (with fp32 features transposed too)
 //   carry  (sequential) S^T at every chunk start; X_K = K S^T, W = U~ - Tp X_K,
 //                       S^T <- g_C S^T + K^T (kappa o W); the final state
 //   output (parallel)   Y = diag(a) Q S_c^T + P W
