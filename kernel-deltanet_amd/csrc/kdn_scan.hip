@@ -31,6 +31,7 @@
 #include "kdn_frag.hpp"
 #include "kdn_internal.hpp"
 #include "kdn_io.hpp"
+#include "kdn_lds_layout.hpp"
 #include "kdn_scan_common.hpp"
 #include "kdn_lift_tile.hpp"
 #include "kdn_tile.hpp"
@@ -50,9 +51,10 @@ namespace kdn {
 // barriers took two and a half times that with four waves: one wave a SIMD waits for every LDS and memory
 // latency, each K^T operand was eight 4-byte reads with eight-fold bank conflicts, and the second of a lane's two
 // L2-prefetch loads was waited for where it was added to the first.  Now two waves share a SIMD, the copy is
-// permuted (f32_slot) so that neither its writes nor its reads conflict, K of the next chunk is loaded as soon as its
+// permuted (kf32_word) so that neither its writes nor its reads conflict, K of the next chunk is loaded as soon as its
 // registers are free, and waves 4-7, idle during the reduction, read their K^T operands and prefetch into L2.
-// 4 heads, 16 chunks: 153 -> 101 us (9.6 -> 6.3 us a chunk).
+// 4 heads, 16 chunks: 153 -> 101 us (9.6 -> 6.3 us a chunk).  64 chunks: 363 us with the reads of the copy conflicting
+// two ways (43.7 % of the kernel's busy LDS cycles), 348 without (0 %).
 //
 // Workgroups are dispatched round-robin over the 8 XCDs (linear id % 8); the value tiles of one head
 // get ids with equal residue so that they share one XCD's L2 for the K fragments they all read.
@@ -68,7 +70,7 @@ struct StateF32 {
   // The partial X_K tiles: tile m of wave v in part[m][v - (v > m)], except wave m's own (it adds it from its
   // registers); part[m][0] takes the reduced tile.  160 KB with the K copies: the whole CU.
   struct Shared {
-    frag k[8][8 * 64];   // wave-private K fragments [4 token tiles x 2 blocks], eight floats per f32_slot
+    frag k[8][8 * 64];   // wave-private K fragments [4 token tiles x 2 blocks], placed by kf32_word
     f32x4 part[4][7][64];
     f32x4 e[4][64];
   };
@@ -93,11 +95,6 @@ struct StateF32 {
   __device__ static void load_g(const unsigned char* ws, Ops& o) { o.gC = reinterpret_cast<const float*>(uni(ws + L::VEC))[128]; }
 };
 
-// Slot (of 64, eight floats each) of the values of token c = 4g + e and features 4q .. 4q + 3 (+ 16) of a K fragment in
-// its LDS copy; the two halves of a slot change places where g >= 2.  The sixteen 16-byte writes of a lane group (16
-// tokens) and the 64 four-byte reads of a K^T operand (fixed e, all g, q and feature & 3) fall on distinct banks.
-__device__ __forceinline__ int f32_slot(int g, int e, int q) { return ((q ^ e) | ((g & 1) << 2)) + 8 * (e | ((g >> 1) << 2)); }
-
 template <int DV, bool DECAY, bool lead>
 __device__ __forceinline__ void state_f32_loop(const ScanParams& p, typename StateF32<DV>::Shared& sh, unsigned char* wsh, int nloc,
                                                int w, int lane, int n, f32x4 (&S)[4]) {
@@ -107,11 +104,10 @@ __device__ __forceinline__ void state_f32_loop(const ScanParams& p, typename Sta
   using frag = typename O::frag;
   constexpr int NV = O::NV;
   float* kl = reinterpret_cast<float*>(sh.k[w]);
-  const int kw = 8 * f32_slot((lane & 15) >> 2, lane & 3, lane >> 4);  // written: token lane & 15, features of lane >> 4
-  const int kflip = 4 * ((lane & 15) >> 3);
-  int kr[4];  // read: feature lane & 15, token 4 (lane >> 4) + e
+  const int kw = kf32_write(lane, 0);
+  int kr[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) kr[e] = 8 * f32_slot(lane >> 4, e, (lane & 15) >> 2) + 4 * (lane >> 5) + (lane & 3);
+  for (int e = 0; e < 4; ++e) kr[e] = kf32_read(lane, e, 0);  // the halves differ in bit 2 of the word
   // K^T operand of feature tile tl (of the wave's four), tokens 32jb + kappa
   auto kt_frag = [&](int tl, int jb) {
     frag f;
@@ -148,7 +144,7 @@ __device__ __forceinline__ void state_f32_loop(const ScanParams& p, typename Sta
         for (int hh = 0; hh < 2; ++hh) {
           const frag& f = o.kx[m][jj];
           const f32x4 v = {f[4 * hh], f[4 * hh + 1], f[4 * hh + 2], f[4 * hh + 3]};
-          *reinterpret_cast<f32x4*>(kl + (2 * m + jj) * 512 + kw + ((4 * hh) ^ kflip)) = v;
+          *reinterpret_cast<f32x4*>(kl + (2 * m + jj) * 512 + (kw ^ (4 * hh))) = v;
         }
 #pragma unroll
     for (int jj = 0; jj < 2; ++jj) store_frag<P>(uni(cur + L::Sfr + (size_t)((2 * w + jj) * NV + n) * 64 * L::FB), lane, sf[jj]);
