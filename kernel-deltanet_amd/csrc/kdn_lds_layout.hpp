@@ -22,4 +22,27 @@ constexpr int kf32_word(int g, int e, int q, int half) {
 constexpr int kf32_write(int lane, int half) { return kf32_word((lane & 15) >> 2, lane & 3, lane >> 4, half); }
 constexpr int kf32_read(int lane, int e, int half) { return kf32_word(lane >> 4, e, (lane & 15) >> 2, half) + (lane & 3); }
 
+// A and T of the 64 x 64 unit-lower inverse in 16 x 16 blocks (unit_lower_inverse_blocked).
+//
+// A by columns, the rows of a column in sixteen groups of four, the groups XORed with the column's low four bits.
+//   4-byte accesses of A[16i + m][16k + 4g + kb] (lane (g, m); the column walk's reads, and the stores of a tile held
+//     with its rows over the lanes): m & 3 on bank bits 0-1, (m >> 2) ^ kb on bits 2-3, (i ^ g) & 1 on bit 4, which
+//     differs over a half-wave's two g;
+//   16-byte accesses of rows 4s .. 4s + 3 of sixteen consecutive columns (the stores of a tile held with its columns over
+//     the lanes): sixteen groups;
+//   16-byte reads of rows 16b + 4p .. + 3 of one column by the lanes p (the substitution): four groups, each broadcast.
+// (In four rows of residue p = row & 3 a column, the stores by columns were four 4-byte ones that met four ways on a bank:
+// prep8_kernel's conflicts 6.7 % of its busy LDS cycles, 2.7 % with this.)
+constexpr int a_word(int row, int col) { return col * 64 + 4 * ((row >> 2) ^ (col & 15)) + (row & 3); }
+
+// T by rows, the 16-byte groups of a row's columns XORed with h(r) = 4 (a ^ p) + a, a = (r >> 2) & 3, p = r & 3, so that
+// each of these falls on distinct banks: 4-byte accesses of rows 4a + 0..3 (a fixed; accumulator tiles) or of rows
+// 4·0..3 + p (p fixed; the substitution's stores) at columns of one 16-column block per instruction (h >> 2 differs over
+// p for fixed a and over a for fixed p), and 16-byte reads of four consecutive columns of 16 consecutive rows (h is a
+// bijection on a 16-row block).
+constexpr int t_swizzle(int r, int c) {
+  const int a = (r >> 2) & 3, p = r & 3;
+  return c ^ (16 * (a ^ p)) ^ (4 * a);
+}
+
 }  // namespace kdn

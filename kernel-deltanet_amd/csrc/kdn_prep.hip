@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(256, (PrepWaves<P, FM>::value)) prep_kernel(Sc
 
   bf16x8* s_omega = reinterpret_cast<bf16x8*>(smem);                 // during the lift (OMEGA_LDS)
   frag* s_phik = reinterpret_cast<frag*>(smem);                       // from the lift to the Gram
-  float* s_A = reinterpret_cast<float*>(smem);                        // [j][p][s'] = A[4s+p][j] (s swizzled, a_swizzle)
+  float* s_A = reinterpret_cast<float*>(smem);                        // A[r][j] at a_word(r, j)
   float* s_T = s_A + 64 * 64;                                          // [t][64] (columns swizzled, t_swizzle)
   InT* s_V = reinterpret_cast<InT*>(s_T + 64 * 64);                    // [t][DVP]
 
@@ -264,7 +264,7 @@ __global__ void __launch_bounds__(256, (PrepWaves<P, FM>::value)) prep_kernel(Sc
           const int j = 16 * m + 4 * (lane >> 4) + i;
           const float gj = s_g[j], skj = s_sk[j];
           const float a = (j < t) ? bt * __expf(fminf(gt - gj, 0.f)) * gkk[m][i] * skt * skj : 0.f;
-          s_A[(j * 4 + (t & 3)) * 16 + a_swizzle(j, t >> 2, t & 3)] = a;
+          s_A[a_word(t, j)] = a;
           if constexpr (!NOQ) pt[m][i] = (j < t) ? __expf(fminf(gtm1 - gj, 0.f)) * gqk[m][i] * sqt * skj : 0.f;
         }
       }
@@ -394,7 +394,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(IsBF16
 
   bf16x8* s_omega = reinterpret_cast<bf16x8*>(smem);                 // during the lift
   frag* s_phik = reinterpret_cast<frag*>(smem);                       // from the lift to the Gram
-  float* s_A = reinterpret_cast<float*>(smem);                        // [j][p][s'] (a_swizzle)
+  float* s_A = reinterpret_cast<float*>(smem);                        // A[r][j] at a_word(r, j)
   float* s_T = s_A + 64 * 64;                                          // [t][64] (t_swizzle)
   f32x4* s_part = reinterpret_cast<f32x4*>(smem + PHIK_BYTES / 2);    // [hf][m][mm][lane] Gram partials
   InT* s_V = reinterpret_cast<InT*>(s_T + 64 * 64);                    // [t][DVP], after the partials
@@ -540,12 +540,13 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(IsBF16
         const int r0 = 16 * mm + 4 * (lane >> 4);
         const f32x4 gr = *reinterpret_cast<const f32x4*>(s_g + r0), skr = *reinterpret_cast<const f32x4*>(s_sk + r0);
         const f32x4 br = *reinterpret_cast<const f32x4*>(s_beta + r0);
+        f32x4 a;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           // the linear rule has no erasure coupling: A = 0, so T = I below
-          const float a = (t < r0 + i && !p.linear) ? br[i] * __expf(fminf(gr[i] - gt, 0.f)) * gk[i] * skr[i] * skt : 0.f;
-          s_A[(t * 4 + i) * 16 + a_swizzle(t, (r0 >> 2), i)] = a;
+          a[i] = (t < r0 + i && !p.linear) ? br[i] * __expf(fminf(gr[i] - gt, 0.f)) * gk[i] * skr[i] * skt : 0.f;
         }
+        *reinterpret_cast<f32x4*>(s_A + a_word(r0, t)) = a;
       }
     } else {
       const float sqt = s_sq[t], gtm1 = t > 0 ? s_g[t - 1] : 0.f;

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "kdn_frag.hpp"
+#include "kdn_lds_layout.hpp"
 
 namespace kdn {
 
@@ -123,32 +124,9 @@ __device__ __forceinline__ void unit_lower_inverse(const float* At, float* T, in
   for (int s2 = 0; s2 < 16; ++s2) T[(4 * s2 + pq) * ldt + col] = -acc[s2];
 }
 
-// Swizzled layouts of A and T for unit_lower_inverse_blocked: At[(j * 4 + p) * 16 + a_swizzle(j, s, p)] =
-// A[4s + p][j] and T[r * 64 + t_swizzle(r, c)] = T[r][c].
-// 4-byte LDS accesses are served per half-wave over 32 banks (16-byte reads per 16 lanes over 64; measured
-// with SQ_LDS_BANK_CONFLICT on a probe of both).  a_swizzle keeps each group of four s (one 16-byte read)
-// contiguous and spreads a half-wave's 4-byte accesses of A over 32 banks: the writer storing one element
-// per lane (p = lane & 3, s & 3 = (lane >> 2) & 3, column group g = lane >> 4) and the column walk reading
-// A[16i + m][16k + 4g + kb] (p = m & 3, s & 3 = m >> 2).  Row j * 4 + p puts p & 1 on bank bit 4; XORing
-// the group index with (j >> 2) & 3 and with 2 (p >> 1) separates the two lane groups of a half-wave and
-// p from p ^ 2.
-__device__ __forceinline__ int a_swizzle(int j, int s, int p) {
-  return 4 * ((s >> 2) ^ ((j >> 2) & 3) ^ (2 * (p >> 1))) + (s & 3);
-}
-// t_swizzle XORs the 16-byte group index of column c in row r (ldt = 64) with h(r) = 4 (a ^ p) + a,
-// a = (r >> 2) & 3, p = r & 3, so that each of these falls on distinct banks: 4-byte accesses of rows
-// 4a + 0..3 (a fixed) or of rows 4·0..3 + p (p fixed) at 16 consecutive columns of one 16-column block per
-// instruction (h >> 2 differs over p for fixed a and over a for fixed p), and 16-byte reads of four
-// consecutive columns of 16 consecutive rows (h is a bijection on a 16-row block).
-__device__ __forceinline__ int t_swizzle(int r, int c) {
-  const int a = (r >> 2) & 3, p = r & 3;
-  return c ^ (16 * (a ^ p)) ^ (4 * a);
-}
-
 // Block column J of T below the diagonal (step 2 of unit_lower_inverse_blocked): T_iJ for i = J+1 .. 3.
 template <int J>
 __device__ __forceinline__ void inverse_block_column(const float* At, float* T, int lane) {
-  auto at_idx = [](int r, int c) { return (c * 4 + (r & 3)) * 16 + a_swizzle(c, r >> 2, r & 3); };
   auto t_idx = [](int r, int c) { return r * 64 + t_swizzle(r, c); };
   const int g = lane >> 4, m = lane & 15;
   // operands read first: L_ik as A operands (depth 4g + kb) and T_ii rows, for every i > J and k in [J, i)
@@ -158,7 +136,7 @@ __device__ __forceinline__ void inverse_block_column(const float* At, float* T, 
 #pragma unroll
     for (int k = J; k < i; ++k)
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) la[i][k][kb] = At[at_idx(16 * i + m, 16 * k + 4 * g + kb)];
+      for (int kb = 0; kb < 4; ++kb) la[i][k][kb] = At[a_word(16 * i + m, 16 * k + 4 * g + kb)];
   f32x4 tii[4];  // T_ii[m][4g .. 4g + 3]
 #pragma unroll
   for (int i = J + 1; i < 4; ++i) tii[i] = *reinterpret_cast<const f32x4*>(T + t_idx(16 * i + m, 16 * i + 4 * g));
@@ -181,7 +159,7 @@ __device__ __forceinline__ void inverse_block_column(const float* At, float* T, 
   }
 }
 
-// The same inverse in 16 x 16 blocks, for the swizzled layouts above (At by a_swizzle, T by t_swizzle with
+// The same inverse in 16 x 16 blocks, for the layouts of kdn_lds_layout.hpp (At by a_word, T by t_swizzle with
 // ldt = 64).  L = I + A with blocks L_ik; T_ii = L_ii^{-1} and T_ij = -T_ii sum_{k=j}^{i-1} L_ik T_kj (i > j).
 //   1. wave b inverts diagonal block b by the column substitution above restricted to 16 rows (15 steps of
 //      one quad broadcast and at most four FMAs), writes T_bb and the zero blocks to its right;
@@ -196,40 +174,37 @@ __device__ __forceinline__ void inverse_block_column(const float* At, float* T, 
 __device__ __forceinline__ void inverse_diag_block(const float* At, float* T, int b, int lane) {
   auto t_idx = [](int r, int c) { return r * 64 + t_swizzle(r, c); };
   {
-    // diagonal block b: lane quad c = lane >> 2 holds column c, lane pq = lane & 3 rows 4s + pq
+    // diagonal block b: lane quad c = lane >> 2 holds column c, lane pq = lane & 3 rows 4pq + s
     const int c = lane >> 2, pq = lane & 3;
-    float acc[4];  // -(partial T_bb[4s + pq][c])
+    float acc[4];  // -(partial T_bb[4pq + s][c])
 #pragma unroll
-    for (int s = 0; s < 4; ++s) acc[s] = (4 * s + pq == c) ? -1.f : 0.f;
-    // column i of L_bb's strict lower part, rows 16b + 4s + pq (s = 0..3): one 16-byte group of At
-    auto col = [&](int i) {
-      const int C = 16 * b + i;
-      return *reinterpret_cast<const f32x4*>(At + (C * 4 + pq) * 16 + 4 * (b ^ ((C >> 2) & 3) ^ (2 * (pq >> 1))));
-    };
-    // every column's read issued before the chain starts (nothing else is live here)
+    for (int s = 0; s < 4; ++s) acc[s] = (4 * pq + s == c) ? -1.f : 0.f;
+    // every column's read issued before the chain starts (nothing else is live here): column i of L_bb's strict lower
+    // part, rows 16b + 4pq .. + 3
     f32x4 acol[15];
 #pragma unroll
-    for (int i = 0; i < 15; ++i) acol[i] = col(i);
+    for (int i = 0; i < 15; ++i) acol[i] = *reinterpret_cast<const f32x4*>(At + a_word(16 * b + 4 * pq, 16 * b + i));
 #pragma unroll
-    for (int i = 0; i < 15; ++i) {
-      const f32x4 a = acol[i];
-      float bc;  // -T[i][c], held by lane pq = i & 3, slot i >> 2 of the quad
-      switch (i & 3) {
-        case 0: bc = quad_bcast<0>(acc[i >> 2]); break;
-        case 1: bc = quad_bcast<1>(acc[i >> 2]); break;
-        case 2: bc = quad_bcast<2>(acc[i >> 2]); break;
-        default: bc = quad_bcast<3>(acc[i >> 2]); break;
+    for (int ib = 0; ib < 4; ++ib) {
+      if (pq >= ib) {  // the rows of the lanes before are final
+#pragma unroll
+        for (int i = 4 * ib; i < 4 * ib + 4 && i < 15; ++i) {
+          float bc;  // -T[i][c], held by lane pq = i >> 2, slot i & 3 of the quad
+          switch (ib) {
+            case 0: bc = quad_bcast<0>(acc[i & 3]); break;
+            case 1: bc = quad_bcast<1>(acc[i & 3]); break;
+            case 2: bc = quad_bcast<2>(acc[i & 3]); break;
+            default: bc = quad_bcast<3>(acc[i & 3]); break;
+          }
+#pragma unroll
+          for (int s = 0; s < 4; ++s) acc[s] = fmaf(-acol[i][s], bc, acc[s]);
+        }
       }
-#pragma unroll
-      for (int s = i >> 2; s < 4; ++s) acc[s] = fmaf(-a[s], bc, acc[s]);
     }
-    // store k writes row 4s + pq with s = k ^ 2 (pq >> 1): a half-wave (columns c = 0..7) then spans bank
-    // bit 3 through s as well as bit 4 through pq, 32 distinct banks (s = k for every lane: 16)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int s = k ^ (2 * (pq >> 1));
-      const int r = 16 * b + 4 * s + pq;
-      T[t_idx(r, 16 * b + c)] = (pq & 2) ? -acc[k ^ 2] : -acc[k];
+    for (int s = 0; s < 4; ++s) {
+      const int r = 16 * b + 4 * pq + s;
+      T[t_idx(r, 16 * b + c)] = -acc[s];
 #pragma unroll
       for (int blk = 0; blk < 4; ++blk)
         if (blk > b) T[t_idx(r, 16 * blk + c)] = 0.f;

@@ -51,6 +51,47 @@ int main() {
           }
   }
   printf("kf32_places %d\nkf32_read %d\nkf32_write %d\n", (int)kf.size(), rd, wr);
+
+  // A of the blocked inverse: rows over the lanes (prep_kernel's stores, the column walk's reads), columns over the
+  // lanes with four rows each (prep8_kernel's stores), the substitution's reads
+  int ar = 0, ac = 0, sub = 0;
+  std::set<int> as;
+  for (int i = 0; i < 4; ++i)
+    for (int k = 0; k < 4; ++k) {
+      up(ac, ways16([&](int l) { return a_word(16 * i + 4 * (l >> 4), 16 * k + (l & 15)); }));
+      for (int e = 0; e < 4; ++e) {
+        up(ar, ways4([&](int l) { return a_word(16 * i + (l & 15), 16 * k + 4 * (l >> 4) + e); }));
+        if (k == i)
+          for (int c = 4 * e; c < 4 * e + 4; ++c) up(sub, ways16([&](int l) { return a_word(16 * i + 4 * (l & 3), 16 * i + c); }));
+      }
+    }
+  for (int r = 0; r < 64; ++r)
+    for (int c = 0; c < 64; ++c) {
+      const int w = a_word(r, c);
+      if (w < 0 || w >= 4096 || w != a_word(r & ~3, c) + (r & 3) || a_word(r & ~3, c) % 4) return 1;
+      as.insert(w);
+    }
+  printf("a_places %d\na_rows %d\na_cols %d\na_substitution %d\n", (int)as.size(), ar, ac, sub);
+
+  // T: the substitution's stores (the block and the zeros to its right), the accumulator-layout accesses, 16-byte rows
+  int td = 0, ta = 0, tr = 0;
+  std::set<int> ts;
+  auto t_word = [](int r, int c) { return r * 64 + t_swizzle(r, c); };
+  for (int b = 0; b < 4; ++b)
+    for (int k = 0; k < 4; ++k) {
+      up(tr, ways16([&](int l) { return t_word(16 * b + (l & 15), 16 * k + 4 * (l >> 4)); }));
+      for (int e = 0; e < 4; ++e) {
+        up(ta, ways4([&](int l) { return t_word(16 * b + 4 * (l >> 4) + e, 16 * k + (l & 15)); }));
+        if (k >= b)
+          up(td, ways4([&](int l) { return t_word(16 * b + 4 * (l & 3) + e, 16 * k + (l >> 2)); }));
+      }
+    }
+  for (int r = 0; r < 64; ++r)
+    for (int c = 0; c < 64; ++c) {
+      if (t_word(r, c) != t_word(r, c & ~3) + (c & 3)) return 1;
+      ts.insert(t_word(r, c));
+    }
+  printf("t_places %d\nt_substitution %d\nt_tiles %d\nt_rows %d\n", (int)ts.size(), td, ta, tr);
   return 0;
 }
 """
@@ -68,11 +109,12 @@ def counts(tmp_path_factory):
     return {k: int(v) for k, v in (line.split() for line in out.splitlines())}
 
 
-@pytest.mark.parametrize("access", ["kf32_read", "kf32_write"])
+@pytest.mark.parametrize("access", ["kf32_read", "kf32_write", "a_rows", "a_cols", "a_substitution",
+                                    "t_substitution", "t_tiles", "t_rows"])
 def test_no_bank_conflicts(counts, access):
     assert counts[access] == 1
 
 
-@pytest.mark.parametrize("layout,words", [("kf32_places", 512)])
+@pytest.mark.parametrize("layout,words", [("kf32_places", 512), ("a_places", 4096), ("t_places", 4096)])
 def test_one_word_per_element(counts, layout, words):
     assert counts[layout] == words
