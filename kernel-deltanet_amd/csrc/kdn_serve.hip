@@ -14,6 +14,7 @@
 #include "kdn_frag.hpp"
 #include "kdn_internal.hpp"
 #include "kdn_io.hpp"
+#include "kdn_serve_rule.hpp"
 
 namespace kdn {
 
@@ -753,9 +754,6 @@ namespace kdn {
 // window, took 5.8 ms for the config-5 step against 3.7 with host offsets), fewer when all fit.
 constexpr int64_t SLOT_WIN_MAX = 1024;
 
-// Tokens up to which a step from a slot map keeps to one stream.
-constexpr int64_t SLOT_ONE_STREAM_TOKENS = 1024;
-
 // Sizes of kdn_slot_step's workspace, all bounds from num_tokens and num_slots: `cap` runs at most (one
 // per slot, and the padding runs between them), n_pre prefills (two tokens or more each), G packed slots
 // (each prefill's chunks and its spare), `nwin` windows of SLOT_WIN slots.
@@ -862,10 +860,10 @@ extern "C" int kdn_slot_step(const kdn_slot_step_args* a, void* stream, void* au
   }
   rc = launch_status();
   if (rc != KDN_OK) return rc;
-  // with an auxiliary stream the decode runs on it after the prefill's prep launches, as in
-  // kdn_ragged_step; a step of few tokens has little to run side by side, and the two events cost more
+  // with an auxiliary stream the decode runs on it after the prefill's prep launches, as in kdn_ragged_step, where
+  // that saves more than its two events cost
   const hipStream_t aux = aux_stream ? as_stream(aux_stream) : nullptr;
-  const bool dec_aux = pl.nwin > 0 && aux && aux != st && a->num_tokens > SLOT_ONE_STREAM_TOKENS;
+  const bool dec_aux = pl.nwin > 0 && aux && aux != st && slot_decode_beside(a->num_tokens, a->num_slots, a->H, a->D, a->d_v);
   EventSet evs;
   if (dec_aux) {
     rc = evs.create(2);

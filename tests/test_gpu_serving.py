@@ -441,6 +441,22 @@ def test_slot_plan_more_runs_than_slots(proj):
     assert int(status) == 1 and torch.equal(sd.cpu(), states) and bool((y == 7.0).all())
 
 
+def test_small_mixed_step_on_two_streams(proj):
+    """A step of few tokens whose decodes are many enough to run beside the prefill: equal to the same step on one
+    stream, bit for bit, over several steps on the same states."""
+    lens = [1] * 20 + [130] + [1] * 13
+    q, k, v, beta, lam, _, slots, states = make_step(lens, 16, 64, torch.bfloat16, len(lens), seed=5)
+    sm = torch.repeat_interleave(slots.to(torch.int64), torch.tensor(lens)).to(DEV)
+    args = [t.to(DEV) for t in (q, k, v, beta, lam)]
+    tab = (proj.device_omega(DEV), proj.device_phase(DEV), proj.tau_star_inv)
+    sa, sb = states.to(DEV), states.to(DEV)
+    for _ in range(3):
+        ya = ops.slot_step(*args, sm, sa, *tab, pipelined=True)
+        yb = ops.slot_step(*args, sm, sb, *tab, pipelined=False)
+        torch.cuda.synchronize()
+        assert torch.equal(ya, yb) and torch.equal(sa, sb)
+
+
 @pytest.mark.parametrize("dv", [16, 32, 64, 128])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rule", [ops.RULE_DELTA, ops.RULE_LINEAR])
