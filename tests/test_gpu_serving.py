@@ -6,6 +6,8 @@ the sequence's slot state; slots that no sequence uses must come back bit-identi
 (relative L2) as for the scan: 1e-4 for fp32 inputs, 2e-2 for bf16 inputs.  The further check the
 serving path calls for: prefill followed by decode steps equals one prefill of the whole sequence.
 """
+import random
+
 import numpy as np
 import pytest
 import torch
@@ -427,6 +429,52 @@ def test_slot_plan_equals_host_offsets(proj, name, slot_dtype):
     assert rel_l2(ya.cpu().numpy(), yb.cpu().numpy()) < 1e-5 and rel_l2(sa.cpu().numpy(), sb.cpu().numpy()) < 1e-5
     rest = [s for s in range(n_slots) if s not in set(int(x) for x in sl)]
     assert torch.equal(sa[rest].cpu(), states[rest])
+
+
+MANY_RUNS = {
+    "pairs": [2] * 4096,                                 # as many prefills as the plan's tables hold; a window past the last
+    "mixed": [random.Random(7).choice([1, 1, 2, 3, 4, 5, 6, -1, -2]) for _ in range(1600)],
+    "cut": [2] * 511 + [300] + [2] * 200 + [1] * 50,     # the window's end falls inside the prefill of 300 tokens
+}
+
+
+@pytest.mark.parametrize("slot_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("name", list(MANY_RUNS))
+def test_slot_plan_many_runs(proj, name, slot_dtype):
+    """As test_slot_plan_equals_host_offsets, with more prefills than the plan has threads and several packed windows
+    (checked over whole tensors)."""
+    runs = torch.tensor(MANY_RUNS[name])
+    lens, n_slots = runs.abs(), len(runs) + 3
+    assert int(lens.sum()) <= 8192
+    q, k, v, beta, lam, cu, slots, states = make_step(lens.tolist(), 1, 16, torch.float32, n_slots, seed=3)
+    i = torch.arange(len(runs), dtype=torch.int32)
+    sl = torch.where(runs < 0, torch.where(i % 2 == 1, -1 - i, n_slots + i), slots)
+    host = torch.where(sl >= n_slots, torch.full_like(sl, -1), sl)
+    sm = torch.repeat_interleave(sl.to(slot_dtype), lens).to(DEV)
+    args = [t.to(DEV) for t in (q, k, v, beta, lam)]
+    ya, yb = (torch.full((q.shape[0], 1, 16), 7.0, device=DEV) for _ in range(2))
+    sa, sb = states.to(DEV), states.to(DEV)
+    status = torch.full((1,), 9, dtype=torch.int32, device=DEV)
+    tab = (proj.device_omega(DEV), proj.device_phase(DEV), proj.tau_star_inv)
+    ops.slot_step(*args, sm, sa, *tab, y=ya, status=status)
+    ops.ragged_step(*args, cu, host, sb, *tab, y=yb)
+    torch.cuda.synchronize()
+    assert int(status) == 0
+    ya, yb, sa, sb = (t.cpu() for t in (ya, yb, sa, sb))
+    row = lambda which: torch.repeat_interleave(which, lens)
+    slot_of = lambda which: sl[which].long()
+    assert torch.equal(ya[row(runs == 1)], yb[row(runs == 1)]) and torch.equal(sa[slot_of(runs == 1)], sb[slot_of(runs == 1)])
+    assert bool((ya[row(runs < 0)] == 7.0).all())
+    used = torch.zeros(n_slots, dtype=torch.bool)
+    used[slot_of(runs > 0)] = True
+    assert torch.equal(sa[~used], states[~used])
+    # each prefill by itself: one among thousands would not show in a norm over all
+    pre = runs >= 2
+    err = torch.zeros(len(runs)).index_add_(0, row(torch.arange(len(runs))), (ya - yb).square().sum((1, 2)))
+    ref = torch.zeros(len(runs)).index_add_(0, row(torch.arange(len(runs))), yb.square().sum((1, 2)))
+    assert bool((err[pre] < 1e-10 * ref[pre]).all())
+    dS, rS = ((t[slot_of(pre)]).square().sum((1, 2, 3)) for t in (sa - sb, sb))
+    assert bool((dS < 1e-10 * rS).all()) and bool(((sa - states)[slot_of(pre)].abs().amax((1, 2, 3)) > 0).all())
 
 
 def test_slot_plan_more_runs_than_slots(proj):
