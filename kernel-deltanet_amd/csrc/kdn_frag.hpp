@@ -95,9 +95,6 @@ __device__ __forceinline__ typename P::frag load_frag_nt(const void* base, int l
   return __builtin_nontemporal_load(reinterpret_cast<const typename P::frag*>(base) + lane);
 }
 
-// Read-only streaming loads that bypass nothing: plain global loads (the workspace is re-read once).
-__device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-
 // Orders one wave's LDS accesses at this point for exchanges between its lanes (a lane reading what
 // another lane of the same wave stored): the hardware performs a wave's LDS operations in order, so no
 // instruction is emitted at wavefront scope, but the compiler may no longer move loads or stores across

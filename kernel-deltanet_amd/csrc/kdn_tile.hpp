@@ -38,22 +38,6 @@ __device__ __forceinline__ f32x8 frag_cols(const float* base, int ld, int c0, in
   for (int s = 0; s < 8; ++s) r[s] = base[(size_t)(k0 + kappa(lane, s)) * ld + c0 + (lane & 15)];
   return r;
 }
-__device__ __forceinline__ f32x8 frag_rows_bf16(const __bf16* base, int ld, int r0, int k0, int lane) {
-  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-  const __bf16* p = base + (size_t)(r0 + (lane & 15)) * ld + k0 + 4 * (lane >> 4);
-  const bf16x4 lo = *reinterpret_cast<const bf16x4*>(p);
-  const bf16x4 hi = *reinterpret_cast<const bf16x4*>(p + 16);
-  f32x8 r;
-#pragma unroll
-  for (int s = 0; s < 4; ++s) { r[s] = (float)lo[s]; r[4 + s] = (float)hi[s]; }
-  return r;
-}
-__device__ __forceinline__ f32x8 frag_cols_bf16(const __bf16* base, int ld, int c0, int k0, int lane) {
-  f32x8 r;
-#pragma unroll
-  for (int s = 0; s < 8; ++s) r[s] = (float)base[(size_t)(k0 + kappa(lane, s)) * ld + c0 + (lane & 15)];
-  return r;
-}
 
 // Fragments in plain depth order (slot s of lane l at depth k0 + 8(l>>4) + s, one 16- or 32-byte run
 // per lane): a product is exact in any depth order as long as both operands use the same one.
