@@ -541,8 +541,10 @@ static void launch_lift_butterfly(const void* x, int64_t rows, int64_t xs, int n
 
 // Up to one 16-row tile per CU the lift takes lift_rows16_kernel, which fills the GPU with one round of
 // workgroups; past that lift_kernel, whose waves keep Omega over several tiles.  D = 512, us per call in a
-// graph, rows16 / persistent: 1021 rows 6.4 / 10.9 (fp32), 5.4 / 9.4 (bf16); 4084 rows 7.7 / 11.4, 6.0 / 9.7;
-// 8192 rows 12.0 / 12.0, 10.4 / 10.1; 16384 rows 19.2 / 13.8, 19.1 / 10.5.
+// graph, rows16 / persistent: 16 rows 5.6 / 9.5 (fp32), 4.7 / 7.3 (bf16); 1021 rows 6.4 / 10.9, 5.4 / 9.4; 4084 rows
+// 7.7 / 11.4, 6.0 / 9.7; 8192 rows 12.0 / 12.0, 10.4 / 10.1; 16384 rows 19.2 / 13.8, 19.1 / 10.5.  Narrower, at 16 and 4084
+// rows: D = 256 3.9 / 5.9 and 4.8 / 7.0 (fp32), 3.7 / 5.2 and 4.3 / 5.9 (bf16); D = 128 3.7 / 4.5 and 4.3 / 5.3, 3.5 / 4.2 and
+// 3.8 / 4.6; from the bf16 table likewise, 0.1 to 1.2 us less on both sides.
 
 template <typename InT, typename OutT, int D>
 static void launch_lift(const void* x, int64_t rows, int64_t xs, int normalize, const void* omega, const int64_t* bits,
