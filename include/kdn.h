@@ -102,8 +102,8 @@ int kdn_fwht_lift(const void* x, int64_t rows, int64_t x_row_stride, int x_dtype
 /* The same lift at the reference's native boundary (ABI 1.5): pybind fwht_forward(input, rademacher_bits,
  * D_lifted, tau_star_inv) of kernels/fwht_cuda.cpp:11-32 takes the packed sign table, not Omega.  Here
  * rademacher_bits is that table, device int64 [D_lifted / 64][3] (column s = stage d1, d2, d3; bit i set
- * <=> entry i is -1; the module buffer of kernels/fwht.py:74-83); every workgroup builds Omega from it in
- * LDS with wave64 butterflies (the sign flips fused into the transform), then lifts as kdn_fwht_lift.
+ * <=> entry i is -1; the module buffer of kernels/fwht.py:74-83); every workgroup builds Omega from it (a
+ * 64-feature block by one wave64 butterfly and exact MFMA products), then lifts as kdn_fwht_lift.
  * The torch-branch semantics this lift implements (kernels/fwht.py:122-131) also need the module's phases
  * b, passed as `phase` (device fp32 [D_lifted]); the reference's CUDA function has no phase argument.
  * normalize_input as kdn_fwht_lift (0 in the reference's call).  d_k must be 64; D_lifted in
@@ -436,8 +436,10 @@ int kdn_ragged_step(const kdn_ragged_args* a, void* stream, void* aux_stream);
  * packed layout are all formed on the device and every launch is sized from num_tokens and num_slots, so
  * distinct runs must have distinct slots (not checked); a map with more than 2 * num_slots + 1 runs is
  * invalid, and then nothing runs and *status (device int32, if not NULL) is set to 1 (else 0).  The
- * prefill runs the split scan over windows of 128 packed chunk slots (each sequence's chunks plus one spare
- * slot), pipelined over aux_stream when it is not NULL. */
+ * prefill runs the chunked scan over windows of at most 1024 packed chunk slots (each sequence's chunks plus
+ * one spare slot), pipelined over aux_stream when it is not NULL; there the decodes run on aux_stream too,
+ * after the prefill's prep launches, unless the step is short and their states few (then before the prefill,
+ * on `stream`).  `stream` finally waits for aux_stream. */
 typedef struct kdn_slot_step_args {
   int64_t num_tokens, H;
   int d_k, D, d_v;             /* d_k = 64, D = 512, d_v in {16, 32, 64, 128} */

@@ -55,7 +55,7 @@ struct Rec {
   static constexpr size_t floats = VEC + 128;
 };
 
-// The backward's record (kdn_delta_scan_bwd at D = 1024): the forward's record (its S field unused) followed
+// The backward's record (kdn_delta_scan_bwd at D = 1024): the forward's record (its S field holding fp32 tiles) followed
 // by the fields of the gradient (offsets in floats).  D x DV matrices in accumulator tiles [n NV][tile D/16][lane]
 // f32x4: lane (g, v = l & 15) holds features feature_of(tile, 4g + i) of value 16n + v.
 template <int D, int DV>
@@ -79,7 +79,7 @@ struct BRec {
                                                                 // [D/32] <Gamma, S> likewise
   static constexpr size_t V_BETA = PART + (D / 32 * 65 + 63) / 64 * 64;  // 64-vectors: beta, dl without the terms of S
   static constexpr size_t V_DL = V_BETA + 64;
-  // The size of a record is what callers have sized workspaces by: kept, though the fields no longer fill it.
+  // The record's size as it was with more fields (workspace queries and the segment rule go by it): a quarter is unused.
   static constexpr size_t floats = T + 3 * D * DV + 7 * C * DV + 4 * C * C;
   static_assert(V_DL + 64 <= floats, "the fields fit the record");
 };

@@ -57,8 +57,9 @@ size_t scan_flat_buffer_bytes(const kdn_scan_args* a, int64_t win);
 // Segment checkpoints of the D = 512, d_v = 64 scan (the backward's first pass): the states at the starts
 // of segments 1 .. n of `seg` chunks each, written as fp32 [B][H][512][64] arrays one after another from
 // `ckpt` (segment s's at ckpt + (s - 1) * B*H*512*64), by the scan's prep and state kernels alone (no
-// output kernel); segment 0 starts from a->initial_state (zeros if NULL).  Each equals, bit for bit, the
-// state that kdn_delta_scan_fwd with segment_chunks = seg carries across that boundary.  `ws` holds `nbuf`
+// output kernel); segment 0 starts from a->initial_state (zeros if NULL).  Each is the state that
+// kdn_delta_scan_fwd with segment_chunks = seg carries across that boundary, up to the order in which prep
+// sums the key norms and Grams (the key-only form over all features, the forward's in two halves).  `ws` holds `nbuf`
 // buffers of `buf_bytes` >= scan_checkpoint_buffer_bytes(a, seg); with aux (not st) and two buffers, prep
 // of segment s + 1 runs on aux beside the state kernel of segment s.  The last launch is on st.
 size_t scan_checkpoint_buffer_bytes(const kdn_scan_args* a, int64_t seg);

@@ -137,7 +137,7 @@ def lift_bits(x: torch.Tensor, rademacher_bits: torch.Tensor, phase: torch.Tenso
               normalize: bool = False, out_dtype: Optional[torch.dtype] = None,
               butterfly: bool = False) -> torch.Tensor:
     """(..., 64) -> (..., D) feature lift from the packed [D/64, 3] sign table (kdn_fwht_lift_bits): each
-    workgroup builds Omega in LDS with wave64 butterflies, then lifts as `lift`.  D = 64 * rows of the
+    workgroup builds Omega from it on the matrix cores, exactly, then lifts as `lift`.  D = 64 * rows of the
     table; phase is the (D,) phase vector b.  butterfly=True projects every row by in-register wave64
     butterflies instead (kdn_fwht_lift_bits_butterfly, the reference's P3 design; slower)."""
     require_device(x, "lift_bits")

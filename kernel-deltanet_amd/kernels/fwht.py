@@ -6,9 +6,9 @@ rademacher_bits (non-persistent), b and Omega, and forward(x) = phi / (||phi|| +
 phi = sqrt(2/D) cos(x Omega^T / tau* + b), tau* = d_k^(1/4).
 
 The forward runs the gfx950 lift kernel at the reference's native boundary (kdn_fwht_lift_bits, the
-replacement of kernel_deltanet_cuda.fwht_forward): every workgroup builds Omega in LDS from the packed
-sign table with wave64 butterflies, then projects on MFMA.  The scan's kernels read a resident bf16 copy
-of Omega instead, built once per device by the same butterflies (kdn_build_omega).  Device tensors only.
+replacement of kernel_deltanet_cuda.fwht_forward): every workgroup builds Omega from the packed sign table
+on the matrix cores, exactly, then projects on MFMA.  The scan's kernels read a resident bf16 copy of Omega
+instead, built once per device by wave64 butterflies (kdn_build_omega).  Device tensors only.
 """
 from __future__ import annotations
 
