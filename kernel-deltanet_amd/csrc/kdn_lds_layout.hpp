@@ -24,16 +24,23 @@ constexpr int kf32_read(int lane, int e, int half) { return kf32_word(lane >> 4,
 
 // A and T of the 64 x 64 unit-lower inverse in 16 x 16 blocks (unit_lower_inverse_blocked).
 //
-// A by columns, the rows of a column in sixteen groups of four, the groups XORed with the column's low four bits.
+// A by columns, the rows of a column in sixteen groups of four, the groups XORed with a permutation of the column's low four
+// bits c3 c2 c1 c0 (c0 to bit 3, c2 to bit 2, c3 to bit 1, c1 to bit 0).
 //   4-byte accesses of A[16i + m][16k + 4g + kb] (lane (g, m); the column walk's reads, and the stores of a tile held
-//     with its rows over the lanes): m & 3 on bank bits 0-1, (m >> 2) ^ kb on bits 2-3, (i ^ g) & 1 on bit 4, which
-//     differs over a half-wave's two g;
+//     with its rows over the lanes): m & 3 on bank bits 0-1, m >> 2 (XORed) on bits 2-3 and (i ^ g) & 1 on bit 4, which
+//     differs over a half-wave's two g; of i and kb only i & 1 and kb >> 1 meet a lane's bits, so that four lane
+//     addresses serve all of a walk's reads;
 //   16-byte accesses of rows 4s .. 4s + 3 of sixteen consecutive columns (the stores of a tile held with its columns over
 //     the lanes): sixteen groups;
 //   16-byte reads of rows 16b + 4p .. + 3 of one column by the lanes p (the substitution): four groups, each broadcast.
 // (In four rows of residue p = row & 3 a column, the stores by columns were four 4-byte ones that met four ways on a bank:
-// prep8_kernel's conflicts 6.7 % of its busy LDS cycles, 2.7 % with this.)
-constexpr int a_word(int row, int col) { return col * 64 + 4 * ((row >> 2) ^ (col & 15)) + (row & 3); }
+// prep8_kernel's conflicts 6.7 % of its busy LDS cycles.  4.1 % with this; 2.7 % with the column's bits unpermuted, where
+// a walk takes twelve lane addresses and the kernel 0.5 us more in a call of 520 chunks, 34.75 for 34.2: the rest is pairs
+// of the walk's reads that the compiler merges, whose two words lie on one bank and are counted, at no cost in time.)
+constexpr int a_word(int row, int col) {
+  const int f = (col >> 1 & 1) | (col >> 3 & 1) << 1 | (col >> 2 & 1) << 2 | (col & 1) << 3;
+  return col * 64 + 4 * ((row >> 2) ^ f) + (row & 3);
+}
 
 // T by rows, the 16-byte groups of a row's columns XORed with h(r) = 4 (a ^ p) + a, a = (r >> 2) & 3, p = r & 3, so that
 // each of these falls on distinct banks: 4-byte accesses of rows 4a + 0..3 (a fixed; accumulator tiles) or of rows

@@ -169,21 +169,17 @@ __device__ __forceinline__ void inverse_diag_block(const float* At, float* T, in
 #pragma unroll
     for (int i = 0; i < 15; ++i) acol[i] = *reinterpret_cast<const f32x4*>(At + a_word(16 * b + 4 * pq, 16 * b + i));
 #pragma unroll
-    for (int ib = 0; ib < 4; ++ib) {
-      if (pq >= ib) {  // the rows of the lanes before are final
-#pragma unroll
-        for (int i = 4 * ib; i < 4 * ib + 4 && i < 15; ++i) {
-          float bc;  // -T[i][c], held by lane pq = i >> 2, slot i & 3 of the quad
-          switch (ib) {
-            case 0: bc = quad_bcast<0>(acc[i & 3]); break;
-            case 1: bc = quad_bcast<1>(acc[i & 3]); break;
-            case 2: bc = quad_bcast<2>(acc[i & 3]); break;
-            default: bc = quad_bcast<3>(acc[i & 3]); break;
-          }
-#pragma unroll
-          for (int s = 0; s < 4; ++s) acc[s] = fmaf(-acol[i][s], bc, acc[s]);
-        }
+    for (int i = 0; i < 15; ++i) {
+      float bc;  // -T[i][c], held by lane pq = i >> 2, slot i & 3 of the quad
+      switch (i >> 2) {
+        case 0: bc = quad_bcast<0>(acc[i & 3]); break;
+        case 1: bc = quad_bcast<1>(acc[i & 3]); break;
+        case 2: bc = quad_bcast<2>(acc[i & 3]); break;
+        default: bc = quad_bcast<3>(acc[i & 3]); break;
       }
+      bc = pq >= (i >> 2) ? bc : 0.f;  // the rows of the lanes before are final, also where a later one is not finite
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc[s] = fmaf(-acol[i][s], bc, acc[s]);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
