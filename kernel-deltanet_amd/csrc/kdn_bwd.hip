@@ -232,8 +232,8 @@ __device__ __forceinline__ float load_x_part(const InT* x, int64_t base, bool va
   }
 #pragma unroll
   for (int e = 0; e < 16; ++e) ss += part[e] * part[e];
-  ss += __shfl_xor(ss, 1);
-  ss += __shfl_xor(ss, 2);
+  ss += xor_shuffle<1>(ss);
+  ss += xor_shuffle<2>(ss);
   const float nrm = sqrtf(ss);
   if (normalize) {
     const float inv = 1.f / fmaxf(nrm, 1e-6f);
@@ -986,8 +986,8 @@ __device__ __forceinline__ void write_dx(const Params& p, const InT* x, int64_t 
     float dot = 0.f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) dot += part[e] * g[e];
-    dot += __shfl_xor(dot, 1);
-    dot += __shfl_xor(dot, 2);
+    dot += xor_shuffle<1>(dot);
+    dot += xor_shuffle<2>(dot);
     if (nrm > 1e-6f) {
       const float inv = 1.f / nrm;
 #pragma unroll
@@ -1501,7 +1501,8 @@ __device__ __forceinline__ void dx_features(const Params& p, DxShared<P>& sh, co
 #pragma unroll
           for (int a = 0; a < 4; ++a) d[a][u] = P::mma(d[a][u], ob[a], bs[wi][jj][u]);
       }
-    float* red = reinterpret_cast<float*>(sh.big) + ((w >> 2) * 2 + W0 + wi) * C * LD;
+    const int le = fresh(lane);
+    float* red = reinterpret_cast<float*>(sh.big) + ((w >> 2) * 2 + W0 + wi) * C * LD + (le & 15) * LD + 4 * (le >> 4);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int a = (w + t) & 3;
@@ -1510,7 +1511,7 @@ __device__ __forceinline__ void dx_features(const Params& p, DxShared<P>& sh, co
         if (aa == a) {  // uniform over the wave
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            f32x4* px = reinterpret_cast<f32x4*>(&red[(16 * u + (lane & 15)) * LD + 16 * aa + 4 * (lane >> 4)]);
+            f32x4* px = reinterpret_cast<f32x4*>(red + 16 * u * LD + 16 * aa);
             *px = t == 0 ? d[aa][u] : *px + d[aa][u];
           }
         }
@@ -1530,7 +1531,7 @@ __global__ void __launch_bounds__(64 * DX_WAVES) bwd_dx_kernel(Params p) {
   const int64_t t0 = (p.c0 + blockIdx.x) * C;
   const float* rec = record(p, b, h, blockIdx.x);
   // loaders: input `which` (0 q, 1 k), row r, features c0 .. c0 + 15
-  const int which = tid >> 8, r = (tid >> 2) & 63, c0 = (tid & 3) * 16;
+  const int which = w >> 2, r = (tid >> 2) & 63, c0 = (tid & 3) * 16;
   const bool rvalid = t0 + r < p.T;
   const InT* x = reinterpret_cast<const InT*>(which == 0 ? p.q : p.k);
   const int64_t xb = which == 0 ? b * p.qs0 + (t0 + r) * p.qs1 + h * p.qs2 + c0 : b * p.ks0 + (t0 + r) * p.ks1 + h * p.ks2 + c0;
@@ -1564,17 +1565,29 @@ __global__ void __launch_bounds__(64 * DX_WAVES) bwd_dx_kernel(Params p) {
     dx_features<P, LO, GEN, 0, 2>(p, sh, rec, h, w, lane, itau, dit);
   } else {
     dx_features<P, LO, GEN, 1, 1>(p, sh, rec, h, w, lane, itau, dit);
-    dx_features<P, LO, GEN, 0, 1>(p, sh, rec, h, w, lane, itau, dit);
+    dx_features<P, LO, GEN, 0, 1>(p, sh, rec, h, w, fresh(lane), itau, dit);
   }
   {
+    const int te = 64 * w + fresh(lane);  // the row and columns again
+    const int re = (te >> 2) & 63, ce = (te & 3) * 16;
+    const int64_t t = t0 + re;
+    const bool valid = t < p.T;
     const float* d0 = reinterpret_cast<const float*>(sh.big) + which * C * LD;
     const float* d1 = d0 + 2 * C * LD;
-    if (which == 0) write_dx<InT>(p, x, xb, p.dq, b * p.dqs0 + (t0 + r) * p.dqs1 + h * p.dqs2 + c0, d0, d1, r, c0, rvalid, itau);
-    else write_dx<InT>(p, x, xb, p.dk, b * p.dks0 + (t0 + r) * p.dks1 + h * p.dks2 + c0, d0, d1, r, c0, rvalid, itau);
+    if (which == 0)
+      write_dx<InT>(p, reinterpret_cast<const InT*>(p.q), b * p.qs0 + t * p.qs1 + h * p.qs2 + ce, p.dq,
+                    b * p.dqs0 + t * p.dqs1 + h * p.dqs2 + ce, d0, d1, re, ce, valid, itau);
+    else
+      write_dx<InT>(p, reinterpret_cast<const InT*>(p.k), b * p.ks0 + t * p.ks1 + h * p.ks2 + ce, p.dk,
+                    b * p.dks0 + t * p.dks1 + h * p.dks2 + ce, d0, d1, re, ce, valid, itau);
   }
   if (GEN && p.dit) {  // fixed order: lanes by a shuffle tree, then the waves in order
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) dit += __shfl_xor(dit, o);
+    dit += xor_shuffle<32>(dit);
+    dit += xor_shuffle<16>(dit);
+    dit += xor_shuffle<8>(dit);
+    dit += xor_shuffle<4>(dit);
+    dit += xor_shuffle<2>(dit);
+    dit += xor_shuffle<1>(dit);
     if (lane == 0) sh.dit[w] = dit;
     __syncthreads();
     if (tid == 0) {

@@ -710,11 +710,14 @@ __global__ void __launch_bounds__(64 * CARRY_WAVES) gen_carry_kernel(Params p, c
   const int vc = 16 * n + (lane & 15);
 
   f32x4 Sg[TPW];
+  // the slice's offsets are formed again at the end where, held through the loop, they would be spilled
+  constexpr bool AGAIN = !O::KEEP || (REV && DV == 64);
+  const int lb = AGAIN ? fresh(lane) : lane;
 #pragma unroll
   for (int t = 0; t < TPW; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      Sg[t][i] = src ? src[b * s0 + h * s1 + feature_of(TPW * w + t, 4 * (lane >> 4) + i) * s2 + vc * s3] : 0.f;
+      Sg[t][i] = src ? src[b * s0 + h * s1 + feature_of(TPW * w + t, 4 * (lb >> 4) + i) * s2 + (16 * n + (lb & 15)) * s3] : 0.f;
   const typename PB::frag sel[2] = {selector<PB>(0, lane), selector<PB>(1, lane)};
   const int nch = (int)p.nch;
   unsigned sink = 0;  // keeps the prefetch loads alive (never stored: nch is positive)
@@ -1189,8 +1192,8 @@ __global__ void __launch_bounds__(64 * DPHI_WAVES) gbwd_dphi_kernel(Params p, Bw
     for (int t = 0; t < 2; ++t) aq[m][t] = ak[m][t] = zero4();
   float dap[4] = {0.f, 0.f, 0.f, 0.f}, gs = 0.f;
   const bool want = g.ddecay != nullptr;
-  const f32x4* st = reinterpret_cast<const f32x4*>(rec + R::SR) + 2 * jf * 64 + lane;
-  const f32x4* gt = reinterpret_cast<const f32x4*>(rec + R::GR) + 2 * jf * 64 + lane;
+  const f32x4* st = reinterpret_cast<const f32x4*>(rec + R::SR) + 2 * jf * 64 + (BF ? lane : 0);
+  const f32x4* gt = reinterpret_cast<const f32x4*>(rec + R::GR) + 2 * jf * 64 + (BF ? lane : 0);
   // contractions over the value columns: S^T (a o dY)^T, Gamma (kappa o W)^T, -S^T Z^T
 #pragma unroll 1
   for (int kb = 0; kb < DV / 32; ++kb) {
@@ -1198,7 +1201,15 @@ __global__ void __launch_bounds__(64 * DPHI_WAVES) gbwd_dphi_kernel(Params p, Bw
 #pragma unroll
     for (int nn = 0; nn < 2; ++nn) {
       const size_t at = (size_t)(2 * kb + nn) * (D / 16) * 64;
-      const f32x8 sv = pair_to8(st[at], st[at + 64]), gv = pair_to8(gt[at], gt[at + 64]);
+      f32x8 sv, gv;
+      if constexpr (BF) {
+        sv = pair_to8(st[at], st[at + 64]);
+        gv = pair_to8(gt[at], gt[at + 64]);
+      } else {  // scalar bases: fp32 fragments leave no vector registers for the addresses
+        const f32x4 *sp = uni(st + at), *gp = uni(gt + at);
+        sv = pair_to8(sp[lane], sp[64 + lane]);
+        gv = pair_to8(gp[lane], gp[64 + lane]);
+      }
 #pragma unroll
       for (int s = 0; s < 8; ++s) gs += sv[s] * gv[s];
       sb[nn] = PB::from_f32(sv);
@@ -1244,12 +1255,13 @@ __global__ void __launch_bounds__(64 * DPHI_WAVES) gbwd_dphi_kernel(Params p, Bw
         }
       }
   }
+  const int le = BF ? lane : fresh(lane);
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
-    const int ri = 16 * m + (lane & 15);
+    const int ri = 16 * m + (le & 15);
     if (ri >= nrows) continue;
     const int64_t t = t0 + ri;
-    const int f = 32 * jf + 8 * (lane >> 4);
+    const int f = 32 * jf + 8 * (le >> 4);
     float* dq = g.dq + b * g.dqs0 + t * g.dqs1 + h * g.dqs2 + f;
     float* dk = g.dk + b * g.dks0 + t * g.dks1 + h * g.dks2 + f;
 #pragma unroll
@@ -1271,10 +1283,10 @@ __global__ void __launch_bounds__(64 * DPHI_WAVES) gbwd_dphi_kernel(Params p, Bw
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       const float s = sum_col4(dap[m]);
-      if (lane < 16) part[jf * 64 + 16 * m + lane] = s;
+      if (le < 16) part[jf * 64 + 16 * m + le] = s;
     }
     gs = wave_sum(gs);
-    if (lane == 0) part[D / 32 * 64 + jf] = gs;
+    if (le == 0) part[D / 32 * 64 + jf] = gs;
   }
 }
 
